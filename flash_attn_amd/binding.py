@@ -101,6 +101,21 @@ def lib():
     return _lib
 
 
+_native = None
+
+
+def _front_end():
+    """The native front end (csrc/py_binding.cpp), bound to the loaded library.  Raises if it has not been built."""
+    global _native
+    L = lib()
+    from . import _native as n
+
+    n.bind(*(C.cast(f, C.c_void_p).value for f in (L.flash_forward, L.flash_forward_splitkv, L.flash_splitkv_resolve_splits)),
+           FlashError)
+    _native = n
+    return n
+
+
 def _ptr(t):
     return None if t is None else t.data_ptr()
 
@@ -175,6 +190,12 @@ def flash_forward(q, k, v, softmax_scale=None, causal=False, window=(-1, -1), al
     [B,H,Nq,Nk] tensor (pre-filled with -inf) that receives the visible scores (debug; slow kernel instance).
     kernel_hint: KERNEL_AUTO / KERNEL_4WAVE / KERNEL_8WAVE.  return_stage_stamps: also return the per-work-group
     time stamps [groups, FLASH_STAMP_WORDS] int64 of the instrumented kernel instance (debug), as the last element."""
+    if not return_keep_mask and scores_out is None and not return_stage_stamps and kernel_hint == KERNEL_AUTO:
+        res = (_native or _front_end()).forward(q, k, v, softmax_scale, causal, window, alibi_slopes, dropout_p, seed, offset,
+                                                stream, out, lse)
+        if res is not NotImplemented:
+            return res
+    # debug outputs, and arguments that the native front end leaves alone (those that raise among them)
     import torch
 
     B, H, Nq, Nk, d = _check_qkv(q, k, v)
@@ -202,6 +223,12 @@ def flash_forward_splitkv(q, k, v, num_splits=0, softmax_scale=None, causal=Fals
     return_partials hands back views of the workspace in the layout the library wrote, for the resolved split count
     S: [B,H,S,Nq,d] / [B,H,S,Nq], or -- one query row with four or more query heads per K/V head, no ALiBi, left
     window or dropout -- [B,H_kv,S,G,d] / [B,H_kv,S,G] with G = H / H_kv; (None, None) when S == 1."""
+    if not return_partials and scores_out is None and not return_stage_stamps and kernel_hint == KERNEL_AUTO:
+        res = (_native or _front_end()).splitkv(q, k, v, num_splits, workspace, softmax_scale, causal, window, alibi_slopes,
+                                                dropout_p, seed, offset, stream, out, lse)
+        if res is not NotImplemented:
+            return res
+    # debug outputs, and arguments that the native front end leaves alone (those that raise among them)
     import torch
 
     B, H, Nq, Nk, d = _check_qkv(q, k, v)
