@@ -27,6 +27,24 @@ typedef __fp16 v4hp __attribute__((__vector_size__(4 * sizeof(__fp16))));
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
+// Division of an index 0 <= n < 2^31 by a divisor that the host knows: n / d = floor(2n M / 2^32) / 2^l with
+// l = ceil(log2 d) and M = ceil(2^(31+l) / d) < 2^32 (exact: M d exceeds 2^(31+l) by less than 2^l, which adds less than
+// 1/d to the quotient).  On the scalar unit that is a shift, a multiply and a shift, where the compiler's division by
+// a run-time divisor is a chain of some thirty instructions through the vector unit's reciprocal.  With the five or six
+// divisions in front of a work-group's first request replaced (315 -> 169 instructions at d = 64), a launch is over 0.3 us
+// earlier (B1 H2 N128 d64 5.1 -> 4.8 us, decode B15 H2 Nk3200 d64 8.9 -> 8.5 us, B2 H8 N2560 d40 causal 34.1 -> 33.6).
+struct FastDiv {
+    uint32_t mul, shift;
+    __device__ __forceinline__ int quotient(int n) const { return (int)(__umulhi(2u * (uint32_t)n, mul) >> shift); }
+};
+inline FastDiv fast_div(long long divisor)
+{
+    const uint64_t d = divisor > 1 ? (uint64_t)divisor : 1u;
+    uint32_t l = 0;
+    while ((1ull << l) < d) ++l;
+    return {(uint32_t)(((1ull << (31 + l)) + d - 1) / d), l};
+}
+
 // Arguments of the tiled forward kernel and of the decode/combine kernels, filled by the host from flash_params
 // (which is itself the superset of the reference's mykernelParamType, include/utils.h:21-44).
 struct FwdArgs {
@@ -58,10 +76,25 @@ struct FwdArgs {
     int snake_end;       // work-groups below this index sit on the GPU together; odd 256-blocks of them run reversed (launcher)
     int group_xcd;       // > 1: query heads per K/V head, and the slice order keeps the heads of a K/V head on one XCD (launcher)
     int split_rotate;    // 1: the split index of a work-group is rotated by its row block (launcher; split_of_rest)
+    // divisions of the work-group index and of the head slice (launcher: set_divisors)
+    FastDiv by_chunk, by_slices, by_splits, by_xcd_group, by_kv_group, by_heads;
 
-    // index of the K/V slice [Nk,d] read by query slice bh = b * H + h
-    __device__ __forceinline__ int kv_slice(int bh) const { return (bh / H) * Hk + (bh % H) / kv_group; }
+    // index of the K/V slice [Nk,d] read by query slice bh = b * H + h: H is a multiple of the heads per K/V head
+    __device__ __forceinline__ int kv_slice(int bh) const { return by_kv_group.quotient(bh); }
+    __device__ __forceinline__ int head(int bh) const { return bh - by_heads.quotient(bh) * H; }
 };
+
+// Divisors of a launch, once its slice order is set (the decode kernel, whose order has no chunks, deals out
+// `slices` groups of query heads per split)
+inline void set_divisors(FwdArgs& b, long long slices)
+{
+    b.by_chunk = fast_div(slices * b.Tr * b.num_splits);
+    b.by_slices = fast_div(slices);
+    b.by_splits = fast_div(b.num_splits);
+    b.by_xcd_group = fast_div(b.group_xcd);
+    b.by_kv_group = fast_div(b.kv_group);
+    b.by_heads = fast_div(b.H);
+}
 
 __device__ __forceinline__ int wave_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
@@ -145,24 +178,47 @@ __device__ __forceinline__ int work_position(int block, int snake_end)
 // The launcher asks for it exactly where the plain order aliases: work-group x + 8 n of XCD x has split
 // (x / c + (8 / c) n) % S for c = 1, 2 or 4 slices per chunk, which reaches every split only if S is odd; other chunk
 // sizes mix by themselves, and rotating an order that already mixes measured 0 ... -14 %.
-__device__ __forceinline__ int split_of_rest(int rest, int num_splits, int rotate, int* row_block_index)
+__device__ __forceinline__ int split_of_rest(const FwdArgs& a, int rest, int* row_block_index)
 {
-    const int mi = rest / num_splits, s0 = rest % num_splits;
+    const int mi = a.by_splits.quotient(rest), s0 = rest - mi * a.num_splits;
     *row_block_index = mi;
-    return rotate ? (s0 + mi) % num_splits : s0;
+    if (!a.split_rotate) return s0;
+    const int s = s0 + mi;
+    return s - a.by_splits.quotient(s) * a.num_splits;
 }
 inline int split_rotate_for(int num_splits, int slice_chunk)
 {
     return num_splits > 1 && num_splits % 2 == 0 && (slice_chunk == 1 || slice_chunk == 2 || slice_chunk == 4) ? 1 : 0;
 }
 
-__device__ __forceinline__ int slice_of_position(int local, int group_xcd)
+__device__ __forceinline__ int slice_of_position(const FwdArgs& a, int local)
 {
-    if (group_xcd > 1) {
-        const int x = local & 7, y = local >> 3;
-        return ((y / group_xcd) * 8 + x) * group_xcd + y % group_xcd;
+    if (a.group_xcd > 1) {
+        const int x = local & 7, y = local >> 3, yg = a.by_xcd_group.quotient(y);
+        return (yg * 8 + x) * a.group_xcd + y - yg * a.group_xcd;
     }
     return local;
+}
+
+// Work-group -> head slice, split and row block.  Slices vary fastest, so that with B*H a multiple of 8 a slice always
+// lands on the same XCD (and L2); the heaviest causal row blocks (largest index) are dispatched first.  Slices are dealt
+// out in chunks of a.slice_chunk (the launcher's choice: all of them unless the problem has far more work-groups than the
+// GPU holds at once), chunk after chunk, so that the row blocks of a slice run closer together in time and find its K
+// and V in the caches.
+struct WorkItem {
+    int bh, split, m_block;
+};
+__device__ __forceinline__ WorkItem work_item(const FwdArgs& a, int block)
+{
+    const int pos = work_position(block, a.snake_end);
+    const int ch = a.by_chunk.quotient(pos), w = pos - ch * (a.slice_chunk * a.Tr * a.num_splits);
+    const int rest = a.by_slices.quotient(w);
+    WorkItem it;
+    it.bh = ch * a.slice_chunk + slice_of_position(a, w - rest * a.slice_chunk);
+    int mi;
+    it.split = split_of_rest(a, rest, &mi);
+    it.m_block = a.Tr - 1 - mi;
+    return it;
 }
 
 // snake_end for a launch of `groups` work-groups with `resident` places on the GPU

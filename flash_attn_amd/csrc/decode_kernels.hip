@@ -50,9 +50,8 @@ __global__ void __launch_bounds__(256) decode_split_kernel(const FwdArgs a)
     const int wave = wave_uniform(tid >> 6);
     const int c = lane % LPK;
     const int kg = lane / LPK;
-    const int BHG = a.B * a.H / G;
-    const int bh0 = (blockIdx.x % BHG) * G;  // first of the G query slices of this work-group
-    const int split = blockIdx.x / BHG;
+    const int split = a.by_slices.quotient(blockIdx.x);
+    const int bh0 = (blockIdx.x - split * (a.B * a.H / G)) * G;  // first of the G query slices of this work-group
     const int d = a.d, Nk = a.Nk;
     // Rows of any length from eight elements on, at any 2-byte alignment: a lane behind the row's whole chunks works
     // on the row's last 16 bytes, columns d - 8 ... d - 1 (no load leaves the row), with q zeroed where the lane before
@@ -82,7 +81,7 @@ __global__ void __launch_bounds__(256) decode_split_kernel(const FwdArgs a)
 #pragma unroll
     for (int gq = 0; gq < G; ++gq) {
         slope2[gq] = 0.0f;
-        if constexpr (kAlibi) slope2[gq] = a.alibi ? a.alibi[(bh0 + gq) % a.H] * kLog2e : 0.0f;
+        if constexpr (kAlibi) slope2[gq] = a.alibi ? a.alibi[a.head(bh0 + gq)] * kLog2e : 0.0f;
     }
 
     float m[G], l[G];
@@ -339,9 +338,12 @@ __global__ void __launch_bounds__(256) keep_mask_kernel(uint8_t* __restrict__ ma
 template <int LPK, int G>
 static hipError_t launch_decode_instance(const FwdArgs& a, hipStream_t st)
 {
-    const unsigned groups = (unsigned)((long long)a.B * a.H / G * a.num_splits);
-    if (a.alibi != nullptr) return launch_kernel(decode_split_kernel<LPK, true, G>, dim3(groups), dim3(256), 0, st, a);
-    return launch_kernel(decode_split_kernel<LPK, false, G>, dim3(groups), dim3(256), 0, st, a);
+    const long long slices = (long long)a.B * a.H / G;
+    const unsigned groups = (unsigned)(slices * a.num_splits);
+    FwdArgs b = a;
+    set_divisors(b, slices);
+    if (a.alibi != nullptr) return launch_kernel(decode_split_kernel<LPK, true, G>, dim3(groups), dim3(256), 0, st, b);
+    return launch_kernel(decode_split_kernel<LPK, false, G>, dim3(groups), dim3(256), 0, st, b);
 }
 
 template <int LPK>

@@ -171,24 +171,8 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
     const int l32 = lane & 31;
     const int g = lane >> 5;
 
-    // work-group -> (head slice, split, row block).  Slices vary fastest, so that with B*H a multiple of 8 a slice
-    // always lands on the same XCD (and L2); the heaviest causal row blocks (largest m) are dispatched first.
-    const int BH = a.B * a.H;
-    // Slices are dealt out in chunks of a.slice_chunk (the launcher's choice: all of them unless the problem has far more
-    // work-groups than the GPU holds at once): inside a chunk as above, chunk after chunk, so that the row blocks of a
-    // slice run closer together in time and find its K and V in the caches.
-    int bh, rest;
-    {
-        const int per_chunk = a.slice_chunk * a.Tr * a.num_splits;
-        const int pos = work_position(blockIdx.x, a.snake_end);
-        const int ch = pos / per_chunk, w = pos % per_chunk;
-        bh = ch * a.slice_chunk + slice_of_position(w % a.slice_chunk, a.group_xcd);
-        rest = w / a.slice_chunk;
-    }
-    int mi;
-    const int split = split_of_rest(rest, a.num_splits, a.split_rotate, &mi);
-    const int m_block = a.Tr - 1 - mi;
-    const int h = bh % a.H;
+    const WorkItem item = work_item(a, blockIdx.x);
+    const int bh = item.bh, split = item.split, m_block = item.m_block;
     const int Nq = a.Nq, Nk = a.Nk, d = kFullD ? D : a.d;
     const int shift = Nk - Nq;
     const int q0 = m_block * BRW;
@@ -445,7 +429,7 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
     auto read_slope = [&]() {
         if constexpr (kAlibi) {
             // (only the kEvery instance is launched without a slope table)
-            slope2 = (!kEvery || a.alibi) ? a.alibi[h] * kLog2e : 0.0f;
+            slope2 = (!kEvery || a.alibi) ? a.alibi[a.head(bh)] * kLog2e : 0.0f;
             nsig = scale_late ? -slope2 / c2 : 0.0f;
             if constexpr (kFoldAlibi) {
 #pragma unroll
@@ -1075,6 +1059,7 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
     set_slice_order(b, a.Tr * a.num_splits, kResident);
     b.split_rotate = split_rotate_for(b.num_splits, b.slice_chunk);
     b.snake_end = snake_end_for(groups, kResident);
+    set_divisors(b, b.slice_chunk);
     return launch_kernel(kern, dim3((unsigned)groups), dim3(256), smem, st, b);
 }
 
@@ -1115,6 +1100,7 @@ inline hipError_t launch_fwd_narrow_instance(const FwdArgs& a, hipStream_t st)
     set_slice_order(b, b.Tr, kNumCus);
     b.split_rotate = 0;
     b.snake_end = snake_end_for(groups, kNumCus);
+    set_divisors(b, b.slice_chunk);
     return launch_kernel(kern, dim3((unsigned)groups), dim3(256), smem, st, b);
 }
 

@@ -88,20 +88,8 @@ __global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const FwdArgs a)
     const int l32 = lane & 31;
     const int g = lane >> 5;
 
-    // work-group -> (head slice, split, row block) as in fwd_kernel: slices fastest inside a chunk of a.slice_chunk
-    // slices, heaviest row blocks first, chunk after chunk
-    int bh, rest;
-    {
-        const int per_chunk = a.slice_chunk * a.Tr * a.num_splits;
-        const int pos = work_position(blockIdx.x, a.snake_end);  // (one work-group per CU: the identity)
-        const int ch = pos / per_chunk, w = pos % per_chunk;
-        bh = ch * a.slice_chunk + slice_of_position(w % a.slice_chunk, a.group_xcd);
-        rest = w / a.slice_chunk;
-    }
-    int mi;
-    const int split = split_of_rest(rest, a.num_splits, a.split_rotate, &mi);
-    const int m_block = a.Tr - 1 - mi;
-    const int h = bh % a.H;
+    const WorkItem item = work_item(a, blockIdx.x);  // (one work-group per CU: the launch order as it is)
+    const int bh = item.bh, split = item.split, m_block = item.m_block;
     const int Nq = a.Nq, Nk = a.Nk;
     const int d = kFullD ? D : a.d;  // 8 <= d <= D
     // byte offset of chunk position c inside a row of global memory
@@ -531,7 +519,7 @@ __global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const FwdArgs a)
             if (ntiles > 2) load_k(2, Ks + 2 * C::KBUF);
         }
         // (a vector load: the wait for it counts every older request too, so it goes last; only launched with a table)
-        if constexpr (kAlibi) nsig = -(a.alibi[h] * kLog2e) / c2;
+        if constexpr (kAlibi) nsig = -(a.alibi[a.head(bh)] * kLog2e) / c2;
         stamps.take(1);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (a memory clobber: the reads below stay below)
         stamps.take(2);
@@ -678,6 +666,7 @@ inline hipError_t launch_fwd_pp_instance(const FwdArgs& a, hipStream_t st)
     set_slice_order(b, b.Tr * a.num_splits, kNumCus);  // one work-group per CU at a time
     b.split_rotate = split_rotate_for(b.num_splits, b.slice_chunk);
     b.snake_end = snake_end_for(groups, kNumCus);
+    set_divisors(b, b.slice_chunk);
     return launch_kernel(kern, dim3((unsigned)groups), dim3(512), C::SMEM, st, b);
 }
 
