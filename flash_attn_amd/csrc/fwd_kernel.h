@@ -39,14 +39,27 @@ struct FwdCfg {
     static constexpr int RW = 32 * NB;        // query rows per wave
     static constexpr int BR = kWaves * RW;    // query rows per work-group
     static constexpr int BC = 64;             // keys per tile
+    static constexpr int CH = D / 8;          // 16-byte chunks per row
     static constexpr int KS = D / 16;         // k-steps of the QK^T contraction
     static constexpr int MB = D / 32;         // 32-wide head-dim blocks of O^T
-    static constexpr int CH = D / 8;          // 16-byte chunks per row
-    // LDS row strides in bytes.  K rows are read 16 bytes per lane by 32 consecutive rows: stride/16 odd spreads
-    // them over all banks.  V rows are read by ds_read_b64_tr_b16, four consecutive rows of 64 bytes per half
-    // wave: a stride of 64 (mod 128) puts the four rows on disjoint bank groups.
-    static constexpr int SK = D * 2 + 16;
+    // LDS rows.  K rows are read 16 bytes per lane by 32 consecutive rows, which have to be spread over all banks.
+    // Either the rows are padded by one 16-byte chunk (kPadK: stride / 16 odd), or the chunks of row r are permuted by
+    // exclusive-or with kswz(r), which gives any 16 consecutive rows 16 different places among the 64 banks.  A
+    // request of permuted rows is one KiB of whole consecutive rows, and a tile takes one request less than with padded
+    // ones, whose requests begin and end anywhere in a row; but a fragment address takes a register per k-step where
+    // padded rows have immediate offsets.  Measured, padded -> permuted: causal with dropout B8 H32 N1000 d96 104.0 -> 95.5
+    // us, B8 H1 N1920 d32 causal 9.96 -> 9.83, B2 H4 N960 d40 causal 9.53 -> 9.36, d = 64 +-1 %; d = 128, eight k-steps, 10
+    // registers more and 1 % slower, keeps its padding.
+    // V rows are read by ds_read_b64_tr_b16, four consecutive rows of 64 bytes per half wave: a stride of 64 (mod 128)
+    // puts the four rows on disjoint bank groups.
+    static constexpr bool kPadK = D == 128;
+    static constexpr int CK = CH + (kPadK ? 1 : 0);  // chunks of a K row in LDS
+    static constexpr int SK = CK * 16;
     static constexpr int SV = D * 2;
+    static constexpr __host__ __device__ int kswz(int r)
+    {
+        return kPadK ? 0 : D == 64 ? (r >> 1) & 7 : (r >> 2) & 3;  // rows of 128 / 192 or 64 bytes
+    }
     // Where the row length is a multiple of 128 bytes, the two 64-byte halves of each 128 bytes are exchanged in rows
     // 2, 3 (mod 4), which has the same effect without padding.
     static constexpr bool VSWZ = (D * 2) % 128 == 0;
@@ -55,7 +68,7 @@ struct FwdCfg {
     static constexpr int SMEM = 2 * KBUF + 2 * VBUF;
     static constexpr int NSTG = 2;
     static constexpr int SMEM_DMA = NSTG * (KBUF + VBUF);
-    static constexpr int NKX = (CH + 1 + 3) / 4;  // 1 KiB blocks of a K tile (CH + 1 of them) per wave, rounded up
+    static constexpr int NKX = (CK + 3) / 4;      // 1 KiB blocks of a K tile (CK of them) per wave, rounded up
     static constexpr int NVX = CH / 4;            // 1 KiB blocks of a V tile (CH of them) per wave
     static constexpr int NLD = BC * CH / 256;  // 16-byte chunks per thread per tile (K and V each)
     static_assert(D % 32 == 0 && D <= 128, "head-dim bucket");
@@ -313,7 +326,7 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
     auto put_k = [&](int buf) {
 #pragma unroll
         for (int x = 0; x < NLD; ++x)
-            *reinterpret_cast<v4u*>(Ks + buf * C::KBUF + ld_row[x] * SK + ld_col[x] * 2) = kreg[x];
+            *reinterpret_cast<v4u*>(Ks + buf * C::KBUF + ld_row[x] * SK + ((ld_col[x] * 2) ^ (C::kswz(ld_row[x]) << 4))) = kreg[x];
     };
     auto put_v = [&](int buf) {
 #pragma unroll
@@ -322,7 +335,7 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
                                     ((ld_col[x] * 2) ^ (C::VSWZ ? ((ld_row[x] >> 1) & 1) << 6 : 0))) = vreg[x];
     };
 
-    // ---- direct global -> LDS path: the tile buffers keep their layout (K rows padded by one chunk, V rows with the
+    // ---- direct global -> LDS path: the tile buffers keep their layout (K rows padded or permuted, V rows with the
     // 64-byte halves exchanged in rows 2, 3 mod 4), and a request fills 64 consecutive 16-byte chunks of a buffer: lane l of
     // block x fetches whatever belongs into chunk 64 x + l (the pad chunk of a K row gets a copy of its neighbour).
     // Blocks go round the four waves; the odd K block goes to the waves that still have a block index left for it.
@@ -331,7 +344,7 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
     const int row_bytes = kFullD ? D * 2 : d * 2;
     auto chunk_offset = [&](int c) { return kFullD ? c * 16 : (c * 8 + 8 <= d ? c * 16 : (d - 8) * 2); };
     // (narrow: every block of a tile is the wave's own, and so is the buffer)
-    constexpr int NKX = kNarrow ? CH + 1 : C::NKX, NVX = kNarrow ? CH : C::NVX;
+    constexpr int NKX = kNarrow ? C::CK : C::NKX, NVX = kNarrow ? CH : C::NVX;
     auto block_of = [&](int i) { return kNarrow ? i : wave + 4 * i; };
     uint32_t koff[NKX], voff[NVX];
     int krow[NKX], vrow[NVX];
@@ -339,9 +352,9 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
 #pragma unroll
         for (int i = 0; i < NKX; ++i) {
             const int q = 64 * block_of(i) + lane;
-            krow[i] = q / (CH + 1);
-            const int col = q % (CH + 1);
-            koff[i] = (uint32_t)(krow[i] * row_bytes + chunk_offset(col < CH ? col : CH - 1));
+            krow[i] = q / C::CK;
+            const int c = q % C::CK;
+            koff[i] = (uint32_t)(krow[i] * row_bytes + chunk_offset((c < CH ? c : CH - 1) ^ C::kswz(krow[i])));
         }
 #pragma unroll
         for (int i = 0; i < NVX; ++i) {
@@ -351,7 +364,7 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
             voff[i] = (uint32_t)(vrow[i] * row_bytes + chunk_offset(C::VSWZ ? c ^ (((vrow[i] >> 1) & 1) << 2) : c));
         }
     }
-    const bool k_extra = kNarrow || wave + 4 * (NKX - 1) <= CH;  // the last round of K blocks exists for this wave
+    const bool k_extra = kNarrow || C::CK % 4 == 0 || wave + 4 * (NKX - 1) < C::CK;  // the last round of K blocks exists for this wave
     auto dma_tile_parts = [&](int tile, int stage, auto k_part, auto v_part) {
         // The tile's offset joins the scalar base address, so that a request of a whole tile needs no vector
         // arithmetic at all; only the last tile of a ragged sequence adjusts rows: keys past Nk re-read key Nk - 1
@@ -439,7 +452,9 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
     };
 
     // LDS read offsets of this lane
-    const int k_rd = l32 * SK + g * 16;                                          // + kb*32*SK + ks*32
+    const int k_rd = l32 * SK + (C::kPadK ? g * 16 : 0);                         // + kb*32*SK + k_step(ks)
+    const int k_ch = C::kPadK ? 0 : (g ^ C::kswz(l32)) << 4;
+    auto k_step = [&](int ks) { return (ks * 32) ^ k_ch; };
     const int v_rd = (4 * g + ((lane & 15) >> 2)) * SV + (((lane >> 4) & 1) * 16 + (lane & 3) * 4) * 2;  // + row/col blocks
     const int v_sw = C::VSWZ ? ((lane >> 3) & 1) << 6 : 0;
 
@@ -455,7 +470,7 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
             constexpr int n = 2 * KS, kAhead = 3;  // step i: k-step i / 2, key block i % 2
             v8h af[n];
 #pragma unroll
-            for (int i = 0; i < kAhead; ++i) af[i] = *reinterpret_cast<const v8h*>(kbase + (i & 1) * 32 * SK + (i >> 1) * 32);
+            for (int i = 0; i < kAhead; ++i) af[i] = *reinterpret_cast<const v8h*>(kbase + (i & 1) * 32 * SK + k_step(i >> 1));
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < n; ++i) {
@@ -463,7 +478,7 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
                 if (ks == 0) asm("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(s[kb][0]) : "v"(af[i]), "v"(qf[0][ks]), "v"(calib));
                 else s[kb][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], qf[0][ks], s[kb][0], 0, 0, 0);
                 if (i + kAhead < n)
-                    af[i + kAhead] = *reinterpret_cast<const v8h*>(kbase + ((i + kAhead) & 1) * 32 * SK + ((i + kAhead) >> 1) * 32);
+                    af[i + kAhead] = *reinterpret_cast<const v8h*>(kbase + ((i + kAhead) & 1) * 32 * SK + k_step((i + kAhead) >> 1));
                 __builtin_amdgcn_sched_barrier(0);
             }
             return;
@@ -472,7 +487,7 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
         for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
-                const v8h af = *reinterpret_cast<const v8h*>(kbase + kb * 32 * SK + ks * 32);
+                const v8h af = *reinterpret_cast<const v8h*>(kbase + kb * 32 * SK + k_step(ks));
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) {
                     if (ks == 0) {
