@@ -78,6 +78,9 @@ struct FwdArgs {
     int split_rotate;    // 1: the split index of a work-group is rotated by its row block (launcher; split_of_rest)
     // divisions of the work-group index and of the head slice (launcher: set_divisors)
     FastDiv by_chunk, by_slices, by_splits, by_xcd_group, by_kv_group, by_heads;
+    int fold_rows;       // > 0: the query heads of a K/V head are the rows of one problem, this many rows each (see RowSpan)
+    int fold_group;      // query heads folded into one
+    FastDiv by_fold;
 
     // index of the K/V slice [Nk,d] read by query slice bh = b * H + h: H is a multiple of the heads per K/V head
     __device__ __forceinline__ int kv_slice(int bh) const { return by_kv_group.quotient(bh); }
@@ -94,6 +97,43 @@ inline void set_divisors(FwdArgs& b, long long slices)
     b.by_xcd_group = fast_div(b.group_xcd);
     b.by_kv_group = fast_div(b.kv_group);
     b.by_heads = fast_div(b.H);
+    b.by_fold = fast_div(b.fold_rows);
+}
+
+// Folded launches: the G query heads of a K/V head, n rows each, are one problem of G n rows over that K/V head -- in
+// memory they are just that, Q [B,H,n,d] is [B,H_kv,G n,d] -- in which row r is query r % n.
+// (kFold: in the instances for such launches.  As a run-time choice in every instance the same code cost each launch
+// 0.15 us.)
+// Position among the queries of row r, and those of rows r0 ... r1 as a range (`straight`: one after the other)
+template <bool kFold>
+__device__ __forceinline__ int row_position(const FwdArgs& a, int r)
+{
+    if constexpr (kFold) return r - a.by_fold.quotient(r) * a.fold_rows;
+    return r;
+}
+struct RowSpan {
+    int first, last;
+    bool straight;
+};
+template <bool kFold>
+__device__ __forceinline__ RowSpan row_span(const FwdArgs& a, int r0, int r1)
+{
+    if constexpr (kFold) {
+        const int h0 = a.by_fold.quotient(r0), h1 = a.by_fold.quotient(r1);
+        if (h0 != h1) return {0, a.fold_rows - 1, false};
+        return {r0 - h0 * a.fold_rows, r1 - h0 * a.fold_rows, true};
+    }
+    return {r0, r1, true};
+}
+// row of the split workspace [B,H,S,n] of row r of slice bh
+template <bool kFold>
+__device__ __forceinline__ size_t partial_row(const FwdArgs& a, int bh, int split, int r)
+{
+    if constexpr (kFold) {
+        const int hq = a.by_fold.quotient(r);
+        return (((size_t)bh * a.fold_group + hq) * a.num_splits + split) * a.fold_rows + (r - hq * a.fold_rows);
+    }
+    return ((size_t)bh * a.num_splits + split) * a.Nq + r;
 }
 
 __device__ __forceinline__ int wave_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -116,11 +156,20 @@ __device__ __forceinline__ v8h mask_q_chunk_anyalign(v4u v, int col, int d)
 // results of split `split`.  The rows are one contiguous piece of memory; it is filled with 16-byte stores at whatever
 // alignment the piece has, the last one ending with the piece.  Called by every thread of the group, before anything else
 // is requested: such a group is done in the time of its stores.
+template <bool kFold = false>
 __device__ __forceinline__ void store_empty_rows(const FwdArgs& a, int bh, int split, int r0, int r1, int tid, int nthreads)
 {
     char* base;
     float* lse;
     size_t bytes;
+    if (kFold && a.num_splits > 1) {  // one piece per head
+        for (int r = r0; r < r1; ++r) {
+            const size_t prow = partial_row<kFold>(a, bh, split, r);
+            for (int i = tid; i < a.d; i += nthreads) a.O_partial[prow * a.d + i] = 0.0f;
+            if (tid == 0) a.LSE_partial[prow] = -INFINITY;
+        }
+        return;
+    }
     if (a.num_splits > 1) {
         const size_t prow = ((size_t)bh * a.num_splits + split) * a.Nq + r0;
         base = reinterpret_cast<char*>(a.O_partial + prow * a.d);

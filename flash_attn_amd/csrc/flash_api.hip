@@ -167,7 +167,7 @@ int launch_tiled(const flash_params* p, const fa::FwdArgs& a, hipStream_t st)
 // work-groups of the tiled launch for the (final) arguments a
 long long tiled_groups(const flash_params* p, const fa::FwdArgs& a)
 {
-    const bool pp = a.d > 96 && fa::fwd_uses_pingpong(a.d, !needs_every_instance(p), a.Nq, a.Nk, a.causal, a.wl, a.wr,
+    const bool pp = a.d > 96 && !a.fold_rows && fa::fwd_uses_pingpong(a.d, !needs_every_instance(p), a.Nq, a.Nk, a.causal, a.wl, a.wr,
                                                       (long long)a.B * a.H * a.num_splits, a.kernel_hint);
     const int rows = pp ? 256 : kRowsPerGroup;
     return (long long)((a.Nq + rows - 1) / rows) * a.B * a.H * a.num_splits;
@@ -192,6 +192,8 @@ long long tiled_groups(const flash_params* p, const fa::FwdArgs& a)
 // on its CU.  Over 21 swept shapes the count it picks is within 5 % of the best measured one on 19 (the others: 6 % and
 // 9 %); the reference's rule with 256 CUs: 9 of 21, the worst 3.1 times slower than the best count.
 int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode);
+bool folds_heads(const flash_params* p);
+void fold_heads(fa::FwdArgs* a);
 
 // The estimate walks the row blocks once per candidate count (up to 0.26 ms on a causal sequence of 65536 rows), and
 // callers in a loop ask for the same few shapes again and again: each thread remembers the answers to its last four
@@ -225,10 +227,12 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
 {
     const int wl = window_left_of(p), wr = window_right_of(p);
     const bool every = needs_every_instance(p);
-    const bool pp = fa::fwd_uses_pingpong(p->d, !every, p->Nq, p->Nk, p->is_causal, wl, wr, (long long)p->B * p->H, p->kernel_hint);
+    const bool fold = folds_heads(p);
+    const bool pp = !fold && fa::fwd_uses_pingpong(p->d, !every, p->Nq, p->Nk, p->is_causal, wl, wr, (long long)p->B * p->H, p->kernel_hint);
     const int rows = pp ? 256 : kRowsPerGroup;
-    const int Tr = (p->Nq + rows - 1) / rows;
-    const long long slices = (long long)p->B * p->H;
+    const int Nq = fold ? p->Nq * (p->H / p->H_kv) : p->Nq;  // rows of a slice
+    const int Tr = (Nq + rows - 1) / rows;
+    const long long slices = (long long)p->B * (fold ? p->H_kv : p->H);
     if (slices * Tr >= 4LL * kNumCU) return 1;  // (the reference's early exit: four rounds of work-groups as they are)
     const int bucket = (p->d + 31) / 32;  // head-dim bucket of the kernel instance: 1 ... 4
     // microseconds per tile of a lone work-group, by bucket; x 1.5 for the instance that serves every request (tiles
@@ -247,7 +251,7 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
     // the split launch; partials: 8 B H Nq d bytes written and read back per split at 4.2 TB/s.  (Fitted to sweeps of
     // explicit counts over 101 shapes, checked on 40 others.)
     const float a = 5.0f, c0 = 4.2f, c1 = decode ? 0.04f : 0.09f;
-    const float partials = 8.0f * (float)slices * (float)p->Nq * (float)p->d / 4.2e6f;  // us per split
+    const float partials = 8.0f * (float)slices * (float)Nq * (float)p->d / 4.2e6f;  // us per split
     const int shift = p->Nk - p->Nq;
     const bool masked = p->is_causal || wl >= 0 || wr >= 0;
     // An unsplit launch may take the narrow instances (fa::fwd_uses_narrow): four times the work-groups, each wave
@@ -257,6 +261,7 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
     if (!pp) {
         fa::FwdArgs unsplit;
         fill_args(p, 1, &unsplit);
+        if (fold) fold_heads(&unsplit);
         narrow = fa::fwd_uses_narrow(unsplit, tiled_variant(p), every);
     }
     int limit = FLASH_MAX_SPLITS;
@@ -274,8 +279,8 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
         for (int m = 0; m < m_end; ++m) {
             long long lo = 0, hi = p->Nk;  // visible keys of the row block: [lo, hi)
             if (masked) {
-                const long long first = (long long)m * rows + shift;
-                const long long last = (long long)((m + 1) * rows < p->Nq ? (m + 1) * rows : p->Nq) - 1 + shift;
+                const long long first = (fold ? 0 : (long long)m * rows) + shift;
+                const long long last = (!fold && (m + 1) * rows < p->Nq ? (m + 1) * rows : p->Nq) - 1 + shift;
                 if (wl >= 0 && first - wl > lo) lo = first - wl;
                 if (p->is_causal && last + 1 < hi) hi = last + 1;
                 if (wr >= 0 && last + wr + 1 < hi) hi = last + wr + 1;
@@ -317,7 +322,7 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
             // odd d (every second row off a 4-byte boundary: slower requests, which a wave on its own cannot hide); under
             // a causal mask with about as many rows as keys the work-groups that follow another on their CU are the
             // light ones of rows that found their tiles in L2 already, and take half of that
-            const long long gn = (groups * ((p->Nq + 31) / 32) + Tr - 1) / Tr;
+            const long long gn = (groups * ((Nq + 31) / 32) + Tr - 1) / Tr;
             const long long kn = (gn + kNumCU - 1) / kNumCU;
             const float rhon = kn >= 2 && p->d <= 32 ? rho2 : 1.0f;
             const float bn = (p->d <= 64 ? 1.15f : bucket == 3 ? 1.3f : 1.6f) * ((p->d & 1) ? 1.7f : 1.0f) * b;
@@ -381,7 +386,8 @@ int resolve_splits(const flash_params* p)
             s = (n_blocks + per - 1) / per;
         }
     } else if (s <= 0) {
-        s = auto_splits_tiled(p, n_blocks);
+        // (a folded launch of one row block per K/V head reads K and V once, as decode launches do)
+        s = auto_splits_tiled(p, n_blocks, folds_heads(p) && p->Nq * (p->H / p->H_kv) <= kRowsPerGroup);
     }
     if (s > n_blocks) s = n_blocks;  // never more splits than key blocks
     if (s > FLASH_MAX_SPLITS) s = FLASH_MAX_SPLITS;
@@ -414,6 +420,30 @@ int scratch_of_current_device(unsigned char** out)
     return FLASH_OK;
 }
 
+// Few query rows per head and grouped K/V heads: the heads of a K/V head become the rows of one problem over it
+// (row_position in common.h), so that the 128-row work-groups are filled and K and V are read once per K/V head instead of
+// once per query head.  Up to 64 rows per head, where that at least halves the work-groups (whole row blocks gain nothing,
+// and a block that holds the end of one head and the start of the next cannot skip tiles for either); a mask depends on
+// the position of a row alone, ALiBi slopes and dropout bits also on the head.  Automatic split counts, before -> after:
+// causal B25 H32 H_kv4 Nq3 Nk8396 d80 294 -> 54 us, B23 H64 H_kv8 Nq21 Nk1664 d112 97 -> 54, B3 H32 H_kv8 Nq14 Nk21440 d100
+// 83 -> 50, B4 H32 H_kv8 Nq16 Nk8192 d128 69 -> 35, B9 H16 H_kv4 Nq61 Nk5184 d80 47 -> 37.
+constexpr int kFoldRows = 64;
+bool folds_heads(const flash_params* p)
+{
+    const int hk = p->H_kv > 0 ? p->H_kv : p->H;
+    return p->Nq > 1 && p->Nq <= kFoldRows && hk < p->H && !p->alibi_slopes && p->dropout_p == 0.0f &&
+           !p->stage_stamps_out && !needs_every_instance(p) && p->kernel_hint == 0;
+}
+void fold_heads(fa::FwdArgs* a)
+{
+    a->fold_rows = a->Nq;
+    a->fold_group = a->kv_group;
+    a->H = a->Hk;
+    a->Nq *= a->kv_group;
+    a->kv_group = 1;
+    a->Tr = (a->Nq + kRowsPerGroup - 1) / kRowsPerGroup;
+}
+
 // Which kernel serves a split-KV call; may reshape the arguments (grouped decode).
 constexpr int kRouteTiled = 0, kRouteStream = 1;
 int splitkv_route(const flash_params* p, fa::FwdArgs* a)
@@ -436,6 +466,7 @@ int splitkv_route(const flash_params* p, fa::FwdArgs* a)
     }
     // one query row per head, rows of eight elements or more, no dropout: bandwidth-bound streaming kernel
     if (p->Nq == 1 && p->d >= 8 && p->dropout_p == 0.0f && p->softmax_scale > 0.0f) return kRouteStream;
+    if (folds_heads(p)) fold_heads(a);
     return kRouteTiled;
 }
 
@@ -450,6 +481,10 @@ int run_splitkv(const flash_params* p, int splits, hipStream_t st)
     const int route = splitkv_route(p, &a);
     const int e = route == kRouteStream ? record_hip(fa::launch_decode_split(a, st)) : launch_tiled(p, a, st);
     if (e != FLASH_OK || splits == 1) return e;
+    if (a.fold_rows) {  // the partial results keep the layout of the heads
+        a.H *= a.fold_group;
+        a.Nq = a.fold_rows;
+    }
     return record_hip(fa::launch_combine(a, st));
 }
 
@@ -470,6 +505,7 @@ FLASH_EXPORT int flash_forward(const flash_params* p, void* stream)
     if ((rc = device_usable()) != FLASH_OK) return rc;
     fa::FwdArgs a;
     fill_args(p, 1, &a);
+    if (folds_heads(p)) fold_heads(&a);
     return launch_tiled(p, a, static_cast<hipStream_t>(stream));
 }
 

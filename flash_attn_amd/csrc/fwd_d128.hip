@@ -31,7 +31,7 @@ bool fwd_uses_pingpong(int d, bool direct, int Nq, int Nk, int causal, int wl, i
 int launch_fwd_d128(const FwdArgs& a, int variant, int nb, hipStream_t st)
 {
     (void)nb;
-    if (fwd_uses_pingpong(a.d, !fwd_needs_every_instance(a, variant), a.Nq, a.Nk, a.causal, a.wl, a.wr, (long long)a.B * a.H * a.num_splits,
+    if (!a.fold_rows && fwd_uses_pingpong(a.d, !fwd_needs_every_instance(a, variant), a.Nq, a.Nk, a.causal, a.wl, a.wr, (long long)a.B * a.H * a.num_splits,
                           a.kernel_hint))
         return launch_fwd_pp_bucket<128>(a, variant, st);
     return launch_fwd_bucket<128, 1>(a, variant, st);

@@ -128,8 +128,9 @@ constexpr float kLazyTau = 8.0f;
 // kVarEvery (with kVarAlibi and kVarDropout, without kVarVec): the instance that serves every request, see kEvery below.
 // kVarNarrow (unsplit launches): the four waves of a work-group share 32 query rows and take every fourth key tile
 // each, see kNarrow below.
+// kVarFold (no other feature): the rows are the query heads of a K/V head, see row_position in common.h.
 constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarStamp = 16, kVarAlibiLeft = 32, kVarKvOnce = 64,
-              kVarEvery = 128, kVarNarrow = 256;
+              kVarEvery = 128, kVarNarrow = 256, kVarFold = 512;
 
 // work-groups per CU: three up to D = 64 (168 VGPRs), except for the instance that serves every request, which stages
 // its tiles through registers
@@ -168,6 +169,8 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
     // of a split -- in the same launch, where a split count of four would need the combine launch behind it.
     constexpr bool kNarrow = (VAR & kVarNarrow) != 0;
     static_assert(!kNarrow || (kDma && NB == 1 && !kStamp && !kKvOnce), "narrow instances");
+    constexpr bool kFold = (VAR & kVarFold) != 0;
+    static_assert(!kFold || (!kAlibi && !kDropout && !kStamp), "folded instances");
     // (narrow: two stages per wave up to D = 64, one above: four waves' tiles of 26 / 33 KiB)
     constexpr int NSTG = kNarrow ? (D <= 64 ? 2 : 1) : kDma ? C::NSTG : 2;
     constexpr int BRW = kNarrow ? 32 : C::BR;  // query rows per work-group
@@ -187,15 +190,16 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
     const WorkItem item = work_item(a, blockIdx.x);
     const int bh = item.bh, split = item.split, m_block = item.m_block;
     const int Nq = a.Nq, Nk = a.Nk, d = kFullD ? D : a.d;
-    const int shift = Nk - Nq;
+    const int shift = Nk - (kFold ? a.fold_rows : Nq);
     const int q0 = m_block * BRW;
     const int wave_row0 = kNarrow ? 0 : wave * C::RW;  // first row of the wave inside the work-group's block
 
     // ---- key range of the work-group (block pruning, src/flash_forward.h:39-48; split range, splitkv.h:40-43)
     int kmin = 0, kmax = Nk;
     {
-        const int last_row = (q0 + BRW - 1 < Nq ? q0 + BRW - 1 : Nq - 1) + shift;
-        if (a.wl >= 0) kmin = max(0, q0 + shift - a.wl);
+        const RowSpan rows = row_span<kFold>(a, q0, q0 + BRW - 1 < Nq ? q0 + BRW - 1 : Nq - 1);
+        const int last_row = rows.last + shift;
+        if (a.wl >= 0) kmin = max(0, rows.first + shift - a.wl);
         if (a.causal) kmax = min(kmax, last_row + 1);
         if (a.wr >= 0) kmax = min(kmax, last_row + a.wr + 1);
         if (a.num_splits > 1) {
@@ -207,7 +211,7 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
     const int tile_begin = kmin / BC;
     const int ntiles = kmax > kmin ? (kmax + BC - 1) / BC - tile_begin : 0;
     if (!kStamp && ntiles == 0) {  // (the instrumented twins take the long way and report their stages)
-        store_empty_rows(a, bh, split, q0, q0 + BRW < Nq ? q0 + BRW : Nq, tid, 256);
+        store_empty_rows<kFold>(a, bh, split, q0, q0 + BRW < Nq ? q0 + BRW : Nq, tid, 256);
         return;
     }
 
@@ -218,7 +222,7 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
     for (int nb = 0; nb < NB; ++nb) {
         const int i = q0 + wave_row0 + nb * 32 + l32;
         row_i[nb] = i;
-        const int ii = (i < Nq ? i : Nq - 1) + shift;
+        const int ii = row_position<kFold>(a, i < Nq ? i : Nq - 1) + shift;
         int l_ = 0, h_ = Nk - 1;
         if (a.wl >= 0) l_ = max(0, ii - a.wl);
         if (a.causal) h_ = min(h_, ii);
@@ -234,9 +238,12 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
     // wave-uniform bounds: [lo_max, hi_min] is visible to every row of the wave (a tile inside it needs no element
     // test), nothing outside [lo_min, hi_max] is visible to any of them (a tile outside it is skipped by the wave)
     int lo_max, hi_min, lo_min, hi_max;
+    bool straight;  // the rows' positions follow each other
     {
         const int first = q0 + wave_row0, last = first + C::RW - 1;
-        const int iif_ = (first < Nq ? first : Nq - 1) + shift, iil_ = (last < Nq ? last : Nq - 1) + shift;
+        const RowSpan rows = row_span<kFold>(a, first < Nq ? first : Nq - 1, last < Nq ? last : Nq - 1);
+        const int iif_ = rows.first + shift, iil_ = rows.last + shift;
+        straight = rows.straight;
         lo_max = lo_min = 0;
         hi_min = hi_max = Nk - 1;
         if (a.wl >= 0) lo_max = max(0, iil_ - a.wl), lo_min = max(0, iif_ - a.wl);
@@ -563,8 +570,8 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
                 // rows not clipped by a sequence or split end): then lane-mask constants per 32-key block do the
                 // masking; otherwise a tile takes one comparison per score and crossed end of the interval.
                 const float ninf = -INFINITY;
-                const bool hi_diag = NB == 1 && hi_max - hi_min == 31 && (hi_min & 31) == 0;
-                const bool lo_diag = NB == 1 && lo_max - lo_min == 31 && (lo_min & 31) == 0;
+                const bool hi_diag = NB == 1 && straight && hi_max - hi_min == 31 && (hi_min & 31) == 0;
+                const bool lo_diag = NB == 1 && straight && lo_max - lo_min == 31 && (lo_min & 31) == 0;
                 if (((mask_sides & 1) == 0 || lo_diag) && ((mask_sides & 2) == 0 || hi_diag)) {
 #pragma unroll
                     for (int kb = 0; kb < 2; ++kb) {
@@ -928,7 +935,7 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
         const int i = row_i[nb];
         if (i >= Nq) continue;
         if (a.num_splits > 1) {
-            const size_t prow = ((size_t)bh * a.num_splits + split) * Nq + i;
+            const size_t prow = partial_row<kFold>(a, bh, split, i);
             if (g == 0) a.LSE_partial[prow] = lse;
             float* op = a.O_partial + prow * d;
 #pragma unroll
@@ -1140,12 +1147,23 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
             if (feat == kVarAlibi) return (int)launch_fwd_narrow_instance<D, F | kVarAlibi>(a, st);
             if (feat == kVarDropout) return (int)launch_fwd_narrow_instance<D, F | kVarDropout>(a, st);
             if (feat != 0) return (int)launch_fwd_narrow_instance<D, F | kVarAlibi | kVarDropout>(a, st);
+            if (a.fold_rows) {
+                if (D > 64 || a.d == D) return (int)launch_fwd_narrow_instance<D, kVarVec | kVarFullD | kVarFold>(a, st);
+                if (variant & kVarVec) return (int)launch_fwd_narrow_instance<D, kVarVec | kVarFold>(a, st);
+                return (int)launch_fwd_narrow_instance<D, kVarFold>(a, st);
+            }
             if (a.d == D) return (int)launch_fwd_narrow_instance<D, kVarVec | kVarFullD>(a, st);
             if constexpr (D <= 64) {  // (above, only rows of the bucket's width come here)
                 if (!(variant & kVarVec)) return (int)launch_fwd_narrow_instance<D, 0>(a, st);
                 return (int)launch_fwd_narrow_instance<D, kVarVec>(a, st);
             }
         }
+    }
+    if (ST == 0 && a.fold_rows) {
+        constexpr int F = ST == 0 ? kVarFold : 0;
+        if (a.d == D) return (int)launch_fwd_instance<D, NB, (ST == 0 ? F | kVarVec | kVarFullD | kVarKvOnce : 0)>(a, st);
+        if (variant & kVarVec) return (int)launch_fwd_instance<D, NB, (ST == 0 ? F | kVarVec : 0)>(a, st);
+        return (int)launch_fwd_instance<D, NB, F>(a, st);
     }
     if (!(variant & kVarVec)) {
         // rows at any alignment: plain, ALiBi, dropout, both, and one more with both features compiled in (slope 0 /
