@@ -44,6 +44,7 @@ class FlashParams(C.Structure):
         ("scores_out", C.c_void_p),
         ("kernel_hint", C.c_int),
         ("stage_stamps_out", C.c_void_p),
+        ("split_counters", C.c_void_p), ("split_counters_len", C.c_int),
     ]
 
 

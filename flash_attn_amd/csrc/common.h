@@ -81,6 +81,8 @@ struct FwdArgs {
     int fold_rows;       // > 0: the query heads of a K/V head are the rows of one problem, this many rows each (see RowSpan)
     int fold_group;      // query heads folded into one
     FastDiv by_fold;
+    uint32_t* counters;  // nullptr, or where the work-groups of a split launch count themselves in (combine.h)
+    int combine_waves;   // waves that merge a row's partial results: 1 or 4 (combine_waves_for)
 
     // index of the K/V slice [Nk,d] read by query slice bh = b * H + h: H is a multiple of the heads per K/V head
     __device__ __forceinline__ int kv_slice(int bh) const { return by_kv_group.quotient(bh); }

@@ -11,26 +11,11 @@
 //     LSE_s = m_s + log l_s go to the workspace (reference: O_tmp, M, L; src/flash_forward_splitkv.h:313-338)
 // combine_kernel replaces forward_kernel_splitkv_combine (src/flash_forward_splitkv.h:347-399) with one wave per
 // query row and coalesced reads of the partials (the reference uses one thread per row).
+#include "combine.h"
 #include "common.h"
 #include "decode_kernels.h"
 
 namespace fa {
-
-template <int CTRL>
-__device__ __forceinline__ float dpp_mov(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
-}
-// sum over the LPK consecutive lanes that share a key; every lane of the group ends with the total
-template <int LPK>
-__device__ __forceinline__ float group_sum(float v)
-{
-    v += dpp_mov<0xB1>(v);                          // quad_perm [1,0,3,2]
-    v += dpp_mov<0x4E>(v);                          // quad_perm [2,3,0,1]
-    if constexpr (LPK >= 8) v += dpp_mov<0x141>(v);   // row_half_mirror
-    if constexpr (LPK >= 16) v += dpp_mov<0x140>(v);  // row_mirror
-    return v;
-}
 
 // G = query heads served by one work-group: the G consecutive heads share one K/V head (grouped-query attention), so
 // the K/V stream is read once for all of them.  G == 1 is the plain one-K/V-head-per-query-head case.
@@ -42,8 +27,9 @@ __global__ void __launch_bounds__(256) decode_split_kernel(const FwdArgs a)
     constexpr int KB = U * KPI;        // keys per wave block
     constexpr int NG = 4 * KPI;        // key groups per work-group
     constexpr int DB = LPK * 8;        // head-dim bucket
-    __shared__ float s_acc[NG][DB];
+    __shared__ __attribute__((aligned(16))) float s_acc[NG][DB];
     __shared__ float s_m[NG], s_l[NG];
+    __shared__ int s_last;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -200,117 +186,39 @@ __global__ void __launch_bounds__(256) decode_split_kernel(const FwdArgs a)
             const bool ok = tid < c0 || (rem != 0 && tid < c0 + 8 && tcol >= c0);
             if (a.num_splits > 1) {
                 const size_t prow = (size_t)bh * a.num_splits + split;  // Nq == 1
-                if (ok) a.O_partial[prow * d + tcol] = o * inv;
-                if (tid == 0) a.LSE_partial[prow] = lse;
+                const bool here = a.counters != nullptr;
+                if (ok) store_partial(a.O_partial + prow * d + tcol, o * inv, here);
+                if (tid == 0) store_partial(a.LSE_partial + prow, lse, here);
             } else {
                 if (ok) a.O[(size_t)bh * d + tcol] = (half_t)(o * inv);
                 if (tid == 0) a.LSE[bh] = lse;
             }
         }
     }
+    if (a.counters != nullptr && last_to_arrive(a.counters + bh0 / G, a.num_splits, &s_last)) {
+        static_assert(NG * DB >= kCombineLds, "the merge fits the buffer of the key groups");
+        float* const lds = &s_acc[0][0];
+        if (a.combine_waves == 1) {
+            for (int gq = wave; gq < G; gq += 4)
+                combine_row<true, 1>(a.O_partial, a.LSE_partial, a.O, a.LSE, bh0 + gq, 0, 1, d, a.num_splits, lds);
+        } else {
+            for (int gq = 0; gq < G; ++gq)
+                combine_row<true, 4>(a.O_partial, a.LSE_partial, a.O, a.LSE, bh0 + gq, 0, 1, d, a.num_splits, lds);
+        }
+    }
 }
 
-// Reductions over the 64 lanes of a wave without LDS: DPP inside the rows of 16 lanes, v_permlane32_swap between the
-// halves, v_readlane for the last two rows; the result is wave-uniform.
-__device__ __forceinline__ float wave_sum(float v)
-{
-    v = xhalf_sum(group_sum<16>(v));  // lanes of rows r and r ^ 2 now hold the total of both rows
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0)) +
-           __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
-}
-__device__ __forceinline__ float wave_max(float v)
-{
-    v = fmaxf(v, dpp_mov<0xB1>(v));
-    v = fmaxf(v, dpp_mov<0x4E>(v));
-    v = fmaxf(v, dpp_mov<0x141>(v));
-    v = fmaxf(v, dpp_mov<0x140>(v));
-    v = xhalf_max(v);
-    return fmaxf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0)),
-                 __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16)));
-}
-
-// One wave per query row: LSE = logsumexp_s LSE_s, O = sum_s exp(LSE_s - LSE) O_s
-// (same value as m = max M_s, l = sum e^{M_s-m} L_s, O = sum (L_s e^{M_s-m} / l) O_s of splitkv.h:359-397).
-// The weights of a row live in LDS that only its wave touches, so no work-group barrier is needed.  With d % 8 == 0
-// a lane holds four consecutive columns, the two halves of the wave take the even and the odd splits, and the first
-// partial rows are requested before the log-sum-exp values they will be weighted with.
+// one wave per query row, or one work-group (W = 4)
+template <int W>
 __global__ void __launch_bounds__(256) combine_kernel(const float* __restrict__ O_partial,
                                                       const float* __restrict__ LSE_partial, half_t* __restrict__ O,
-                                                      float* __restrict__ LSE, int BH, int Nq, int d, int S)
+                                                      float* __restrict__ LSE, int rows, int Nq, FastDiv by_Nq, int d, int S)
 {
-    __shared__ float s_w[4][FLASH_MAX_SPLITS_K];
-    const int lane = threadIdx.x & 63;
-    const int wave = wave_uniform(threadIdx.x >> 6);
-    const long long row = (long long)blockIdx.x * 4 + wave;
-    if (row >= (long long)BH * Nq) return;
-    const int bh = (int)(row / Nq), i = (int)(row % Nq);
-    const float* lp = LSE_partial + (size_t)bh * S * Nq + i;  // stride Nq between splits
-    const size_t sstride = (size_t)Nq * d;                     // floats between the partial rows of two splits
-    const float* op = O_partial + ((size_t)bh * S * Nq + i) * d;
-    const bool vec = (d & 7) == 0;  // rows of the partials and of O are 16-byte aligned (the host checks the bases)
-    constexpr int U = 8;            // partial rows in flight per half-wave
-    const int c4 = (lane & 31) * 4, grp = lane >> 5;
-    const bool act = c4 < d;
-    float4 pre[U];
-    if (vec) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int s = grp + 2 * u;
-            pre[u] = (act && s < S) ? *reinterpret_cast<const float4*>(op + s * sstride + c4) : float4{0.f, 0.f, 0.f, 0.f};
-        }
-    }
-    float mx = -INFINITY;
-    for (int s = lane; s < S; s += 64) mx = fmaxf(mx, lp[(size_t)s * Nq]);
-    mx = wave_max(mx);
-    const float mu = (mx == -INFINITY) ? 0.0f : mx;
-    float sum = 0.0f;
-    for (int s = lane; s < S; s += 64) {
-        const float w = __expf(lp[(size_t)s * Nq] - mu);
-        s_w[wave][s] = w;
-        sum += w;
-    }
-    sum = wave_sum(sum);
-    const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
-    if (lane == 0) LSE[(size_t)bh * Nq + i] = sum > 0.0f ? mx + __logf(sum) : -INFINITY;
-    if (vec) {
-        float4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int s = grp + 2 * u;
-            const float w = s < S ? s_w[wave][s] : 0.0f;
-            acc.x += w * pre[u].x, acc.y += w * pre[u].y, acc.z += w * pre[u].z, acc.w += w * pre[u].w;
-        }
-        // the remaining partial rows, U at a time, requested together (one by one, every request waited for its
-        // predecessor's arithmetic: with 64 splits and more the combine took longer than the split kernel)
-        for (int s0 = grp + 2 * U; s0 < S; s0 += 2 * U) {  // (wave-uniform trip count: the first half-wave's)
-            float4 nxt[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int s = s0 + 2 * u;
-                nxt[u] = (act && s < S) ? *reinterpret_cast<const float4*>(op + s * sstride + c4) : float4{0.f, 0.f, 0.f, 0.f};
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int s = s0 + 2 * u;
-                const float w = s < S ? s_w[wave][s] : 0.0f;
-                acc.x += w * nxt[u].x, acc.y += w * nxt[u].y, acc.z += w * nxt[u].z, acc.w += w * nxt[u].w;
-            }
-        }
-        acc.x = xhalf_sum(acc.x), acc.y = xhalf_sum(acc.y), acc.z = xhalf_sum(acc.z), acc.w = xhalf_sum(acc.w);
-        if (act && grp == 0) {
-            union { v2h h[2]; uint2 u; } r;
-            r.h[0] = pack_f16(acc.x * inv, acc.y * inv);
-            r.h[1] = pack_f16(acc.z * inv, acc.w * inv);
-            *reinterpret_cast<uint2*>(O + ((size_t)bh * Nq + i) * d + c4) = r.u;
-        }
-    } else {
-        for (int dc = lane; dc < d; dc += 64) {
-            float o = 0.0f;
-            for (int s = 0; s < S; ++s) o += s_w[wave][s] * op[s * sstride + dc];
-            O[((size_t)bh * Nq + i) * d + dc] = (half_t)(o * inv);
-        }
-    }
+    __shared__ __attribute__((aligned(16))) float lds[kCombineLds];
+    const int row = W == 1 ? blockIdx.x * 4 + wave_uniform(threadIdx.x >> 6) : blockIdx.x;
+    if (row >= rows) return;
+    const int bh = by_Nq.quotient(row);
+    combine_row<false, W>(O_partial, LSE_partial, O, LSE, bh, row - bh * Nq, Nq, d, S, lds);
 }
 
 // keep[b,h,i,j] = (16-bit field dropout_field(j) of the Philox call dropout_call(j) of row (b*H + h, i)) >= threshold;
@@ -335,6 +243,8 @@ __global__ void __launch_bounds__(256) keep_mask_kernel(uint8_t* __restrict__ ma
     }
 }
 
+int decode_heads_per_group(int kv_group) { return kv_group % 8 == 0 ? 8 : kv_group % 4 == 0 ? 4 : kv_group % 2 == 0 ? 2 : 1; }
+
 template <int LPK, int G>
 static hipError_t launch_decode_instance(const FwdArgs& a, hipStream_t st)
 {
@@ -350,10 +260,12 @@ template <int LPK>
 static hipError_t launch_decode_bucket(const FwdArgs& a, hipStream_t st)
 {
     // as many of the query heads of a K/V head per work-group as divide the group (up to 8)
-    if (a.kv_group % 8 == 0) return launch_decode_instance<LPK, 8>(a, st);
-    if (a.kv_group % 4 == 0) return launch_decode_instance<LPK, 4>(a, st);
-    if (a.kv_group % 2 == 0) return launch_decode_instance<LPK, 2>(a, st);
-    return launch_decode_instance<LPK, 1>(a, st);
+    switch (decode_heads_per_group(a.kv_group)) {
+        case 8: return launch_decode_instance<LPK, 8>(a, st);
+        case 4: return launch_decode_instance<LPK, 4>(a, st);
+        case 2: return launch_decode_instance<LPK, 2>(a, st);
+        default: return launch_decode_instance<LPK, 1>(a, st);
+    }
 }
 
 int launch_decode_split(const FwdArgs& a, hipStream_t st)
@@ -365,10 +277,13 @@ int launch_decode_split(const FwdArgs& a, hipStream_t st)
 
 int launch_combine(const FwdArgs& a, hipStream_t st)
 {
-    const long long rows = (long long)a.B * a.H * a.Nq;
-    const unsigned groups = (unsigned)((rows + 3) / 4);
-    return (int)launch_kernel(combine_kernel, dim3(groups), dim3(256), 0, st, a.O_partial, a.LSE_partial, a.O, a.LSE,
-                              a.B * a.H, a.Nq, a.d, a.num_splits);
+    const int rows = (int)((long long)a.B * a.H * a.Nq);  // < 2^31: validate_shape
+    const FastDiv by_Nq = fast_div(a.Nq);
+    if (a.combine_waves == 1)
+        return (int)launch_kernel(combine_kernel<1>, dim3((unsigned)(rows + 3) / 4), dim3(256), 0, st, a.O_partial, a.LSE_partial, a.O,
+                                  a.LSE, rows, a.Nq, by_Nq, a.d, a.num_splits);
+    return (int)launch_kernel(combine_kernel<4>, dim3((unsigned)rows), dim3(256), 0, st, a.O_partial, a.LSE_partial, a.O, a.LSE, rows,
+                              a.Nq, by_Nq, a.d, a.num_splits);
 }
 
 int launch_keep_mask(uint8_t* mask, int B, int H, int Nq, int Nk, uint32_t thr, uint64_t seed, uint64_t offset,

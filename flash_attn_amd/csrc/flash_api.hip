@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstring>
 
+#include "combine.h"
 #include "common.h"
 #include "decode_kernels.h"
 #include "fwd_kernel.h"
@@ -83,6 +84,7 @@ int validate(const flash_params* p, bool* empty)
     if (p->alibi_slopes && misaligned(p->alibi_slopes, 4)) return FLASH_EALIGN;
     if (p->scores_out && misaligned(p->scores_out, 4)) return FLASH_EALIGN;
     if (p->stage_stamps_out && misaligned(p->stage_stamps_out, 8)) return FLASH_EALIGN;
+    if (p->split_counters && misaligned(p->split_counters, 4)) return FLASH_EALIGN;
     return FLASH_OK;
 }
 
@@ -356,7 +358,7 @@ int resolve_splits(const flash_params* p)
             // heads and key count (B1 H32 Nk16384 d128: 1 / 4 / 6 / 8 / 16 / 32 splits 142 / 48 / 42 / 42 / 45 / 48 us;
             // B4 H8 Nk65536: best at 6; B16 H32 and B64 H32: unsplit); and every split adds to the combine, which
             // bounds the useful count by about sqrt(Nk / 3).
-            const int per_group = G % 8 == 0 ? 8 : G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;  // query heads per work-group
+            const int per_group = fa::decode_heads_per_group(G);
             const long long groups = (long long)p->B * p->H / per_group;
             // (twice that where a work-group serves four or eight query heads, which only ALiBi or a window send here: it
             // then spends as long on arithmetic as on loads; B16 H32 H_kv8 Nk16384 with ALiBi 2 / 4 splits 185 / 171 us)
@@ -479,8 +481,12 @@ int run_splitkv(const flash_params* p, int splits, hipStream_t st)
     fa::FwdArgs a;
     fill_args(p, splits, &a);
     const int route = splitkv_route(p, &a);
+    // (a slice of the decode kernel has one row per query head, which its last work-group merges in a microsecond)
+    if (route == kRouteStream && splits > 1 && p->split_counters && (long long)p->B * p->H <= p->split_counters_len)
+        a.counters = p->split_counters;
+    a.combine_waves = fa::combine_waves_for(splits, route == kRouteStream ? fa::decode_heads_per_group(a.kv_group) : 1);
     const int e = route == kRouteStream ? record_hip(fa::launch_decode_split(a, st)) : launch_tiled(p, a, st);
-    if (e != FLASH_OK || splits == 1) return e;
+    if (e != FLASH_OK || splits == 1 || a.counters) return e;
     if (a.fold_rows) {  // the partial results keep the layout of the heads
         a.H *= a.fold_group;
         a.Nq = a.fold_rows;

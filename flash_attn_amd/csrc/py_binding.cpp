@@ -14,8 +14,10 @@
 
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <vector>
 
 #include "flash_attn_mi355.h"
 
@@ -69,11 +71,48 @@ bool optional_tensor(PyObject* o, const at::Tensor** t)
     return o == Py_None || (*t = tensor_of(o)) != nullptr;
 }
 
+// Arrival counters (flash_params::split_counters) of the calls on one stream: a region of kCountersPerStream zeros for
+// each of up to kCounterStreams streams of a device, 1 MiB per device that ever needs one, allocated and cleared once.
+// Only the default stream and torch's own pooled streams get one: those exist until the process ends, so calls that share a
+// region are ordered for good.  Other streams, calls under graph capture (a graph may be replayed beside other work)
+// and whoever comes too late merge in a launch of their own.  (All of this runs with the interpreter lock held.)
+constexpr int kCountersPerStream = 4096, kCounterStreams = 64;
+struct DeviceCounters {
+    at::Tensor zeros;
+    std::vector<void*> streams;
+};
+uint32_t* counters_of(at::Device device, void* stream, bool pooled)
+{
+    static std::vector<DeviceCounters>* all = new std::vector<DeviceCounters>;  // (never freed: outlives the runtime's own end)
+    if (stream != nullptr && !pooled) return nullptr;
+    hipStreamCaptureStatus capture;
+    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &capture) != hipSuccess || capture != hipStreamCaptureStatusNone)
+        return nullptr;
+    const size_t dev = (size_t)device.index();
+    if (dev >= all->size()) all->resize(dev + 1);
+    DeviceCounters& c = (*all)[dev];
+    size_t i = 0;
+    while (i < c.streams.size() && c.streams[i] != stream) ++i;
+    if (i == c.streams.size()) {
+        if (i == (size_t)kCounterStreams) return nullptr;
+        if (!c.zeros.defined()) {
+            at::Tensor z = at::detail::empty_cuda({(int64_t)kCountersPerStream * kCounterStreams}, at::kInt, device, std::nullopt);
+            const auto current = c10::hip::getCurrentHIPStream(device.index()).stream();
+            if (hipMemsetAsync(z.data_ptr(), 0, z.nbytes(), current) != hipSuccess || hipStreamSynchronize(current) != hipSuccess)
+                return nullptr;
+            c.zeros = z;
+        }
+        c.streams.push_back(stream);
+    }
+    return static_cast<uint32_t*>(c.zeros.data_ptr()) + i * kCountersPerStream;
+}
+
 struct Call {
     flash_params p{};
     const at::Tensor* q = nullptr;
     const at::Tensor *out = nullptr, *lse = nullptr;
     void* stream = nullptr;
+    bool pooled_stream = false;  // one of torch's own
 };
 
 // Arguments that both entry points share: q, k, v and the array (softmax_scale, causal, window, alibi_slopes, dropout_p,
@@ -102,13 +141,21 @@ Parsed parse(PyObject* const* qkv, PyObject* const* a, Call* c)
     p.offset = PyLong_AsUnsignedLongLongMask(a[6]);
     if (!optional_tensor(a[8], &c->out) || !optional_tensor(a[9], &c->lse)) return kPython;
     if (a[7] == Py_None) {
-        c->stream = c10::hip::getCurrentHIPStream().stream();
+        const auto current = c10::hip::getCurrentHIPStream();
+        c->stream = current.stream();
+        c->pooled_stream = (current.id() & 1) != 0;  // (the id of a stream from outside is its handle, an aligned pointer)
     } else {
         PyObject* h = PyObject_GetAttrString(a[7], "cuda_stream");
         if (!h) return kRaised;
         c->stream = PyLong_AsVoidPtr(h);
         Py_DECREF(h);
         if (PyErr_Occurred()) return kRaised;
+        if (PyObject* id = PyObject_GetAttrString(a[7], "stream_id")) {
+            c->pooled_stream = PyLong_Check(id) && (PyLong_AsUnsignedLongLongMask(id) & 1) != 0;
+            Py_DECREF(id);
+        } else {
+            PyErr_Clear();
+        }
     }
     p.Q = q->data_ptr(), p.K = k->data_ptr(), p.V = v->data_ptr();
     p.alibi_slopes = slopes ? static_cast<const float*>(slopes->data_ptr()) : nullptr;
@@ -204,6 +251,10 @@ PyObject* splitkv(PyObject*, PyObject* const* args, Py_ssize_t n)
             own = empty_like_q(c, {o_floats + rows}, at::kFloat);
             p.O_partial = static_cast<float*>(own.data_ptr());
             p.LSE_partial = p.O_partial + o_floats;
+        }
+        if (S > 1 && (c.stream == nullptr || c.pooled_stream)) {
+            p.split_counters = counters_of(c.q->device(), c.stream, c.pooled_stream);
+            p.split_counters_len = p.split_counters ? kCountersPerStream : 0;
         }
         return launch(g_splitkv, "flash_forward_splitkv", &c);
     });

@@ -109,6 +109,13 @@ typedef struct flash_params {
      * split count above 1 the combine step is not stamped.  The only instrumentation of the reference is the event
      * pair around its launches (src/main.cu:195-213). */
     uint64_t *stage_stamps_out;
+    /* Optional: device memory of split_counters_len 32-bit words, all zero, which lets flash_forward_splitkv merge the
+     * partial results of few query rows (16 or fewer per K/V head or query head) inside the split kernel instead of in a
+     * second launch; the results are the same bit by bit.  The call leaves the words zero.  Calls that may overlap on the GPU must
+     * not share them: one such array per stream will do (and none for calls captured into a graph that may be replayed
+     * beside others).  Used where there are at least B * H words; NULL, or fewer words: the second launch. */
+    uint32_t *split_counters;
+    int split_counters_len;
 } flash_params;
 
 #define FLASH_STAMP_WORDS 9
