@@ -33,7 +33,7 @@
 namespace fa {
 
 
-template <int D, int NB>
+template <int D, int NB, bool kNarrow = false>
 struct FwdCfg {
     static constexpr int kWaves = 4;
     static constexpr int RW = 32 * NB;        // query rows per wave
@@ -49,16 +49,17 @@ struct FwdCfg {
     // ones, whose requests begin and end anywhere in a row; but a fragment address takes a register per k-step where
     // padded rows have immediate offsets.  Measured, padded -> permuted: causal with dropout B8 H32 N1000 d96 104.0 -> 95.5
     // us, B8 H1 N1920 d32 causal 9.96 -> 9.83, B2 H4 N960 d40 causal 9.53 -> 9.36, d = 64 +-1 %; d = 128, eight k-steps, 10
-    // registers more and 1 % slower, keeps its padding.
+    // registers more and 1-4 % slower, keeps its padding, except in the narrow instances, where a wave requests whole
+    // tiles and the period of the permutation saves offsets (NPX below).
     // V rows are read by ds_read_b64_tr_b16, four consecutive rows of 64 bytes per half wave: a stride of 64 (mod 128)
     // puts the four rows on disjoint bank groups.
-    static constexpr bool kPadK = D == 128;
+    static constexpr bool kPadK = D == 128 && !kNarrow;
     static constexpr int CK = CH + (kPadK ? 1 : 0);  // chunks of a K row in LDS
     static constexpr int SK = CK * 16;
     static constexpr int SV = D * 2;
     static constexpr __host__ __device__ int kswz(int r)
     {
-        return kPadK ? 0 : D == 64 ? (r >> 1) & 7 : (r >> 2) & 3;  // rows of 128 / 192 or 64 bytes
+        return kPadK ? 0 : D == 128 ? r & 15 : D == 64 ? (r >> 1) & 7 : (r >> 2) & 3;  // rows of 256 / 128 / 192 or 64 bytes
     }
     // Where the row length is a multiple of 128 bytes, the two 64-byte halves of each 128 bytes are exchanged in rows
     // 2, 3 (mod 4), which has the same effect without padding.
@@ -132,11 +133,12 @@ constexpr float kLazyTau = 8.0f;
 constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarStamp = 16, kVarAlibiLeft = 32, kVarKvOnce = 64,
               kVarEvery = 128, kVarNarrow = 256, kVarFold = 512;
 
-// work-groups per CU: three up to D = 64 (168 VGPRs), except for the instance that serves every request, which stages
+// work-groups per CU (narrow: one or two by their LDS; held to 256 VGPRs all the same, without which the compiler keeps more
+// than there are and moves them to and from accumulation registers): three up to D = 64 (168 VGPRs), except for the instance that serves every request, which stages
 // its tiles through registers
 constexpr int fwd_groups_per_cu(int D, int NB, int VAR)
 {
-    if ((VAR & kVarNarrow) != 0) return 1;
+    if ((VAR & kVarNarrow) != 0) return 2;
     return NB == 1 ? (D <= 64 && (VAR & kVarEvery) == 0 ? 3 : 2) : 1;
 }
 
@@ -145,7 +147,7 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
 {
     constexpr bool kVec = (VAR & kVarVec) != 0, kAlibi = (VAR & kVarAlibi) != 0, kDropout = (VAR & kVarDropout) != 0,
                    kFullD = (VAR & kVarFullD) != 0, kStamp = (VAR & kVarStamp) != 0, kKvOnce = (VAR & kVarKvOnce) != 0;
-    using C = FwdCfg<D, NB>;
+    using C = FwdCfg<D, NB, (VAR & kVarNarrow) != 0>;
     Stamps<kStamp> stamps;
     stamps.take(0);
     constexpr int BC = C::BC, KS = C::KS, MB = C::MB, CH = C::CH, SK = C::SK, SV = C::SV, NLD = C::NLD;
@@ -357,21 +359,24 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
     // load_chunk_anyalign): for K they meet zero columns of Q, for V they only reach rows of O^T that are never stored.
     const int row_bytes = kFullD ? D * 2 : d * 2;
     auto chunk_offset = [&](int c) { return kFullD ? c * 16 : (c * 8 + 8 <= d ? c * 16 : (d - 8) * 2); };
-    // (narrow: every block of a tile is the wave's own, and so is the buffer)
-    constexpr int NKX = kNarrow ? C::CK : C::NKX, NVX = kNarrow ? CH : C::NVX;
+    // (narrow: every block of a tile is the wave's own, and so is the buffer; both permutations repeat every 16 rows, which are
+    // CH / 4 blocks, so that only the first CH / 4 requests need offsets of their own and all others are the same some
+    // multiple of 16 rows further on, which goes into the scalar base address: 66 registers less at D = 128)
+    constexpr int NKX = kNarrow ? CH : C::NKX, NVX = kNarrow ? CH : C::NVX;
+    constexpr int NKO = kNarrow ? CH / 4 : NKX, NVO = kNarrow ? CH / 4 : NVX;  // offsets held
     auto block_of = [&](int i) { return kNarrow ? i : wave + 4 * i; };
-    uint32_t koff[NKX], voff[NVX];
-    int krow[NKX], vrow[NVX];
+    uint32_t koff[NKO], voff[NVO];
+    int krow[NKO], vrow[NVO];
     if constexpr (kDma) {
 #pragma unroll
-        for (int i = 0; i < NKX; ++i) {
+        for (int i = 0; i < NKO; ++i) {
             const int q = 64 * block_of(i) + lane;
             krow[i] = q / C::CK;
             const int c = q % C::CK;
             koff[i] = (uint32_t)(krow[i] * row_bytes + chunk_offset((c < CH ? c : CH - 1) ^ C::kswz(krow[i])));
         }
 #pragma unroll
-        for (int i = 0; i < NVX; ++i) {
+        for (int i = 0; i < NVO; ++i) {
             const int q = 64 * block_of(i) + lane;
             vrow[i] = q / CH;
             const int c = q % CH;
@@ -395,21 +400,26 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
             // for the sake of this one)
             int rows_left = Nk - tile * BC;
             if constexpr (kRagged) asm volatile("" : "+s"(rows_left));
+            // request i of a tensor: offset i % n, i / n times 16 rows further on
+            auto request = [&](const char* base, uint32_t off, int row, int further, FA_LDS char* dst) __attribute__((always_inline)) {
+                if constexpr (kRagged) {  // (all of it in the offset, which is unsigned)
+                    row += further;
+                    off += (uint32_t)((further - (row >= rows_left ? row - rows_left + 1 : 0)) * row_bytes);
+                } else {
+                    base += (size_t)further * (size_t)row_bytes;
+                }
+                if constexpr (kKvOnce) dma_kib_nt(base, off, dst);
+                else dma_kib(base, off, dst);
+            };
 #pragma unroll
             for (int i = 0; i < NKX; ++i) {
                 if (!decltype(k_part)::value || (i == NKX - 1 && !k_extra)) break;
-                uint32_t o = koff[i];
-                if (kRagged && krow[i] >= rows_left) o -= (uint32_t)((krow[i] - rows_left + 1) * row_bytes);
-                if constexpr (kKvOnce) dma_kib_nt(Kb, o, kst + block_of(i) * 1024);
-                else dma_kib(Kb, o, kst + block_of(i) * 1024);
+                request(Kb, koff[i % NKO], krow[i % NKO], i / NKO * 16, kst + block_of(i) * 1024);
             }
 #pragma unroll
             for (int i = 0; i < NVX; ++i) {
                 if (!decltype(v_part)::value) break;
-                uint32_t o = voff[i];
-                if (kRagged && vrow[i] >= rows_left) o -= (uint32_t)((vrow[i] - rows_left + 1) * row_bytes);
-                if constexpr (kKvOnce) dma_kib_nt(Vb, o, vst + block_of(i) * 1024);
-                else dma_kib(Vb, o, vst + block_of(i) * 1024);
+                request(Vb, voff[i % NVO], vrow[i % NVO], i / NVO * 16, vst + block_of(i) * 1024);
             }
         };
         if (rows_left >= BC) issue(std::false_type{});
@@ -1098,30 +1108,47 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
 // The instances of a bucket: {d == bucket, d % 8 == 0} x {plain, ALiBi, ALiBi with every visible key at or left of its
 // row, dropout, both}, for rows at any alignment (d % 8 != 0) {plain, ALiBi, dropout, both}, and the one that serves
 // every other request.  ST = kVarStamp selects their instrumented twins (debug time stamps).
-// The narrow instances (kNarrow in fwd_kernel): unsplit launches that would
-// occupy at most half the CUs with work-groups of 128 rows, each of them with 16 key tiles or more ahead of it (8 where
-// they occupy a quarter of the CUs).  Measured against the 128-row instances, same box: B1 H8 N1021 d31 (the reference's
-// own run) 14.2 -> 11.8 us, B1 H8 N1024 d64 15.0 -> 10.2, B1 H8 N2048 d64 causal 27.3 -> 17.8, B1 H1 N2048 d32 causal
-// 22.2 -> 10.5, B1 H4 N4096 d64 50.1 -> 38.0, B1 H8 N1024 d128 20.9 -> 14.3; with 128 work-groups of 8 tiles (B1 H32
-// N512 d64) 10.3 -> 11.8, hence the limit.
+// The narrow instances (kNarrow in fwd_kernel) serve unsplit launches whose time is the chain of key tiles that a work-group
+// walks through, which they cut to a quarter for a fixed cost of 0.5-2 us (a wave's own requests, the merge of four).  Per
+// tile of a wave on its own: 0.5 / 1.0 / 1.3 / 1.6 us at D = 32 / 64 / 96 / 128, against 0.45 / 0.65 / 0.8 / 1.0 us of a
+// 128-row work-group alone on its CU.  Measured against the 128-row instances on 400 random launches of up to 400 of those
+// work-groups; the lines below lie where the ratio of the two crosses one:
+//  * One round -- no more 32-row work-groups than places for them, one per CU by their LDS, two at D = 32: from 4 tiles
+//    on, 5 under a window (B4 H2 N256 d64: 6.0 -> 4.8 us, B1 H4 N640 d128 causal 14.8 -> 10.5, B1 H2 N3264 d128 56 -> 26), from 6 or 10
+//    where rows are shorter than a bucket above 64, whose requests of unaligned pieces a wave cannot hide (B1 H4 N960 d80
+//    16.6 -> 11.0, B2 H4 N960 d100 20.2 -> 16.2; B3 H2 N112 d112, two tiles: 6.8 -> 10.2).
+//  * More rounds only where the later work-groups are the light ones of a causal mask, the longer the sequence the more of
+//    them (B1 H8 N2423 d64, 608 of them: 31.4 -> 22.4 us, but B3 H8 N1344 d64, 1008 of them: 19.2 -> 25.4), or the
+//    chain is so long that two rounds of a quarter are still shorter (B1 H4 N4096 d64 50 -> 38, B2 H4 N4736 d32 69 -> 53).
 inline bool fwd_uses_narrow(const FwdArgs& a, int variant, bool every)
 {
+    (void)variant;
     if (every || a.num_splits != 1 || a.stamps != nullptr || a.kernel_hint != 0) return false;
-    const long long groups = (long long)a.B * a.H * ((a.Nq + 127) / 128);
-    if (2 * groups > kNumCus) return false;
-    // (above d = 64 a wave has one LDS stage and waits for most of every tile request: rows shorter than the bucket,
-    // whose requests take longer, measured slower than the 128-row instances there, and so did launches of more 32-row
-    // work-groups than CUs unless causal -- B2 H2 Nq4096 Nk1024 d128 25.6 against 20.9 us, the same causal shapes 39.5
-    // against 69.0 us)
-    if (a.d > 64 && (a.d % 32 != 0 || (!a.causal && (long long)a.B * a.H * ((a.Nq + 31) / 32) > kNumCus))) return false;
-    const int keys = 4 * groups <= kNumCus ? 512 : 1024;  // visible keys per row that make the chain worth cutting
-    return a.Nk >= keys && (a.wl < 0 || a.wl >= keys - 64);
+    const long long groups = (long long)a.B * a.H * ((a.Nq + 31) / 32);
+    if (groups > 1280) return false;
+    const int bucket = (a.d + 31) / 32;
+    const bool whole = a.d == 32 * bucket;
+    // keys that the rows of a 128-row work-group see, at most
+    const long long left = a.wl >= 0 ? a.wl : a.Nk, right = a.causal ? 0 : a.wr >= 0 ? a.wr : a.Nk;
+    const long long keys = left + right + 128 < a.Nk ? left + right + 128 : a.Nk;
+    const int tiles = (int)((keys + 63) / 64);
+    if (groups <= (bucket == 1 ? 2 * kNumCus : kNumCus)) {
+        if (bucket >= 3 && !whole) return tiles >= (bucket == 3 ? 6 : 10);
+        return tiles >= (groups > kNumCus || keys < a.Nk ? 5 : 4);
+    }
+    if (keys < a.Nk) return false;  // a window: the later work-groups are as heavy as the first
+    if (a.causal && 2 * (long long)(a.fold_rows ? a.fold_rows : a.Nq) >= a.Nk) {
+        if (bucket == 1) return groups <= 576 ? tiles >= 9 : groups <= 800 && tiles >= 16;
+        if (bucket == 4 && !whole) return false;
+        return groups <= 384 ? tiles >= (bucket == 3 && !whole ? 20 : 14) : groups <= 640 && tiles >= 36;
+    }
+    return bucket == 1 ? tiles >= 64 : bucket == 2 && groups <= 512 && tiles >= 24;
 }
 
 template <int D, int VAR>
 inline hipError_t launch_fwd_narrow_instance(const FwdArgs& a, hipStream_t st)
 {
-    using C = FwdCfg<D, 1>;
+    using C = FwdCfg<D, 1, true>;
     auto kern = fwd_kernel<D, 1, VAR | kVarNarrow>;
     static DeviceFlags attr_done;  // per instantiation and device
     constexpr int smem = 4 * (D <= 64 ? 2 : 1) * (C::KBUF + C::VBUF);  // two stages per wave up to D = 64, one above
@@ -1150,23 +1177,26 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
     constexpr int AL = kVarAlibi | kVarAlibiLeft;  // ALiBi with no visible key right of its row
     if constexpr (ST == 0) {
         if (fwd_uses_narrow(a, variant, fwd_needs_every_instance(a, variant))) {
-            // plain: by row length like the others; with ALiBi or dropout: up to d = 64 the instances for rows at any
-            // alignment, which serve every row length from eight elements on, above the ones for rows of the bucket's
-            // width (the only rows that come here)
-            constexpr int F = D <= 64 ? 0 : kVarVec | kVarFullD;
-            if (feat == kVarAlibi) return (int)launch_fwd_narrow_instance<D, F | kVarAlibi>(a, st);
-            if (feat == kVarDropout) return (int)launch_fwd_narrow_instance<D, F | kVarDropout>(a, st);
-            if (feat != 0) return (int)launch_fwd_narrow_instance<D, F | kVarAlibi | kVarDropout>(a, st);
+            // plain: by row length like the others; with ALiBi or dropout: the instances for rows at any alignment, which serve
+            // every row length from eight elements on, and above 64 the ones for rows of the bucket's width
+            auto with_features = [&](auto full_c) {
+                constexpr int F = decltype(full_c)::value ? kVarVec | kVarFullD : 0;
+                if (feat == kVarAlibi) return (int)launch_fwd_narrow_instance<D, F | kVarAlibi>(a, st);
+                if (feat == kVarDropout) return (int)launch_fwd_narrow_instance<D, F | kVarDropout>(a, st);
+                return (int)launch_fwd_narrow_instance<D, F | kVarAlibi | kVarDropout>(a, st);
+            };
+            if constexpr (D > 64) {
+                if (feat != 0 && a.d == D) return with_features(std::true_type{});
+            }
+            if (feat != 0) return with_features(std::false_type{});
             if (a.fold_rows) {
-                if (D > 64 || a.d == D) return (int)launch_fwd_narrow_instance<D, kVarVec | kVarFullD | kVarFold>(a, st);
+                if (a.d == D) return (int)launch_fwd_narrow_instance<D, kVarVec | kVarFullD | kVarFold>(a, st);
                 if (variant & kVarVec) return (int)launch_fwd_narrow_instance<D, kVarVec | kVarFold>(a, st);
                 return (int)launch_fwd_narrow_instance<D, kVarFold>(a, st);
             }
             if (a.d == D) return (int)launch_fwd_narrow_instance<D, kVarVec | kVarFullD>(a, st);
-            if constexpr (D <= 64) {  // (above, only rows of the bucket's width come here)
-                if (!(variant & kVarVec)) return (int)launch_fwd_narrow_instance<D, 0>(a, st);
-                return (int)launch_fwd_narrow_instance<D, kVarVec>(a, st);
-            }
+            if (variant & kVarVec) return (int)launch_fwd_narrow_instance<D, kVarVec>(a, st);
+            return (int)launch_fwd_narrow_instance<D, 0>(a, st);
         }
     }
     if (ST == 0 && a.fold_rows) {

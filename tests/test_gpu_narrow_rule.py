@@ -1,0 +1,41 @@
+"""Launches on both sides of the lines that the rule for the 32-row work-groups draws (fwd_uses_narrow): tile counts, work-group
+counts, windows and row lengths around them, every feature combination in every head-dim bucket, against the oracle."""
+import pytest
+
+from helpers import check_o_lse, oracle_forward_batched, randn_f16_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,H,N,d,kw", [
+    (2, 4, 192, 64, dict()), (2, 4, 193, 64, dict()),                          # 3 | 4 tiles
+    (2, 32, 256, 32, dict(causal=True)), (1, 32, 272, 32, dict()),             # more 32-row groups than CUs: 4 | 5 tiles
+    (2, 3, 300, 64, dict(window=(100, 0))), (2, 3, 300, 64, dict(window=(140, 0))),  # 4 | 5 tiles under a window
+    (1, 4, 320, 80, dict()), (1, 4, 321, 80, dict(causal=True)),               # 5 | 6 tiles, row shorter than its bucket
+    (1, 2, 576, 100, dict()), (1, 2, 577, 100, dict(causal=True)), (1, 2, 577, 112, dict()),  # 9 | 10 tiles
+    (1, 32, 256, 128, dict()), (1, 33, 256, 128, dict()),                      # 256 | 264 groups
+    (1, 12, 832, 64, dict(causal=True)), (1, 12, 833, 96, dict(causal=True)),  # two rounds, causal: 13 | 14 tiles
+    (1, 18, 576, 31, dict(causal=True)),                                       # 324 groups at two per CU, any alignment
+])
+def test_around_the_lines(fa, oracle, B, H, N, d, kw):
+    q, k, v = (randn_f16_gpu((B, H, N, d), s) for s in (1, 2, 3))
+    O, L = oracle_forward_batched(oracle, q, k, v, **kw)
+    check_o_lse(*fa.flash_forward(q, k, v, **kw), O, L, f"{B} {H} {N} {d} {kw}")
+
+
+@pytest.mark.parametrize("d", [31, 40, 64, 72, 96, 99, 112, 128])
+@pytest.mark.parametrize("alibi,p", [(True, 0.0), (False, 0.2), (True, 0.2)])
+def test_features_in_every_bucket(fa, oracle, d, alibi, p):
+    import torch
+
+    B, H, N = 1, 3, 700  # 66 groups of 32 rows, 11 tiles
+    q, k, v = (randn_f16_gpu((B, H, N, d), s) for s in (4, 5, 6))
+    kw, okw = dict(causal=True), dict(causal=True)
+    if alibi:
+        sl = oracle.alibi_slopes(H)
+        kw, okw = dict(kw, alibi_slopes=torch.from_numpy(sl).cuda()), dict(okw, slopes=sl)
+    if p:
+        keep = oracle.dropout_keep_mask(7, 8, p, B, H, N, N)
+        kw, okw = dict(kw, dropout_p=p, seed=7, offset=8), dict(okw, keep_mask=torch.from_numpy(keep), p_drop=p)
+    O, L = oracle_forward_batched(oracle, q, k, v, **okw)
+    check_o_lse(*fa.flash_forward(q, k, v, **kw), O, L, f"d {d} {sorted(kw)}")
