@@ -129,21 +129,22 @@ constexpr float kLazyTau = 8.0f;
 // kVarEvery (with kVarAlibi and kVarDropout, without kVarVec): the instance that serves every request, see kEvery below.
 // kVarNarrow (unsplit launches): the four waves of a work-group share 32 query rows and take every fourth key tile
 // each, see kNarrow below.
+// kVarPair (no other feature): eight waves in two halves that take every other tile each, see kPair below.
 // kVarFold (no other feature): the rows are the query heads of a K/V head, see row_position in common.h.
 constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarStamp = 16, kVarAlibiLeft = 32, kVarKvOnce = 64,
-              kVarEvery = 128, kVarNarrow = 256, kVarFold = 512;
+              kVarEvery = 128, kVarNarrow = 256, kVarFold = 512, kVarPair = 1024;
 
 // work-groups per CU (narrow: one or two by their LDS; held to 256 VGPRs all the same, without which the compiler keeps more
 // than there are and moves them to and from accumulation registers): three up to D = 64 (168 VGPRs), except for the instance that serves every request, which stages
 // its tiles through registers
 constexpr int fwd_groups_per_cu(int D, int NB, int VAR)
 {
-    if ((VAR & kVarNarrow) != 0) return 2;
+    if ((VAR & (kVarNarrow | kVarPair)) != 0) return 2;
     return NB == 1 ? (D <= 64 && (VAR & kVarEvery) == 0 ? 3 : 2) : 1;
 }
 
 template <int D, int NB, int VAR>
-__global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel(const FwdArgs a)
+__global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel(const FwdArgs a)
 {
     constexpr bool kVec = (VAR & kVarVec) != 0, kAlibi = (VAR & kVarAlibi) != 0, kDropout = (VAR & kVarDropout) != 0,
                    kFullD = (VAR & kVarFullD) != 0, kStamp = (VAR & kVarStamp) != 0, kKvOnce = (VAR & kVarKvOnce) != 0;
@@ -173,6 +174,11 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
     static_assert(!kNarrow || (kDma && NB == 1 && !kStamp && !kKvOnce), "narrow instances");
     constexpr bool kFold = (VAR & kVarFold) != 0;
     static_assert(!kFold || (!kAlibi && !kDropout && !kStamp), "folded instances");
+    // A launch of one work-group per CU leaves a SIMD one wave, whose score, softmax and output phases follow one another:
+    // a paired work-group has eight waves.  Waves 0 ... 3 walk the even tiles of the range, waves 4 ... 7, which hold the same
+    // rows and have LDS stages of their own, the odd ones, and the two partial results are merged through LDS at the end.
+    constexpr bool kPair = (VAR & kVarPair) != 0;
+    static_assert(!kPair || (kDma && NB == 1 && !kStamp && !kNarrow), "paired instances");
     // (narrow: two stages per wave up to D = 64, one above: four waves' tiles of 26 / 33 KiB)
     constexpr int NSTG = kNarrow ? (D <= 64 ? 2 : 1) : kDma ? C::NSTG : 2;
     constexpr int BRW = kNarrow ? 32 : C::BR;  // query rows per work-group
@@ -180,10 +186,11 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = wave_uniform(tid >> 6);
-    // tile buffers: of the work-group, or (narrow) of the wave
+    const int wave = wave_uniform(kPair ? (tid >> 6) & 3 : tid >> 6);
+    const int half = kPair ? wave_uniform(tid >> 8) : 0;
+    // tile buffers: of the work-group, or (narrow) of the wave, or (paired) of four waves
     constexpr int kWaveLds = NSTG * (C::KBUF + C::VBUF);
-    const int lds_base = kNarrow ? wave * kWaveLds : 0;
+    const int lds_base = kNarrow ? wave * kWaveLds : kPair ? half * kWaveLds : 0;
     char* const Ks = smem + lds_base;
     char* const Vs = Ks + NSTG * C::KBUF;
     const int l32 = lane & 31;
@@ -213,7 +220,7 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
     const int tile_begin = kmin / BC;
     const int ntiles = kmax > kmin ? (kmax + BC - 1) / BC - tile_begin : 0;
     if (!kStamp && ntiles == 0) {  // (the instrumented twins take the long way and report their stages)
-        store_empty_rows<kFold>(a, bh, split, q0, q0 + BRW < Nq ? q0 + BRW : Nq, tid, 256);
+        store_empty_rows<kFold>(a, bh, split, q0, q0 + BRW < Nq ? q0 + BRW : Nq, tid, kPair ? 512 : 256);
         return;
     }
 
@@ -833,13 +840,15 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
         // grows towards the row, so in rising order the row maximum outgrew kLazyTau, and O was rescaled, in tile after
         // tile.  Causal window of 1650 keys B9 H3 N5649 d72: 112.3 -> 104.4 us, B4 H4 N3392 d128 with 704 keys 32.8 -> 31.0,
         // B2 H16 N4096 d64 with 256 keys (a third of whose heads rescaled per tile) 23.8 -> 23.3.
-        auto nth = [&](int t) { return kFoldAlibi ? ntiles - 1 - t : t; };
+        auto nth = [&](int t) { return kFoldAlibi ? ntiles - 1 - t : kPair ? 2 * t + half : t; };
+        // (paired: both halves go round as often, for the barrier; the second one's last tile may not exist)
+        const int rounds = kPair ? (ntiles + 1) / 2 : ntiles;
         constexpr int PF = NSTG - 1;
         static_assert(PF == 1 || PF == 2, "prefetch distance");
         static_assert(NKX + NVX <= 63, "vmcnt immediate");
 #pragma unroll
         for (int u = 0; u < NSTG; ++u)
-            if (u < ntiles) dma_tile(tile_begin + nth(u), u);
+            if (u < rounds && (!kPair || nth(u) < ntiles)) dma_tile(tile_begin + nth(u), u);
         set_bounds();
         read_slope();
         stamps.take(1);
@@ -849,10 +858,10 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
         __syncthreads();
         stamps.take(3);
         int buf = 0, nbuf = PF % NSTG;  // stages of tile t and of tile t + PF
-        for (int t = 0; t < ntiles; ++t) {
-            const bool more = t + PF < ntiles;
+        for (int t = 0; t < rounds; ++t) {
+            const bool more = kPair ? nth(t + PF) < ntiles : t + PF < ntiles;
             if (more && t > 0) dma_tile(tile_begin + nth(t + PF), nbuf);
-            tile_math(nth(t), buf);
+            if (!kPair || nth(t) < ntiles) tile_math(nth(t), buf);
             if (kStamp && t == 0) stamps.take(4);
             dma_wait(PF == 2 && more);
             __syncthreads();
@@ -948,6 +957,32 @@ __global__ void __launch_bounds__(256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel
                 a.LSE[(size_t)bh * Nq + gi] = L > 0.0f ? __builtin_fmaf(M, kLn2, fast_log2(L) * kLn2) : -INFINITY;
         }
         return;
+    }
+
+    if constexpr (kPair) {
+        // ---------------- merge of the two halves' partial results, register by register, as the merge above
+        // (behind the loop's last barrier; the buffer lies behind the O staging of the epilogue, which other waves may be in)
+        constexpr int kOut = 4 * 32 * (2 * D + 16);
+        static_assert(kOut + 4 * (16 * MB + 2) * 256 <= 2 * kWaveLds, "merge buffer fits the tile buffers");
+        float* const mine = reinterpret_cast<float*>(smem + kOut) + wave * (16 * MB + 2) * 64 + lane;
+        if (half == 1) {
+            mine[0] = m_ref[0];
+            mine[64] = l_run[0];
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) mine[(2 + 16 * mb + r) * 64] = oacc[mb][0][r];
+        }
+        __syncthreads();
+        if (half == 1) return;
+        const float m1 = mine[0], M = fmaxf(m_ref[0], m1), Mu = (M == -INFINITY) ? 0.0f : M;
+        const float w0 = fast_exp2(m_ref[0] - Mu), w1 = fast_exp2(m1 - Mu);
+        m_ref[0] = M;
+        l_run[0] = __builtin_fmaf(w1, mine[64], w0 * l_run[0]);
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) oacc[mb][0][r] = __builtin_fmaf(w1, mine[(2 + 16 * mb + r) * 64], w0 * oacc[mb][0][r]);
     }
 
     // ---------------- epilogue: normalise once, store O (fp16) + LSE, or the fp32 split partials
@@ -1098,16 +1133,17 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
     using C = FwdCfg<D, NB>;
     auto kern = fwd_kernel<D, NB, VAR>;
     static DeviceFlags attr_done;  // per instantiation and device
-    constexpr int smem = C::SMEM_DMA > C::SMEM ? C::SMEM_DMA : C::SMEM;  // (equal: both paths use two stages)
+    constexpr bool kPair = (VAR & kVarPair) != 0;
+    constexpr int smem = (kPair ? 2 : 1) * (C::SMEM_DMA > C::SMEM ? C::SMEM_DMA : C::SMEM);  // (equal: both paths use two stages)
     if (hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), smem, attr_done); e != hipSuccess) return e;
     const long long groups = (long long)a.Tr * a.B * a.H * a.num_splits;
     FwdArgs b = a;
-    constexpr int kResident = (NB == 1 ? fwd_groups_per_cu(D, NB, VAR) : 2) * kNumCus;
+    constexpr int kResident = (kPair ? 1 : NB == 1 ? fwd_groups_per_cu(D, NB, VAR) : 2) * kNumCus;
     set_slice_order(b, a.Tr * a.num_splits, kResident);
     b.split_rotate = split_rotate_for(b.num_splits, b.slice_chunk);
     b.snake_end = snake_end_for(groups, kResident);
     set_divisors(b, b.slice_chunk);
-    return launch_kernel(kern, dim3((unsigned)groups), dim3(256), smem, st, b);
+    return launch_kernel(kern, dim3((unsigned)groups), dim3(kPair ? 512 : 256), smem, st, b);
 }
 
 // The instances of a bucket: {d == bucket, d % 8 == 0} x {plain, ALiBi, ALiBi with every visible key at or left of its
@@ -1168,6 +1204,21 @@ inline hipError_t launch_fwd_narrow_instance(const FwdArgs& a, hipStream_t st)
     return launch_kernel(kern, dim3((unsigned)groups), dim3(256), smem, st, b);
 }
 
+// Paired work-groups (kPair in fwd_kernel): launches of at most one 128-row work-group per CU, whose SIMDs would have one
+// wave each.  Measured against the unpaired instances on 60 random launches (unsplit / split):
+//  * causal, 64-256 work-groups that the narrow instances leave: B2 H4 N1909 d100 36.3 -> 28.8 us, B1 H8 N1664 d100 32.0 ->
+//    25.8, B1 H16 N768 d112 17.1 -> 15.0, B1 H16 N1244 d31 16.6 -> 14.3; split: B1 H64 Nq185 Nk3840 d112 46.8 -> 40.9, B1 H32
+//    Nq128 Nk16384 d128 63.3 -> 60.6 (bound by HBM for half of it).
+//  * eight tiles or more per work-group: with fewer the merge costs what the shorter chain saves.
+//  * up to 32 rows only one wave of four has any, and a second one beside it gained 7-11 % at d = 32, but lost 4 % at
+//    d = 112 (B2 H16 H_kv4 Nq2 Nk16960 18.2 -> 19.0).
+inline bool fwd_uses_pair(const FwdArgs& a, int bucket_d, int feat)
+{
+    if (feat != 0 || a.kernel_hint != 0 || (a.Nq <= 32 && bucket_d > 32)) return false;
+    const long long groups = (long long)a.Tr * a.B * a.H * a.num_splits;
+    return groups <= kNumCus && a.Nk >= 8 * 64 * a.num_splits;
+}
+
 // requests that only the instance which serves every request takes (kEvery in fwd_kernel)
 inline bool fwd_needs_every_instance(const FwdArgs& a, int variant)
 {
@@ -1204,11 +1255,19 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
             return (int)launch_fwd_narrow_instance<D, 0>(a, st);
         }
     }
+    const bool pair = ST == 0 && fwd_uses_pair(a, D, feat);
+    auto plain = [&](auto var) {
+        constexpr int V = decltype(var)::value;
+        if constexpr (ST == 0) {
+            if (pair) return launch_fwd_instance<D, NB, V | kVarPair>(a, st);
+        }
+        return launch_fwd_instance<D, NB, V>(a, st);
+    };
     if (ST == 0 && a.fold_rows) {
         constexpr int F = ST == 0 ? kVarFold : 0;
-        if (a.d == D) return (int)launch_fwd_instance<D, NB, (ST == 0 ? F | kVarVec | kVarFullD | kVarKvOnce : 0)>(a, st);
-        if (variant & kVarVec) return (int)launch_fwd_instance<D, NB, (ST == 0 ? F | kVarVec : 0)>(a, st);
-        return (int)launch_fwd_instance<D, NB, F>(a, st);
+        if (a.d == D) return (int)plain(std::integral_constant<int, (ST == 0 ? F | kVarVec | kVarFullD | kVarKvOnce : 0)>{});
+        if (variant & kVarVec) return (int)plain(std::integral_constant<int, (ST == 0 ? F | kVarVec : 0)>{});
+        return (int)plain(std::integral_constant<int, F>{});
     }
     if (!(variant & kVarVec)) {
         // rows at any alignment: plain, ALiBi, dropout, both, and one more with both features compiled in (slope 0 /
@@ -1216,20 +1275,20 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
         // scores are scaled ahead of the row maximum), the score dump, rows of fewer than eight elements, a dropout
         // threshold of 0
         if (fwd_needs_every_instance(a, variant)) e = launch_fwd_instance<D, NB, ST | kVarAlibi | kVarDropout | kVarEvery>(a, st);
-        else if (feat == 0) e = launch_fwd_instance<D, NB, ST>(a, st);
+        else if (feat == 0) e = plain(std::integral_constant<int, ST>{});
         else if (feat == kVarAlibi) e = launch_fwd_instance<D, NB, ST | kVarAlibi>(a, st);
         else if (feat == kVarDropout) e = launch_fwd_instance<D, NB, ST | kVarDropout>(a, st);
         else e = launch_fwd_instance<D, NB, ST | kVarAlibi | kVarDropout>(a, st);
     } else if (a.d == D) {
         constexpr int V = ST | kVarVec | kVarFullD;
         const bool kv_once = ST == 0 && a.Tr == 1 && a.kv_group == 1;
-        if (feat == 0) e = kv_once ? launch_fwd_instance<D, NB, V | (ST == 0 ? kVarKvOnce : 0)>(a, st) : launch_fwd_instance<D, NB, V>(a, st);
+        if (feat == 0) e = kv_once ? plain(std::integral_constant<int, V | (ST == 0 ? kVarKvOnce : 0)>{}) : plain(std::integral_constant<int, V>{});
         else if (feat == kVarAlibi) e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi>(a, st);
         else if (feat == kVarDropout) e = launch_fwd_instance<D, NB, V | kVarDropout>(a, st);
         else e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL | kVarDropout>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi | kVarDropout>(a, st);
     } else {
         constexpr int V = ST | kVarVec;
-        if (feat == 0) e = launch_fwd_instance<D, NB, V>(a, st);
+        if (feat == 0) e = plain(std::integral_constant<int, V>{});
         else if (feat == kVarAlibi) e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi>(a, st);
         else if (feat == kVarDropout) e = launch_fwd_instance<D, NB, V | kVarDropout>(a, st);
         else e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL | kVarDropout>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi | kVarDropout>(a, st);

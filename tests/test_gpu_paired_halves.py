@@ -1,0 +1,28 @@
+"""Paired work-groups: eight waves in two halves that take every other key tile.  Row counts at the edges of a wave and of a
+work-group, odd and even tile counts (a window leaves one to four), whole and split, every row alignment and folded
+heads, against the oracle."""
+import pytest
+
+from helpers import check_o_lse, oracle_forward_batched, randn_f16_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("Nq,G,d", [(33, 1, 128), (128, 1, 64), (129, 1, 96), (200, 1, 31), (140, 1, 100), (135, 1, 80),
+                                    (20, 2, 128), (30, 4, 72), (64, 2, 40), (5, 1, 32)])
+@pytest.mark.parametrize("kw", [dict(), dict(causal=True), dict(causal=True, window=(40, -1)), dict(window=(90, 30))])
+def test_paired_halves(fa, oracle, Nq, G, d, kw):
+    B, Hk, Nk = 1, 2, 1740
+    q, k, v = randn_f16_gpu((B, Hk * G, Nq, d), 1), randn_f16_gpu((B, Hk, Nk, d), 2), randn_f16_gpu((B, Hk, Nk, d), 3)
+    kr, vr = (t.repeat_interleave(G, dim=1).contiguous() for t in (k, v))
+    O, L = oracle_forward_batched(oracle, q, kr, vr, **kw)
+    for S in (2, 3):
+        check_o_lse(*fa.flash_forward_splitkv(q, k, v, num_splits=S, **kw), O, L, f"split {S}")
+
+
+@pytest.mark.parametrize("B,H,N,d", [(1, 8, 1664, 100), (2, 4, 1311, 112), (1, 16, 1244, 31), (1, 11, 1090, 64)])
+def test_paired_halves_unsplit(fa, oracle, B, H, N, d):
+    """Unsplit causal launches of 64 to 256 work-groups, too many rows for the narrow instances."""
+    q, k, v = (randn_f16_gpu((B, H, N, d), s) for s in (4, 5, 6))
+    O, L = oracle_forward_batched(oracle, q, k, v, causal=True)
+    check_o_lse(*fa.flash_forward(q, k, v, causal=True), O, L, "unsplit")
