@@ -66,7 +66,8 @@ struct FwdCfg {
     static constexpr bool VSWZ = (D * 2) % 128 == 0;
     static constexpr int KBUF = BC * SK;
     static constexpr int VBUF = BC * SV;
-    static constexpr int SMEM = 2 * KBUF + 2 * VBUF;
+    static constexpr int kTiles = 2 * KBUF + 2 * VBUF, kOut = 4 * NB * 32 * (2 * D + 16);
+    static constexpr int SMEM = kTiles > kOut ? kTiles : kOut;
     static constexpr int NSTG = 2;
     static constexpr int SMEM_DMA = NSTG * (KBUF + VBUF);
     static constexpr int NKX = (CK + 3) / 4;      // 1 KiB blocks of a K tile (CK of them) per wave, rounded up
@@ -140,7 +141,7 @@ constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarSt
 constexpr int fwd_groups_per_cu(int D, int NB, int VAR)
 {
     if ((VAR & (kVarNarrow | kVarPair)) != 0) return 2;
-    return NB == 1 ? (D <= 64 && (VAR & kVarEvery) == 0 ? 3 : 2) : 1;
+    return NB == 1 && D <= 64 && (VAR & kVarEvery) == 0 ? 3 : 2;
 }
 
 template <int D, int NB, int VAR>
@@ -1219,6 +1220,19 @@ inline bool fwd_uses_pair(const FwdArgs& a, int bucket_d, int feat)
     return groups <= kNumCus && a.Nk >= 8 * 64 * a.num_splits;
 }
 
+// 64 query rows per wave at d = 64 (NB = 2, 202 VGPRs, two work-groups of 256 rows per CU): a K or V fragment read from LDS
+// feeds two MFMAs.  Only without a mask -- causal it measured -9 %, with a window of 256 keys -21 %: wider diagonals -- and
+// where 256-row blocks add no more than 4 % of empty rows to what 128-row blocks have (B32 H32 N384 52.8 -> 60.3 us, N300
+// -7 %, N640 +-0) and no more than an eighth of the rows is empty (B32 H64 N140 -6 %, N200 +-0), from two rounds of
+// work-groups on.  B32 H32 N512 107.1 -> 99.8 us (688 TFLOP/s), B16 H16 N1024 96.1 -> 87.2,
+// B8 H32 N2048 333.6 -> 313.3, B2 H16 N8192 607 -> 577 (953 TFLOP/s), B31 H64 H_kv8 N705 361 -> 356 us; same bits.
+inline bool fwd_uses_tall(const FwdArgs& a, int feat)
+{
+    if (feat != 0 || a.num_splits != 1 || a.fold_rows || a.causal || a.wl >= 0 || a.wr >= 0 || a.kernel_hint != 0) return false;
+    const long long blocks = (a.Nq + 255) / 256, added = 2 * blocks - (a.Nq + 127) / 128;  // in blocks of 128 rows
+    return (long long)a.B * a.H * blocks >= 4 * kNumCus && 25 * added <= 2 * blocks && 8 * (256 * blocks - a.Nq) <= 256 * blocks;
+}
+
 // requests that only the instance which serves every request takes (kEvery in fwd_kernel)
 inline bool fwd_needs_every_instance(const FwdArgs& a, int variant)
 {
@@ -1281,6 +1295,13 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
         else e = launch_fwd_instance<D, NB, ST | kVarAlibi | kVarDropout>(a, st);
     } else if (a.d == D) {
         constexpr int V = ST | kVarVec | kVarFullD;
+        if constexpr (D == 64 && ST == 0) {
+            if (fwd_uses_tall(a, feat)) {
+                FwdArgs b = a;
+                b.Tr = (a.Nq + 255) / 256;
+                return (int)launch_fwd_instance<D, 2, V>(b, st);
+            }
+        }
         const bool kv_once = ST == 0 && a.Tr == 1 && a.kv_group == 1;
         if (feat == 0) e = kv_once ? plain(std::integral_constant<int, V | (ST == 0 ? kVarKvOnce : 0)>{}) : plain(std::integral_constant<int, V>{});
         else if (feat == kVarAlibi) e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi>(a, st);

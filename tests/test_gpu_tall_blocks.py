@@ -1,0 +1,20 @@
+"""Unmasked d = 64 launches of many heads take 256-row work-groups: bit for bit the results of the 128-row ones (which
+kernel_hint = 1 asks for), whole and ragged row counts, key counts that differ, grouped heads; and the oracle on a head."""
+import pytest
+
+from helpers import check_o_lse, randn_f16_gpu, to_f32_np
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,H,Hk,Nq,Nk", [(32, 32, 32, 256, 256), (32, 32, 8, 225, 225), (16, 32, 32, 512, 64),
+                                          (16, 32, 32, 385, 130), (3, 28, 28, 3329, 65)])
+def test_tall_blocks(fa, oracle, B, H, Hk, Nq, Nk):
+    import torch
+
+    q, k, v = randn_f16_gpu((B, H, Nq, 64), 1), randn_f16_gpu((B, Hk, Nk, 64), 2), randn_f16_gpu((B, Hk, Nk, 64), 3)
+    o, lse = fa.flash_forward(q, k, v)
+    o4, lse4 = fa.flash_forward(q, k, v, kernel_hint=1)
+    assert torch.equal(o, o4) and torch.equal(lse, lse4)
+    O, L = oracle.attention_forward(*(to_f32_np(t[-1:, -1:]) for t in (q, k, v)))
+    check_o_lse(o[-1:, -1:], lse[-1:, -1:], O, L, "last head")
