@@ -130,7 +130,7 @@ constexpr float kLazyTau = 8.0f;
 // kVarEvery (with kVarAlibi and kVarDropout, without kVarVec): the instance that serves every request, see kEvery below.
 // kVarNarrow (unsplit launches): the four waves of a work-group share 32 query rows and take every fourth key tile
 // each, see kNarrow below.
-// kVarPair (no other feature): eight waves in two halves that take every other tile each, see kPair below.
+// kVarPair (without ALiBi): eight waves in two halves that take every other tile each, see kPair below.
 // kVarFold (no other feature): the rows are the query heads of a K/V head, see row_position in common.h.
 constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarStamp = 16, kVarAlibiLeft = 32, kVarKvOnce = 64,
               kVarEvery = 128, kVarNarrow = 256, kVarFold = 512, kVarPair = 1024;
@@ -1210,12 +1210,14 @@ inline hipError_t launch_fwd_narrow_instance(const FwdArgs& a, hipStream_t st)
 //  * causal, 64-256 work-groups that the narrow instances leave: B2 H4 N1909 d100 36.3 -> 28.8 us, B1 H8 N1664 d100 32.0 ->
 //    25.8, B1 H16 N768 d112 17.1 -> 15.0, B1 H16 N1244 d31 16.6 -> 14.3; split: B1 H64 Nq185 Nk3840 d112 46.8 -> 40.9, B1 H32
 //    Nq128 Nk16384 d128 63.3 -> 60.6 (bound by HBM for half of it).
+//  * causal with dropout: B2 H2 N2112 d100 59.9 -> 46.2 us, B2 H4 N1986 d96 50.1 -> 38.9, B1 H8 N3061 d64 65.2 -> 52.6, B4 H8
+//    N683 d128 22.7 -> 20.1.
 //  * eight tiles or more per work-group: with fewer the merge costs what the shorter chain saves.
 //  * up to 32 rows only one wave of four has any, and a second one beside it gained 7-11 % at d = 32, but lost 4 % at
 //    d = 112 (B2 H16 H_kv4 Nq2 Nk16960 18.2 -> 19.0).
 inline bool fwd_uses_pair(const FwdArgs& a, int bucket_d, int feat)
 {
-    if (feat != 0 || a.kernel_hint != 0 || (a.Nq <= 32 && bucket_d > 32)) return false;
+    if ((feat & kVarAlibi) != 0 || a.kernel_hint != 0 || (a.Nq <= 32 && bucket_d > 32)) return false;
     const long long groups = (long long)a.Tr * a.B * a.H * a.num_splits;
     return groups <= kNumCus && a.Nk >= 8 * 64 * a.num_splits;
 }
@@ -1270,7 +1272,7 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
         }
     }
     const bool pair = ST == 0 && fwd_uses_pair(a, D, feat);
-    auto plain = [&](auto var) {
+    auto halves = [&](auto var) {
         constexpr int V = decltype(var)::value;
         if constexpr (ST == 0) {
             if (pair) return launch_fwd_instance<D, NB, V | kVarPair>(a, st);
@@ -1279,9 +1281,9 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
     };
     if (ST == 0 && a.fold_rows) {
         constexpr int F = ST == 0 ? kVarFold : 0;
-        if (a.d == D) return (int)plain(std::integral_constant<int, (ST == 0 ? F | kVarVec | kVarFullD | kVarKvOnce : 0)>{});
-        if (variant & kVarVec) return (int)plain(std::integral_constant<int, (ST == 0 ? F | kVarVec : 0)>{});
-        return (int)plain(std::integral_constant<int, F>{});
+        if (a.d == D) return (int)halves(std::integral_constant<int, (ST == 0 ? F | kVarVec | kVarFullD | kVarKvOnce : 0)>{});
+        if (variant & kVarVec) return (int)halves(std::integral_constant<int, (ST == 0 ? F | kVarVec : 0)>{});
+        return (int)halves(std::integral_constant<int, F>{});
     }
     if (!(variant & kVarVec)) {
         // rows at any alignment: plain, ALiBi, dropout, both, and one more with both features compiled in (slope 0 /
@@ -1289,9 +1291,9 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
         // scores are scaled ahead of the row maximum), the score dump, rows of fewer than eight elements, a dropout
         // threshold of 0
         if (fwd_needs_every_instance(a, variant)) e = launch_fwd_instance<D, NB, ST | kVarAlibi | kVarDropout | kVarEvery>(a, st);
-        else if (feat == 0) e = plain(std::integral_constant<int, ST>{});
+        else if (feat == 0) e = halves(std::integral_constant<int, ST>{});
         else if (feat == kVarAlibi) e = launch_fwd_instance<D, NB, ST | kVarAlibi>(a, st);
-        else if (feat == kVarDropout) e = launch_fwd_instance<D, NB, ST | kVarDropout>(a, st);
+        else if (feat == kVarDropout) e = halves(std::integral_constant<int, ST | kVarDropout>{});
         else e = launch_fwd_instance<D, NB, ST | kVarAlibi | kVarDropout>(a, st);
     } else if (a.d == D) {
         constexpr int V = ST | kVarVec | kVarFullD;
@@ -1303,15 +1305,15 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
             }
         }
         const bool kv_once = ST == 0 && a.Tr == 1 && a.kv_group == 1;
-        if (feat == 0) e = kv_once ? plain(std::integral_constant<int, V | (ST == 0 ? kVarKvOnce : 0)>{}) : plain(std::integral_constant<int, V>{});
+        if (feat == 0) e = kv_once ? halves(std::integral_constant<int, V | (ST == 0 ? kVarKvOnce : 0)>{}) : halves(std::integral_constant<int, V>{});
         else if (feat == kVarAlibi) e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi>(a, st);
-        else if (feat == kVarDropout) e = launch_fwd_instance<D, NB, V | kVarDropout>(a, st);
+        else if (feat == kVarDropout) e = halves(std::integral_constant<int, V | kVarDropout>{});
         else e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL | kVarDropout>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi | kVarDropout>(a, st);
     } else {
         constexpr int V = ST | kVarVec;
-        if (feat == 0) e = plain(std::integral_constant<int, V>{});
+        if (feat == 0) e = halves(std::integral_constant<int, V>{});
         else if (feat == kVarAlibi) e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi>(a, st);
-        else if (feat == kVarDropout) e = launch_fwd_instance<D, NB, V | kVarDropout>(a, st);
+        else if (feat == kVarDropout) e = halves(std::integral_constant<int, V | kVarDropout>{});
         else e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL | kVarDropout>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi | kVarDropout>(a, st);
     }
     return (int)e;

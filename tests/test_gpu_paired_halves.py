@@ -26,3 +26,14 @@ def test_paired_halves_unsplit(fa, oracle, B, H, N, d):
     q, k, v = (randn_f16_gpu((B, H, N, d), s) for s in (4, 5, 6))
     O, L = oracle_forward_batched(oracle, q, k, v, causal=True)
     check_o_lse(*fa.flash_forward(q, k, v, causal=True), O, L, "unsplit")
+
+
+@pytest.mark.parametrize("Nq,d", [(33, 128), (129, 96), (140, 100), (200, 31), (128, 64)])
+def test_paired_halves_dropout(fa, oracle, Nq, d):
+    import torch
+
+    B, H, Nk, p = 1, 2, 1740, 0.2
+    q, k, v = randn_f16_gpu((B, H, Nq, d), 1), randn_f16_gpu((B, H, Nk, d), 2), randn_f16_gpu((B, H, Nk, d), 3)
+    keep = torch.from_numpy(oracle.dropout_keep_mask(9, 0, p, B, H, Nq, Nk))
+    O, L = oracle_forward_batched(oracle, q, k, v, causal=True, keep_mask=keep, p_drop=p)
+    check_o_lse(*fa.flash_forward_splitkv(q, k, v, num_splits=3, causal=True, dropout_p=p, seed=9), O, L, "dropout")
