@@ -1212,14 +1212,16 @@ inline hipError_t launch_fwd_narrow_instance(const FwdArgs& a, hipStream_t st)
 //    Nq128 Nk16384 d128 63.3 -> 60.6 (bound by HBM for half of it).
 //  * causal with dropout: B2 H2 N2112 d100 59.9 -> 46.2 us, B2 H4 N1986 d96 50.1 -> 38.9, B1 H8 N3061 d64 65.2 -> 52.6, B4 H8
 //    N683 d128 22.7 -> 20.1.
-//  * eight tiles or more per work-group: with fewer the merge costs what the shorter chain saves.
+//  * eight tiles or more per work-group, a window's included: with fewer the merge costs what the shorter chain saves.
+//    (Window of 500 keys B1 H16 N1500 d64 12.7 -> 10.7 us, of 1000 B2 H4 N2500 d96 21.5 -> 18.0.)
 //  * up to 32 rows only one wave of four has any, and a second one beside it gained 7-11 % at d = 32, but lost 4 % at
 //    d = 112 (B2 H16 H_kv4 Nq2 Nk16960 18.2 -> 19.0).
 inline bool fwd_uses_pair(const FwdArgs& a, int bucket_d, int feat)
 {
     if ((feat & kVarAlibi) != 0 || a.kernel_hint != 0 || (a.Nq <= 32 && bucket_d > 32)) return false;
     const long long groups = (long long)a.Tr * a.B * a.H * a.num_splits;
-    return groups <= kNumCus && a.Nk >= 8 * 64 * a.num_splits;
+    const long long left = a.wl >= 0 ? a.wl : a.Nk, right = a.causal ? 0 : a.wr >= 0 ? a.wr : a.Nk;
+    return groups <= kNumCus && a.Nk >= 8 * 64 * a.num_splits && left + right + 128 >= 8 * 64;
 }
 
 // 64 query rows per wave at d = 64 (NB = 2, 202 VGPRs, two work-groups of 256 rows per CU): a K or V fragment read from LDS
