@@ -240,6 +240,7 @@ def flash_forward_splitkv(q, k, v, num_splits=0, softmax_scale=None, causal=Fals
     S = lib().flash_splitkv_resolve_splits(C.byref(p))
     if S < 0:
         raise FlashError(S, "flash_splitkv_resolve_splits")
+    p.num_splits = S  # (the launch and the stamp buffer go by the count that the workspace is sized for)
     rows = B * H * S * Nq if S > 1 else 0
     if workspace is None and rows:
         workspace = (torch.empty(rows * d, dtype=torch.float32, device=q.device),

@@ -199,7 +199,8 @@ void fold_heads(fa::FwdArgs* a);
 
 // The estimate walks the row blocks once per candidate count (up to 0.26 ms on a causal sequence of 65536 rows), and
 // callers in a loop ask for the same few shapes again and again: each thread remembers the answers to its last four
-// distinct requests.  Everything the estimate reads is part of the key.
+// distinct requests.  Everything the estimate reads is part of the key.  The stage-stamp pointer is not among it: callers
+// size the workspace before they set it, and both times the count has to be the same.
 int auto_splits_tiled(const flash_params* p, int n_blocks, bool decode = false)
 {
     struct Key {
@@ -215,8 +216,7 @@ int auto_splits_tiled(const flash_params* p, int n_blocks, bool decode = false)
     static thread_local int next = 0;
     const Key key = {p->B, p->H, p->H_kv, p->Nq, p->Nk, p->d, p->is_causal, window_left_of(p), window_right_of(p), p->kernel_hint,
                      tiled_variant(p) | (p->softmax_scale > 0.0f ? 8 : 0) | (p->scores_out ? 16 : 0) | (decode ? 32 : 0) |
-                         (p->dropout_p > 0.0f && flash_dropout_threshold(p->dropout_p) == 0 ? 64 : 0) |
-                         (p->stage_stamps_out ? 128 : 0)};
+                         (p->dropout_p > 0.0f && flash_dropout_threshold(p->dropout_p) == 0 ? 64 : 0)};
     for (const Entry& e : memo)
         if (e.valid && e.key == key) return e.splits;
     const int splits = auto_splits_tiled_uncached(p, n_blocks, decode);
@@ -263,6 +263,7 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
     if (!pp) {
         fa::FwdArgs unsplit;
         fill_args(p, 1, &unsplit);
+        unsplit.stamps = nullptr;
         if (fold) fold_heads(&unsplit);
         narrow = fa::fwd_uses_narrow(unsplit, tiled_variant(p), every);
     }
@@ -434,7 +435,7 @@ bool folds_heads(const flash_params* p)
 {
     const int hk = p->H_kv > 0 ? p->H_kv : p->H;
     return p->Nq > 1 && p->Nq <= kFoldRows && hk < p->H && !p->alibi_slopes && p->dropout_p == 0.0f &&
-           !p->stage_stamps_out && !needs_every_instance(p) && p->kernel_hint == 0;
+           !needs_every_instance(p) && p->kernel_hint == 0;
 }
 void fold_heads(fa::FwdArgs* a)
 {
@@ -468,7 +469,7 @@ int splitkv_route(const flash_params* p, fa::FwdArgs* a)
     }
     // one query row per head, rows of eight elements or more, no dropout: bandwidth-bound streaming kernel
     if (p->Nq == 1 && p->d >= 8 && p->dropout_p == 0.0f && p->softmax_scale > 0.0f) return kRouteStream;
-    if (folds_heads(p)) fold_heads(a);
+    if (folds_heads(p) && !p->stage_stamps_out) fold_heads(a);
     return kRouteTiled;
 }
 
@@ -511,7 +512,7 @@ FLASH_EXPORT int flash_forward(const flash_params* p, void* stream)
     if ((rc = device_usable()) != FLASH_OK) return rc;
     fa::FwdArgs a;
     fill_args(p, 1, &a);
-    if (folds_heads(p)) fold_heads(&a);
+    if (folds_heads(p) && !p->stage_stamps_out) fold_heads(&a);
     return launch_tiled(p, a, static_cast<hipStream_t>(stream));
 }
 

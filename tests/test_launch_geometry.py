@@ -1,0 +1,52 @@
+"""What the library launches against the buffers it told the caller to bring, without a GPU (tests/launch_recorder.py)."""
+import numpy as np
+
+from launch_recorder import record
+
+STAMPS = 0x900000  # a stage-stamp buffer
+
+
+def random_calls(seed, n, **fixed):
+    """Calls of both entry points over every head-dim bucket, mask, feature and kernel hint, few and many rows, grouped heads."""
+    rng = np.random.default_rng(seed)
+    calls = []
+    while len(calls) < n:
+        Hk = int(rng.choice([1, 2, 4, 8]))
+        B, H = int(rng.integers(1, 30)), Hk * int(rng.choice([1, 1, 2, 3, 4, 8]))
+        Nq = int(rng.choice([int(rng.integers(2, 70)), int(rng.integers(1, 600)), int(rng.integers(100, 5000))]))
+        Nk = Nq if rng.random() < 0.3 else int(round(2 ** rng.uniform(4, 15)))
+        c = dict(entry=str(rng.choice(["forward", "splitkv"])), B=B, H=H, H_kv=Hk, Nq=Nq, Nk=Nk,
+                 d=int(rng.choice([7, 31, 32, 40, 64, 64, 72, 96, 100, 128, 128])), is_causal=int(rng.integers(0, 2)),
+                 num_splits=int(rng.choice([0, 0, 1, 4, 17])))
+        if rng.random() < 0.3:
+            c.update(window_left=int(rng.integers(0, 2000)), window_right=int(rng.choice([-1, 0, 100])))
+        if rng.random() < 0.2:
+            c.update(alibi_slopes=0xA00000)
+        if rng.random() < 0.2:
+            c.update(dropout_p=float(rng.choice([0.1, 1e-6])), seed=3)
+        if rng.random() < 0.2:
+            c.update(kernel_hint=int(rng.integers(1, 3)))
+        if rng.random() < 0.05:
+            c.update(softmax_scale=-0.1)
+        c.update(fixed)
+        calls.append(c)
+    return calls
+
+
+def split_rows(c, r):
+    """Rows of partial results that the launches write, over the split count that the combine step was given."""
+    S = max(launch["split_count"] for launch in r["launches"])
+    return c["B"] * c["H"] * c["Nq"] * S if S > 1 else 0
+
+
+def test_workspace_does_not_depend_on_the_stage_stamps():
+    """The workspace is sized before the stamp buffer is there, and the launch that sees the buffer needs no more of it."""
+    calls = random_calls(1, 1500, entry="splitkv", num_splits=0, stage_stamps_out=STAMPS)
+    calls.append(dict(entry="splitkv", B=14, H=64, H_kv=8, Nq=36, Nk=27335, d=128, num_splits=0, stage_stamps_out=STAMPS))
+    split = 0
+    for c, r in zip(calls, record(calls)):
+        assert r["rc"] == 0, c
+        rows = split_rows(c, r)
+        split += rows > 0
+        assert r["workspace"] == [rows * c["d"] * 4, rows * 4], c
+    assert split > 150  # (the sample is of the kind that it is about)
