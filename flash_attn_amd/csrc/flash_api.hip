@@ -555,10 +555,14 @@ FLASH_EXPORT int flash_stage_stamps_bytes(const flash_params* p, int split, size
     bool empty;
     const int rc = validate_shape(p, &empty);
     if (rc != FLASH_OK || empty) return rc;
+    // the route of the call that will carry the buffer, which the caller does not have yet
+    flash_params with = *p;
+    uint64_t any;
+    with.stage_stamps_out = &any;
     fa::FwdArgs a;
-    fill_args(p, split ? resolve_splits(p) : 1, &a);
-    if ((split || p->Nq == 1) && splitkv_route(p, &a) == kRouteStream) return FLASH_OK;  // (flash_forward routes Nq == 1 too)
-    *bytes = (size_t)tiled_groups(p, a) * FLASH_STAMP_WORDS * sizeof(uint64_t);
+    fill_args(&with, split ? resolve_splits(&with) : 1, &a);
+    if ((split || p->Nq == 1) && splitkv_route(&with, &a) == kRouteStream) return FLASH_OK;  // (flash_forward routes Nq == 1 too)
+    *bytes = (size_t)tiled_groups(&with, a) * FLASH_STAMP_WORDS * sizeof(uint64_t);
     return FLASH_OK;
 }
 

@@ -50,3 +50,15 @@ def test_workspace_does_not_depend_on_the_stage_stamps():
         split += rows > 0
         assert r["workspace"] == [rows * c["d"] * 4, rows * 4], c
     assert split > 150  # (the sample is of the kind that it is about)
+
+
+def test_stage_stamp_buffer_holds_every_work_group():
+    """FLASH_STAMP_WORDS words for each work-group of the tiled launch, whichever entry point and route: heads folded into the
+    rows of one problem among them."""
+    calls = random_calls(2, 3000, stage_stamps_out=STAMPS)
+    calls.append(dict(entry="splitkv", B=4, H=32, H_kv=8, Nq=16, Nk=8192, d=128, num_splits=8, stage_stamps_out=STAMPS))
+    for c, r in zip(calls, record(calls)):
+        assert r["rc"] == 0, c
+        first = r["launches"][0]
+        groups = first["groups"] if first["variant"] is not None else 0  # (the decode stream is not stamped)
+        assert r["stamp_bytes"] == groups * 9 * 8, (c, r)
