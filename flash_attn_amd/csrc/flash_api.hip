@@ -169,9 +169,7 @@ int launch_tiled(const flash_params* p, const fa::FwdArgs& a, hipStream_t st)
 // work-groups of the tiled launch for the (final) arguments a
 long long tiled_groups(const flash_params* p, const fa::FwdArgs& a)
 {
-    const bool pp = a.d > 96 && !a.fold_rows && fa::fwd_uses_pingpong(a.d, !needs_every_instance(p), a.Nq, a.Nk, a.causal, a.wl, a.wr,
-                                                      (long long)a.B * a.H * a.num_splits, a.kernel_hint);
-    const int rows = pp ? 256 : kRowsPerGroup;
+    const int rows = fa::fwd_rows_per_group(a, tiled_variant(p));
     return (long long)((a.Nq + rows - 1) / rows) * a.B * a.H * a.num_splits;
 }
 
@@ -263,9 +261,8 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
     if (!pp) {
         fa::FwdArgs unsplit;
         fill_args(p, 1, &unsplit);
-        unsplit.stamps = nullptr;
         if (fold) fold_heads(&unsplit);
-        narrow = fa::fwd_uses_narrow(unsplit, tiled_variant(p), every);
+        narrow = fa::fwd_uses_narrow(unsplit, every);
     }
     int limit = FLASH_MAX_SPLITS;
     if (n_blocks < limit) limit = n_blocks;
@@ -469,7 +466,7 @@ int splitkv_route(const flash_params* p, fa::FwdArgs* a)
     }
     // one query row per head, rows of eight elements or more, no dropout: bandwidth-bound streaming kernel
     if (p->Nq == 1 && p->d >= 8 && p->dropout_p == 0.0f && p->softmax_scale > 0.0f) return kRouteStream;
-    if (folds_heads(p) && !p->stage_stamps_out) fold_heads(a);
+    if (folds_heads(p)) fold_heads(a);
     return kRouteTiled;
 }
 
@@ -512,7 +509,7 @@ FLASH_EXPORT int flash_forward(const flash_params* p, void* stream)
     if ((rc = device_usable()) != FLASH_OK) return rc;
     fa::FwdArgs a;
     fill_args(p, 1, &a);
-    if (folds_heads(p) && !p->stage_stamps_out) fold_heads(&a);
+    if (folds_heads(p)) fold_heads(&a);
     return launch_tiled(p, a, static_cast<hipStream_t>(stream));
 }
 
@@ -555,14 +552,14 @@ FLASH_EXPORT int flash_stage_stamps_bytes(const flash_params* p, int split, size
     bool empty;
     const int rc = validate_shape(p, &empty);
     if (rc != FLASH_OK || empty) return rc;
-    // the route of the call that will carry the buffer, which the caller does not have yet
-    flash_params with = *p;
-    uint64_t any;
-    with.stage_stamps_out = &any;
     fa::FwdArgs a;
-    fill_args(&with, split ? resolve_splits(&with) : 1, &a);
-    if ((split || p->Nq == 1) && splitkv_route(&with, &a) == kRouteStream) return FLASH_OK;  // (flash_forward routes Nq == 1 too)
-    *bytes = (size_t)tiled_groups(&with, a) * FLASH_STAMP_WORDS * sizeof(uint64_t);
+    fill_args(p, split ? resolve_splits(p) : 1, &a);
+    if (split || p->Nq == 1) {  // (flash_forward routes Nq == 1 too)
+        if (splitkv_route(p, &a) == kRouteStream) return FLASH_OK;
+    } else if (folds_heads(p)) {
+        fold_heads(&a);
+    }
+    *bytes = (size_t)tiled_groups(p, a) * FLASH_STAMP_WORDS * sizeof(uint64_t);
     return FLASH_OK;
 }
 

@@ -172,14 +172,14 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // for its own requests only), and the four partial results are merged through LDS at the end like the partial results
     // of a split -- in the same launch, where a split count of four would need the combine launch behind it.
     constexpr bool kNarrow = (VAR & kVarNarrow) != 0;
-    static_assert(!kNarrow || (kDma && NB == 1 && !kStamp && !kKvOnce), "narrow instances");
+    static_assert(!kNarrow || (kDma && NB == 1 && !kKvOnce), "narrow instances");
     constexpr bool kFold = (VAR & kVarFold) != 0;
-    static_assert(!kFold || (!kAlibi && !kDropout && !kStamp), "folded instances");
+    static_assert(!kFold || (!kAlibi && !kDropout), "folded instances");
     // A launch of one work-group per CU leaves a SIMD one wave, whose score, softmax and output phases follow one another:
     // a paired work-group has eight waves.  Waves 0 ... 3 walk the even tiles of the range, waves 4 ... 7, which hold the same
     // rows and have LDS stages of their own, the odd ones, and the two partial results are merged through LDS at the end.
     constexpr bool kPair = (VAR & kVarPair) != 0;
-    static_assert(!kPair || (kDma && NB == 1 && !kStamp && !kNarrow), "paired instances");
+    static_assert(!kPair || (kDma && NB == 1 && !kNarrow), "paired instances");
     // (narrow: two stages per wave up to D = 64, one above: four waves' tiles of 26 / 33 KiB)
     constexpr int NSTG = kNarrow ? (D <= 64 ? 2 : 1) : kDma ? C::NSTG : 2;
     constexpr int BRW = kNarrow ? 32 : C::BR;  // query rows per work-group
@@ -789,12 +789,16 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
             if (u < nt) dma_tile(tile_begin + wave + 4 * u, u);
         set_bounds();
         read_slope();
+        stamps.take(1);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         pin_q();
+        stamps.take(2);
+        stamps.take(3);  // (no barrier in front of the loop)
         if constexpr (NSTG == 2) {
             int buf = 0;
             for (int n = 0; n < nt; ++n) {
                 tile_math(wave + 4 * n, buf);
+                if (kStamp && n == 0) stamps.take(4);
                 if (n + 2 < nt) {
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage has been read
                     dma_tile(tile_begin + wave + 4 * (n + 2), buf);
@@ -824,6 +828,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                 if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NKX) : "memory");
                 else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 if (live) pv(0, pf);
+                if (kStamp && n == 0) stamps.take(4);
                 if (more) {
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                     dma_tile_parts(tile_begin + wave + 4 * (n + 1), 0, std::false_type{}, std::true_type{});
@@ -903,6 +908,15 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         }
     }
 
+    stamps.take(5);
+    auto store_stamps = [&]() {
+        if constexpr (kStamp) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the result stores of this wave have left
+            stamps.take(6);
+            stamps.store(a.stamps, ntiles);
+        }
+    };
+
     if constexpr (kNarrow) {
         // ---------------- merge of the four waves' partial results (same rows, disjoint keys), then O and LSE.
         // Like the combine of split partials: weights 2^(m_w - M) on the row sums and on the unnormalised O.
@@ -957,6 +971,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
             if ((tid & 7) == 0)
                 a.LSE[(size_t)bh * Nq + gi] = L > 0.0f ? __builtin_fmaf(M, kLn2, fast_log2(L) * kLn2) : -INFINITY;
         }
+        store_stamps();
         return;
     }
 
@@ -987,7 +1002,6 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     }
 
     // ---------------- epilogue: normalise once, store O (fp16) + LSE, or the fp32 split partials
-    stamps.take(5);
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
         const float l = xhalf_sum(l_run[nb]);
@@ -1080,11 +1094,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
             }
         }
     }
-    if constexpr (kStamp) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the result stores of this wave have left
-        stamps.take(6);
-        stamps.store(a.stamps, ntiles);
-    }
+    store_stamps();
 }
 
 // Launcher of one head-dim bucket, defined in fwd_d{32,64,96,128}.hip.
@@ -1149,7 +1159,8 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
 
 // The instances of a bucket: {d == bucket, d % 8 == 0} x {plain, ALiBi, ALiBi with every visible key at or left of its
 // row, dropout, both}, for rows at any alignment (d % 8 != 0) {plain, ALiBi, dropout, both}, and the one that serves
-// every other request.  ST = kVarStamp selects their instrumented twins (debug time stamps).
+// every other request; the narrow, paired and folded ones below.  ST = kVarStamp selects their instrumented twins (debug
+// time stamps).  Nothing else looks at the stamp pointer: a stamped call is launched as the same call without.
 // The narrow instances (kNarrow in fwd_kernel) serve unsplit launches whose time is the chain of key tiles that a work-group
 // walks through, which they cut to a quarter for a fixed cost of 0.5-2 us (a wave's own requests, the merge of four).  Per
 // tile of a wave on its own: 0.5 / 1.0 / 1.3 / 1.6 us at D = 32 / 64 / 96 / 128, against 0.45 / 0.65 / 0.8 / 1.0 us of a
@@ -1162,10 +1173,9 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
 //  * More rounds only where the later work-groups are the light ones of a causal mask, the longer the sequence the more of
 //    them (B1 H8 N2423 d64, 608 of them: 31.4 -> 22.4 us, but B3 H8 N1344 d64, 1008 of them: 19.2 -> 25.4), or the
 //    chain is so long that two rounds of a quarter are still shorter (B1 H4 N4096 d64 50 -> 38, B2 H4 N4736 d32 69 -> 53).
-inline bool fwd_uses_narrow(const FwdArgs& a, int variant, bool every)
+inline bool fwd_uses_narrow(const FwdArgs& a, bool every)
 {
-    (void)variant;
-    if (every || a.num_splits != 1 || a.stamps != nullptr || a.kernel_hint != 0) return false;
+    if (every || a.num_splits != 1 || a.kernel_hint != 0) return false;
     const long long groups = (long long)a.B * a.H * ((a.Nq + 31) / 32);
     if (groups > 1280) return false;
     const int bucket = (a.d + 31) / 32;
@@ -1230,9 +1240,9 @@ inline bool fwd_uses_pair(const FwdArgs& a, int bucket_d, int feat)
 // -7 %, N640 +-0) and no more than an eighth of the rows is empty (B32 H64 N140 -6 %, N200 +-0), from two rounds of
 // work-groups on.  B32 H32 N512 107.1 -> 99.8 us (688 TFLOP/s), B16 H16 N1024 96.1 -> 87.2,
 // B8 H32 N2048 333.6 -> 313.3, B2 H16 N8192 607 -> 577 (953 TFLOP/s), B31 H64 H_kv8 N705 361 -> 356 us; same bits.
-inline bool fwd_uses_tall(const FwdArgs& a, int feat)
+inline bool fwd_uses_tall(const FwdArgs& a, int variant)
 {
-    if (feat != 0 || a.num_splits != 1 || a.fold_rows || a.causal || a.wl >= 0 || a.wr >= 0 || a.kernel_hint != 0) return false;
+    if (variant != kVarVec || a.d != 64 || a.num_splits != 1 || a.fold_rows || a.causal || a.wl >= 0 || a.wr >= 0 || a.kernel_hint != 0) return false;
     const long long blocks = (a.Nq + 255) / 256, added = 2 * blocks - (a.Nq + 127) / 128;  // in blocks of 128 rows
     return (long long)a.B * a.H * blocks >= 4 * kNumCus && 25 * added <= 2 * blocks && 8 * (256 * blocks - a.Nq) <= 256 * blocks;
 }
@@ -1243,48 +1253,53 @@ inline bool fwd_needs_every_instance(const FwdArgs& a, int variant)
     return a.scale_log2 <= 0.0f || a.scores_out != nullptr || a.d < 8 || ((variant & kVarDropout) && a.drop_thr == 0);
 }
 
+// query rows per work-group of the launch that a takes (what the launchers below and launch_fwd_d128 do)
+inline int fwd_rows_per_group(const FwdArgs& a, int variant)
+{
+    const bool every = fwd_needs_every_instance(a, variant);
+    if (!a.fold_rows && fwd_uses_pingpong(a.d, !every, a.Nq, a.Nk, a.causal, a.wl, a.wr, (long long)a.B * a.H * a.num_splits, a.kernel_hint))
+        return 256;
+    if (fwd_uses_narrow(a, every)) return 32;
+    return fwd_uses_tall(a, variant) ? 256 : 128;
+}
+
 template <int D, int NB, int ST>
 inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
 {
     hipError_t e;
     const int feat = variant & (kVarAlibi | kVarDropout);
     constexpr int AL = kVarAlibi | kVarAlibiLeft;  // ALiBi with no visible key right of its row
-    if constexpr (ST == 0) {
-        if (fwd_uses_narrow(a, variant, fwd_needs_every_instance(a, variant))) {
-            // plain: by row length like the others; with ALiBi or dropout: the instances for rows at any alignment, which serve
-            // every row length from eight elements on, and above 64 the ones for rows of the bucket's width
-            auto with_features = [&](auto full_c) {
-                constexpr int F = decltype(full_c)::value ? kVarVec | kVarFullD : 0;
-                if (feat == kVarAlibi) return (int)launch_fwd_narrow_instance<D, F | kVarAlibi>(a, st);
-                if (feat == kVarDropout) return (int)launch_fwd_narrow_instance<D, F | kVarDropout>(a, st);
-                return (int)launch_fwd_narrow_instance<D, F | kVarAlibi | kVarDropout>(a, st);
-            };
-            if constexpr (D > 64) {
-                if (feat != 0 && a.d == D) return with_features(std::true_type{});
-            }
-            if (feat != 0) return with_features(std::false_type{});
-            if (a.fold_rows) {
-                if (a.d == D) return (int)launch_fwd_narrow_instance<D, kVarVec | kVarFullD | kVarFold>(a, st);
-                if (variant & kVarVec) return (int)launch_fwd_narrow_instance<D, kVarVec | kVarFold>(a, st);
-                return (int)launch_fwd_narrow_instance<D, kVarFold>(a, st);
-            }
-            if (a.d == D) return (int)launch_fwd_narrow_instance<D, kVarVec | kVarFullD>(a, st);
-            if (variant & kVarVec) return (int)launch_fwd_narrow_instance<D, kVarVec>(a, st);
-            return (int)launch_fwd_narrow_instance<D, 0>(a, st);
+    if (fwd_uses_narrow(a, fwd_needs_every_instance(a, variant))) {
+        // plain: by row length like the others; with ALiBi or dropout: the instances for rows at any alignment, which serve
+        // every row length from eight elements on, and above 64 the ones for rows of the bucket's width
+        auto with_features = [&](auto full_c) {
+            constexpr int F = ST | (decltype(full_c)::value ? kVarVec | kVarFullD : 0);
+            if (feat == kVarAlibi) return (int)launch_fwd_narrow_instance<D, F | kVarAlibi>(a, st);
+            if (feat == kVarDropout) return (int)launch_fwd_narrow_instance<D, F | kVarDropout>(a, st);
+            return (int)launch_fwd_narrow_instance<D, F | kVarAlibi | kVarDropout>(a, st);
+        };
+        if constexpr (D > 64) {
+            if (feat != 0 && a.d == D) return with_features(std::true_type{});
         }
+        if (feat != 0) return with_features(std::false_type{});
+        if (a.fold_rows) {
+            if (a.d == D) return (int)launch_fwd_narrow_instance<D, ST | kVarVec | kVarFullD | kVarFold>(a, st);
+            if (variant & kVarVec) return (int)launch_fwd_narrow_instance<D, ST | kVarVec | kVarFold>(a, st);
+            return (int)launch_fwd_narrow_instance<D, ST | kVarFold>(a, st);
+        }
+        if (a.d == D) return (int)launch_fwd_narrow_instance<D, ST | kVarVec | kVarFullD>(a, st);
+        if (variant & kVarVec) return (int)launch_fwd_narrow_instance<D, ST | kVarVec>(a, st);
+        return (int)launch_fwd_narrow_instance<D, ST>(a, st);
     }
-    const bool pair = ST == 0 && fwd_uses_pair(a, D, feat);
+    const bool pair = fwd_uses_pair(a, D, feat);
     auto halves = [&](auto var) {
         constexpr int V = decltype(var)::value;
-        if constexpr (ST == 0) {
-            if (pair) return launch_fwd_instance<D, NB, V | kVarPair>(a, st);
-        }
-        return launch_fwd_instance<D, NB, V>(a, st);
+        return pair ? launch_fwd_instance<D, NB, V | kVarPair>(a, st) : launch_fwd_instance<D, NB, V>(a, st);
     };
-    if (ST == 0 && a.fold_rows) {
-        constexpr int F = ST == 0 ? kVarFold : 0;
-        if (a.d == D) return (int)halves(std::integral_constant<int, (ST == 0 ? F | kVarVec | kVarFullD | kVarKvOnce : 0)>{});
-        if (variant & kVarVec) return (int)halves(std::integral_constant<int, (ST == 0 ? F | kVarVec : 0)>{});
+    if (a.fold_rows) {
+        constexpr int F = ST | kVarFold;
+        if (a.d == D) return (int)halves(std::integral_constant<int, F | kVarVec | kVarFullD | kVarKvOnce>{});
+        if (variant & kVarVec) return (int)halves(std::integral_constant<int, F | kVarVec>{});
         return (int)halves(std::integral_constant<int, F>{});
     }
     if (!(variant & kVarVec)) {
@@ -1299,15 +1314,15 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
         else e = launch_fwd_instance<D, NB, ST | kVarAlibi | kVarDropout>(a, st);
     } else if (a.d == D) {
         constexpr int V = ST | kVarVec | kVarFullD;
-        if constexpr (D == 64 && ST == 0) {
-            if (fwd_uses_tall(a, feat)) {
+        if constexpr (D == 64) {
+            if (fwd_uses_tall(a, variant)) {
                 FwdArgs b = a;
                 b.Tr = (a.Nq + 255) / 256;
                 return (int)launch_fwd_instance<D, 2, V>(b, st);
             }
         }
-        const bool kv_once = ST == 0 && a.Tr == 1 && a.kv_group == 1;
-        if (feat == 0) e = kv_once ? halves(std::integral_constant<int, V | (ST == 0 ? kVarKvOnce : 0)>{}) : halves(std::integral_constant<int, V>{});
+        const bool kv_once = a.Tr == 1 && a.kv_group == 1;
+        if (feat == 0) e = kv_once ? halves(std::integral_constant<int, V | kVarKvOnce>{}) : halves(std::integral_constant<int, V>{});
         else if (feat == kVarAlibi) e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi>(a, st);
         else if (feat == kVarDropout) e = halves(std::integral_constant<int, V | kVarDropout>{});
         else e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL | kVarDropout>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi | kVarDropout>(a, st);
@@ -1321,6 +1336,7 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
     return (int)e;
 }
 
+// every instance has an instrumented twin: the same launch, with time stamps
 template <int D, int NB>
 inline int launch_fwd_bucket(const FwdArgs& a, int variant, hipStream_t st)
 {

@@ -93,9 +93,12 @@ typedef struct flash_params {
      * feature and head dim, which is about 20 % slower.  No counterpart in the reference. */
     float *scores_out;
     /* Which tiled kernel serves the call, for A/B measurements and tests: 0 = the library chooses (by shape),
-     * 1 = the 4-wave kernel with 128 query rows per work-group (left to itself the library gives small unsplit
-     * problems work-groups of 32 rows whose waves share out the key tiles), 2 = the 8-wave ping-pong kernel (256 rows; needs
-     * 96 < d <= 128, a positive scale and more than 128 query rows, and is ignored otherwise).  Any other value: FLASH_EINVAL.
+     * 1 = the 4-wave kernel with 128 query rows of one head per work-group, 2 = the 8-wave ping-pong kernel (256 rows; needs
+     * 96 < d <= 128, a positive scale and more than 128 query rows, and is 1 otherwise).  Left to itself the library also
+     * gives small unsplit problems work-groups of 32 rows whose waves share out the key tiles, launches of one work-group per
+     * CU a second set of four waves that takes every other tile, unmasked d = 64 launches of many rows 256 rows per work-group,
+     * and a few query rows per head of grouped heads one problem per K/V head; either hint turns all four off.  Any other
+     * value: FLASH_EINVAL.
      * The reference selects its kernel by template flags alone (src/main.cu:141-178) and has no such switch. */
     int kernel_hint;
     /* Optional debug output: when non-NULL, every work-group of the tiled kernel stores FLASH_STAMP_WORDS 64-bit words
@@ -105,8 +108,11 @@ typedef struct flash_params {
      * word 7 packs (tiles of the work-group) << 32 | hardware id of the CU (bits 0-15 of HW_ID; bits 16-19 the
      * XCC), and word 8 is the number of shader-clock cycles (s_memtime) between readings 3 and 5: divided by their
      * distance in time it is the clock the CU ran at while the work-group was in its key-tile loop (the power
-     * management lowers it when the MFMA operands change from instruction to instruction).  The call then runs instrumented instances of the same kernels (same arithmetic, same results).  With a
-     * split count above 1 the combine step is not stamped.  The only instrumentation of the reference is the event
+     * management lowers it when the MFMA operands change from instruction to instruction).  The call is launched as it is
+     * without the buffer, with the instrumented twin of the same kernel instance: same split count, same work-groups, same
+     * results bit by bit.  Where the waves of a work-group share out its key tiles (see kernel_hint) the readings are those of
+     * its first wave, which has every fourth or every other tile; with 32 rows per work-group there is no barrier in front of
+     * the loop, and reading 3 follows reading 2.  With a split count above 1 the combine step is not stamped.  The only instrumentation of the reference is the event
      * pair around its launches (src/main.cu:195-213). */
     uint64_t *stage_stamps_out;
     /* Optional: device memory of split_counters_len 32-bit words, all zero, which lets flash_forward_splitkv merge the

@@ -682,6 +682,35 @@ def test_stage_stamps(fa, oracle, hint, N, d, kw):
     assert (np.diff(st2.cpu().numpy()[:, :7], axis=1) >= 0).all()
 
 
+@pytest.mark.parametrize("B,H,Hk,Nq,Nk,d,S,kw", [
+    (1, 3, 3, 700, 700, 64, 1, dict(causal=True)),      # 32-row work-groups, two stages per wave
+    (1, 3, 3, 700, 700, 128, 1, dict()),                # 32-row work-groups, one stage
+    (2, 2, 2, 200, 1740, 31, 3, dict(causal=True)),     # eight waves in two halves
+    (1, 8, 8, 1664, 1664, 100, 1, dict(causal=True)),
+    (2, 16, 4, 20, 700, 128, 3, dict(causal=True)),     # folded heads
+    (1, 8, 2, 30, 1740, 72, 2, dict()),                 # folded heads in two halves
+    (2, 32, 4, 64, 64, 96, 1, dict(window=(20, 5))),    # folded heads, several row blocks
+    (4, 16, 16, 1, 700, 128, 2, dict(dropout_p=0.1)),
+    (1, 8, 8, 100, 2000, 64, 12, dict(causal=True, window=(60, -1))),  # splits without a key
+    (1, 2, 2, 300, 40, 64, 1, dict(causal=True)),       # row blocks without a key
+    (32, 32, 32, 256, 70, 64, 1, dict()),               # 256-row work-groups
+])
+def test_stage_stamps_of_every_launch_form(fa, B, H, Hk, Nq, Nk, d, S, kw):
+    """The instrumented twin of whatever instance serves the call: the same results bit by bit, and a row of ordered
+    stamps from each work-group."""
+    import torch
+
+    q, k, v = randn_f16_gpu((B, H, Nq, d), 1), randn_f16_gpu((B, Hk, Nk, d), 2), randn_f16_gpu((B, Hk, Nk, d), 3)
+    call = fa.flash_forward if S == 1 else fa.flash_forward_splitkv
+    kw = dict(kw, num_splits=S) if S > 1 else kw
+    o0, l0 = call(q, k, v, **kw)
+    o, l, st = call(q, k, v, return_stage_stamps=True, **kw)
+    assert torch.equal(o, o0) and torch.equal(l, l0)
+    t = st.cpu().numpy()
+    assert (t[:, 0] > 0).all() and (np.diff(t[:, :7], axis=1) >= 0).all()
+    assert ((t[:, 6] - t[:, 0]) < 100_000_000).all() and (t[:, 7] >> 32).max() <= (Nk + 63) // 64
+
+
 def test_grouped_query_head_counts_must_divide(fa):
     with pytest.raises(ValueError):
         fa.flash_forward(randn_f16_gpu((1, 6, 8, 64), 1), randn_f16_gpu((1, 4, 8, 64), 2), randn_f16_gpu((1, 4, 8, 64), 3))

@@ -1,7 +1,7 @@
 """What the library launches against the buffers it told the caller to bring, without a GPU (tests/launch_recorder.py)."""
 import numpy as np
 
-from launch_recorder import record
+from launch_recorder import EVERY, FOLD, NARROW, PAIR, STAMP, record
 
 STAMPS = 0x900000  # a stage-stamp buffer
 
@@ -62,3 +62,19 @@ def test_stage_stamp_buffer_holds_every_work_group():
         first = r["launches"][0]
         groups = first["groups"] if first["variant"] is not None else 0  # (the decode stream is not stamped)
         assert r["stamp_bytes"] == groups * 9 * 8, (c, r)
+
+
+def test_stage_stamps_do_not_change_the_launch():
+    """A stamped call runs the instrumented twin of the instance that the call without stamps runs, on the same grid."""
+    calls = random_calls(3, 3000) + [dict(entry="forward", B=32, H=32, Nq=512, Nk=512, d=64)]
+    seen = set()
+    for c, plain, stamped in zip(calls, record(calls), record([dict(c, stage_stamps_out=STAMPS) for c in calls])):
+        assert len(plain["launches"]) == len(stamped["launches"])
+        for a, b in zip(plain["launches"], stamped["launches"]):
+            if a["variant"] is not None:
+                assert b["variant"] == a["variant"] | STAMP, (c, a, b)
+                kind = "pp" if "_pp_" in a["kernel"] else a["kernel"].split("ELi")[1]  # (the other argument: 2 = tall)
+                seen.add((kind, a["variant"] & (EVERY | NARROW | FOLD | PAIR)))
+            assert (b["groups"], b["threads"]) == (a["groups"], a["threads"]), (c, a, b)
+    assert {("1", 0), ("2", 0), ("pp", 0), ("1", EVERY), ("1", NARROW), ("1", FOLD), ("1", PAIR), ("1", NARROW | FOLD),
+            ("1", PAIR | FOLD)} <= seen
