@@ -150,7 +150,7 @@ def make_step(fa, c, q, k, v):
     ws = (None, None)
     if c["splits"]:  # > 0: that many splits; < 0: split entry point with the library's own count
         S = fa.resolve_splits(B, H, Nq, Nk, d, max(0, c["splits"]), causal=c["causal"], window=c["window"],
-                              H_kv=c.get("Hk", 0))
+                              H_kv=c.get("Hk", 0), alibi=c["alibi"], dropout_p=c["p"])
         if S > 1:
             ws = (torch.empty((B, H, S, Nq, d), dtype=torch.float32, device="cuda"),
                   torch.empty((B, H, S, Nq), dtype=torch.float32, device="cuda"))

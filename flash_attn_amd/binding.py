@@ -298,33 +298,48 @@ def stage_stamp_names():
             "tiles<<32|xcc<<16|hw_id", "shader_cycles_first_barrier_to_loop_done")
 
 
-def _shape_params(B, H, Nq, Nk, d, num_splits, causal=False, window=(-1, -1), H_kv=0, kernel_hint=KERNEL_AUTO):
+def _shape_params(B, H, Nq, Nk, d, num_splits, causal=False, window=(-1, -1), H_kv=0, kernel_hint=KERNEL_AUTO,
+                  alibi=False, dropout_p=0.0, softmax_scale=1.0):
     p = FlashParams()
     lib().flash_params_init(C.byref(p))
     p.B, p.H, p.Nq, p.Nk, p.d = B, H, Nq, Nk, d
-    p.softmax_scale = 1.0
+    p.softmax_scale = softmax_scale
     p.num_splits = num_splits
     p.is_causal = int(bool(causal))
     p.window_left, p.window_right = int(window[0]), int(window[1])
     p.H_kv = int(H_kv)
     p.kernel_hint = int(kernel_hint)
+    p.alibi_slopes = 4 if alibi else None  # (the size queries only ask whether there is one)
+    p.dropout_p = float(dropout_p)
     return p
 
 
-def resolve_splits(B, H, Nq, Nk, d, num_splits=0, causal=False, window=(-1, -1), H_kv=0, kernel_hint=KERNEL_AUTO):
+def resolve_splits(B, H, Nq, Nk, d, num_splits=0, causal=False, window=(-1, -1), H_kv=0, kernel_hint=KERNEL_AUTO,
+                   alibi=False, dropout_p=0.0):
     """The split count flash_forward_splitkv will use for such a call (num_splits <= 0: the library's choice)."""
     rc = lib().flash_splitkv_resolve_splits(C.byref(_shape_params(B, H, Nq, Nk, d, num_splits, causal, window, H_kv,
-                                                                kernel_hint)))
+                                                                kernel_hint, alibi, dropout_p)))
     if rc < 0:
         raise FlashError(rc, "flash_splitkv_resolve_splits")
     return rc
 
 
-def workspace_bytes(B, H, Nq, Nk, d, num_splits=0, causal=False, window=(-1, -1), H_kv=0, kernel_hint=KERNEL_AUTO):
+def workspace_bytes(B, H, Nq, Nk, d, num_splits=0, causal=False, window=(-1, -1), H_kv=0, kernel_hint=KERNEL_AUTO,
+                    alibi=None, dropout_p=None):
+    """Bytes of (O_partial, LSE_partial) for flash_forward_splitkv calls of this shape, mask and hint.  The library's
+    choice of split count also looks at ALiBi, dropout and whether the scale is positive: with alibi and dropout_p given the
+    sizes are those of such calls, with one left at None they are enough whatever the call asks for there."""
     ob, lb = C.c_size_t(), C.c_size_t()
-    rc = lib().flash_splitkv_workspace_bytes(C.byref(_shape_params(B, H, Nq, Nk, d, num_splits, causal, window, H_kv,
-                                                                kernel_hint)),
-                                             C.byref(ob), C.byref(lb))
-    if rc != FLASH_OK:
-        raise FlashError(rc, "flash_splitkv_workspace_bytes")
-    return ob.value, lb.value
+    most = (0, 0)
+    for with_alibi in ((False, True) if alibi is None else (alibi,)):
+        for p_drop in ((0.0, 0.5) if dropout_p is None else (dropout_p,)):
+            # (a score dump and a dropout probability below 2^-16 count like a scale that is not positive)
+            for scale in (1.0, -1.0):
+                p = _shape_params(B, H, Nq, Nk, d, num_splits, causal, window, H_kv, kernel_hint, with_alibi, p_drop, scale)
+                rc = lib().flash_splitkv_workspace_bytes(C.byref(p), C.byref(ob), C.byref(lb))
+                if rc != FLASH_OK:
+                    raise FlashError(rc, "flash_splitkv_workspace_bytes")
+                most = max(most, (ob.value, lb.value))  # (both grow with the split count)
+            if num_splits > 0:
+                return most  # (a count that is asked for depends on the key blocks alone)
+    return most

@@ -78,3 +78,26 @@ def test_stage_stamps_do_not_change_the_launch():
             assert (b["groups"], b["threads"]) == (a["groups"], a["threads"]), (c, a, b)
     assert {("1", 0), ("2", 0), ("pp", 0), ("1", EVERY), ("1", NARROW), ("1", FOLD), ("1", PAIR), ("1", NARROW | FOLD),
             ("1", PAIR | FOLD)} <= seen
+
+
+def test_workspace_helper_covers_the_calls_it_knows_nothing_of(fa):
+    """workspace_bytes() of a shape is enough for the launch whatever the call's features are, and so is the size for the
+    features that it is given."""
+    calls = [c for c in random_calls(4, 3000, entry="splitkv", num_splits=0) if c.get("dropout_p") != 1e-6]
+    for Nq in range(2, 65):  # rows whose heads are folded unless a feature keeps them apart
+        for feature in (dict(), dict(alibi_slopes=0xA00000), dict(dropout_p=0.1)):
+            calls.append(dict(entry="splitkv", B=14, H=64, H_kv=8, Nq=Nq, Nk=27335, d=128, num_splits=0, **feature))
+    calls += [dict(c, dropout_p=1e-6) for c in calls[:300]] + [dict(c, scores_out=0xB00000) for c in calls[:300]]
+    for c, r in zip(calls, record(calls)):
+        assert r["rc"] == 0, c
+        rows = split_rows(c, r)
+        shape = [c[x] for x in ("B", "H", "Nq", "Nk", "d")]
+        kw = dict(causal=c.get("is_causal", 0), window=(c.get("window_left", -1), c.get("window_right", -1)), H_kv=c["H_kv"],
+                  kernel_hint=c.get("kernel_hint", 0))
+        ob, lb = fa.workspace_bytes(*shape, **kw)
+        assert ob >= rows * c["d"] * 4 and lb >= rows * 4, c
+        alibi, p = "alibi_slopes" in c, c.get("dropout_p", 0.0)
+        ob, lb = fa.workspace_bytes(*shape, alibi=alibi, dropout_p=p, **kw)
+        assert ob >= rows * c["d"] * 4 and lb >= rows * 4, c
+        if p != 1e-6 and c.get("softmax_scale", 1) > 0 and "scores_out" not in c:
+            assert fa.resolve_splits(*shape, alibi=alibi, dropout_p=p, **kw) == r["splits"], c
