@@ -483,6 +483,8 @@ int run_splitkv(const flash_params* p, int splits, hipStream_t st)
     if (route == kRouteStream && splits > 1 && p->split_counters && (long long)p->B * p->H <= p->split_counters_len)
         a.counters = p->split_counters;
     a.combine_waves = fa::combine_waves_for(splits, route == kRouteStream ? fa::decode_heads_per_group(a.kv_group) : 1);
+    // (a launch is limited to 2^32 - 1 threads: a work-group per row reaches 2^24 rows, a wave per row 2^26)
+    if ((long long)p->B * p->H * p->Nq >= 1LL << 24) a.combine_waves = 1;
     const int e = route == kRouteStream ? record_hip(fa::launch_decode_split(a, st)) : launch_tiled(p, a, st);
     if (e != FLASH_OK || splits == 1 || a.counters) return e;
     if (a.fold_rows) {  // the partial results keep the layout of the heads

@@ -711,6 +711,20 @@ def test_stage_stamps_of_every_launch_form(fa, B, H, Hk, Nq, Nk, d, S, kw):
     assert ((t[:, 6] - t[:, 0]) < 100_000_000).all() and (t[:, 7] >> 32).max() <= (Nk + 63) // 64
 
 
+def test_combine_of_more_rows_than_work_groups_fit_a_launch(fa):
+    """2^24 rows in 17 splits: the merge takes a wave per row.  Against the unsplit launch (fp16 results, one rounding of
+    at most 2^-11 each)."""
+    import torch
+
+    Nq, Nk, d = 2 ** 24, 17 * 128, 8
+    q = torch.randn((1, 1, Nq, d), generator=torch.Generator(device="cuda").manual_seed(1), dtype=torch.float16, device="cuda")
+    k, v = randn_f16_gpu((1, 1, Nk, d), 2), randn_f16_gpu((1, 1, Nk, d), 3)
+    o, lse = fa.flash_forward_splitkv(q, k, v, num_splits=17)
+    o1, lse1 = fa.flash_forward(q, k, v)
+    torch.testing.assert_close(o, o1, rtol=2e-3, atol=2e-3)
+    torch.testing.assert_close(lse, lse1, rtol=0, atol=1e-4)
+
+
 def test_grouped_query_head_counts_must_divide(fa):
     with pytest.raises(ValueError):
         fa.flash_forward(randn_f16_gpu((1, 6, 8, 64), 1), randn_f16_gpu((1, 4, 8, 64), 2), randn_f16_gpu((1, 4, 8, 64), 3))

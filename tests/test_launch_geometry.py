@@ -101,3 +101,11 @@ def test_workspace_helper_covers_the_calls_it_knows_nothing_of(fa):
         assert ob >= rows * c["d"] * 4 and lb >= rows * 4, c
         if p != 1e-6 and c.get("softmax_scale", 1) > 0 and "scores_out" not in c:
             assert fa.resolve_splits(*shape, alibi=alibi, dropout_p=p, **kw) == r["splits"], c
+
+
+def test_combine_launch_fits_a_grid_up_to_2_to_the_26_rows():
+    """More than 16 splits take a work-group per row up to the 2^32 threads of a launch, and a wave per row beyond."""
+    for Nq, S, waves in ((4096, 17, 4), (2 ** 24 - 1, 17, 4), (2 ** 24, 17, 1), (2 ** 24, 16, 1), (2 ** 26 - 4, 20, 1)):
+        r, = record([dict(entry="splitkv", B=1, H=1, Nq=Nq, Nk=128 * S, d=8, num_splits=S)])
+        assert r["rc"] == 0, (Nq, S, r)
+        assert f"combine_kernelILi{waves}E" in r["launches"][1]["kernel"] and r["launches"][1]["split_count"] == S
