@@ -125,8 +125,9 @@ constexpr float kLazyTau = 8.0f;
 // variant bits of the kernel template
 // kVarStamp: debug time stamps.  kVarAlibiLeft (with kVarAlibi, kVarVec): every visible key lies at or left of its row
 // (causal mask or a right window of 0), which lets the bias ride in the MFMA accumulator (see calib below).
-// kVarKvOnce (with kVarVec, kVarFullD, no other feature): every K/V tile is requested by this work-group alone -- one row
-// block per slice and one query head per K/V head, the shape of a decode launch -- and its requests are non-temporal.
+// kVarKvOnce (with kVarVec, kVarFullD, no other feature but kVarFold): every K/V tile is requested by this work-group alone --
+// one row block per slice and one query head (folded: all the query heads) per K/V head, the shape of a decode launch -- and
+// its requests are non-temporal.
 // kVarEvery (with kVarAlibi and kVarDropout, without kVarVec): the instance that serves every request, see kEvery below.
 // kVarNarrow (unsplit launches): the four waves of a work-group share 32 query rows and take every fourth key tile
 // each, see kNarrow below.
@@ -1296,9 +1297,14 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
         constexpr int V = decltype(var)::value;
         return pair ? launch_fwd_instance<D, NB, V | kVarPair>(a, st) : launch_fwd_instance<D, NB, V>(a, st);
     };
+    // (several row blocks per K/V head ask for the same tiles and have to find them in L2: folded launches of 129 rows or more,
+    // non-temporal -> ordinary, 24 random shapes -1 ... +15 %, +4.4 % in the mean: B2 H32 H_kv8 Nq42 Nk3937 d128 23.5 -> 20.5 us, B16
+    // H16 H_kv2 Nq50 Nk5711 d128 70.0 -> 62.9)
+    const bool kv_once = a.Tr == 1 && a.kv_group == 1;
     if (a.fold_rows) {
         constexpr int F = ST | kVarFold;
-        if (a.d == D) return (int)halves(std::integral_constant<int, F | kVarVec | kVarFullD | kVarKvOnce>{});
+        if (a.d == D && kv_once) return (int)halves(std::integral_constant<int, F | kVarVec | kVarFullD | kVarKvOnce>{});
+        if (a.d == D) return (int)halves(std::integral_constant<int, F | kVarVec | kVarFullD>{});
         if (variant & kVarVec) return (int)halves(std::integral_constant<int, F | kVarVec>{});
         return (int)halves(std::integral_constant<int, F>{});
     }
@@ -1321,7 +1327,6 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
                 return (int)launch_fwd_instance<D, 2, V>(b, st);
             }
         }
-        const bool kv_once = a.Tr == 1 && a.kv_group == 1;
         if (feat == 0) e = kv_once ? halves(std::integral_constant<int, V | kVarKvOnce>{}) : halves(std::integral_constant<int, V>{});
         else if (feat == kVarAlibi) e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi>(a, st);
         else if (feat == kVarDropout) e = halves(std::integral_constant<int, V | kVarDropout>{});

@@ -1,7 +1,7 @@
 """What the library launches against the buffers it told the caller to bring, without a GPU (tests/launch_recorder.py)."""
 import numpy as np
 
-from launch_recorder import EVERY, FOLD, NARROW, PAIR, STAMP, record
+from launch_recorder import ALIBI, DROPOUT, EVERY, FOLD, FULL_D, KV_ONCE, NARROW, PAIR, STAMP, record
 
 STAMPS = 0x900000  # a stage-stamp buffer
 
@@ -109,3 +109,24 @@ def test_combine_launch_fits_a_grid_up_to_2_to_the_26_rows():
         r, = record([dict(entry="splitkv", B=1, H=1, Nq=Nq, Nk=128 * S, d=8, num_splits=S)])
         assert r["rc"] == 0, (Nq, S, r)
         assert f"combine_kernelILi{waves}E" in r["launches"][1]["kernel"] and r["launches"][1]["split_count"] == S
+
+
+def test_non_temporal_requests_only_where_no_other_work_group_asks_for_the_tiles():
+    """One row block per K/V head: K and V pass once, whether the rows are a head's own, folded heads or a decode launch's."""
+    calls = random_calls(5, 3000)
+    for G, Nq in ((2, 64), (4, 32), (4, 33), (8, 16), (8, 17), (16, 64)):  # 128 rows | more
+        for d in (32, 64, 96, 128):
+            for S in (1, 8):
+                calls.append(dict(entry="splitkv", B=3, H=8 * G, H_kv=8, Nq=Nq, Nk=9000, d=d, num_splits=S))
+    seen = set()
+    for c, r in zip(calls, record(calls)):
+        if r["rc"] != 0 or not r["launches"] or r["launches"][0]["variant"] is None or "_pp_" in r["launches"][0]["kernel"]:
+            continue
+        v, G = r["launches"][0]["variant"], c["H"] // c["H_kv"]
+        heads_as_rows = v & FOLD or (c["Nq"] == 1 and G >= 4 and not c.get("alibi_slopes") and not c.get("dropout_p")
+                                     and c.get("window_left", -1) < 0)
+        once = (c["Nq"] * G if heads_as_rows else c["Nq"] if G == 1 else 1 << 30) <= 128
+        may = v & FULL_D and not v & (NARROW | ALIBI | DROPOUT)
+        assert bool(v & KV_ONCE) == bool(once and may), (c, r)
+        seen.add((bool(v & FOLD), bool(v & KV_ONCE), bool(v & PAIR), bool(may)))
+    assert {(True, True, False, True), (True, False, False, True), (True, False, True, True), (True, True, True, True)} <= seen
