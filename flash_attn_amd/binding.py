@@ -7,6 +7,7 @@ exits, src/main.cu:18-25,182-185).
 """
 import ctypes as C
 import os
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.path.join(_HERE, "lib", "libflash_attn_mi355.so")
@@ -105,14 +106,33 @@ def lib():
 _native = None
 
 
+class _NoFrontEnd:
+    """Leaves every call to binding.py's own path."""
+
+    @staticmethod
+    def forward(*args):
+        return NotImplemented
+
+    splitkv = forward
+
+
 def _front_end():
-    """The native front end (csrc/py_binding.cpp), bound to the loaded library.  Raises if it has not been built."""
+    """The native front end (csrc/py_binding.cpp), bound to the loaded library.  Where it has not been built (it needs a Python
+    with torch, the library does not), or for another torch, calls go through ctypes: the same launches, 10 us later."""
     global _native
     L = lib()
-    from . import _native as n
+    try:
+        import torch
+        from . import _native as n
 
-    n.bind(*(C.cast(f, C.c_void_p).value for f in (L.flash_forward, L.flash_forward_splitkv, L.flash_splitkv_resolve_splits)),
-           FlashError)
+        if n.torch_version.split("+")[0] != torch.__version__.split("+")[0]:
+            raise ImportError(f"built for torch {n.torch_version}, this is {torch.__version__}")
+        n.bind(*(C.cast(f, C.c_void_p).value for f in (L.flash_forward, L.flash_forward_splitkv, L.flash_splitkv_resolve_splits)),
+               FlashError)
+    except ImportError as e:
+        warnings.warn(f"flash_attn_amd: no native front end ({e}), every call takes some 10 us more host time; build it with "
+                      "`make -C flash_attn_amd/csrc native`", RuntimeWarning, stacklevel=3)
+        n = _NoFrontEnd
     _native = n
     return n
 

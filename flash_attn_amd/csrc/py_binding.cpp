@@ -11,6 +11,7 @@
 // small -- returns NotImplemented with nothing allocated or launched; binding.py then takes its own path, which raises the
 // errors (and serves the debug outputs).
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
@@ -285,4 +286,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nu
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__native(void)
+{
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) != 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

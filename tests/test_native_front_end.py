@@ -1,5 +1,10 @@
 """The native front end of the binding (csrc/py_binding.cpp) against binding.py's own path, which the debug outputs take:
 same kernels, so bit-identical results whatever way the arguments come."""
+import os
+import subprocess
+import sys
+import types
+
 import pytest
 
 from helpers import randn_f16_gpu
@@ -78,3 +83,51 @@ def test_leaves_what_it_cannot_serve_to_the_binding(fa):
         fa.flash_forward(z, z, z)
     with pytest.raises(ValueError, match="fp16"):
         fa.flash_forward_splitkv(z, z, z)
+
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "flash_attn_amd", "csrc")
+
+
+def _dry_run(*args):
+    r = subprocess.run(["make", "-n", "-C", CSRC, *args], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr
+    return r.stdout
+
+
+def test_the_library_builds_without_python():
+    assert "flash_api.hip" in (out := _dry_run("-B", "PYTHON=false")) and "py_binding.cpp" not in out
+
+
+def test_the_front_end_is_rebuilt_for_another_torch():
+    import torch
+
+    assert "py_binding.cpp" not in _dry_run("native", "-o", "../../include/flash_attn_mi355.h", "-o", "py_binding.cpp")
+    assert "py_binding.cpp" in _dry_run("native", "-W", os.path.join(os.path.dirname(torch.__file__), "version.py"))
+
+
+@pytest.mark.parametrize("found", [None, types.SimpleNamespace(torch_version="1.0.0")])  # not built | built for another torch
+def test_calls_are_served_without_the_front_end(fa, monkeypatch, found):
+    import flash_attn_amd
+    import torch
+
+    monkeypatch.setitem(sys.modules, "flash_attn_amd._native", found)
+    monkeypatch.delattr(flash_attn_amd, "_native", raising=False)
+    if found is not None:
+        monkeypatch.setattr(flash_attn_amd, "_native", found, raising=False)
+    monkeypatch.setattr(fa.binding, "_native", None)
+    z = torch.zeros(1, 1, 2, 8)
+    with pytest.warns(RuntimeWarning, match="make -C flash_attn_amd/csrc native"), pytest.raises(ValueError, match="fp16"):
+        fa.flash_forward(z, z, z)
+    with pytest.raises(ValueError, match="fp16"):  # (and says so once)
+        fa.flash_forward_splitkv(z, z, z)
+
+
+@pytest.mark.gpu
+def test_results_without_the_front_end(fa, monkeypatch):
+    import torch
+
+    q, k, v = randn_f16_gpu((2, 4, 70, 40), 1), randn_f16_gpu((2, 2, 900, 40), 2), randn_f16_gpu((2, 2, 900, 40), 3)
+    with_it = fa.flash_forward(q, k, v, causal=True) + fa.flash_forward_splitkv(q, k, v)
+    monkeypatch.setattr(fa.binding, "_native", fa.binding._NoFrontEnd)
+    without = fa.flash_forward(q, k, v, causal=True) + fa.flash_forward_splitkv(q, k, v)
+    assert all(torch.equal(a, b) for a, b in zip(with_it, without))
