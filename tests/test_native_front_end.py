@@ -1,5 +1,6 @@
 """The native front end of the binding (csrc/py_binding.cpp) against binding.py's own path, which the debug outputs take:
 same kernels, so bit-identical results whatever way the arguments come."""
+import contextlib
 import os
 import subprocess
 import sys
@@ -12,6 +13,28 @@ from helpers import randn_f16_gpu
 
 def _call(fa, entry, tensors, **kw):
     return (fa.flash_forward if entry == "forward" else fa.flash_forward_splitkv)(*tensors, **kw)
+
+
+@contextlib.contextmanager
+def _front_end_watched(fa):
+    """Yields a list that collects, call by call, whether the front end served it."""
+    front = fa.binding._front_end()
+    seen = []
+    real = fa.binding._native
+
+    class Spy:
+        def __getattr__(self, name):
+            def f(*a):
+                r = getattr(front, name)(*a)
+                seen.append(r is not NotImplemented)
+                return r
+            return f
+
+    fa.binding._native = Spy()
+    try:
+        yield seen
+    finally:
+        fa.binding._native = real
 
 
 @pytest.mark.gpu
@@ -42,23 +65,8 @@ def test_matches_the_binding_s_own_path(fa, entry, Nq, kw, own_buffers):
         extra = dict(out=torch.empty_like(o0), lse=torch.empty_like(l0), stream=s)
         if entry == "splitkv":
             extra["workspace"] = (torch.empty(2 * 4 * 8 * Nq * 40, device="cuda"), torch.empty(2 * 4 * 8 * Nq, device="cuda"))
-    front = fa.binding._front_end()
-    seen = []
-    real = fa.binding._native
-
-    class Spy:
-        def __getattr__(self, name):
-            def f(*a):
-                r = getattr(front, name)(*a)
-                seen.append(r is not NotImplemented)
-                return r
-            return f
-
-    fa.binding._native = Spy()
-    try:
+    with _front_end_watched(fa) as seen:
         o1, l1 = _call(fa, entry, (q, k, v), **extra, **kw)
-    finally:
-        fa.binding._native = real
     torch.cuda.synchronize()
     assert seen == [True]
     if entry == "forward":  # (a hint can change the automatic split count and with it the rounding)
@@ -131,3 +139,34 @@ def test_results_without_the_front_end(fa, monkeypatch):
     monkeypatch.setattr(fa.binding, "_native", fa.binding._NoFrontEnd)
     without = fa.flash_forward(q, k, v, causal=True) + fa.flash_forward_splitkv(q, k, v)
     assert all(torch.equal(a, b) for a, b in zip(with_it, without))
+
+
+@pytest.mark.gpu
+def test_allocations_are_seen_by_those_who_look(fa):
+    """A dispatch mode sees results and workspace being allocated, and deterministic mode fills them."""
+    import torch
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if func is torch.ops.aten.empty.memory_format:
+                sizes.append(tuple(args[0]))
+            return func(*args, **(kwargs or {}))
+
+    q, k, v = randn_f16_gpu((1, 2, 3, 40), 1), randn_f16_gpu((1, 2, 500, 40), 2), randn_f16_gpu((1, 2, 500, 40), 3)
+    sizes = []
+    want = fa.flash_forward(q, k, v), fa.flash_forward_splitkv(q, k, v, num_splits=2)
+    with Watch():
+        got = fa.flash_forward(q, k, v), fa.flash_forward_splitkv(q, k, v, num_splits=2)
+    assert sizes == [(1, 2, 3, 40), (1, 2, 3), (1, 2, 3, 40), (1, 2, 3), (2 * 2 * 3 * 40,), (2 * 2 * 3,)]
+    assert all(torch.equal(a, b) for w, g in zip(want, got) for a, b in zip(w, g))
+    before = torch.utils.deterministic.fill_uninitialized_memory
+    with _front_end_watched(fa) as seen:
+        torch.use_deterministic_algorithms(True)
+        try:
+            for torch.utils.deterministic.fill_uninitialized_memory in (True, False):
+                assert torch.equal(fa.flash_forward(q, k, v)[0], want[0][0])
+        finally:
+            torch.use_deterministic_algorithms(False)
+            torch.utils.deterministic.fill_uninitialized_memory = before
+    assert seen == [False, True]
