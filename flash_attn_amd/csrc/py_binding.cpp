@@ -20,9 +20,9 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
-#include <vector>
 
 #include "flash_attn_mi355.h"
+#include "split_counters.h"
 
 namespace {
 
@@ -74,40 +74,35 @@ bool optional_tensor(PyObject* o, const at::Tensor** t)
     return o == Py_None || (*t = tensor_of(o)) != nullptr;
 }
 
-// Arrival counters (flash_params::split_counters) of the calls on one stream: a region of kCountersPerStream zeros for
-// each of up to kCounterStreams streams of a device, 1 MiB per device that ever needs one, allocated and cleared once.
-// Only the default stream and torch's own pooled streams get one: those exist until the process ends, so calls that share a
-// region are ordered for good.  Other streams, calls under graph capture (a graph may be replayed beside other work)
-// and whoever comes too late merge in a launch of their own.  (All of this runs with the interpreter lock held.)
-constexpr int kCountersPerStream = 4096, kCounterStreams = 64;
-struct DeviceCounters {
-    at::Tensor zeros;
-    std::vector<void*> streams;
+// What the table of split_counters.h asks for: 1 MiB of zeros per device that ever needs some, allocated and cleared once and
+// kept until the process ends.  (All of this runs with the interpreter lock held.)
+struct TorchRuntime {
+    int current_device() const
+    {
+        int d = -1;
+        return hipGetDevice(&d) == hipSuccess ? d : -1;
+    }
+    bool capturing(void* stream) const
+    {
+        hipStreamCaptureStatus c;
+        return hipStreamIsCapturing(static_cast<hipStream_t>(stream), &c) != hipSuccess || c != hipStreamCaptureStatusNone;
+    }
+    uint32_t* zeros(int device, size_t words) const
+    {
+        const at::Device on(at::kCUDA, (c10::DeviceIndex)device);
+        at::Tensor* z = new at::Tensor(at::detail::empty_cuda({(int64_t)words}, at::kInt, on, std::nullopt));
+        const auto current = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
+        if (hipMemsetAsync(z->data_ptr(), 0, z->nbytes(), current) == hipSuccess && hipStreamSynchronize(current) == hipSuccess)
+            return static_cast<uint32_t*>(z->data_ptr());
+        delete z;
+        return nullptr;
+    }
 };
 uint32_t* counters_of(at::Device device, void* stream, bool pooled)
 {
-    static std::vector<DeviceCounters>* all = new std::vector<DeviceCounters>;  // (never freed: outlives the runtime's own end)
-    if (stream != nullptr && !pooled) return nullptr;
-    hipStreamCaptureStatus capture;
-    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &capture) != hipSuccess || capture != hipStreamCaptureStatusNone)
-        return nullptr;
-    const size_t dev = (size_t)device.index();
-    if (dev >= all->size()) all->resize(dev + 1);
-    DeviceCounters& c = (*all)[dev];
-    size_t i = 0;
-    while (i < c.streams.size() && c.streams[i] != stream) ++i;
-    if (i == c.streams.size()) {
-        if (i == (size_t)kCounterStreams) return nullptr;
-        if (!c.zeros.defined()) {
-            at::Tensor z = at::detail::empty_cuda({(int64_t)kCountersPerStream * kCounterStreams}, at::kInt, device, std::nullopt);
-            const auto current = c10::hip::getCurrentHIPStream(device.index()).stream();
-            if (hipMemsetAsync(z.data_ptr(), 0, z.nbytes(), current) != hipSuccess || hipStreamSynchronize(current) != hipSuccess)
-                return nullptr;
-            c.zeros = z;
-        }
-        c.streams.push_back(stream);
-    }
-    return static_cast<uint32_t*>(c.zeros.data_ptr()) + i * kCountersPerStream;
+    static auto* table = new fa::CounterTable<TorchRuntime>;  // (never freed: outlives the runtime's own end)
+    TorchRuntime rt;
+    return table->of(rt, device.index(), stream, pooled);
 }
 
 struct Call {
@@ -267,7 +262,7 @@ PyObject* splitkv(PyObject*, PyObject* const* args, Py_ssize_t n)
         }
         if (S > 1 && (c.stream == nullptr || c.pooled_stream)) {
             p.split_counters = counters_of(c.q->device(), c.stream, c.pooled_stream);
-            p.split_counters_len = p.split_counters ? kCountersPerStream : 0;
+            p.split_counters_len = p.split_counters ? fa::kCountersPerStream : 0;
         }
         return launch(g_splitkv, "flash_forward_splitkv", &c);
     });

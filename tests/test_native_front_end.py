@@ -113,6 +113,14 @@ def test_the_front_end_is_rebuilt_for_another_torch():
     assert "py_binding.cpp" in _dry_run("native", "-W", os.path.join(os.path.dirname(torch.__file__), "version.py"))
 
 
+def test_counters_of_streams(tmp_path):
+    exe = str(tmp_path / "split_counters_test")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-Wall", "-I", CSRC, os.path.join(os.path.dirname(__file__), "split_counters_test.cpp"),
+                           "-o", exe])
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
+
+
 @pytest.mark.parametrize("found", [None, types.SimpleNamespace(torch_version="1.0.0")])  # not built | built for another torch
 def test_calls_are_served_without_the_front_end(fa, monkeypatch, found):
     import flash_attn_amd
