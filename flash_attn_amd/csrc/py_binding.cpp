@@ -16,6 +16,7 @@
 #include <ATen/Context.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 
@@ -74,8 +75,8 @@ bool optional_tensor(PyObject* o, const at::Tensor** t)
     return o == Py_None || (*t = tensor_of(o)) != nullptr;
 }
 
-// What the table of split_counters.h asks for: 1 MiB of zeros per device that ever needs some, allocated and cleared once and
-// kept until the process ends.  (All of this runs with the interpreter lock held.)
+// What the table of split_counters.h asks for.  A region is 16 KiB of the stream's own pool, kept until the process ends, at
+// most 1 MiB per device.  (All of this runs with the interpreter lock held.)
 struct TorchRuntime {
     int current_device() const
     {
@@ -87,15 +88,19 @@ struct TorchRuntime {
         hipStreamCaptureStatus c;
         return hipStreamIsCapturing(static_cast<hipStream_t>(stream), &c) != hipSuccess || c != hipStreamCaptureStatusNone;
     }
-    uint32_t* zeros(int device, size_t words) const
+    uint32_t* allocate(size_t words, void* stream) const
     {
-        const at::Device on(at::kCUDA, (c10::DeviceIndex)device);
-        at::Tensor* z = new at::Tensor(at::detail::empty_cuda({(int64_t)words}, at::kInt, on, std::nullopt));
-        const auto current = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
-        if (hipMemsetAsync(z->data_ptr(), 0, z->nbytes(), current) == hipSuccess && hipStreamSynchronize(current) == hipSuccess)
-            return static_cast<uint32_t*>(z->data_ptr());
-        delete z;
-        return nullptr;
+        try {
+            return static_cast<uint32_t*>(
+                c10::hip::HIPCachingAllocator::raw_alloc_with_stream(words * sizeof(uint32_t), static_cast<hipStream_t>(stream)));
+        } catch (const c10::Error&) {
+            return nullptr;
+        }
+    }
+    void release(uint32_t* p) const { c10::hip::HIPCachingAllocator::raw_delete(p); }
+    bool clear(uint32_t* p, size_t words, void* stream) const
+    {
+        return hipMemsetAsync(p, 0, words * sizeof(uint32_t), static_cast<hipStream_t>(stream)) == hipSuccess;
     }
 };
 uint32_t* counters_of(at::Device device, void* stream, bool pooled)

@@ -24,23 +24,28 @@ public:
         if (rt.current_device() != device) return nullptr;
         if (rt.capturing(stream)) return nullptr;
         if ((size_t)device >= devices_.size()) devices_.resize((size_t)device + 1);
-        Device& d = devices_[(size_t)device];
-        size_t i = 0;
-        while (i < d.streams.size() && d.streams[i] != stream) ++i;
-        if (i == d.streams.size()) {
-            if (i == (size_t)kCounterStreams) return nullptr;
-            if (!d.zeros && !(d.zeros = rt.zeros(device, (size_t)kCountersPerStream * kCounterStreams))) return nullptr;
-            d.streams.push_back(stream);
+        std::vector<Region>& regions = devices_[(size_t)device];
+        for (const Region& r : regions)
+            if (r.stream == stream) return r.counters;
+        if (regions.size() == (size_t)kCounterStreams) return nullptr;
+        // Allocated and cleared on the stream itself, in front of the launches that count in it: no other stream is touched, none
+        // waited for (the current one may be another, and under capture).
+        uint32_t* const fresh = rt.allocate(kCountersPerStream, stream);
+        if (fresh == nullptr) return nullptr;
+        if (!rt.clear(fresh, kCountersPerStream, stream)) {
+            rt.release(fresh);
+            return nullptr;
         }
-        return d.zeros + i * kCountersPerStream;
+        regions.push_back({stream, fresh});
+        return fresh;
     }
 
 private:
-    struct Device {
-        uint32_t* zeros = nullptr;
-        std::vector<void*> streams;
+    struct Region {
+        void* stream;
+        uint32_t* counters;
     };
-    std::vector<Device> devices_;
+    std::vector<std::vector<Region>> devices_;
 };
 
 }  // namespace fa

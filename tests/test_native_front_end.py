@@ -178,3 +178,56 @@ def test_allocations_are_seen_by_those_who_look(fa):
             torch.use_deterministic_algorithms(False)
             torch.utils.deterministic.fill_uninitialized_memory = before
     assert seen == [False, True]
+
+
+@pytest.mark.gpu
+def test_first_call_on_a_stream_while_another_is_captured(fa):
+    """Split calls on streams that have not been used yet, issued inside a capture of the current stream: they run beside it,
+    and the captured graph is whole."""
+    import torch
+
+    q, k, v = randn_f16_gpu((1, 2, 1, 64), 1), randn_f16_gpu((1, 2, 3000, 64), 2), randn_f16_gpu((1, 2, 3000, 64), 3)
+    want = fa.flash_forward_splitkv(q, k, v, num_splits=4)
+    captured = torch.cuda.Stream()
+    # (torch deals out 32 streams in turn: all of them but the captured one)
+    sides = [s for s in (torch.cuda.Stream() for _ in range(32)) if s.cuda_stream != captured.cuda_stream]
+    bufs = [(torch.zeros_like(want[0]), torch.zeros_like(want[1]), (torch.empty(4 * 2 * 64, device="cuda"), torch.empty(4 * 2, device="cuda")))
+            for _ in sides]
+    x = torch.ones(1000, device="cuda")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=captured):
+        y = x + 1
+        for s, (o, lse, ws) in zip(sides, bufs):
+            fa.flash_forward_splitkv(q, k, v, num_splits=4, stream=s, out=o, lse=lse, workspace=ws)
+        z = y * 2
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, want[0]) and torch.equal(lse, want[1]) for o, lse, _ in bufs)
+    for i in range(3):
+        x.fill_(i)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(z, torch.full_like(z, 2.0 * (i + 1)))
+
+
+@pytest.mark.gpu
+def test_counters_on_two_streams_at_once(fa):
+    """Decode calls that merge in the split launch, many of them in flight on each of two streams."""
+    import torch
+
+    shapes = [(2, 3, 2500, 64, 8), (1, 4, 9000, 128, 40)]
+    sets, wants = [], []
+    for i, (B, H, Nk, d, S) in enumerate(shapes):
+        t = randn_f16_gpu((B, H, 1, d), 3 * i), randn_f16_gpu((B, H, Nk, d), 3 * i + 1), randn_f16_gpu((B, H, Nk, d), 3 * i + 2)
+        sets.append((t, S))
+        wants.append(fa.flash_forward_splitkv(*t, num_splits=S))
+    streams = [torch.cuda.Stream() for _ in shapes]
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(50):
+        for i, ((t, S), s) in enumerate(zip(sets, streams)):
+            with torch.cuda.stream(s):
+                got[i].append(fa.flash_forward_splitkv(*t, num_splits=S))
+    torch.cuda.synchronize()
+    for want, results in zip(wants, got):
+        assert all(torch.equal(o, want[0]) and torch.equal(lse, want[1]) for o, lse in results)
