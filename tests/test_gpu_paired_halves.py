@@ -37,3 +37,34 @@ def test_paired_halves_dropout(fa, oracle, Nq, d):
     keep = torch.from_numpy(oracle.dropout_keep_mask(9, 0, p, B, H, Nq, Nk))
     O, L = oracle_forward_batched(oracle, q, k, v, causal=True, keep_mask=keep, p_drop=p)
     check_o_lse(*fa.flash_forward_splitkv(q, k, v, num_splits=3, causal=True, dropout_p=p, seed=9), O, L, "dropout")
+
+
+@pytest.mark.parametrize("B,H,N,d,kw", [(1, 20, 700, 128, dict(causal=True)), (1, 11, 1090, 64, dict(causal=True)),
+                                        (1, 20, 900, 100, dict(causal=True, window=(390, -1))), (1, 16, 1100, 96, dict(window=(600, 0))),
+                                        (1, 34, 800, 31, dict(causal=True))])
+def test_paired_halves_unsplit_dropout(fa, oracle, B, H, N, d, kw):
+    """Whole launches with dropout, under a mask and under a window, and the decisions that the two halves store."""
+    import torch
+
+    p = 0.2
+    q, k, v = (randn_f16_gpu((B, H, N, d), s) for s in (4, 5, 6))
+    keep = torch.from_numpy(oracle.dropout_keep_mask(9, 0, p, B, H, N, N))
+    O, L = oracle_forward_batched(oracle, q, k, v, keep_mask=keep, p_drop=p, **kw)
+    o, lse = fa.flash_forward(q, k, v, dropout_p=p, seed=9, **kw)
+    check_o_lse(o, lse, O, L, "unsplit dropout")
+    o1, lse1, stored = fa.flash_forward(q, k, v, dropout_p=p, seed=9, return_keep_mask=True, **kw)
+    assert torch.equal(o1, o) and torch.equal(lse1, lse)
+    i, j = torch.arange(N).view(-1, 1), torch.arange(N).view(1, -1)
+    visible = (j <= i) & (i - j <= (kw.get("window", (N,))[0] if kw.get("window", (-1,))[0] >= 0 else N))
+    assert torch.equal(stored.cpu()[..., visible], keep[..., visible])
+
+
+@pytest.mark.parametrize("Nq,d", [(33, 128), (140, 100), (128, 64)])
+def test_paired_halves_windowed_dropout(fa, oracle, Nq, d):
+    import torch
+
+    B, H, Nk, p, kw = 1, 2, 1740, 0.2, dict(causal=True, window=(390, -1))
+    q, k, v = randn_f16_gpu((B, H, Nq, d), 1), randn_f16_gpu((B, H, Nk, d), 2), randn_f16_gpu((B, H, Nk, d), 3)
+    keep = torch.from_numpy(oracle.dropout_keep_mask(9, 0, p, B, H, Nq, Nk))
+    O, L = oracle_forward_batched(oracle, q, k, v, keep_mask=keep, p_drop=p, **kw)
+    check_o_lse(*fa.flash_forward_splitkv(q, k, v, num_splits=3, dropout_p=p, seed=9, **kw), O, L, "windowed dropout")

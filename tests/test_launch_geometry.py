@@ -130,3 +130,14 @@ def test_non_temporal_requests_only_where_no_other_work_group_asks_for_the_tiles
         assert bool(v & KV_ONCE) == bool(once and may), (c, r)
         seen.add((bool(v & FOLD), bool(v & KV_ONCE), bool(v & PAIR), bool(may)))
     assert {(True, True, False, True), (True, False, False, True), (True, False, True, True), (True, True, True, True)} <= seen
+
+
+def test_paired_launches_of_the_dropout_tests():
+    """The shapes of tests/test_gpu_paired_halves.py that are about paired launches with dropout are such launches."""
+    calls = [dict(entry="forward", B=1, H=H, Nq=N, Nk=N, d=d, is_causal=c, window_left=left, window_right=right, dropout_p=0.2)
+             for H, N, d, c, left, right in ((20, 700, 128, 1, -1, -1), (11, 1090, 64, 1, -1, -1), (20, 900, 100, 1, 390, -1),
+                                             (16, 1100, 96, 0, 600, 0), (34, 800, 31, 1, -1, -1))]
+    calls += [dict(entry="splitkv", B=1, H=2, Nq=Nq, Nk=1740, d=d, num_splits=3, is_causal=1, window_left=390, dropout_p=0.2)
+              for Nq, d in ((33, 128), (140, 100), (128, 64))]
+    for c, r in zip(calls, record(calls)):
+        assert r["launches"][0]["variant"] & (PAIR | NARROW | DROPOUT) == PAIR | DROPOUT, c
