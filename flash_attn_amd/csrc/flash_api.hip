@@ -190,7 +190,9 @@ long long tiled_groups(const flash_params* p, const fa::FwdArgs& a)
 // tiles (the heaviest one plus k - 1 average ones) taken in rounds of as many as the CU has places for, a round of n
 // side by side costing the sum of its tiles over the gain of n, b = microseconds per 64-key tile of a work-group alone
 // on its CU.  Over 21 swept shapes the count it picks is within 5 % of the best measured one on 19 (the others: 6 % and
-// 9 %); the reference's rule with 256 CUs: 9 of 21, the worst 3.1 times slower than the best count.
+// 9 %); the reference's rule with 256 CUs: 9 of 21, the worst 3.1 times slower than the best count.  It does not know which
+// launches will be paired: a cheaper tile for those made the counts of 300 random shapes 0.2 % worse.  Its constants and the lines
+// of fwd_uses_narrow are fits to the kernels as they are; a change of either wants both measured again.
 int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode);
 bool folds_heads(const flash_params* p);
 void fold_heads(fa::FwdArgs* a);

@@ -166,8 +166,8 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // the score dump among them.
     constexpr bool kEvery = (VAR & kVarEvery) != 0;
     static_assert(!kEvery || (!kVec && kAlibi && kDropout), "the instance that serves every request");
-    // Small problems -- fewer work-groups of 128 rows than half the CUs -- are bound by the chain of tiles that a
-    // work-group walks through one after the other.  The narrow instances cut that chain to a quarter: a work-group owns
+    // Problems of few work-groups are bound by the chain of tiles that a work-group walks through one after the other
+    // (fwd_uses_narrow says which).  The narrow instances cut that chain to a quarter: a work-group owns
     // 32 query rows, all four waves hold those rows, and wave w takes the key tiles w, w + 4, w + 8, ... of the range on
     // its own: it requests them into LDS stages of its own (no work-group barrier inside the loop, every wave waits
     // for its own requests only), and the four partial results are merged through LDS at the end like the partial results
@@ -1240,7 +1240,10 @@ inline bool fwd_uses_pair(const FwdArgs& a, int bucket_d, int feat)
 // where 256-row blocks add no more than 4 % of empty rows to what 128-row blocks have (B32 H32 N384 52.8 -> 60.3 us, N300
 // -7 %, N640 +-0) and no more than an eighth of the rows is empty (B32 H64 N140 -6 %, N200 +-0), from two rounds of
 // work-groups on.  B32 H32 N512 107.1 -> 99.8 us (688 TFLOP/s), B16 H16 N1024 96.1 -> 87.2,
-// B8 H32 N2048 333.6 -> 313.3, B2 H16 N8192 607 -> 577 (953 TFLOP/s), B31 H64 H_kv8 N705 361 -> 356 us; same bits.
+// B8 H32 N2048 333.6 -> 313.3, B2 H16 N8192 607 -> 577 (953 TFLOP/s), B31 H64 H_kv8 N705 361 -> 356 us; same bits.  On another
+// card the first two were 108.3 -> 105.6 and 94.8 -> 92.5, and B2 H16 N8192 641 -> 629: the launch needs no fewer cycles than with
+// 128 rows, 16 % of which have neither a VALU instruction nor an MFMA, but half the LDS instructions and 0.57 of the bytes
+// fetched, and what those save in power comes back as clock.
 inline bool fwd_uses_tall(const FwdArgs& a, int variant)
 {
     if (variant != kVarVec || a.d != 64 || a.num_splits != 1 || a.fold_rows || a.causal || a.wl >= 0 || a.wr >= 0 || a.kernel_hint != 0) return false;

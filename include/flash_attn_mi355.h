@@ -136,9 +136,10 @@ int flash_forward(const flash_params *p, void *stream);
  *     forward_kernel_splitkv_combine<<<dim3(Tr,H,B),Br>>>(param);          (src/flash_forward_splitkv.h:14-16,347-348,
  *                                                                          src/main.cu:189-192)
  * Uses p->num_splits; needs the workspace when the resulting split count is > 1.  With num_splits <= 0 the library
- * chooses: flash_num_splits_heuristic with 256 CUs (the reference's rule, src/main.cu:125) for Nq > 1; for Nq == 1,
- * which streams K and V once and is bound by memory bandwidth, enough splits of at least 512 keys to give every CU
- * several work-groups.  flash_splitkv_resolve_splits returns the count either way. */
+ * chooses (the reference asks num_splits_heuristic, src/main.cu:125): the count with the lowest estimated time for Nq > 1
+ * and for the Nq == 1 calls that the tiled kernel serves; otherwise for Nq == 1, which streams K and V once and is bound by
+ * memory bandwidth, about one work-group per CU, at most sqrt(Nk / 3) splits.  flash_splitkv_resolve_splits returns the
+ * count either way; it depends on the sizes, masks, scale, kernel_hint, scores_out and on whether ALiBi and dropout are on. */
 int flash_forward_splitkv(const flash_params *p, void *stream);
 
 /* flash_forward_splitkv for callers that cannot allocate device memory (code under HIP graph capture, tight serving
@@ -155,7 +156,8 @@ int flash_forward_splitkv(const flash_params *p, void *stream);
 #define FLASH_STATIC_SCRATCH_BYTES (32u << 20)
 int flash_forward_splitkv_static(const flash_params *p, void *stream);
 
-/* Bytes of O_partial and of LSE_partial needed for p (the cudaMallocs of src/main.cu:160-162). Either may be NULL. */
+/* Bytes of O_partial and of LSE_partial needed for p (the cudaMallocs of src/main.cu:160-162). Either may be NULL.
+ * With num_splits <= 0 set the fields that the split count depends on first (see above; the other pointers do not matter). */
 int flash_splitkv_workspace_bytes(const flash_params *p, size_t *o_partial_bytes, size_t *lse_partial_bytes);
 
 /* The split count flash_forward_splitkv will use for p (after the heuristic and clamping). */
