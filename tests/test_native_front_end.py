@@ -109,8 +109,10 @@ def test_the_library_builds_without_python():
 def test_the_front_end_is_rebuilt_for_another_torch():
     import torch
 
-    assert "py_binding.cpp" not in _dry_run("native", "-o", "../../include/flash_attn_mi355.h", "-o", "py_binding.cpp")
-    assert "py_binding.cpp" in _dry_run("native", "-W", os.path.join(os.path.dirname(torch.__file__), "version.py"))
+    version = os.path.join(os.path.dirname(torch.__file__), "version.py")
+    settled = [x for f in ("../../include/flash_attn_mi355.h", "py_binding.cpp", "split_counters.h") for x in ("-o", f)]
+    assert "py_binding.cpp" not in _dry_run("native", *settled, "-o", version)
+    assert "py_binding.cpp" in _dry_run("native", *settled, "-W", version)
 
 
 def test_counters_of_streams(tmp_path):
