@@ -788,9 +788,10 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
 #pragma unroll
         for (int u = 0; u < NSTG; ++u)
             if (u < nt) dma_tile(tile_begin + wave + 4 * u, u);
+        stamps.take(1);
+        if constexpr (kStamp) __builtin_amdgcn_sched_barrier(0);  // (ahead of the work on Q, whose wait drains the requests too)
         set_bounds();
         read_slope();
-        stamps.take(1);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         pin_q();
         stamps.take(2);
