@@ -1,6 +1,5 @@
 """The native front end of the binding (csrc/py_binding.cpp) against binding.py's own path, which the debug outputs take:
 same kernels, so bit-identical results whatever way the arguments come."""
-import contextlib
 import os
 import subprocess
 import sys
@@ -13,28 +12,6 @@ from helpers import randn_f16_gpu
 
 def _call(fa, entry, tensors, **kw):
     return (fa.flash_forward if entry == "forward" else fa.flash_forward_splitkv)(*tensors, **kw)
-
-
-@contextlib.contextmanager
-def _front_end_watched(fa):
-    """Yields a list that collects, call by call, whether the front end served it."""
-    front = fa.binding._front_end()
-    seen = []
-    real = fa.binding._native
-
-    class Spy:
-        def __getattr__(self, name):
-            def f(*a):
-                r = getattr(front, name)(*a)
-                seen.append(r is not NotImplemented)
-                return r
-            return f
-
-    fa.binding._native = Spy()
-    try:
-        yield seen
-    finally:
-        fa.binding._native = real
 
 
 @pytest.mark.gpu
@@ -65,8 +42,23 @@ def test_matches_the_binding_s_own_path(fa, entry, Nq, kw, own_buffers):
         extra = dict(out=torch.empty_like(o0), lse=torch.empty_like(l0), stream=s)
         if entry == "splitkv":
             extra["workspace"] = (torch.empty(2 * 4 * 8 * Nq * 40, device="cuda"), torch.empty(2 * 4 * 8 * Nq, device="cuda"))
-    with _front_end_watched(fa) as seen:
+    front = fa.binding._front_end()
+    seen = []
+    real = fa.binding._native
+
+    class Spy:
+        def __getattr__(self, name):
+            def f(*a):
+                r = getattr(front, name)(*a)
+                seen.append(r is not NotImplemented)
+                return r
+            return f
+
+    fa.binding._native = Spy()
+    try:
         o1, l1 = _call(fa, entry, (q, k, v), **extra, **kw)
+    finally:
+        fa.binding._native = real
     torch.cuda.synchronize()
     assert seen == [True]
     if entry == "forward":  # (a hint can change the automatic split count and with it the rounding)
@@ -171,15 +163,16 @@ def test_allocations_are_seen_by_those_who_look(fa):
     assert sizes == [(1, 2, 3, 40), (1, 2, 3), (1, 2, 3, 40), (1, 2, 3), (2 * 2 * 3 * 40,), (2 * 2 * 3,)]
     assert all(torch.equal(a, b) for w, g in zip(want, got) for a, b in zip(w, g))
     before = torch.utils.deterministic.fill_uninitialized_memory
-    with _front_end_watched(fa) as seen:
-        torch.use_deterministic_algorithms(True)
-        try:
-            for torch.utils.deterministic.fill_uninitialized_memory in (True, False):
-                assert torch.equal(fa.flash_forward(q, k, v)[0], want[0][0])
-        finally:
-            torch.use_deterministic_algorithms(False)
-            torch.utils.deterministic.fill_uninitialized_memory = before
-    assert seen == [False, True]
+    front, rest = fa.binding._front_end(), (None, False, (-1, -1), None, 0.0, 0, 0, None, None, None)
+    torch.use_deterministic_algorithms(True)
+    try:
+        for torch.utils.deterministic.fill_uninitialized_memory in (True, False):
+            served = front.forward(q, k, v, *rest) is not NotImplemented
+            assert served != torch.utils.deterministic.fill_uninitialized_memory
+            assert torch.equal(fa.flash_forward(q, k, v)[0], want[0][0])
+    finally:
+        torch.use_deterministic_algorithms(False)
+        torch.utils.deterministic.fill_uninitialized_memory = before
 
 
 @pytest.mark.gpu
