@@ -121,6 +121,9 @@ __device__ __forceinline__ v4u load_chunk_anyalign(const half_t* __restrict__ ro
 // until then probabilities are taken relative to the stale maximum (bounded by 2^kLazyTau, exact in the end
 // because numerator and denominator carry the same factor).  Saves the per-tile rescale of the O accumulators.
 constexpr float kLazyTau = 8.0f;
+// Running maximum (log2 units) of a row that has seen no key: the lowest finite number, relative to which a masked score is
+// still 2^-inf = 0 and every visible one raises it; -inf would need a case of its own wherever it is subtracted.
+constexpr float kNothingSeen = -3.402823466e38f;
 
 // variant bits of the kernel template
 // kVarStamp: debug time stamps.  kVarAlibiLeft (with kVarAlibi, kVarVec): every visible key lies at or left of its row
@@ -238,6 +241,9 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // test), nothing outside [lo_min, hi_max] is visible to any of them (a tile outside it is skipped by the wave)
     int lo_max, hi_min, lo_min, hi_max;
     bool straight;  // the rows' positions follow each other
+    // the same in tiles of the work-group's range: first one and number of those that some row of the wave sees, and of those
+    // that every row sees whole
+    int live0, nlive, clean0, nclean;
     auto set_bounds = [&]() __attribute__((always_inline)) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -273,6 +279,11 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                 hi_max = min(hi_max, kmax - 1);
             }
         }
+        // (a wave whose rows all lie past Nq sees nothing: it only helps to stage the tiles)
+        live0 = (lo_min >> 6) - tile_begin;
+        nlive = q0 + wave_row0 < Nq ? max(0, (hi_max >> 6) - tile_begin - live0 + 1) : 0;
+        clean0 = ((lo_max + 63) >> 6) - tile_begin;
+        nclean = max(0, ((hi_min - 63) >> 6) - tile_begin - clean0 + 1);
     };
 
     const half_t* __restrict__ Qbh = a.Q + (size_t)bh * Nq * d;
@@ -367,6 +378,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // Rows shorter than the bucket: chunk positions past the row's whole chunks fetch the row's last 16 bytes (see
     // load_chunk_anyalign): for K they meet zero columns of Q, for V they only reach rows of O^T that are never stored.
     const int row_bytes = kFullD ? D * 2 : d * 2;
+    const int whole_tiles = Nk / BC;  // tiles of the sequence that hold BC keys
     auto chunk_offset = [&](int c) { return kFullD ? c * 16 : (c * 8 + 8 <= d ? c * 16 : (d - 8) * 2); };
     // (narrow: every block of a tile is the wave's own, and so is the buffer; both permutations repeat every 16 rows, which are
     // CH / 4 blocks, so that only the first CH / 4 requests need offsets of their own and all others are the same some
@@ -398,7 +410,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         // arithmetic at all; only the last tile of a ragged sequence adjusts rows: keys past Nk re-read key Nk - 1
         // (their scores are masked).
         const size_t tb = (size_t)tile * (size_t)(BC * row_bytes);
-        const int rows_left = Nk - tile * BC;  // >= 1
+        const bool whole = tile < whole_tiles;
         FA_LDS char* const kst = (FA_LDS char*)smem + lds_base + stage * C::KBUF;
         FA_LDS char* const vst = (FA_LDS char*)smem + lds_base + NSTG * C::KBUF + stage * C::VBUF;
         const char* const Kb = reinterpret_cast<const char*>(Kbh) + tb;
@@ -431,7 +443,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                 request(Vb, voff[i % NVO], vrow[i % NVO], i / NVO * 16, vst + block_of(i) * 1024);
             }
         };
-        if (rows_left >= BC) issue(std::false_type{});
+        if (whole) issue(std::false_type{});
         else issue(std::true_type{});
     };
     auto dma_tile = [&](int tile, int stage) { dma_tile_parts(tile, stage, std::true_type{}, std::true_type{}); };
@@ -444,10 +456,11 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
 
     // ---- accumulators
     v16f oacc[MB][NB];
-    float m_ref[NB], l_run[NB];
+    float m_ref[NB], m_thr[NB], l_run[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-        m_ref[nb] = -INFINITY;
+        m_ref[nb] = kNothingSeen;
+        m_thr[nb] = -INFINITY;
         l_run[nb] = 0.0f;
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
@@ -462,6 +475,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     const float c2 = a.scale_log2;
     const bool scale_late = !kEvery || c2 > 0.0f;
     const float cs = scale_late ? c2 : 1.0f;
+    const float inv_cs = __builtin_amdgcn_rcpf(cs);  // (of the raise threshold alone: whether a row is rescaled is no matter of its last bit)
     // The ALiBi slope of the head is read once the first tile requests are on their way (read_slope below): it is a
     // vector load, the wait for it counts every older request as well, and nothing before the first softmax needs it.
     float slope2 = 0.0f, nsig = 0.0f;
@@ -560,9 +574,9 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     };
 
     // online softmax of one tile (per query row = per lane); leaves P^T packed to fp16 in pf
-    // mask_sides: bit 0 = some row of the wave has its first allowed key inside or after this tile, bit 1 = some row
-    // has its last allowed key inside or before it (both wave-uniform)
-    auto softmax = [&](int mask_sides, int kb0, v16f (&s)[2][NB], v8h (&pf)[2][2][NB]) {
+    // masked: some row of the wave does not see all of the tile; then mask_sides: bit 0 = some row of the wave has its first
+    // allowed key inside or after this tile, bit 1 = some row has its last allowed key inside or before it (wave-uniform)
+    auto softmax = [&](bool masked, int kb0, v16f (&s)[2][NB], v8h (&pf)[2][2][NB]) {
         constexpr bool folded = kFoldAlibi;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
@@ -589,13 +603,16 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                             s[kb][nb][r] = s[kb][nb][r] * c2 - slope2 * __builtin_fabsf(jb + (float)(32 * kb + 8 * (r >> 2) + (r & 3)));
                 }
             }
-            if (mask_sides != 0) {
+            if (masked) {
                 // Wave-uniform and rare (boundary tiles only); the masking itself is inline asm (common.h), which keeps
                 // these real branches.  The bounds of the wave's rows run along block diagonals when they move by one
                 // key per row and start at a multiple of 32 (causal masks and windows whose offsets are multiples of 32,
                 // rows not clipped by a sequence or split end): then lane-mask constants per 32-key block do the
                 // masking; otherwise a tile takes one comparison per score and crossed end of the interval.
+                // (kb0 is laundered: the compiler otherwise carries what it makes of it here through every tile)
                 const float ninf = -INFINITY;
+                asm volatile("" : "+s"(kb0));
+                const int mask_sides = (kb0 < lo_max ? 1 : 0) | (kb0 + BC - 1 > hi_min ? 2 : 0);
                 const bool hi_diag = NB == 1 && straight && hi_max - hi_min == 31 && (hi_min & 31) == 0;
                 const bool lo_diag = NB == 1 && straight && lo_max - lo_min == 31 && (lo_min & 31) == 0;
                 if (((mask_sides & 1) == 0 || lo_diag) && ((mask_sides & 2) == 0 || hi_diag)) {
@@ -633,42 +650,36 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                         }
                 }
             }
-            float mx = -INFINITY;
-            if constexpr (folded) {
-                float mk[2] = {-INFINITY, -INFINITY};
+            // Row maximum of the lane's own scores (half of the row's keys: the other half sits in lane l ^ 32), two chains side
+            // by side.  Whether some row outgrows the running maximum is asked without the exchange between the two lanes and
+            // in score units, against a threshold that is worked out where the maximum is raised: one comparison per tile,
+            // where exchange, scaling and sum took ten dependent instructions.
+            float mk[2] = {-INFINITY, -INFINITY};
 #pragma unroll
-                for (int kb = 0; kb < 2; ++kb)
+            for (int r = 0; r < 16; ++r)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) mk[kb] = fmaxf(mk[kb], s[kb][nb][r]);
-                mx = fmaxf(mk[0] + abias[0], mk[1] + abias[1]);
-            } else {
-#pragma unroll
-                for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kb][nb][r]);
-            }
-            mx = xhalf_max(mx);
-            mx *= cs;  // cs > 0
-            if (__builtin_amdgcn_ballot_w64(mx > m_ref[nb] + kLazyTau) != 0ull) {
-                const float m_new = fmaxf(m_ref[nb], mx);
-                float alpha = (m_new == -INFINITY) ? 1.0f : fast_exp2(m_ref[nb] - m_new);
+                for (int kb = 0; kb < 2; ++kb) mk[kb] = fmaxf(mk[kb], s[kb][nb][r]);
+            float mx = folded ? fmaxf(mk[0] + abias[0], mk[1] + abias[1]) : fmaxf(mk[0], mk[1]);
+            if (__builtin_amdgcn_ballot_w64(mx > m_thr[nb]) != 0ull) {
+                const float m_new = fmaxf(m_ref[nb], xhalf_max(mx) * cs);  // cs > 0
+                float alpha = fast_exp2(m_ref[nb] - m_new);
                 asm volatile("; raise running max" : "+v"(alpha));  // keeps the rescale inside this rare branch
                 m_ref[nb] = m_new;
+                m_thr[nb] = (m_new + kLazyTau) * inv_cs;
                 l_run[nb] *= alpha;
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) oacc[mb][nb][r] *= alpha;
             }
-            const float m_use = (m_ref[nb] == -INFINITY) ? 0.0f : m_ref[nb];  // nothing seen yet: exp2(-inf - 0) = 0
             float rs = 0.0f;
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
-                const float addend = folded ? __builtin_fmaf(abias[kb], cs, -m_use) : -m_use;
+                const float addend = folded ? __builtin_fmaf(abias[kb], cs, -m_ref[nb]) : -m_ref[nb];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const float p = fast_exp2(__builtin_fmaf(s[kb][nb][r], cs, addend));
-                    rs += p;
+                    rs = kb == 0 && r == 0 ? p : rs + p;
                     s[kb][nb][r] = p;
                 }
             }
@@ -767,15 +778,14 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // A wave whose rows all lie past Nq (fewer than 128 query rows: short prompts, or the heads of one K/V head decoding
     // together) only helps to stage the tiles, and so does any wave for a tile that none of its rows can see (the far
     // end of the causal diagonal block, the near end of a sliding window).
-    const bool wave_live = q0 + wave_row0 < Nq;
+    auto tile_live = [&](int t) { return (unsigned)(t - live0) < (unsigned)nlive; };
+    auto tile_masked = [&](int t) { return (unsigned)(t - clean0) >= (unsigned)nclean; };
     auto tile_math = [&](int t, int buf) {
-        const int kb0 = (tile_begin + t) * BC;
-        if (wave_live && kb0 <= hi_max && kb0 + BC - 1 >= lo_min) {
+        if (tile_live(t)) {
             v16f s[2][NB];
             v8h pf[2][2][NB];
-            const int mask_sides = (kb0 < lo_max ? 1 : 0) | (kb0 + BC - 1 > hi_min ? 2 : 0);
             qk(buf, s);
-            softmax(mask_sides, kb0, s, pf);
+            softmax(tile_masked(t), (tile_begin + t) * BC, s, pf);
             pv(buf, pf);
         }
     };
@@ -815,8 +825,8 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
             // as the V buffer has been read; each is waited for right before its first use, the younger request of the
             // other tensor staying in flight.
             for (int n = 0; n < nt; ++n) {
-                const int kb0 = (tile_begin + wave + 4 * n) * BC;
-                const bool live = wave_live && kb0 <= hi_max && kb0 + BC - 1 >= lo_min;
+                const int t = wave + 4 * n;
+                const bool live = tile_live(t);
                 const bool more = n + 1 < nt;
                 v16f s[2][NB];
                 v8h pf[2][2][NB];
@@ -825,7 +835,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                     dma_tile_parts(tile_begin + wave + 4 * (n + 1), 0, std::true_type{}, std::false_type{});
                 }
-                if (live) softmax((kb0 < lo_max ? 1 : 0) | (kb0 + BC - 1 > hi_min ? 2 : 0), kb0, s, pf);
+                if (live) softmax(tile_masked(t), (tile_begin + t) * BC, s, pf);
                 // V(n): older than the K request just issued
                 if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NKX) : "memory");
                 else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -839,8 +849,8 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
             }
         }
     } else if constexpr (kDma) {
-        // Tile t + PF is requested when tile t starts (its stage was read last during tile t - 1, behind a barrier);
-        // before the barrier that ends tile t, the requests of tile t + 1 have landed, those of t + 2 may be in flight.
+        // Tile t + 2 is requested when tile t is done (its stage has been read, behind a barrier); before the barrier that ends
+        // tile t, the requests of tile t + 1 have landed.
         // Before tile 0 every stage is free: the prologue requests one tile per stage, so that the request which
         // tile 0 would issue is already on its way (a work-group with few tiles otherwise pays the memory latency a
         // second time at the end of its first tile).
@@ -851,9 +861,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         auto nth = [&](int t) { return kFoldAlibi ? ntiles - 1 - t : kPair ? 2 * t + half : t; };
         // (paired: both halves go round as often, for the barrier; the second one's last tile may not exist)
         const int rounds = kPair ? (ntiles + 1) / 2 : ntiles;
-        constexpr int PF = NSTG - 1;
-        static_assert(PF == 1 || PF == 2, "prefetch distance");
-        static_assert(NKX + NVX <= 63, "vmcnt immediate");
+        static_assert(NSTG == 2, "a stage that is read and one that is filled");
 #pragma unroll
         for (int u = 0; u < NSTG; ++u)
             if (u < rounds && (!kPair || nth(u) < ntiles)) dma_tile(tile_begin + nth(u), u);
@@ -865,16 +873,16 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         stamps.take(2);
         __syncthreads();
         stamps.take(3);
-        int buf = 0, nbuf = PF % NSTG;  // stages of tile t and of tile t + PF
+        int buf = 0;  // stage of tile t
         for (int t = 0; t < rounds; ++t) {
-            const bool more = kPair ? nth(t + PF) < ntiles : t + PF < ntiles;
-            if (more && t > 0) dma_tile(tile_begin + nth(t + PF), nbuf);
             if (!kPair || nth(t) < ntiles) tile_math(nth(t), buf);
             if (kStamp && t == 0) stamps.take(4);
-            dma_wait(PF == 2 && more);
+            dma_wait(false);
             __syncthreads();
-            buf = buf + 1 == NSTG ? 0 : buf + 1;
-            nbuf = nbuf + 1 == NSTG ? 0 : nbuf + 1;
+            // (the request stands at the end so that the first tile, whose successor is on its way already, is no case of its own:
+            // a copy of the tile's code costs a launch of few tiles its way through a cold instruction cache)
+            if (kPair ? nth(t + 2) < ntiles : t + 2 < ntiles) dma_tile(tile_begin + nth(t + 2), buf);
+            buf ^= 1;
         }
     } else {
         // double-buffered through registers: tile t+1 is fetched from global memory while tile t is computed
@@ -943,14 +951,13 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         // thread -> one row and D / 8 consecutive chunk positions of it
         constexpr int CPT = D / 8;
         const int row = tid >> 3, cp0 = (tid & 7) * CPT;
-        float M = -INFINITY;
+        float M = kNothingSeen;
 #pragma unroll
         for (int w = 0; w < 4; ++w) M = fmaxf(M, sm[w * 32 + row]);
-        const float Mu = (M == -INFINITY) ? 0.0f : M;
         float L = 0.0f, wgt[4];
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
-            wgt[w] = fast_exp2(sm[w * 32 + row] - Mu);
+            wgt[w] = fast_exp2(sm[w * 32 + row] - M);
             L += wgt[w] * sl[w * 32 + row];
         }
         const float inv = L > 0.0f ? (kDropout ? a.drop_rscale : 1.0f) / L : 0.0f;
@@ -993,8 +1000,8 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         }
         __syncthreads();
         if (half == 1) return;
-        const float m1 = mine[0], M = fmaxf(m_ref[0], m1), Mu = (M == -INFINITY) ? 0.0f : M;
-        const float w0 = fast_exp2(m_ref[0] - Mu), w1 = fast_exp2(m1 - Mu);
+        const float m1 = mine[0], M = fmaxf(m_ref[0], m1);
+        const float w0 = fast_exp2(m_ref[0] - M), w1 = fast_exp2(m1 - M);
         m_ref[0] = M;
         l_run[0] = __builtin_fmaf(w1, mine[64], w0 * l_run[0]);
 #pragma unroll

@@ -214,7 +214,7 @@ __global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const FwdArgs a)
 
     // ---- accumulators
     v16f oacc[MB];
-    float m_ref = -INFINITY, l_run = 0.0f;
+    float m_ref = kNothingSeen, m_thr = -INFINITY, l_run = 0.0f;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -224,6 +224,7 @@ __global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const FwdArgs a)
     // into the exponent (one fma per score): cs = scale, and the ALiBi bias is added beforehand divided by the scale.
     // (The host sends a non-positive scale to the element-wise instance of the 4-wave kernel.)
     const float c2 = a.scale_log2, cs = c2;
+    const float inv_cs = __builtin_amdgcn_rcpf(cs);  // (of the raise threshold alone)
     float nsig = 0.0f;  // ALiBi slope / scale, negated: read behind the prologue requests (below)
 
     // Lane parts of the fragment addresses (layout above).  K fragment (ks, kb): key 32 kb + l32, chunk 2 ks + g
@@ -385,32 +386,31 @@ __global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const FwdArgs a)
                 }
             }
         }
+        // (the lane's half of the row's keys alone, in score units: see fwd_kernel.h)
         float mx = -INFINITY;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kb][r]);
-        mx = xhalf_max(mx);
-        mx *= cs;  // cs > 0
-        if (__builtin_amdgcn_ballot_w64(mx > m_ref + kLazyTau) != 0ull) {
-            const float m_new = fmaxf(m_ref, mx);
-            float alpha = (m_new == -INFINITY) ? 1.0f : fast_exp2(m_ref - m_new);
+        if (__builtin_amdgcn_ballot_w64(mx > m_thr) != 0ull) {
+            const float m_new = fmaxf(m_ref, xhalf_max(mx) * cs);  // cs > 0
+            float alpha = fast_exp2(m_ref - m_new);
             asm volatile("; raise running max" : "+v"(alpha));
             m_ref = m_new;
+            m_thr = (m_new + kLazyTau) * inv_cs;
             l_run *= alpha;
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) oacc[mb][r] *= alpha;
         }
-        const float m_use = (m_ref == -INFINITY) ? 0.0f : m_ref;
         float rs = 0.0f;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const float p = fast_exp2(__builtin_fmaf(s[kb][r], cs, -m_use));
-                rs += p;
+                const float p = fast_exp2(__builtin_fmaf(s[kb][r], cs, -m_ref));
+                rs = kb == 0 && r == 0 ? p : rs + p;
                 s[kb][r] = p;
             }
         l_run += rs;
