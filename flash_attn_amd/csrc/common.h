@@ -138,6 +138,16 @@ __device__ __forceinline__ size_t partial_row(const FwdArgs& a, int bh, int spli
     return ((size_t)bh * a.num_splits + split) * a.Nq + r;
 }
 
+// Index of this lane in its wave, worked out where it is asked for: in rare branches and behind loops, so that nothing made of
+// it occupies a register throughout a loop (as an ordinary expression the compiler moves it, and whatever follows from it,
+// in front of the loop).
+__device__ __forceinline__ int lane_here()
+{
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    return l;
+}
+
 __device__ __forceinline__ int wave_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // Q chunk for the chunk position at column col (a multiple of 8) of a row of d >= 8 elements at any alignment, where the
@@ -369,56 +379,92 @@ __device__ __forceinline__ void mul_wide_u32(uint32_t m, uint32_t x, uint32_t& h
     lo = (uint32_t)r;
 }
 
-// Element masks of a 32 x 32 score block whose boundary runs along its diagonal.  In the accumulator layout lane
+// Element masks of a tile: two 32 x 32 score blocks (keys 0 ... 31 and 32 ... 63 of the tile).  In the accumulator layout lane
 // (l32 = lane % 32, g = lane / 32) holds in register r the score of query row l32 and key 8 (r / 4) + r % 4 + 4 g of the
-// block, so "key right of the diagonal" (key > row) and "key left of it" (key < row) are fixed sets of lanes per register:
-// sixteen 64-bit constants each, applied with one v_cndmask per register on a constant lane mask instead of a comparison
-// and a select per score.
-constexpr uint64_t diag_lane_mask(int r, bool right)
+// block.  A block's mode is a sum of
+//   kMaskRight, kMaskLeft   the boundary runs along the block's diagonal, and the keys right of it (key > row) or left of it
+//                           (key < row) go: a fixed set of lanes per register, in either half of the lanes the first so many
+//                           rows or all but these, which s_bfm makes; one v_cndmask per score
+//   kMaskAbove, kMaskBelow  keys above `hi` or below `lo` go (the lane's own bounds, counted from the tile's first key plus the
+//                           lane's 4 g): a comparison and a v_cndmask per score
+//   kMaskWhole              all of it goes
+// and 0 leaves the block alone; `modes` holds the first block's in bits 0-7, the second one's in bits 8-15.
+// One statement with its branches inside, and a block's sixteen registers as one operand, on purpose: with branches that the
+// compiler sees, or with an operand per register, one path or the other ends in copies of the accumulators, 64 v_mov per
+// boundary tile and as many registers to copy into, which cost the instances for d <= 96 registers and a work-group per CU.  The assembler
+// takes the number of the first register out of the operand's name.
+// (The wait states at the head: whoever produced the scores may have been an MFMA right in front, which the compiler does not
+// account for where it cannot see who reads them.)
+constexpr int kMaskRight = 1, kMaskLeft = 2, kMaskAbove = 4, kMaskBelow = 8, kMaskWhole = 16;
+// SYM: the first number of the operand's "v[first:last]"; anything but sixteen vector registers is an error
+#define FA_FIRST_REGISTER(SYM, OPERAND) \
+    ".set " SYM ", 0\n\t.set fa_last, 0\n\t.set fa_in, 0\n\t.irpc fa_c, \"" OPERAND "\"\n\t" \
+    ".ifc \\fa_c,:\n\t.set fa_in, 2\n\t.endif\n\t.ifc \\fa_c,]\n\t.set fa_in, 3\n\t.endif\n\t" \
+    ".if fa_in == 1\n\t.set " SYM ", " SYM " * 10 + \\fa_c\n\t.endif\n\t" \
+    ".if fa_in == 2\n\t.ifnc \\fa_c,:\n\t.set fa_last, fa_last * 10 + \\fa_c\n\t.endif\n\t.endif\n\t" \
+    ".ifc \\fa_c,[\n\t.set fa_in, 1\n\t.endif\n\t.endr\n\t" \
+    ".if fa_last - " SYM " - 15\n\t.error \"an accumulator of sixteen registers\"\n\t.endif\n\t"
+// register, its key in the lower half of the lanes, in the upper half, and the lower one counted from the tile's start
+#define FA_MASK_16A(X) X("fa_a+0", 0, 4, 0) X("fa_a+1", 1, 5, 1) X("fa_a+2", 2, 6, 2) X("fa_a+3", 3, 7, 3) X("fa_a+4", 8, 12, 8) \
+    X("fa_a+5", 9, 13, 9) X("fa_a+6", 10, 14, 10) X("fa_a+7", 11, 15, 11) X("fa_a+8", 16, 20, 16) X("fa_a+9", 17, 21, 17) \
+    X("fa_a+10", 18, 22, 18) X("fa_a+11", 19, 23, 19) X("fa_a+12", 24, 28, 24) X("fa_a+13", 25, 29, 25) X("fa_a+14", 26, 30, 26) \
+    X("fa_a+15", 27, 31, 27)
+#define FA_MASK_16B(X) X("fa_b+0", 0, 4, 32) X("fa_b+1", 1, 5, 33) X("fa_b+2", 2, 6, 34) X("fa_b+3", 3, 7, 35) X("fa_b+4", 8, 12, 40) \
+    X("fa_b+5", 9, 13, 41) X("fa_b+6", 10, 14, 42) X("fa_b+7", 11, 15, 43) X("fa_b+8", 16, 20, 48) X("fa_b+9", 17, 21, 49) \
+    X("fa_b+10", 18, 22, 50) X("fa_b+11", 19, 23, 51) X("fa_b+12", 24, 28, 56) X("fa_b+13", 25, 29, 57) X("fa_b+14", 26, 30, 58) \
+    X("fa_b+15", 27, 31, 59)
+#define FA_MASK_RIGHT(R, K, K4, T) \
+    "s_bfm_b32 vcc_lo, " #K ", 0\n\ts_bfm_b32 vcc_hi, " #K4 ", 0\n\tv_cndmask_b32_e32 v[" R "], v[" R "], %[ninf], vcc\n\t"
+#define FA_MASK_LEFT(R, K, K4, T) \
+    "s_bfm_b64 vcc, " #K4 "+1, 32\n\ts_bfm_b32 vcc_lo, " #K "+1, 0\n\tv_cndmask_b32_e32 v[" R "], %[ninf], v[" R "], vcc\n\t"
+#define FA_MASK_ABOVE(R, K, K4, T) "v_cmp_gt_i32_e32 vcc, " #T ", %[hi]\n\tv_cndmask_b32_e32 v[" R "], v[" R "], %[ninf], vcc\n\t"
+#define FA_MASK_BELOW(R, K, K4, T) "v_cmp_lt_i32_e32 vcc, " #T ", %[lo]\n\tv_cndmask_b32_e32 v[" R "], v[" R "], %[ninf], vcc\n\t"
+#define FA_MASK_WHOLE(R, K, K4, T) "v_mov_b32 v[" R "], %[ninf]\n\t"
+#define FA_MASK_IF(BIT, NAME, BODY) "s_bitcmp1_b32 %[modes], " #BIT "\n\ts_cbranch_scc0 .Lfa_" NAME "%=\n\t" BODY ".Lfa_" NAME "%=:\n\t"
+template <bool kDiagonals>
+__device__ __forceinline__ void mask_tile(v16f& s0, v16f& s1, int modes, int lo, int hi, float ninf)
 {
-    uint64_t m = 0;
-    for (int lane = 0; lane < 64; ++lane) {
-        const int row = lane & 31, key = 8 * (r >> 2) + (r & 3) + 4 * (lane >> 5);
-        if (right ? key > row : key < row) m |= 1ull << lane;
-    }
-    return m;
+    if constexpr (kDiagonals)
+        asm(FA_FIRST_REGISTER("fa_a", "%[s0]") FA_FIRST_REGISTER("fa_b", "%[s1]") "s_nop 15\n\t"
+            FA_MASK_IF(0, "ar", FA_MASK_16A(FA_MASK_RIGHT)) FA_MASK_IF(1, "al", FA_MASK_16A(FA_MASK_LEFT))
+            FA_MASK_IF(2, "aa", FA_MASK_16A(FA_MASK_ABOVE)) FA_MASK_IF(3, "ab", FA_MASK_16A(FA_MASK_BELOW))
+            FA_MASK_IF(4, "aw", FA_MASK_16A(FA_MASK_WHOLE))
+            FA_MASK_IF(8, "br", FA_MASK_16B(FA_MASK_RIGHT)) FA_MASK_IF(9, "bl", FA_MASK_16B(FA_MASK_LEFT))
+            FA_MASK_IF(10, "ba", FA_MASK_16B(FA_MASK_ABOVE)) FA_MASK_IF(11, "bb", FA_MASK_16B(FA_MASK_BELOW))
+            FA_MASK_IF(12, "bw", FA_MASK_16B(FA_MASK_WHOLE))
+            : [s0] "+v"(s0), [s1] "+v"(s1)
+            : [modes] "s"(modes), [lo] "v"(lo), [hi] "v"(hi), [ninf] "v"(ninf)
+            : "vcc", "scc");
+    else
+        asm(FA_FIRST_REGISTER("fa_a", "%[s0]") FA_FIRST_REGISTER("fa_b", "%[s1]") "s_nop 15\n\t"
+            FA_MASK_IF(2, "a", FA_MASK_16A(FA_MASK_ABOVE) FA_MASK_16B(FA_MASK_ABOVE))
+            FA_MASK_IF(3, "b", FA_MASK_16A(FA_MASK_BELOW) FA_MASK_16B(FA_MASK_BELOW))
+            : [s0] "+v"(s0), [s1] "+v"(s1)
+            : [modes] "s"(modes), [lo] "v"(lo), [hi] "v"(hi), [ninf] "v"(ninf)
+            : "vcc", "scc");
 }
-template <bool kRight, int R = 0>
-__device__ __forceinline__ void mask_off_diagonal(v16f& s, float ninf)
+// Modes of a tile whose first key is kb0, for rows that see keys from lo_min ... lo_max on and up to hi_min ... hi_max (their
+// bounds, which one after the other moves by one key per row where `straight`); sides: bit 0, the first key matters here,
+// bit 1, the last one does.
+template <bool kDiagonals>
+__device__ __forceinline__ int mask_modes(int kb0, int sides, bool straight, int lo_min, int lo_max, int hi_min, int hi_max)
 {
-    if constexpr (R < 16) {
-        // (the constant goes into vcc inside the statement: as an operand the compiler would keep all thirty-two
-        // constants in scalar registers across the key loop and spill them)
-        constexpr uint64_t m = diag_lane_mask(R, kRight);
-        asm("s_mov_b32 vcc_lo, %2\n\ts_mov_b32 vcc_hi, %3\n\tv_cndmask_b32_e32 %0, %0, %1, vcc"
-            : "+v"(s[R])
-            : "v"(ninf), "n"((uint32_t)m), "n"((uint32_t)(m >> 32))
-            : "vcc");
-        mask_off_diagonal<kRight, R + 1>(s, ninf);
-    }
-}
-
-// The general case: the score in register R belongs to key 8 (R / 4) + R % 4 of the block (the caller folds the lane's
-// 4 g and the block's position into the bound); scores of keys above (below) the lane's bound become -inf.  In place
-// and as inline asm on purpose: written as selects the compiler copies the sixteen accumulator registers first, and
-// turns a rare wave-uniform branch around them into selects that every tile executes.
-template <bool kAbove, int R = 0>
-__device__ __forceinline__ void mask_beyond(v16f& s, int bound, float ninf)
-{
-    if constexpr (R < 16) {
-        constexpr int key = 8 * (R >> 2) + (R & 3);
-        if constexpr (kAbove)
-            asm("v_cmp_gt_i32_e32 vcc, %2, %1\n\tv_cndmask_b32_e32 %0, %0, %3, vcc" : "+v"(s[R]) : "v"(bound), "n"(key), "v"(ninf) : "vcc");
-        else
-            asm("v_cmp_lt_i32_e32 vcc, %2, %1\n\tv_cndmask_b32_e32 %0, %0, %3, vcc" : "+v"(s[R]) : "v"(bound), "n"(key), "v"(ninf) : "vcc");
-        mask_beyond<kAbove, R + 1>(s, bound, ninf);
-    }
-}
-
-__device__ __forceinline__ void mask_whole_block(v16f& s, float ninf)
-{
+    const bool hi_diag = straight && hi_max - hi_min == 31 && (hi_min & 31) == 0;
+    const bool lo_diag = straight && lo_max - lo_min == 31 && (lo_min & 31) == 0;
+    if (kDiagonals && ((sides & 1) == 0 || lo_diag) && ((sides & 2) == 0 || hi_diag)) {
+        int modes = 0;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) asm("v_mov_b32 %0, %1" : "=v"(s[r]) : "v"(ninf));
+        for (int kb = 0; kb < 2; ++kb) {
+            // last / first visible key of the wave's first row relative to the block: multiples of 32
+            const int dh = (sides & 2) ? hi_min - (kb0 + 32 * kb) : 64;
+            const int dl = (sides & 1) ? lo_min - (kb0 + 32 * kb) : -64;
+            const int m = dh < 0 || dl >= 32 ? kMaskWhole : (dh == 0 ? kMaskRight : 0) + (dl == 0 ? kMaskLeft : 0);
+            modes |= m << (8 * kb);
+        }
+        return wave_uniform(modes);  // (it is; said, because the compiler may hold it in a vector register)
+    }
+    const int m = ((sides & 1) ? kMaskBelow : 0) + ((sides & 2) ? kMaskAbove : 0);
+    return wave_uniform(m | m << 8);
 }
 
 // three-input exclusive or in one instruction (v_bitop3_b32, truth table 0x96)

@@ -233,10 +233,24 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // are worked out behind the first requests (set_bounds, called below), like everything else that can wait.  A
     // launch of few tiles is bound by its instructions up to there, fetched through a cold instruction cache: 0.1 us per
     // launch (B3 H4 N73 d64 4.92 -> 4.83 us), and B32 H32 N512 d64, whose work-groups have eight tiles each, 107.4 -> 105.9.
-    int row_i[NB], lo[NB], hi[NB];
+    int row_i[NB];
     float iif[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) row_i[nb] = q0 + wave_row0 + nb * 32 + l32;
+    // first and last key that row i sees (asked for in boundary tiles, and worked out there: two registers less in the loop)
+    auto row_bounds = [&](int i, int* lo, int* hi) __attribute__((always_inline)) {
+        const int ii = row_position<kFold>(a, i < Nq ? i : Nq - 1) + shift;
+        int l_ = 0, h_ = Nk - 1;
+        if (a.wl >= 0) l_ = max(0, ii - a.wl);
+        if (a.causal) h_ = min(h_, ii);
+        if (a.wr >= 0) h_ = min(h_, ii + a.wr);
+        if (a.num_splits > 1) {
+            l_ = max(l_, kmin);
+            h_ = min(h_, kmax - 1);
+        }
+        *lo = l_;
+        *hi = h_;
+    };
     // wave-uniform bounds: [lo_max, hi_min] is visible to every row of the wave (a tile inside it needs no element
     // test), nothing outside [lo_min, hi_max] is visible to any of them (a tile outside it is skipped by the wave)
     int lo_max, hi_min, lo_min, hi_max;
@@ -249,18 +263,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             const int i = row_i[nb];
-            const int ii = row_position<kFold>(a, i < Nq ? i : Nq - 1) + shift;
-            int l_ = 0, h_ = Nk - 1;
-            if (a.wl >= 0) l_ = max(0, ii - a.wl);
-            if (a.causal) h_ = min(h_, ii);
-            if (a.wr >= 0) h_ = min(h_, ii + a.wr);
-            if (a.num_splits > 1) {
-                l_ = max(l_, kmin);
-                h_ = min(h_, kmax - 1);
-            }
-            lo[nb] = l_;
-            hi[nb] = h_;
-            iif[nb] = (float)ii;
+            iif[nb] = (float)(row_position<kFold>(a, i < Nq ? i : Nq - 1) + shift);
         }
         {
             const int first = q0 + wave_row0, last = first + C::RW - 1;
@@ -443,7 +446,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                 request(Vb, voff[i % NVO], vrow[i % NVO], i / NVO * 16, vst + block_of(i) * 1024);
             }
         };
-        if (whole) issue(std::false_type{});
+        if (__builtin_expect(whole, 1)) issue(std::false_type{});
         else issue(std::true_type{});
     };
     auto dma_tile = [&](int tile, int stage) { dma_tile_parts(tile, stage, std::true_type{}, std::true_type{}); };
@@ -603,50 +606,31 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                             s[kb][nb][r] = s[kb][nb][r] * c2 - slope2 * __builtin_fabsf(jb + (float)(32 * kb + 8 * (r >> 2) + (r & 3)));
                 }
             }
-            if (masked) {
-                // Wave-uniform and rare (boundary tiles only); the masking itself is inline asm (common.h), which keeps
-                // these real branches.  The bounds of the wave's rows run along block diagonals when they move by one
-                // key per row and start at a multiple of 32 (causal masks and windows whose offsets are multiples of 32,
-                // rows not clipped by a sequence or split end): then lane-mask constants per 32-key block do the
-                // masking; otherwise a tile takes one comparison per score and crossed end of the interval.
+            if (__builtin_expect(masked, 0)) {
+                // (common.h: mask_tile.)  The bounds of the wave's rows run along block diagonals when they move by one key per
+                // row and start at a multiple of 32: causal masks and windows whose offsets are multiples of 32, rows not
+                // clipped by a sequence or split end.
                 // (kb0 is laundered: the compiler otherwise carries what it makes of it here through every tile)
-                const float ninf = -INFINITY;
                 asm volatile("" : "+s"(kb0));
-                const int mask_sides = (kb0 < lo_max ? 1 : 0) | (kb0 + BC - 1 > hi_min ? 2 : 0);
-                const bool hi_diag = NB == 1 && straight && hi_max - hi_min == 31 && (hi_min & 31) == 0;
-                const bool lo_diag = NB == 1 && straight && lo_max - lo_min == 31 && (lo_min & 31) == 0;
-                if (((mask_sides & 1) == 0 || lo_diag) && ((mask_sides & 2) == 0 || hi_diag)) {
-#pragma unroll
-                    for (int kb = 0; kb < 2; ++kb) {
-                        // last / first visible key of the wave's first row relative to the block: multiples of 32
-                        const int dh = (mask_sides & 2) ? hi_min - (kb0 + 32 * kb) : 64;
-                        const int dl = (mask_sides & 1) ? lo_min - (kb0 + 32 * kb) : -64;
-                        if (dh < 0 || dl >= 32) {
-                            mask_whole_block(s[kb][nb], ninf);
-                        } else {
-                            if (dh == 0) mask_off_diagonal<true>(s[kb][nb], ninf);
-                            if (dl == 0) mask_off_diagonal<false>(s[kb][nb], ninf);
-                        }
-                    }
-                } else {
-                    const int lo_rel = lo[nb] - kb0 - 4 * g, hi_rel = hi[nb] - kb0 - 4 * g;
-#pragma unroll
-                    for (int kb = 0; kb < 2; ++kb) {
-                        if (mask_sides & 1) mask_beyond<false>(s[kb][nb], lo_rel - 32 * kb, ninf);
-                        if (mask_sides & 2) mask_beyond<true>(s[kb][nb], hi_rel - 32 * kb, ninf);
-                    }
-                }
+                const int sides = (kb0 < lo_max ? 1 : 0) | (kb0 + BC - 1 > hi_min ? 2 : 0);
+                const int modes = mask_modes<NB == 1>(kb0, sides, straight, lo_min, lo_max, hi_min, hi_max);
+                const int ln = lane_here();
+                int lo, hi;
+                row_bounds(q0 + wave_row0 + nb * 32 + (ln & 31), &lo, &hi);
+                mask_tile<NB == 1>(s[0][nb], s[1][nb], modes, lo - kb0 - 4 * (ln >> 5), hi - kb0 - 4 * (ln >> 5), -INFINITY);
             }
             if constexpr (kEvery) {
                 if (a.scores_out != nullptr && row_i[nb] < Nq) {  // debug dump of the visible scores, natural-log units
                     float* srow = a.scores_out + ((size_t)bh * Nq + row_i[nb]) * Nk;
+                    int lo, hi;
+                    row_bounds(row_i[nb], &lo, &hi);
                     const float unit = (scale_late ? cs : 1.0f) * kLn2;
 #pragma unroll
                     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
                         for (int r = 0; r < 16; ++r) {
                             const int j = kb0 + 4 * g + 32 * kb + 8 * (r >> 2) + (r & 3);
-                            if (j >= lo[nb] && j <= hi[nb]) srow[j] = s[kb][nb][r] * unit;
+                            if (j >= lo && j <= hi) srow[j] = s[kb][nb][r] * unit;
                         }
                 }
             }
@@ -660,7 +644,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
 #pragma unroll
                 for (int kb = 0; kb < 2; ++kb) mk[kb] = fmaxf(mk[kb], s[kb][nb][r]);
             float mx = folded ? fmaxf(mk[0] + abias[0], mk[1] + abias[1]) : fmaxf(mk[0], mk[1]);
-            if (__builtin_amdgcn_ballot_w64(mx > m_thr[nb]) != 0ull) {
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(mx > m_thr[nb]) != 0ull, 0)) {
                 const float m_new = fmaxf(m_ref[nb], xhalf_max(mx) * cs);  // cs > 0
                 float alpha = fast_exp2(m_ref[nb] - m_new);
                 asm volatile("; raise running max" : "+v"(alpha));  // keeps the rescale inside this rare branch
@@ -781,11 +765,12 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     auto tile_live = [&](int t) { return (unsigned)(t - live0) < (unsigned)nlive; };
     auto tile_masked = [&](int t) { return (unsigned)(t - clean0) >= (unsigned)nclean; };
     auto tile_math = [&](int t, int buf) {
-        if (tile_live(t)) {
+        if (__builtin_expect(tile_live(t), 1)) {
             v16f s[2][NB];
             v8h pf[2][2][NB];
+            const int kb0 = (tile_begin + t) * BC;
             qk(buf, s);
-            softmax(tile_masked(t), (tile_begin + t) * BC, s, pf);
+            softmax(tile_masked(t), kb0, s, pf);
             pv(buf, pf);
         }
     };
@@ -1016,7 +1001,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         const float l = xhalf_sum(l_run[nb]);
         const float inv = l > 0.0f ? (kDropout ? a.drop_rscale : 1.0f) / l : 0.0f;
         const float lse = l > 0.0f ? __builtin_fmaf(m_ref[nb], kLn2, fast_log2(l) * kLn2) : -INFINITY;  // (one rounding at the size of m)
-        const int i = row_i[nb];
+        const int i = q0 + wave_row0 + nb * 32 + (lane_here() & 31);
         if (i >= Nq) continue;
         if (a.num_splits > 1) {
             const size_t prow = partial_row<kFold>(a, bh, split, i);
