@@ -379,6 +379,19 @@ __device__ __forceinline__ void mul_wide_u32(uint32_t m, uint32_t x, uint32_t& h
     lo = (uint32_t)r;
 }
 
+// both products of a Philox round (one statement: between two of the above the compiler puts a wait state that nothing needs)
+__device__ __forceinline__ void mul_wide_pair(uint32_t m0, uint32_t x0, uint32_t m1, uint32_t x1, uint32_t& hi0, uint32_t& lo0,
+                                              uint32_t& hi1, uint32_t& lo1)
+{
+    uint64_t r0, r1;
+    asm("v_mad_u64_u32 %0, vcc, %2, %3, 0\n\tv_mad_u64_u32 %1, vcc, %4, %5, 0"
+        : "=&v"(r0), "=v"(r1)
+        : "s"(m0), "v"(x0), "s"(m1), "v"(x1)
+        : "vcc");
+    hi0 = (uint32_t)(r0 >> 32), lo0 = (uint32_t)r0;
+    hi1 = (uint32_t)(r1 >> 32), lo1 = (uint32_t)r1;
+}
+
 // Element masks of a tile: two 32 x 32 score blocks (keys 0 ... 31 and 32 ... 63 of the tile).  In the accumulator layout lane
 // (l32 = lane % 32, g = lane / 32) holds in register r the score of query row l32 and key 8 (r / 4) + r % 4 + 4 g of the
 // block.  A block's mode is a sum of
@@ -391,7 +404,7 @@ __device__ __forceinline__ void mul_wide_u32(uint32_t m, uint32_t x, uint32_t& h
 // and 0 leaves the block alone; `modes` holds the first block's in bits 0-7, the second one's in bits 8-15.
 // One statement with its branches inside, and a block's sixteen registers as one operand, on purpose: with branches that the
 // compiler sees, or with an operand per register, one path or the other ends in copies of the accumulators, 64 v_mov per
-// boundary tile and as many registers to copy into, which cost the instances for d <= 96 registers and a work-group per CU.  The assembler
+// boundary tile and as many registers to copy into, which cost the instances for d <= 96 a work-group per CU.  The assembler
 // takes the number of the first register out of the operand's name.
 // (The wait states at the head: whoever produced the scores may have been an MFMA right in front, which the compiler does not
 // account for where it cannot see who reads them.)
@@ -488,44 +501,77 @@ __device__ __forceinline__ v4u philox4x32_10(uint32_t c0, uint32_t c1, uint32_t 
     return o;
 }
 
-// The same function for callers whose third counter word is the same in every lane (the head slice of a work-group):
-// they pass its first-round product 0xCD9E8D57 * c2 as (c2_hi, c2_lo), computed once on the scalar unit, and the first
-// round is left with one vector multiply; the exclusive-ors of uniform words fold into scalar ones as well.
-__device__ __forceinline__ v4u philox4x32_10_c2(uint32_t c0, uint32_t c1, uint32_t c2_hi, uint32_t c2_lo, uint32_t c3, uint32_t k0,
-                                                uint32_t k1)
+// The same function for the tiled kernels, where a work-group holds one head slice, a lane one query row, and all lanes of a
+// half wave ask for the same call.  Written out, the words that the first three rounds leave depend on the row alone (the
+// first-round word that holds the row number, and its product), on the call and the head slice alone (every other
+// product up to the third round's first), or on both by an exclusive-or -- so a wave works out the call's part for 64 calls
+// at once, a lane each, into LDS (CallTable below), and a call is left with 15 of its 20 integer multiplies, which are what
+// bounds a launch with dropout.  Causal with dropout, 19 multiplies per call -> 15 (and the rounds interleaved with the MFMAs
+// of the second product, see pv in fwd_kernel.h): B8 H16 N1300 d80 77.3 -> 69.4 us, B16 H16 N2048 d64 265 -> 250, B2 H4 N1986 d96
+// (paired) 38.4 -> 35.0, B4 H16 N900 d31 20.5 -> 18.7, B8 H32 N1000 d96 92 -> 89, B4 H16 N2048 d128 (8-wave kernel) 99.7 -> 97.2.
+//   round 1   A0 = hi(M1 bh) ^ i ^ k0   A1 = lo(M1 bh)            A2 = hi(M0 c) ^ off ^ k1    A3 = lo(M0 c)
+//   round 2   B0 = hi(M1 A2) ^ A1 ^ k0' B1 = lo(M1 A2)            B2 = hi(M0 A0) ^ A3 ^ k1'   B3 = lo(M0 A0)
+//   round 3   hi(M1 B2) ^ B1 ^ k0"      lo(M1 B2)                 hi(M0 B0) ^ B3 ^ k1"        lo(M0 B0)
+constexpr uint32_t kPhiloxM0 = 0xD2511F53u, kPhiloxM1 = 0xCD9E8D57u, kPhiloxW0 = 0x9E3779B9u, kPhiloxW1 = 0xBB67AE85u;
+struct PhiloxRow {
+    uint32_t hi, lo;  // M0 A0
+};
+__device__ __forceinline__ PhiloxRow philox_row_part(uint32_t i, uint32_t bh, uint32_t k0)
+{
+    PhiloxRow r;
+    mul_wide_u32(kPhiloxM0, (uint32_t)(((uint64_t)kPhiloxM1 * bh) >> 32) ^ i ^ k0, r.hi, r.lo);
+    return r;
+}
+// {A3 ^ k1', B1 ^ k0", hi(M0 B0) ^ k1", lo(M0 B0)}
+__device__ __forceinline__ v4u philox_call_part(uint32_t c, uint32_t bh, uint32_t off, uint32_t k0, uint32_t k1)
+{
+    uint32_t hi, a3, b1, lo;
+    mul_wide_u32(kPhiloxM0, c, hi, a3);
+    mul_wide_u32(kPhiloxM1, hi ^ (off ^ k1), hi, b1);
+    mul_wide_u32(kPhiloxM0, hi ^ (kPhiloxM1 * bh ^ (k0 + kPhiloxW0)), hi, lo);
+    const v4u r = {a3 ^ (k1 + kPhiloxW1), b1 ^ (k0 + 2 * kPhiloxW0), hi ^ (k1 + 2 * kPhiloxW1), lo};
+    return r;
+}
+__device__ __forceinline__ v4u philox_from_parts(const PhiloxRow& row, const v4u& call, uint32_t k0, uint32_t k1)
 {
     uint32_t hi0, lo0, hi1, lo1;
-    // first Philox round
-    mul_wide_u32(0xD2511F53u, c0, hi0, lo0);
-    uint32_t n0 = c1 ^ (c2_hi ^ k0);
-    const uint32_t u1 = c2_lo;  // uniform
-    uint32_t n2 = hi0 ^ (c3 ^ k1);
-    uint32_t n3 = lo0;
-    k0 += 0x9E3779B9u;
-    k1 += 0xBB67AE85u;
-    // second Philox round: its second word is still uniform
-    mul_wide_u32(0xD2511F53u, n0, hi0, lo0);
-    mul_wide_u32(0xCD9E8D57u, n2, hi1, lo1);
-    c0 = hi1 ^ (u1 ^ k0);
-    c1 = lo1;
-    uint32_t c2 = xor3(hi0, n3, k1);
-    c3 = lo0;
-    k0 += 0x9E3779B9u;
-    k1 += 0xBB67AE85u;
+    mul_wide_u32(kPhiloxM1, row.hi ^ call[0], hi1, lo1);
+    uint32_t c0 = hi1 ^ call[1], c1 = lo1, c2 = call[2] ^ row.lo, c3 = call[3];
 #pragma unroll
-    for (int r = 2; r < 10; ++r) {
-        mul_wide_u32(0xD2511F53u, c0, hi0, lo0);
-        mul_wide_u32(0xCD9E8D57u, c2, hi1, lo1);
-        c0 = xor3(hi1, c1, k0);
+    for (int r = 3; r < 10; ++r) {
+        const uint32_t q0 = k0 + r * kPhiloxW0, q1 = k1 + r * kPhiloxW1;
+        mul_wide_pair(kPhiloxM0, c0, kPhiloxM1, c2, hi0, lo0, hi1, lo1);
+        c0 = xor3(hi1, c1, q0);
         c1 = lo1;
-        c2 = xor3(hi0, c3, k1);
+        c2 = xor3(hi0, c3, q1);
         c3 = lo0;
-        k0 += 0x9E3779B9u;
-        k1 += 0xBB67AE85u;
     }
-    v4u o = {c0, c1, c2, c3};
+    const v4u o = {c0, c1, c2, c3};
     return o;
 }
+
+// The call parts of 64 calls (512 keys, eight tiles) in LDS, one table per wave: nobody else reads it, so nothing but the
+// order of the wave's own LDS operations stands between a refill and the reads.
+template <int kWaves>
+__device__ __forceinline__ v4u* call_table_memory()
+{
+    __shared__ v4u t[kWaves * 64];
+    return t;
+}
+struct CallTable {
+    v4u* mem;    // of the wave
+    int chunk;   // calls 64 chunk ... 64 chunk + 63 are in it
+    // in front of the reads of the tile at key kb0 (wave-uniform)
+    __device__ __forceinline__ void cover(int kb0, int lane, uint32_t bh, uint32_t off, uint32_t k0, uint32_t k1)
+    {
+        if ((kb0 >> 9) != chunk) {
+            chunk = kb0 >> 9;
+            mem[lane] = philox_call_part((uint32_t)(64 * chunk + lane), bh, off, k0, k1);
+        }
+    }
+    // call of the keys jg + 4 g ... (jg a multiple of 16): index 2 (jg / 16) + g
+    __device__ __forceinline__ v4u at(int kb0, int within, int g) const { return mem[((kb0 >> 3) & 63) + (within >> 3) + g]; }
+};
 
 // Keep decisions of two scores at once: p2 holds their probabilities as packed fp16, w the two 16-bit Philox fields in the
 // same halves, sub2 = threshold - 1 in both halves (threshold >= 1).  A saturating subtraction leaves a half non-zero

@@ -140,12 +140,14 @@ constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarSt
               kVarEvery = 128, kVarNarrow = 256, kVarFold = 512, kVarPair = 1024;
 
 // work-groups per CU (narrow: one or two by their LDS; held to 256 VGPRs all the same, without which the compiler keeps more
-// than there are and moves them to and from accumulation registers): three up to D = 64 (168 VGPRs), except for the instance that serves every request, which stages
-// its tiles through registers
+// than there are and moves them to and from accumulation registers): three up to D = 96 (168 VGPRs), except for the instance that
+// serves every request, which stages its tiles through registers, and at D = 96 those with sixteen registers of bias constants,
+// which would spill (window with ALiBi B2 H16 N4096 d96 50 -> 57 us)
 constexpr int fwd_groups_per_cu(int D, int NB, int VAR)
 {
     if ((VAR & (kVarNarrow | kVarPair)) != 0) return 2;
-    return NB == 1 && D <= 64 && (VAR & kVarEvery) == 0 ? 3 : 2;
+    if (D == 96 && (VAR & kVarAlibiLeft) != 0) return 2;
+    return NB == 1 && D <= 96 && (VAR & kVarEvery) == 0 ? 3 : 2;
 }
 
 template <int D, int NB, int VAR>
@@ -501,6 +503,40 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         }
     };
 
+    // dropout: the parts of the Philox calls that depend on the row alone and on the call alone (common.h)
+    PhiloxRow drop_row[NB];
+    CallTable calls;
+    v4u first_part;  // of the tile at hand
+    if constexpr (kDropout) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) drop_row[nb] = philox_row_part((uint32_t)row_i[nb], (uint32_t)bh, a.seed_lo);
+        constexpr int kWaves = kPair ? 8 : 4;
+        calls.mem = call_table_memory<kWaves>() + 64 * (kPair ? 4 * half + wave : wave);
+        calls.chunk = -1;
+    }
+
+    // debug dump of the tile's keep decisions: the words once more, so that the ordinary path need not keep them
+    auto dump_keep = [&](int kb0) {
+        if constexpr (kDropout) {
+            if (__builtin_expect(a.keep_out == nullptr, 1)) return;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                const int ln = lane_here(), g = ln >> 5, row = q0 + wave_row0 + nb * 32 + (ln & 31);
+                if (row >= Nq) continue;
+                uint8_t* const kout = a.keep_out + ((size_t)bh * Nq + row) * Nk;
+#pragma unroll 1
+                for (int jg = 0; jg < BC; jg += 16) {
+                    const v4u w = philox_from_parts(drop_row[nb], calls.at(kb0, jg, g), a.seed_lo, a.seed_hi);
+#pragma unroll
+                    for (int f = 0; f < 8; ++f) {
+                        const int j = kb0 + jg + 8 * (f >> 2) + 4 * g + (f & 3);
+                        if (j < Nk) kout[j] = philox_field16(w, f) >= a.drop_thr ? 1 : 0;
+                    }
+                }
+            }
+        }
+    };
+
     // LDS read offsets of this lane
     const int k_rd = l32 * SK + (C::kPadK ? g * 16 : 0);                         // + kb*32*SK + k_step(ks)
     const int k_ch = C::kPadK ? 0 : (g ^ C::kswz(l32)) << 4;
@@ -577,10 +613,11 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     };
 
     // online softmax of one tile (per query row = per lane); leaves P^T packed to fp16 in pf
-    // masked: some row of the wave does not see all of the tile; then mask_sides: bit 0 = some row of the wave has its first
-    // allowed key inside or after this tile, bit 1 = some row has its last allowed key inside or before it (wave-uniform)
+    // masked: some row of the wave does not see all of the tile (wave-uniform)
     auto softmax = [&](bool masked, int kb0, v16f (&s)[2][NB], v8h (&pf)[2][2][NB]) {
         constexpr bool folded = kFoldAlibi;
+        if constexpr (kDropout) calls.cover(kb0, lane, (uint32_t)bh, a.off_lo, a.seed_lo, a.seed_hi);
+        if constexpr (kDropout && !kEvery) first_part = calls.at(kb0, 0, g);  // (in time for pv)
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             // folded ALiBi: bias of 32-key block kb that is common to the lane's 16 scores there (score units)
@@ -668,49 +705,23 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                 }
             }
             l_run[nb] += rs;  // per-lane partial; the two half-waves are added in the epilogue
-            if constexpr (kDropout) {
+            if constexpr (kDropout && kEvery) {  // (the other instances: pv below)
                 // drop iff field < threshold, row sum left undropped (src/flash_forward.h:221-237); the survivors' factor
                 // 1/(1-p) is common to the whole row and multiplies O once in the epilogue instead of every score here
-                const uint32_t i_u = (uint32_t)row_i[nb];
-                // first-round Philox product of the head-slice word: the same for the whole work-group, so a scalar multiply
-                const uint64_t bh_prod = (uint64_t)0xCD9E8D57u * (uint64_t)(uint32_t)bh;
-                const uint32_t bh_hi = (uint32_t)(bh_prod >> 32), bh_lo = (uint32_t)bh_prod;
-                uint8_t* kout = a.keep_out ? a.keep_out + ((size_t)bh * Nq + row_i[nb]) * Nk : nullptr;
 #pragma unroll
                 for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
                     for (int q = 0; q < 2; ++q) {
-                        // the lane's eight keys among the 16 from jg on: field f belongs to key jg + 8*(f>>2) + 4*g + (f&3)
-                        const int jg = kb0 + 32 * kb + 16 * q;
-                        const v4u w = philox4x32_10_c2(dropout_call((uint32_t)(jg + 4 * g)), i_u, bh_hi, bh_lo, a.off_lo, a.seed_lo, a.seed_hi);
-                        if constexpr (!kEvery) {
-                            // registers 8q + 2k and 8q + 2k + 1 become one packed fp16 word, fields 2k and 2k + 1 are the
-                            // halves of Philox word k: the decisions are applied to the packed word (keep_pair)
+                        // the lane's eight keys among the 16 from kb0 + 32 kb + 16 q on: field f belongs to the (8*(f>>2) + 4*g + (f&3))th
+                        const v4u w = philox_from_parts(drop_row[nb], calls.at(kb0, 32 * kb + 16 * q, g), a.seed_lo, a.seed_hi);
 #pragma unroll
-                            for (int k = 0; k < 4; ++k) {
-                                union { v2h h; uint32_t u; } pk;
-                                pk.h = pack_f16(s[kb][nb][8 * q + 2 * k], s[kb][nb][8 * q + 2 * k + 1]);
-                                pk.u = keep_pair(pk.u, w[k], a.drop_sub2);
-                                pf[kb][q][nb][2 * k] = pk.h[0];
-                                pf[kb][q][nb][2 * k + 1] = pk.h[1];
-                            }
-                        } else {
-#pragma unroll
-                            for (int f = 0; f < 8; ++f) {
-                                const int r = 8 * q + f;
-                                s[kb][nb][r] = philox_field16(w, f) >= a.drop_thr ? s[kb][nb][r] : 0.0f;
-                            }
-                        }
-                        if (a.keep_out != nullptr) {  // debug dump: one uniform branch per call, none per score
-#pragma unroll
-                            for (int f = 0; f < 8; ++f) {
-                                const int j = jg + 8 * (f >> 2) + 4 * g + (f & 3);
-                                if (row_i[nb] < Nq && j < Nk) kout[j] = philox_field16(w, f) >= a.drop_thr ? 1 : 0;
-                            }
+                        for (int f = 0; f < 8; ++f) {
+                            const int r = 8 * q + f;
+                            s[kb][nb][r] = philox_field16(w, f) >= a.drop_thr ? s[kb][nb][r] : 0.0f;
                         }
                     }
             }
-            if constexpr (!(kDropout && !kEvery)) {  // (there the dropout step has packed them already)
+            if constexpr (!(kDropout && !kEvery)) {  // (there pv packs them)
 #pragma unroll
                 for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -726,23 +737,61 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     };
 
     // O^T += V^T P^T with the tile in V buffer `buf`
-    auto pv = [&](int buf, v8h (&pf)[2][2][NB]) {
+    auto pv = [&](int buf, int kb0, v16f (&s)[2][NB], v8h (&pf)[2][2][NB]) {
         // (a lane's rows all share bit 1 of the row index: the swizzle is one per-lane choice between two bases)
         const char* const vb[2] = {Vs + buf * C::VBUF + v_rd + v_sw, Vs + buf * C::VBUF + v_rd + (v_sw ^ (C::VSWZ ? 64 : 0))};
+        auto v_frag = [&](int kb, int tt, int mb) __attribute__((always_inline)) {
+            const char* p0 = C::VSWZ ? vb[mb & 1] + (32 * kb + 16 * tt) * SV + (mb >> 1) * 128 : vb[0] + (32 * kb + 16 * tt) * SV + mb * 64;
+            union { v4hp p[2]; v8h v; } af;
+            af.p[0] = __builtin_amdgcn_ds_read_tr16_b64_v4f16((FA_LDS v4hp*)(p0));
+            af.p[1] = __builtin_amdgcn_ds_read_tr16_b64_v4f16((FA_LDS v4hp*)(p0 + 8 * SV));
+            return af.v;
+        };
+        if constexpr (kDropout && !kEvery) {
+            // Dropout, 16 keys at a time (a step): drop iff field < threshold, row sum left undropped
+            // (src/flash_forward.h:221-237); the survivors' factor 1/(1-p) is common to the whole row and multiplies O once in
+            // the epilogue.  The steps are fenced off from each other, so that the matrix units work on one step while the
+            // vector unit is at the next one's Philox rounds: left to itself the compiler put all MFMAs behind all rounds.
+            static_assert(NB == 1, "one row per lane");
+            v4u part = first_part;
+#pragma unroll
+            for (int st = 0; st < 4; ++st) {
+                const int kb = st >> 1, q = st & 1;
+                v8h af[MB];
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) af[mb] = v_frag(kb, q, mb);
+                const v4u mine = part;
+                if (st < 3) part = calls.at(kb0, 16 * (st + 1), g);
+                __builtin_amdgcn_sched_barrier(0);
+                // the lane's eight keys among the step's 16: field f belongs to the (8*(f>>2) + 4*g + (f&3))th.  Registers 8q + 2k
+                // and 8q + 2k + 1 become one packed fp16 word, fields 2k and 2k + 1 are the halves of Philox word k: the
+                // decisions are applied to the packed word (keep_pair)
+                const v4u w = philox_from_parts(drop_row[0], mine, a.seed_lo, a.seed_hi);
+                v8h p;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    union { v2h h; uint32_t u; } pk;
+                    pk.h = pack_f16(s[kb][0][8 * q + 2 * k], s[kb][0][8 * q + 2 * k + 1]);
+                    pk.u = keep_pair(pk.u, w[k], a.drop_sub2);
+                    p[2 * k] = pk.h[0];
+                    p[2 * k + 1] = pk.h[1];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) oacc[mb][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mb], p, oacc[mb][0], 0, 0, 0);
+            }
+            return;
+        }
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt) {
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb) {
-                    const char* p0 = C::VSWZ ? vb[mb & 1] + (32 * kb + 16 * tt) * SV + (mb >> 1) * 128
-                                             : vb[0] + (32 * kb + 16 * tt) * SV + mb * 64;
-                    union { v4hp p[2]; v8h v; } af;
-                    af.p[0] = __builtin_amdgcn_ds_read_tr16_b64_v4f16((FA_LDS v4hp*)(p0));
-                    af.p[1] = __builtin_amdgcn_ds_read_tr16_b64_v4f16((FA_LDS v4hp*)(p0 + 8 * SV));
+                    const v8h af = v_frag(kb, tt, mb);
 #pragma unroll
                     for (int nb = 0; nb < NB; ++nb)
-                        oacc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af.v, pf[kb][tt][nb], oacc[mb][nb], 0, 0, 0);
+                        oacc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, pf[kb][tt][nb], oacc[mb][nb], 0, 0, 0);
                 }
             }
         }
@@ -771,7 +820,8 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
             const int kb0 = (tile_begin + t) * BC;
             qk(buf, s);
             softmax(tile_masked(t), kb0, s, pf);
-            pv(buf, pf);
+            pv(buf, kb0, s, pf);
+            dump_keep(kb0);
         }
     };
     if constexpr (kNarrow) {
@@ -824,7 +874,10 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                 // V(n): older than the K request just issued
                 if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NKX) : "memory");
                 else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                if (live) pv(0, pf);
+                if (live) {
+                    pv(0, (tile_begin + t) * BC, s, pf);
+                    dump_keep((tile_begin + t) * BC);
+                }
                 if (kStamp && n == 0) stamps.take(4);
                 if (more) {
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -1144,7 +1197,9 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
     const long long groups = (long long)a.Tr * a.B * a.H * a.num_splits;
     FwdArgs b = a;
     constexpr int kResident = (kPair ? 1 : NB == 1 ? fwd_groups_per_cu(D, NB, VAR) : 2) * kNumCus;
-    set_slice_order(b, a.Tr * a.num_splits, kResident);
+    // (D = 96: chunks as for two work-groups per CU.  For three, causal B8 H32 N1000 d96 takes all its 256 slices as one chunk
+    // instead of 128 and finds fewer tiles in the caches: 74.9 -> 79.0 us, unmasked N = 1024 119.9 -> 133.7)
+    set_slice_order(b, a.Tr * a.num_splits, D == 96 ? 2 * kNumCus : kResident);
     b.split_rotate = split_rotate_for(b.num_splits, b.slice_chunk);
     b.snake_end = snake_end_for(groups, kResident);
     set_divisors(b, b.slice_chunk);

@@ -227,6 +227,33 @@ __global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const FwdArgs a)
     const float inv_cs = __builtin_amdgcn_rcpf(cs);  // (of the raise threshold alone)
     float nsig = 0.0f;  // ALiBi slope / scale, negated: read behind the prologue requests (below)
 
+    // dropout: the parts of the Philox calls that depend on the row alone and on the call alone (common.h)
+    PhiloxRow drop_row;
+    CallTable calls;
+    if constexpr (kDropout) {
+        drop_row = philox_row_part((uint32_t)row_i, (uint32_t)bh, a.seed_lo);
+        static_assert(C::SMEM + C::kWaves * 64 * 16 <= 160 * 1024, "stages, Q and call tables");
+        calls.mem = call_table_memory<C::kWaves>() + 64 * wave;
+        calls.chunk = -1;
+    }
+
+    // debug dump of the tile's keep decisions: the words once more, so that the ordinary path need not keep them
+    auto dump_keep = [&](int kb0) {
+        if constexpr (kDropout) {
+            if (a.keep_out == nullptr || row_i >= Nq) return;
+            uint8_t* const kout = a.keep_out + ((size_t)bh * Nq + row_i) * Nk;
+#pragma unroll 1
+            for (int jg = 0; jg < BC; jg += 16) {
+                const v4u w = philox_from_parts(drop_row, calls.at(kb0, jg, g), a.seed_lo, a.seed_hi);
+#pragma unroll
+                for (int f = 0; f < 8; ++f) {
+                    const int j = kb0 + jg + 8 * (f >> 2) + 4 * g + (f & 3);
+                    if (j < Nk) kout[j] = philox_field16(w, f) >= a.drop_thr ? 1 : 0;
+                }
+            }
+        }
+    };
+
     // Lane parts of the fragment addresses (layout above).  K fragment (ks, kb): key 32 kb + l32, chunk 2 ks + g
     // -> k_rd ^ (32 ks) + 8192 kb.  V transpose read (st, mb, half h) of lane (G = lane / 16, e = lane / 4 % 4,
     // j = lane % 4): key 16 st + 8 h + 4 (G / 2) + e, 32-byte chunk 2 mb + G % 2, bytes 8 j .. 8 j + 7
@@ -344,6 +371,7 @@ __global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const FwdArgs a)
     // mask_sides: bit 0 = some row of the wave has its first allowed key inside or after this tile, bit 1 = some row has
     // its last allowed key inside or before it (both wave-uniform)
     auto softmax = [&](int mask_sides, int kb0) __attribute__((always_inline)) {
+        if constexpr (kDropout) calls.cover(kb0, lane, (uint32_t)bh, a.off_lo, a.seed_lo, a.seed_hi);
         if constexpr (kAlibi) {
             // score*scale - slope*|i - j|  (src/main.cu:315,324), in the log2 domain
             const float jb = (float)(kb0 + 4 * g) - iif;
@@ -387,18 +415,12 @@ __global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const FwdArgs a)
             }
         l_run += rs;
         if constexpr (kDropout) {
-            const uint32_t i_u = (uint32_t)row_i;
-            // first-round Philox product of the head-slice word: the same for the whole work-group, so a scalar multiply
-            const uint64_t bh_prod = (uint64_t)0xCD9E8D57u * (uint64_t)(uint32_t)bh;
-            const uint32_t bh_hi = (uint32_t)(bh_prod >> 32), bh_lo = (uint32_t)bh_prod;
-            uint8_t* kout = a.keep_out ? a.keep_out + ((size_t)bh * Nq + row_i) * Nk : nullptr;
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
                 for (int q = 0; q < 2; ++q) {
-                    // the lane's eight keys among the 16 from jg on: field f belongs to key jg + 8*(f>>2) + 4*g + (f&3)
-                    const int jg = kb0 + 32 * kb + 16 * q;
-                    const v4u w = philox4x32_10_c2(dropout_call((uint32_t)(jg + 4 * g)), i_u, bh_hi, bh_lo, a.off_lo, a.seed_lo, a.seed_hi);
+                    // the lane's eight keys among the 16 from kb0 + 32 kb + 16 q on: field f belongs to the (8*(f>>2) + 4*g + (f&3))th
+                    const v4u w = philox_from_parts(drop_row, calls.at(kb0, 32 * kb + 16 * q, g), a.seed_lo, a.seed_hi);
                     // the decisions are applied to the packed fp16 words (keep_pair); the 1/(1-p) waits for the epilogue
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
@@ -408,14 +430,8 @@ __global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const FwdArgs a)
                         pf[kb][q][2 * k] = pk.h[0];
                         pf[kb][q][2 * k + 1] = pk.h[1];
                     }
-                    if (a.keep_out != nullptr) {  // debug dump: one uniform branch per call, none per score
-#pragma unroll
-                        for (int f = 0; f < 8; ++f) {
-                            const int j = jg + 8 * (f >> 2) + 4 * g + (f & 3);
-                            if (row_i < Nq && j < Nk) kout[j] = philox_field16(w, f) >= a.drop_thr ? 1 : 0;
-                        }
-                    }
                 }
+            dump_keep(kb0);
         }
         if constexpr (!kDropout) {  // (there the dropout step has packed them already)
 #pragma unroll
