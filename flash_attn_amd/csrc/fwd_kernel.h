@@ -142,11 +142,14 @@ constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarSt
 // work-groups per CU (narrow: one or two by their LDS; held to 256 VGPRs all the same, without which the compiler keeps more
 // than there are and moves them to and from accumulation registers): three up to D = 96 (168 VGPRs), except for the instance that
 // serves every request, which stages its tiles through registers, and at D = 96 those with sixteen registers of bias constants,
-// which would spill (window with ALiBi B2 H16 N4096 d96 50 -> 57 us)
+// which would spill (window with ALiBi B2 H16 N4096 d96 50 -> 57 us).  Four at D = 64 without dropout (128 VGPRs): the plain
+// instances fit by themselves, those with ALiBi do when told so (B32 H32 N512 d64 in 128-row blocks 100.3 -> 91.1 us together with the
+// shorter chunks below, causal window of 256 keys with ALiBi B2 H16 N4096 24.2 -> 23.7)
 constexpr int fwd_groups_per_cu(int D, int NB, int VAR)
 {
     if ((VAR & (kVarNarrow | kVarPair)) != 0) return 2;
     if (D == 96 && (VAR & kVarAlibiLeft) != 0) return 2;
+    if (NB == 1 && D == 64 && (VAR & (kVarEvery | kVarDropout)) == 0) return 4;
     return NB == 1 && D <= 96 && (VAR & kVarEvery) == 0 ? 3 : 2;
 }
 
@@ -1161,11 +1164,15 @@ bool fwd_uses_pingpong(int d, bool direct, int Nq, int Nk, int causal, int wl, i
 // slices +3-5 %; 64: +-0; 32: -2 %; 16: -9 %; 96 and 192 (a ragged last chunk): -1 %.  With this rule, against all
 // slices in one chunk: causal B16 H32 N1024 d128 +5 %, B8 H32 N2048 d64 +4 %, B8 H32 N4096 d128 (8-wave kernel) +16 %;
 // once or four times the resident work-groups per chunk instead of twice: 0 ... -4 %.
+// Where all work-groups weigh alike (no mask, one split) there is no tail to balance and the chunk is sixteen slices, whose
+// row blocks follow each other closely enough to find the slices' K and V in L2.  Chunks of 8 / 16 / 32 / 64 / 128 / 256 /
+// all: B32 H32 N512 d64 101.0 / 100.9 / 100.5 / 101.7 / 101.8 / 103.1 / 104.7 us, B8 H32 N1024 d96 118.9 / 118.1 / 119.0 / 119.8 /
+// 119.9 / 133.7, B8 H32 N2048 d64 320 / 318 / 318 / 321 / 325 / 332, B16 H16 N1024 d128 161 / 163 / 162 / 163 / 164 / 170.
 constexpr int kNumCus = 256;  // MI355X
-inline int slice_chunk_for(int slices, int groups_per_slice, int resident, int step = 8)
+inline int slice_chunk_for(int slices, int groups_per_slice, int resident, bool alike, int step = 8)
 {
     if (slices <= 0 || groups_per_slice <= 0) return 1;
-    const long long want = (2LL * resident + groups_per_slice - 1) / groups_per_slice;
+    const long long want = alike ? 16 : (2LL * resident + groups_per_slice - 1) / groups_per_slice;
     for (long long c = (want + step - 1) / step * step; c < slices; c += step)
         if (slices % c == 0) return (int)c;
     return slices;
@@ -1176,12 +1183,13 @@ inline int slice_chunk_for(int slices, int groups_per_slice, int resident, int s
 inline void set_slice_order(FwdArgs& b, int groups_per_slice, int resident)
 {
     const int slices = b.B * b.H;
+    const bool alike = !b.causal && b.wl < 0 && b.wr < 0 && b.num_splits == 1;
     b.group_xcd = 0;
     if (b.kv_group > 1 && slices % (8 * b.kv_group) == 0) {
-        b.slice_chunk = slice_chunk_for(slices, groups_per_slice, resident, 8 * b.kv_group);
+        b.slice_chunk = slice_chunk_for(slices, groups_per_slice, resident, alike, 8 * b.kv_group);
         if (b.slice_chunk % (8 * b.kv_group) == 0) b.group_xcd = b.kv_group;
     } else {
-        b.slice_chunk = slice_chunk_for(slices, groups_per_slice, resident);
+        b.slice_chunk = slice_chunk_for(slices, groups_per_slice, resident, alike);
     }
 }
 
@@ -1196,7 +1204,9 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
     if (hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), smem, attr_done); e != hipSuccess) return e;
     const long long groups = (long long)a.Tr * a.B * a.H * a.num_splits;
     FwdArgs b = a;
-    constexpr int kResident = (kPair ? 1 : NB == 1 ? fwd_groups_per_cu(D, NB, VAR) : 2) * kNumCus;
+    // (the order of the work-groups counts three places per CU at D = 64 as well: measured +-1 % causal)
+    constexpr int kPlaces = fwd_groups_per_cu(D, NB, VAR) < 3 ? fwd_groups_per_cu(D, NB, VAR) : 3;
+    constexpr int kResident = (kPair ? 1 : NB == 1 ? kPlaces : 2) * kNumCus;
     // (D = 96: chunks as for two work-groups per CU.  For three, causal B8 H32 N1000 d96 takes all its 256 slices as one chunk
     // instead of 128 and finds fewer tiles in the caches: 74.9 -> 79.0 us, unmasked N = 1024 119.9 -> 133.7)
     set_slice_order(b, a.Tr * a.num_splits, D == 96 ? 2 * kNumCus : kResident);
@@ -1283,18 +1293,16 @@ inline bool fwd_uses_pair(const FwdArgs& a, int bucket_d, int feat)
     return groups <= kNumCus && a.Nk >= 8 * 64 * a.num_splits && left + right + 128 >= 8 * 64;
 }
 
-// 64 query rows per wave at d = 64 (NB = 2, 202 VGPRs, two work-groups of 256 rows per CU): a K or V fragment read from LDS
-// feeds two MFMAs.  Only without a mask -- causal it measured -9 %, with a window of 256 keys -21 %: wider diagonals -- and
-// where 256-row blocks add no more than 4 % of empty rows to what 128-row blocks have (B32 H32 N384 52.8 -> 60.3 us, N300
-// -7 %, N640 +-0) and no more than an eighth of the rows is empty (B32 H64 N140 -6 %, N200 +-0), from two rounds of
-// work-groups on.  B32 H32 N512 107.1 -> 99.8 us (688 TFLOP/s), B16 H16 N1024 96.1 -> 87.2,
-// B8 H32 N2048 333.6 -> 313.3, B2 H16 N8192 607 -> 577 (953 TFLOP/s), B31 H64 H_kv8 N705 361 -> 356 us; same bits.  On another
-// card the first two were 108.3 -> 105.6 and 94.8 -> 92.5, and B2 H16 N8192 641 -> 629: the launch needs no fewer cycles than with
-// 128 rows, 16 % of which have neither a VALU instruction nor an MFMA, but half the LDS instructions and 0.57 of the bytes
-// fetched, and what those save in power comes back as clock.
+// 64 query rows per wave at d = 64 (NB = 2, 199 VGPRs, two work-groups of 256 rows per CU): a K or V fragment read from LDS
+// feeds two MFMAs; the launch needs no fewer cycles than with 128 rows, but half the LDS instructions and 0.57 of the bytes
+// fetched, and what those save in power comes back as clock.  Only without a mask -- causal it measured -9 %, with a window of
+// 256 keys -21 %: wider diagonals --, where 256-row blocks add no more than 4 % of empty rows to what 128-row blocks have (N300
+// -7 %) and no more than an eighth of the rows is empty, from two rounds of work-groups on, and from sixteen tiles on: shorter
+// work-groups are better off four to a CU.  Tall / 128 rows: B32 H32 N512 96.6 / 91.1 us, B24 H16 N768 70.8 / 68.3, B16 H16 N768 46.5 /
+// 46.9, B12 H16 N896 51.0 / 51.1, B16 H16 N1024 75.9 / 79.3, B8 H32 N2048 287 / 298, B4 H16 N4096 281 / 296; same bits.
 inline bool fwd_uses_tall(const FwdArgs& a, int variant)
 {
-    if (variant != kVarVec || a.d != 64 || a.num_splits != 1 || a.fold_rows || a.causal || a.wl >= 0 || a.wr >= 0 || a.kernel_hint != 0) return false;
+    if (variant != kVarVec || a.d != 64 || a.Nk < 1024 || a.num_splits != 1 || a.fold_rows || a.causal || a.wl >= 0 || a.wr >= 0 || a.kernel_hint != 0) return false;
     const long long blocks = (a.Nq + 255) / 256, added = 2 * blocks - (a.Nq + 127) / 128;  // in blocks of 128 rows
     return (long long)a.B * a.H * blocks >= 4 * kNumCus && 25 * added <= 2 * blocks && 8 * (256 * blocks - a.Nq) <= 256 * blocks;
 }

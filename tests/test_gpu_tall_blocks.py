@@ -18,3 +18,9 @@ def test_tall_blocks(fa, oracle, B, H, Hk, Nq, Nk):
     assert torch.equal(o, o4) and torch.equal(lse, lse4)
     O, L = oracle.attention_forward(*(to_f32_np(t[-1:, -1:]) for t in (q, k, v)))
     check_o_lse(o[-1:, -1:], lse[-1:, -1:], O, L, "last head")
+
+
+@pytest.mark.parametrize("B,H,Hk,Nq,Nk", [(16, 32, 32, 512, 1024), (16, 32, 8, 481, 1090), (3, 28, 28, 3329, 1025), (13, 40, 40, 512, 1087)])
+def test_tall_blocks_and_slice_chunks_of_long_key_ranges(fa, oracle, B, H, Hk, Nq, Nk):
+    """The rule takes them from 1024 keys on; slice counts that do and do not divide into chunks of sixteen."""
+    test_tall_blocks(fa, oracle, B, H, Hk, Nq, Nk)
