@@ -1285,11 +1285,19 @@ inline hipError_t launch_fwd_narrow_instance(const FwdArgs& a, hipStream_t st)
 //    (Window of 500 keys B1 H16 N1500 d64 12.7 -> 10.7 us, of 1000 B2 H4 N2500 d96 21.5 -> 18.0.)
 //  * up to 32 rows only one wave of four has any, and a second one beside it gained 7-11 % at d = 32, but lost 4 % at
 //    d = 112 (B2 H16 H_kv4 Nq2 Nk16960 18.2 -> 19.0).
+//  * causal, unsplit and up to twice as many: two work-groups of a CU side by side last as long as the longer one, whose SIMDs
+//    have one wave each once its light neighbour is done; as paired ones they follow each other, eight waves at a time.  From
+//    1280 keys on up to 384 work-groups (1.0 ... 1.2 times as fast over d = 40 ... 128), with dropout up to 512, from 1856 on up to
+//    512 without (0.98 ... 1.1): B1 H32 N1500 d128 32.5 -> 29.2 us, B3 H8 N1777 d100 34.4 -> 29.3, B1 H16 N4096 d128 83.1 -> 75.2, B4 H8
+//    N2000 d96 35.3 -> 33.3, with dropout B3 H12 N1777 d80 45.1 -> 41.8.  Below (B2 H24 N1000 d128 23.3 -> 24.1) and above (B5 H8 N1777
+//    d100 42.5 -> 47.8, 560 of them) it loses.
 inline bool fwd_uses_pair(const FwdArgs& a, int bucket_d, int feat)
 {
     if ((feat & kVarAlibi) != 0 || a.kernel_hint != 0 || (a.Nq <= 32 && bucket_d > 32)) return false;
     const long long groups = (long long)a.Tr * a.B * a.H * a.num_splits;
     const long long left = a.wl >= 0 ? a.wl : a.Nk, right = a.causal ? 0 : a.wr >= 0 ? a.wr : a.Nk;
+    if (a.causal && a.wl < 0 && a.num_splits == 1 && !a.fold_rows && 2 * (long long)a.Nq >= a.Nk && groups > kNumCus)
+        return groups <= 2 * kNumCus && a.Nk >= (groups <= 384 || feat != 0 ? 1280 : 1856);
     return groups <= kNumCus && a.Nk >= 8 * 64 * a.num_splits && left + right + 128 >= 8 * 64;
 }
 

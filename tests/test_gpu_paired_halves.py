@@ -68,3 +68,21 @@ def test_paired_halves_windowed_dropout(fa, oracle, Nq, d):
     keep = torch.from_numpy(oracle.dropout_keep_mask(9, 0, p, B, H, Nq, Nk))
     O, L = oracle_forward_batched(oracle, q, k, v, keep_mask=keep, p_drop=p, **kw)
     check_o_lse(*fa.flash_forward_splitkv(q, k, v, num_splits=3, dropout_p=p, seed=9, **kw), O, L, "windowed dropout")
+
+
+@pytest.mark.parametrize("B,H,Hk,Nq,Nk,d,p", [(1, 28, 28, 1283, 1283, 100, 0.0), (2, 12, 4, 1700, 1921, 40, 0.0), (1, 26, 26, 1281, 1300, 64, 0.2),
+                                              (1, 24, 24, 1925, 1870, 72, 0.0)])
+def test_paired_halves_one_after_the_other(fa, oracle, B, H, Hk, Nq, Nk, d, p):
+    """Causal launches of 257 to 512 work-groups, two of them one after the other on a CU; rows that see no key among them."""
+    import torch
+
+    q, k, v = randn_f16_gpu((B, H, Nq, d), 4), randn_f16_gpu((B, Hk, Nk, d), 5), randn_f16_gpu((B, Hk, Nk, d), 6)
+    kr, vr = (t.repeat_interleave(H // Hk, dim=1).contiguous() for t in (k, v))
+    okw, kw = dict(causal=True), dict(causal=True)
+    if p:
+        kw.update(dropout_p=p, seed=9)
+        okw.update(keep_mask=torch.from_numpy(oracle.dropout_keep_mask(9, 0, p, B, H, Nq, Nk)), p_drop=p)
+    O, L = oracle_forward_batched(oracle, q, kr, vr, **okw)
+    o, lse = fa.flash_forward(q, k, v, **kw)
+    check_o_lse(o, lse, O, L, "two paired work-groups per CU")
+    assert all(torch.equal(a, b) for a, b in zip(fa.flash_forward(q, k, v, **kw), (o, lse)))
