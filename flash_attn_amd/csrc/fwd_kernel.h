@@ -903,15 +903,23 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         // (paired: both halves go round as often, for the barrier; the second one's last tile may not exist)
         const int rounds = kPair ? (ntiles + 1) / 2 : ntiles;
         static_assert(NSTG == 2, "a stage that is read and one that is filled");
-#pragma unroll
-        for (int u = 0; u < NSTG; ++u)
-            if (u < rounds && (!kPair || nth(u) < ntiles)) dma_tile(tile_begin + nth(u), u);
+        // (Launches whose every tile has one reader take them from HBM, all work-groups at once: they request the second tile only
+        // when the first one is there, since both at once arrive in twice the time of one.  B8 H32 H_kv8 Nq1 Nk5003 d128 30.6 -> 29.4
+        // us, B1 H32 H_kv8 Nq16 Nk8192 d128 17.3 -> 16.8, B16 H32 H_kv4 Nq3 Nk6000 d80 24.4 -> 23.9; other split launches +-1 %, paired
+        // work-groups, whose halves have a tile each on its way, -2 %.)
+        constexpr bool late = (kFold || kKvOnce) && !kPair;
+        auto second_tile = [&](bool now) {
+            if (now && 1 < rounds && (!kPair || nth(1) < ntiles)) dma_tile(tile_begin + nth(1), 1);
+        };
+        if (0 < rounds && (!kPair || nth(0) < ntiles)) dma_tile(tile_begin + nth(0), 0);
+        second_tile(!late);
         set_bounds();
         read_slope();
         stamps.take(1);
         dma_wait(false);
         pin_q();
         stamps.take(2);
+        second_tile(late);
         __syncthreads();
         stamps.take(3);
         int buf = 0;  // stage of tile t
