@@ -19,6 +19,7 @@ typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 // 16 bytes at any 2-byte / 4-byte boundary (the hardware runs in unaligned access mode): rows of d % 8 != 0 elements
 typedef v4u __attribute__((aligned(2))) v4u_anyalign;
 typedef v4f __attribute__((aligned(4))) v4f_anyalign;
+typedef v4h __attribute__((aligned(2))) v4h_anyalign;
 // operand type of the ds_read_b64_tr_b16 builtin
 typedef __fp16 v4hp __attribute__((__vector_size__(4 * sizeof(__fp16))));
 

@@ -982,8 +982,12 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         __syncthreads();  // every wave is done with its tile buffers
         float* const sm = reinterpret_cast<float*>(smem);  // [4][32] running maxima (log2 units)
         float* const sl = sm + 4 * 32;                      // [4][32] row sums
-        float* const so = sl + 4 * 32;                      // [4][32][D] unnormalised O, by chunk position
-        static_assert((2 * 4 * 32 + 4 * 32 * D) * 4 <= 4 * kWaveLds, "merge buffers fit the tile buffers");
+        // (Rows four floats apart from each other's banks, four columns per access and 8-byte stores of O: with a stride of D every
+        // row of a store began at the same bank, and single floats and halves took 2 us of a launch.  B1 H8 N1021 d31 9.07 -> 8.45
+        // us, B1 H8 N1024 d64 8.55 -> 7.76, d128 13.2 -> 11.6, B1 H4 N700 d100 causal 15.5 -> 11.4, B2 H4 N256 d64 5.47 -> 4.41.)
+        constexpr int SM = D + 4;
+        float* const so = sl + 4 * 32;                      // [4][32][SM] unnormalised O, by chunk position
+        static_assert((2 * 4 * 32 + 4 * 32 * SM) * 4 <= 4 * kWaveLds, "merge buffers fit the tile buffers");
         const float l = xhalf_sum(l_run[0]);
         if (g == 0) {
             sm[wave * 32 + l32] = m_ref[0];
@@ -994,12 +998,11 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
 #pragma unroll
             for (int rg = 0; rg < 4; ++rg) {
                 const v4f o = {oacc[mb][0][4 * rg], oacc[mb][0][4 * rg + 1], oacc[mb][0][4 * rg + 2], oacc[mb][0][4 * rg + 3]};
-                *reinterpret_cast<v4f*>(so + (wave * 32 + l32) * D + 32 * mb + 8 * rg + 4 * g) = o;
+                *reinterpret_cast<v4f*>(so + (wave * 32 + l32) * SM + 32 * mb + 8 * rg + 4 * g) = o;
             }
         __syncthreads();
-        // thread -> one row and D / 8 consecutive chunk positions of it
-        constexpr int CPT = D / 8;
-        const int row = tid >> 3, cp0 = (tid & 7) * CPT;
+        // eight threads per row, four consecutive chunk positions at a time: 128 bytes of each partial result per row and read
+        const int row = tid >> 3;
         float M = kNothingSeen;
 #pragma unroll
         for (int w = 0; w < 4; ++w) M = fmaxf(M, sm[w * 32 + row]);
@@ -1015,16 +1018,20 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
             half_t* const op = a.O + ((size_t)bh * Nq + gi) * d;
             const int cfull = d & ~7, rem = d & 7;
 #pragma unroll
-            for (int c = 0; c < CPT; ++c) {
-                const int cc = cp0 + c;
-                float o = 0.0f;
+            for (int k = 0; k < D / 32; ++k) {
+                const int cc = 4 * ((tid & 7) + 8 * k);
+                v4f o = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int w = 0; w < 4; ++w) o = __builtin_fmaf(wgt[w], so[(w * 32 + row) * D + cc], o);
-                // column of chunk position cc: behind the row's whole chunks sit the columns d - 8 ... d - 1, of which
-                // the first 8 - d % 8 belong to the positions before
-                const int col = kFullD || cc < cfull ? cc : cc - (8 - rem);
-                const bool ok = kFullD || cc < cfull || (rem != 0 && cc < cfull + 8 && col >= cfull);
-                if (ok) op[col] = (half_t)(o * inv);
+                for (int w = 0; w < 4; ++w) {
+                    const v4f p = *reinterpret_cast<const v4f*>(so + (w * 32 + row) * SM + cc);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(wgt[w], p[e], o[e]);
+                }
+                const v4h r = {(half_t)(o[0] * inv), (half_t)(o[1] * inv), (half_t)(o[2] * inv), (half_t)(o[3] * inv)};
+                // (behind the row's whole chunks sit the columns d - 8 ... d - 1; those that a position before holds as well are
+                // the same)
+                if constexpr (kFullD) *reinterpret_cast<v4h*>(op + cc) = r;
+                else if (cc < cfull || (rem != 0 && cc < cfull + 8)) *reinterpret_cast<v4h_anyalign*>(op + (cc < cfull ? cc : cc - (8 - rem))) = r;
             }
             if ((tid & 7) == 0)
                 a.LSE[(size_t)bh * Nq + gi] = L > 0.0f ? __builtin_fmaf(M, kLn2, fast_log2(L) * kLn2) : -INFINITY;
@@ -1038,25 +1045,33 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         // (behind the loop's last barrier; the buffer lies behind the O staging of the epilogue, which other waves may be in)
         constexpr int kOut = 4 * 32 * (2 * D + 16);
         static_assert(kOut + 4 * (16 * MB + 2) * 256 <= 2 * kWaveLds, "merge buffer fits the tile buffers");
-        float* const mine = reinterpret_cast<float*>(smem + kOut) + wave * (16 * MB + 2) * 64 + lane;
+        // (four registers per access, a wave's 64 lanes one after the other)
+        float* const mine = reinterpret_cast<float*>(smem + kOut) + wave * (16 * MB + 2) * 64;
+        v4f* const mine_o = reinterpret_cast<v4f*>(mine) + lane;
+        float* const mine_ml = mine + 16 * MB * 64 + lane;
         if (half == 1) {
-            mine[0] = m_ref[0];
-            mine[64] = l_run[0];
+            mine_ml[0] = m_ref[0];
+            mine_ml[64] = l_run[0];
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) mine[(2 + 16 * mb + r) * 64] = oacc[mb][0][r];
+                for (int rg = 0; rg < 4; ++rg)
+                    mine_o[(4 * mb + rg) * 64] = v4f{oacc[mb][0][4 * rg], oacc[mb][0][4 * rg + 1], oacc[mb][0][4 * rg + 2], oacc[mb][0][4 * rg + 3]};
         }
         __syncthreads();
         if (half == 1) return;
-        const float m1 = mine[0], M = fmaxf(m_ref[0], m1);
+        const float m1 = mine_ml[0], M = fmaxf(m_ref[0], m1);
         const float w0 = fast_exp2(m_ref[0] - M), w1 = fast_exp2(m1 - M);
         m_ref[0] = M;
-        l_run[0] = __builtin_fmaf(w1, mine[64], w0 * l_run[0]);
+        l_run[0] = __builtin_fmaf(w1, mine_ml[64], w0 * l_run[0]);
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) oacc[mb][0][r] = __builtin_fmaf(w1, mine[(2 + 16 * mb + r) * 64], w0 * oacc[mb][0][r]);
+            for (int rg = 0; rg < 4; ++rg) {
+                const v4f o = mine_o[(4 * mb + rg) * 64];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) oacc[mb][0][4 * rg + e] = __builtin_fmaf(w1, o[e], w0 * oacc[mb][0][4 * rg + e]);
+            }
     }
 
     // ---------------- epilogue: normalise once, store O (fp16) + LSE, or the fp32 split partials
