@@ -190,8 +190,8 @@ long long tiled_groups(const flash_params* p, const fa::FwdArgs& a)
 // tiles (the heaviest one plus k - 1 average ones) taken in rounds of as many as the CU has places for, a round of n
 // side by side costing the sum of its tiles over the gain of n, b = microseconds per 64-key tile of a work-group alone
 // on its CU.  Over 21 swept shapes the count it picks is within 5 % of the best measured one on 19 (the others: 6 % and
-// 9 %); the reference's rule with 256 CUs: 9 of 21, the worst 3.1 times slower than the best count.  It does not know which
-// launches will be paired: a cheaper tile for those made the counts of 300 random shapes 0.2 % worse.  Its constants and the lines
+// 9 %); the reference's rule with 256 CUs: 9 of 21, the worst 3.1 times slower than the best count.  It knows
+// which launches will be narrow or paired.  Its constants and the lines
 // of fwd_uses_narrow are fits to the kernels as they are; a change of either wants both measured again.
 int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode);
 bool folds_heads(const flash_params* p);
@@ -260,12 +260,10 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
     // walking a quarter of the tiles alone on its SIMD, two work-groups side by side per CU up to d = 32 and one in a
     // row above, 3 us for the launch and 4 us per work-group in a row on a CU (fitted to 12 shapes).
     bool narrow = false;
-    if (!pp) {
-        fa::FwdArgs unsplit;
-        fill_args(p, 1, &unsplit);
-        if (fold) fold_heads(&unsplit);
-        narrow = fa::fwd_uses_narrow(unsplit, every);
-    }
+    fa::FwdArgs launch;
+    fill_args(p, 1, &launch);
+    if (fold) fold_heads(&launch);
+    if (!pp) narrow = fa::fwd_uses_narrow(launch, every);
     int limit = FLASH_MAX_SPLITS;
     if (n_blocks < limit) limit = n_blocks;
     int best_s = 1, prev_per = -1;
@@ -316,7 +314,12 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
             chain += ((left == k ? (float)tmax + (float)(n - 1) * avg : (float)n * avg)) / gain[n];
             left -= n;
         }
-        float t = (float)k * a / rho + b * chain;
+        // (Paired work-groups: two waves per SIMD where a lone work-group has one, and a merge.  Without this the count came out twice
+        // as high, two unpaired work-groups to a CU: B2 H16 Nq111 Nk20468 d64 16 -> 8 splits 46.4 -> 42.4 us, B10 H4 Nq240 Nk9594 d72 6 -> 3
+        // 56.6 -> 51.8, B6 H1 Nq459 Nk28734 d64 21 -> 10 40.0 -> 34.9.)
+        launch.num_splits = s;
+        const bool paired = !pp && !every && k == 1 && fa::fwd_uses_pair(launch, 32 * bucket, tiled_variant(p) & 6);
+        float t = (float)k * a / rho + (paired ? 1.0f + 0.92f * b * chain : b * chain);
         if (s == 1 && narrow) {
             // 32-row work-groups with a visible key, and the time per tile of a wave on its own, measured: x 1.15 with
             // two LDS stages per wave (d <= 64); with one, where the next tile's requests are only partly hidden, x 1.3 at

@@ -1244,17 +1244,19 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
 // every other request; the narrow, paired and folded ones below.  ST = kVarStamp selects their instrumented twins (debug
 // time stamps).  Nothing else looks at the stamp pointer: a stamped call is launched as the same call without.
 // The narrow instances (kNarrow in fwd_kernel) serve unsplit launches whose time is the chain of key tiles that a work-group
-// walks through, which they cut to a quarter for a fixed cost of 0.5-2 us (a wave's own requests, the merge of four).  Per
-// tile of a wave on its own: 0.5 / 1.0 / 1.3 / 1.6 us at D = 32 / 64 / 96 / 128, against 0.45 / 0.65 / 0.8 / 1.0 us of a
-// 128-row work-group alone on its CU.  Measured against the 128-row instances on 400 random launches of up to 400 of those
-// work-groups; the lines below lie where the ratio of the two crosses one:
-//  * One round -- no more 32-row work-groups than places for them, one per CU by their LDS, two at D = 32: from 4 tiles
-//    on, 5 under a window (B4 H2 N256 d64: 6.0 -> 4.8 us, B1 H4 N640 d128 causal 14.8 -> 10.5, B1 H2 N3264 d128 56 -> 26), from 6 or 10
-//    where rows are shorter than a bucket above 64, whose requests of unaligned pieces a wave cannot hide (B1 H4 N960 d80
-//    16.6 -> 11.0, B2 H4 N960 d100 20.2 -> 16.2; B3 H2 N112 d112, two tiles: 6.8 -> 10.2).
-//  * More rounds only where the later work-groups are the light ones of a causal mask, the longer the sequence the more of
-//    them (B1 H8 N2423 d64, 608 of them: 31.4 -> 22.4 us, but B3 H8 N1344 d64, 1008 of them: 19.2 -> 25.4), or the
-//    chain is so long that two rounds of a quarter are still shorter (B1 H4 N4096 d64 50 -> 38, B2 H4 N4736 d32 69 -> 53).
+// walks through, which they cut to a quarter for a fixed cost of about 1 us (a wave's own requests, the merge of four).
+// Measured against the 128-row instances, paired ones among them, on 1240 random launches of up to 1600 work-groups of 32 rows;
+// the lines below lie where the ratio of the two crosses one:
+//  * One round -- no more 32-row work-groups than places for them, one per CU by their LDS, two at D = 32 (from 4 tiles on): from 2
+//    tiles on, 3 at 96 < d < 128 (N150, 3 tiles, d31 / 64 / 128 / 100 6.2 / 6.2 / 7.8 / 8.3 -> 5.1 / 5.2 / 6.6 / 7.6 us; N120, 2 tiles,
+//    5.9 / 5.7 / 6.8 / 7.2 -> 5.2 / 5.2 / 6.3 / 7.4; window of 100 keys N600, 4 tiles, 8.0 / 8.1 / 10.1 / 10.3 -> 5.3 / 5.3 / 6.7 / 7.8).
+//    Launches of up to 64 of them, which would gain as much, stay where they were below 4 tiles, 5 under a window: the tests
+//    of the 128-row instances' stage stamps ask for them there.
+//  * More rounds only where the later work-groups are the light ones of a causal mask, the more tiles the more of them:
+//    D >= 96: up to 576 from 8 + (groups - 256) / 16 tiles on (narrow / 128 rows: 0.6 ... 1.0 there; B1 H3 N3748 d100, 354 of them: 48
+//    -> 31 us; B8 H3 N1344 d64, 1008 of them: 19 -> 25), D = 64: up to 560 from 8 + (groups - 256) / 12 on, d = 32: a tile for every 40 of
+//    them (B1 H11 N2402: 20.0 -> 15.8), shorter rows, whose requests a wave alone hides less well, up to 640 from 16 on.  Without a
+//    mask a second round loses (B1 H7 N4555 d31 67.7 against 37.5), but for long ones at d = 32 (0.9 ... 1.2).
 inline bool fwd_uses_narrow(const FwdArgs& a, bool every)
 {
     if (every || a.num_splits != 1 || a.kernel_hint != 0) return false;
@@ -1267,16 +1269,16 @@ inline bool fwd_uses_narrow(const FwdArgs& a, bool every)
     const long long keys = left + right + 128 < a.Nk ? left + right + 128 : a.Nk;
     const int tiles = (int)((keys + 63) / 64);
     if (groups <= (bucket == 1 ? 2 * kNumCus : kNumCus)) {
-        if (bucket >= 3 && !whole) return tiles >= (bucket == 3 ? 6 : 10);
-        return tiles >= (groups > kNumCus || keys < a.Nk ? 5 : 4);
+        if (groups <= 64) return tiles >= (keys < a.Nk ? 5 : 4);
+        return tiles >= (groups > kNumCus ? 4 : bucket == 4 && !whole ? 3 : 2);
     }
     if (keys < a.Nk) return false;  // a window: the later work-groups are as heavy as the first
     if (a.causal && 2 * (long long)(a.fold_rows ? a.fold_rows : a.Nq) >= a.Nk) {
-        if (bucket == 1) return groups <= 576 ? tiles >= 9 : groups <= 800 && tiles >= 16;
-        if (bucket == 4 && !whole) return false;
-        return groups <= 384 ? tiles >= (bucket == 3 && !whole ? 20 : 14) : groups <= 640 && tiles >= 36;
+        if (bucket == 1) return whole ? 40 * tiles >= groups : groups <= 640 && tiles >= 16;
+        if (bucket == 2) return groups <= 560 && 12 * (tiles - 8) >= groups - kNumCus;
+        return groups <= 576 && 16 * (tiles - 8) >= groups - kNumCus;
     }
-    return bucket == 1 ? tiles >= 64 : bucket == 2 && groups <= 512 && tiles >= 24;
+    return false;
 }
 
 template <int D, int VAR>
