@@ -1255,7 +1255,9 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
 //  * More rounds only where the later work-groups are the light ones of a causal mask, the more tiles the more of them:
 //    D >= 96: up to 576 from 8 + (groups - 256) / 16 tiles on (narrow / 128 rows: 0.6 ... 1.0 there; B1 H3 N3748 d100, 354 of them: 48
 //    -> 31 us; B8 H3 N1344 d64, 1008 of them: 19 -> 25), D = 64: up to 560 from 8 + (groups - 256) / 12 on, d = 32: a tile for every 40 of
-//    them (B1 H11 N2402: 20.0 -> 15.8), shorter rows, whose requests a wave alone hides less well, up to 640 from 16 on.  Without a
+//    them (B1 H11 N2402: 20.0 -> 15.8), shorter rows, whose requests a wave alone hides less well, up to 640 from 16 on; with dropout,
+//    whose tiles cost more beside the same fixed part, D >= 96 up to 512 from 8 + (groups - 256) / 32 on and up to 640 from 26 on, D = 64 the
+//    same beyond 18 tiles (B1 H11 N1267 21.9 -> 16.2), D = 32 up to 640 from 10 on (B1 H12 N1261 d128 30.1 -> 23.0, B1 H7 N2635 d96 45.2 -> 39.6).  Without a
 //    mask a second round loses (B1 H7 N4555 d31 67.7 against 37.5), but for long ones at d = 32 (0.9 ... 1.2).
 inline bool fwd_uses_narrow(const FwdArgs& a, bool every)
 {
@@ -1274,8 +1276,10 @@ inline bool fwd_uses_narrow(const FwdArgs& a, bool every)
     }
     if (keys < a.Nk) return false;  // a window: the later work-groups are as heavy as the first
     if (a.causal && 2 * (long long)(a.fold_rows ? a.fold_rows : a.Nq) >= a.Nk) {
-        if (bucket == 1) return whole ? 40 * tiles >= groups : groups <= 640 && tiles >= 16;
-        if (bucket == 2) return groups <= 560 && 12 * (tiles - 8) >= groups - kNumCus;
+        const bool dropout = a.drop_thr != 0;
+        if (bucket == 1) return (whole && 40 * tiles >= groups) || (groups <= 640 && tiles >= (dropout ? 10 : 16));
+        if (bucket == 2 && !(dropout && tiles > 18)) return groups <= 560 && 12 * (tiles - 8) >= groups - kNumCus;
+        if (dropout) return groups <= 640 && (32 * (tiles - 8) >= groups - kNumCus) && (groups <= 512 || tiles >= 26);
         return groups <= 576 && 16 * (tiles - 8) >= groups - kNumCus;
     }
     return false;
