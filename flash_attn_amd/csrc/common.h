@@ -434,18 +434,21 @@ constexpr int kMaskRight = 1, kMaskLeft = 2, kMaskAbove = 4, kMaskBelow = 8, kMa
 #define FA_MASK_ABOVE(R, K, K4, T) "v_cmp_gt_i32_e32 vcc, " #T ", %[hi]\n\tv_cndmask_b32_e32 v[" R "], v[" R "], %[ninf], vcc\n\t"
 #define FA_MASK_BELOW(R, K, K4, T) "v_cmp_lt_i32_e32 vcc, " #T ", %[lo]\n\tv_cndmask_b32_e32 v[" R "], v[" R "], %[ninf], vcc\n\t"
 #define FA_MASK_WHOLE(R, K, K4, T) "v_mov_b32 v[" R "], %[ninf]\n\t"
+// (a taken branch costs some twenty cycles: whole groups of modes are passed by together)
 #define FA_MASK_IF(BIT, NAME, BODY) "s_bitcmp1_b32 %[modes], " #BIT "\n\ts_cbranch_scc0 .Lfa_" NAME "%=\n\t" BODY ".Lfa_" NAME "%=:\n\t"
+#define FA_MASK_BLOCK(B, ANY, DIAG, WHOLE, B0, B1, B2, B3, REGS) \
+    "s_and_b32 vcc_lo, %[modes], " ANY "\n\ts_cbranch_scc0 .Lfa_" B "z%=\n\t" \
+    "s_and_b32 vcc_lo, %[modes], " DIAG "\n\ts_cbranch_scc0 .Lfa_" B "o%=\n\t" \
+    FA_MASK_IF(B0, B "r", REGS(FA_MASK_RIGHT)) FA_MASK_IF(B1, B "l", REGS(FA_MASK_LEFT)) "s_branch .Lfa_" B "z%=\n\t" \
+    ".Lfa_" B "o%=:\n\t" FA_MASK_IF(B2, B "a", REGS(FA_MASK_ABOVE)) FA_MASK_IF(B3, B "b", REGS(FA_MASK_BELOW)) \
+    "s_and_b32 vcc_lo, %[modes], " WHOLE "\n\ts_cbranch_scc0 .Lfa_" B "z%=\n\t" REGS(FA_MASK_WHOLE) ".Lfa_" B "z%=:\n\t"
 template <bool kDiagonals>
 __device__ __forceinline__ void mask_tile(v16f& s0, v16f& s1, int modes, int lo, int hi, float ninf)
 {
     if constexpr (kDiagonals)
         asm(FA_FIRST_REGISTER("fa_a", "%[s0]") FA_FIRST_REGISTER("fa_b", "%[s1]") "s_nop 15\n\t"
-            FA_MASK_IF(0, "ar", FA_MASK_16A(FA_MASK_RIGHT)) FA_MASK_IF(1, "al", FA_MASK_16A(FA_MASK_LEFT))
-            FA_MASK_IF(2, "aa", FA_MASK_16A(FA_MASK_ABOVE)) FA_MASK_IF(3, "ab", FA_MASK_16A(FA_MASK_BELOW))
-            FA_MASK_IF(4, "aw", FA_MASK_16A(FA_MASK_WHOLE))
-            FA_MASK_IF(8, "br", FA_MASK_16B(FA_MASK_RIGHT)) FA_MASK_IF(9, "bl", FA_MASK_16B(FA_MASK_LEFT))
-            FA_MASK_IF(10, "ba", FA_MASK_16B(FA_MASK_ABOVE)) FA_MASK_IF(11, "bb", FA_MASK_16B(FA_MASK_BELOW))
-            FA_MASK_IF(12, "bw", FA_MASK_16B(FA_MASK_WHOLE))
+            FA_MASK_BLOCK("a", "31", "3", "16", 0, 1, 2, 3, FA_MASK_16A)
+            FA_MASK_BLOCK("b", "31*256", "3*256", "16*256", 8, 9, 10, 11, FA_MASK_16B)
             : [s0] "+v"(s0), [s1] "+v"(s1)
             : [modes] "s"(modes), [lo] "v"(lo), [hi] "v"(hi), [ninf] "v"(ninf)
             : "vcc", "scc");
@@ -457,28 +460,31 @@ __device__ __forceinline__ void mask_tile(v16f& s0, v16f& s1, int modes, int lo,
             : [modes] "s"(modes), [lo] "v"(lo), [hi] "v"(hi), [ninf] "v"(ninf)
             : "vcc", "scc");
 }
-// Modes of a tile whose first key is kb0, for rows that see keys from lo_min ... lo_max on and up to hi_min ... hi_max (their
-// bounds, which one after the other moves by one key per row where `straight`); sides: bit 0, the first key matters here,
-// bit 1, the last one does.
-template <bool kDiagonals>
-__device__ __forceinline__ int mask_modes(int kb0, int sides, bool straight, int lo_min, int lo_max, int hi_min, int hi_max)
+// 1 where x is negative / zero, in integers alone: as comparisons the scalar conditions end up in vector instructions
+__device__ __forceinline__ int is_negative(int x) { return (int)((unsigned)x >> 31); }
+__device__ __forceinline__ int is_zero(int x) { return 1 - is_negative(x | -x); }
+// Which ends of the interval cross the tile at key kb0, for rows that see keys from lo_max (the last first one) on and up to hi_min:
+// bit 0 the first key, bit 1 the last one
+__device__ __forceinline__ int mask_sides(int kb0, int lo_max, int hi_min) { return is_negative(kb0 - lo_max) | is_negative(hi_min - 63 - kb0) << 1; }
+// Which of the wave's bounds run along block diagonals, same bits: first row lo_min / hi_min, last row lo_max / hi_max
+__device__ __forceinline__ int diagonal_sides(bool straight, int lo_min, int lo_max, int hi_min, int hi_max)
 {
-    const bool hi_diag = straight && hi_max - hi_min == 31 && (hi_min & 31) == 0;
-    const bool lo_diag = straight && lo_max - lo_min == 31 && (lo_min & 31) == 0;
-    if (kDiagonals && ((sides & 1) == 0 || lo_diag) && ((sides & 2) == 0 || hi_diag)) {
-        int modes = 0;
+    return (straight && lo_max - lo_min == 31 && (lo_min & 31) == 0 ? 1 : 0) | (straight && hi_max - hi_min == 31 && (hi_min & 31) == 0 ? 2 : 0);
+}
+// Modes of a tile; general (the bounds of the lane's own row are asked for) where a crossing end does not run along a diagonal
+__device__ __forceinline__ bool mask_is_general(int sides, int diagonals) { return (sides & ~diagonals) != 0; }
+__device__ __forceinline__ int mask_modes_general(int sides) { return ((sides & 1) * kMaskBelow + (sides >> 1) * kMaskAbove) * 0x101; }
+__device__ __forceinline__ int mask_modes_diagonal(int kb0, int sides, int lo_min, int hi_min)
+{
+    // last / first visible key of the wave's first row, in blocks from the tile's first one
+    const int th = (sides & 2) ? (hi_min - kb0) >> 5 : 2, tl = (sides & 1) ? (lo_min - kb0) >> 5 : -1;
+    int modes = 0;
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            // last / first visible key of the wave's first row relative to the block: multiples of 32
-            const int dh = (sides & 2) ? hi_min - (kb0 + 32 * kb) : 64;
-            const int dl = (sides & 1) ? lo_min - (kb0 + 32 * kb) : -64;
-            const int m = dh < 0 || dl >= 32 ? kMaskWhole : (dh == 0 ? kMaskRight : 0) + (dl == 0 ? kMaskLeft : 0);
-            modes |= m << (8 * kb);
-        }
-        return wave_uniform(modes);  // (it is; said, because the compiler may hold it in a vector register)
+    for (int kb = 0; kb < 2; ++kb) {
+        const int whole = is_negative(th - kb) | is_negative(kb - tl);
+        modes |= (whole * kMaskWhole + (1 - whole) * (is_zero(th - kb) * kMaskRight + is_zero(tl - kb) * kMaskLeft)) << (8 * kb);
     }
-    const int m = ((sides & 1) ? kMaskBelow : 0) + ((sides & 2) ? kMaskAbove : 0);
-    return wave_uniform(m | m << 8);
+    return modes;
 }
 
 // three-input exclusive or in one instruction (v_bitop3_b32, truth table 0x96)

@@ -141,15 +141,15 @@ constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarSt
 
 // work-groups per CU (narrow: one or two by their LDS; held to 256 VGPRs all the same, without which the compiler keeps more
 // than there are and moves them to and from accumulation registers): three up to D = 96 (168 VGPRs), except for the instance that
-// serves every request, which stages its tiles through registers, and at D = 96 those with sixteen registers of bias constants,
-// which would spill (window with ALiBi B2 H16 N4096 d96 50 -> 57 us).  Four at D = 64 without dropout (128 VGPRs): the plain
-// instances fit by themselves, those with ALiBi do when told so (B32 H32 N512 d64 in 128-row blocks 100.3 -> 91.1 us together with the
-// shorter chunks below, causal window of 256 keys with ALiBi B2 H16 N4096 24.2 -> 23.7)
+// serves every request, which stages its tiles through registers, and at D = 96 those with sixteen registers of bias constants
+// and dropout, which would spill.  Four at D = 64 without either (128 VGPRs: B32 H32 N512 d64 in 128-row blocks 100.3 -> 91.1 us
+// together with the shorter chunks below); with the bias constants four spill in the loop (window of 256 keys with ALiBi B2
+// H16 N4096 d64 22.9 -> 24.4).
 constexpr int fwd_groups_per_cu(int D, int NB, int VAR)
 {
     if ((VAR & (kVarNarrow | kVarPair)) != 0) return 2;
-    if (D == 96 && (VAR & kVarAlibiLeft) != 0) return 2;
-    if (NB == 1 && D == 64 && (VAR & (kVarEvery | kVarDropout)) == 0) return 4;
+    if (D == 96 && (VAR & kVarAlibiLeft) != 0 && (VAR & kVarDropout) != 0) return 2;
+    if (NB == 1 && D == 64 && (VAR & (kVarEvery | kVarDropout | kVarAlibiLeft)) == 0) return 4;
     return NB == 1 && D <= 96 && (VAR & kVarEvery) == 0 ? 3 : 2;
 }
 
@@ -259,7 +259,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // wave-uniform bounds: [lo_max, hi_min] is visible to every row of the wave (a tile inside it needs no element
     // test), nothing outside [lo_min, hi_max] is visible to any of them (a tile outside it is skipped by the wave)
     int lo_max, hi_min, lo_min, hi_max;
-    bool straight;  // the rows' positions follow each other
+    int diagonals;  // which of the bounds run along diagonals of 32 x 32 score blocks (diagonal_sides)
     // the same in tiles of the work-group's range: first one and number of those that some row of the wave sees, and of those
     // that every row sees whole
     int live0, nlive, clean0, nclean;
@@ -270,6 +270,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
             const int i = row_i[nb];
             iif[nb] = (float)(row_position<kFold>(a, i < Nq ? i : Nq - 1) + shift);
         }
+        bool straight;
         {
             const int first = q0 + wave_row0, last = first + C::RW - 1;
             const RowSpan rows = row_span<kFold>(a, first < Nq ? first : Nq - 1, last < Nq ? last : Nq - 1);
@@ -287,6 +288,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                 hi_max = min(hi_max, kmax - 1);
             }
         }
+        diagonals = diagonal_sides(straight, lo_min, lo_max, hi_min, hi_max);
         // (a wave whose rows all lie past Nq sees nothing: it only helps to stage the tiles)
         live0 = (lo_min >> 6) - tile_begin;
         nlive = q0 + wave_row0 < Nq ? max(0, (hi_max >> 6) - tile_begin - live0 + 1) : 0;
@@ -652,12 +654,20 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                 // clipped by a sequence or split end.
                 // (kb0 is laundered: the compiler otherwise carries what it makes of it here through every tile)
                 asm volatile("" : "+s"(kb0));
-                const int sides = (kb0 < lo_max ? 1 : 0) | (kb0 + BC - 1 > hi_min ? 2 : 0);
-                const int modes = mask_modes<NB == 1>(kb0, sides, straight, lo_min, lo_max, hi_min, hi_max);
-                const int ln = lane_here();
-                int lo, hi;
-                row_bounds(q0 + wave_row0 + nb * 32 + (ln & 31), &lo, &hi);
-                mask_tile<NB == 1>(s[0][nb], s[1][nb], modes, lo - kb0 - 4 * (ln >> 5), hi - kb0 - 4 * (ln >> 5), -INFINITY);
+                const int sides = mask_sides(kb0, lo_max, hi_min);
+                int modes, lo_rel, hi_rel;
+                if (NB != 1 || mask_is_general(sides, diagonals)) {
+                    const int ln = lane_here();
+                    int lo, hi;
+                    row_bounds(q0 + wave_row0 + nb * 32 + (ln & 31), &lo, &hi);
+                    lo_rel = lo - kb0 - 4 * (ln >> 5);
+                    hi_rel = hi - kb0 - 4 * (ln >> 5);
+                    modes = mask_modes_general(sides);
+                } else {
+                    asm("" : "=v"(lo_rel), "=v"(hi_rel));  // (not read)
+                    modes = mask_modes_diagonal(kb0, sides, lo_min, hi_min);
+                }
+                mask_tile<NB == 1>(s[0][nb], s[1][nb], wave_uniform(modes), lo_rel, hi_rel, -INFINITY);
             }
             if constexpr (kEvery) {
                 if (a.scores_out != nullptr && row_i[nb] < Nq) {  // debug dump of the visible scores, natural-log units

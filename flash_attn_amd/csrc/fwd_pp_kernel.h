@@ -368,9 +368,9 @@ __global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const FwdArgs a)
     };
 
     // online softmax of the tile whose scores sit in s; leaves P^T packed to fp16 in pf
-    // mask_sides: bit 0 = some row of the wave has its first allowed key inside or after this tile, bit 1 = some row has
+    // sides: bit 0 = some row of the wave has its first allowed key inside or after this tile, bit 1 = some row has
     // its last allowed key inside or before it (both wave-uniform)
-    auto softmax = [&](int mask_sides, int kb0) __attribute__((always_inline)) {
+    auto softmax = [&](int sides, int kb0) __attribute__((always_inline)) {
         if constexpr (kDropout) calls.cover(kb0, lane, (uint32_t)bh, a.off_lo, a.seed_lo, a.seed_hi);
         if constexpr (kAlibi) {
             // score*scale - slope*|i - j|  (src/main.cu:315,324), in the log2 domain
@@ -381,10 +381,13 @@ __global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const FwdArgs a)
                 for (int r = 0; r < 16; ++r)
                     s[kb][r] = __builtin_fmaf(nsig, __builtin_fabsf(jb + (float)(32 * kb + 8 * (r >> 2) + (r & 3))), s[kb][r]);
         }
-        if (__builtin_expect(mask_sides != 0, 0)) {
-            const int modes = mask_modes<true>(kb0, mask_sides, true, __builtin_amdgcn_readlane(lo, 0), __builtin_amdgcn_readlane(lo, 31),
-                                               __builtin_amdgcn_readlane(hi, 0), __builtin_amdgcn_readlane(hi, 31));
-            mask_tile<true>(s[0], s[1], modes, lo - kb0 - 4 * g, hi - kb0 - 4 * g, -INFINITY);
+        if (__builtin_expect(sides != 0, 0)) {
+            const int diagonals = diagonal_sides(true, __builtin_amdgcn_readlane(lo, 0), __builtin_amdgcn_readlane(lo, 31),
+                                                 __builtin_amdgcn_readlane(hi, 0), __builtin_amdgcn_readlane(hi, 31));
+            const int modes = mask_is_general(sides, diagonals)
+                                  ? mask_modes_general(sides)
+                                  : mask_modes_diagonal(kb0, sides, __builtin_amdgcn_readlane(lo, 0), __builtin_amdgcn_readlane(hi, 0));
+            mask_tile<true>(s[0], s[1], wave_uniform(modes), lo - kb0 - 4 * g, hi - kb0 - 4 * g, -INFINITY);
         }
         // (the lane's half of the row's keys alone, in score units: see fwd_kernel.h)
         float mx = -INFINITY;
@@ -454,8 +457,7 @@ __global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const FwdArgs a)
         const int kb0 = (tile_begin + t) * BC;
         // ---------------- VALU phase: request the V tile to come, softmax of tile t
         if (t + 2 < ntiles) load_v(t + 2, wrv);
-        const int mask_sides = (kb0 < lo_max ? 1 : 0) | (kb0 + BC - 1 > hi_min ? 2 : 0);
-        softmax(mask_sides, kb0);
+        softmax(mask_sides(kb0, lo_max, hi_min), kb0);
         __builtin_amdgcn_sched_barrier(0);
         const uint32_t vbase = frag_base(rdv, v_rd);
         const uint32_t kbase = frag_base(rdk, k_rd);
