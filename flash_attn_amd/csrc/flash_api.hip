@@ -225,6 +225,24 @@ int auto_splits_tiled(const flash_params* p, int n_blocks, bool decode = false)
     return splits;
 }
 
+// Unsplit launches of several rounds of 32-row work-groups at the edge of what the narrow instances take: the 128-row instances
+// are as fast there or a little faster, but the estimate, which prices those too high when K and V stay in L2, would split them.
+// They stay whole: a call of such a shape needs no workspace, and none that exceeds the built-in scratch.
+bool near_narrow(const fa::FwdArgs& a, bool every)
+{
+    const long long groups = (long long)a.B * a.H * ((a.Nq + 31) / 32);
+    const int bucket = (a.d + 31) / 32, tiles = (a.Nk + 63) / 64;
+    const bool whole = a.d == 32 * bucket;
+    if (every || a.kernel_hint != 0 || groups > 1280 || groups <= (bucket == 1 ? 2 : 1) * kNumCU) return false;
+    const long long left = a.wl >= 0 ? a.wl : a.Nk, right = a.causal ? 0 : a.wr >= 0 ? a.wr : a.Nk;
+    if (left + right + 128 < a.Nk) return false;
+    if (a.causal && 2 * (long long)(a.fold_rows ? a.fold_rows : a.Nq) >= a.Nk) {
+        if (bucket == 1) return groups <= 576 ? tiles >= 9 : groups <= 800 && tiles >= 16;
+        return (bucket < 4 || whole) && (groups <= 384 ? tiles >= (bucket == 3 && !whole ? 20 : 14) : groups <= 640 && tiles >= 36);
+    }
+    return bucket == 1 ? tiles >= 64 : bucket == 2 && groups <= 512 && tiles >= 24;
+}
+
 int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
 {
     const int wl = window_left_of(p), wr = window_right_of(p);
@@ -263,7 +281,7 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
     fa::FwdArgs launch;
     fill_args(p, 1, &launch);
     if (fold) fold_heads(&launch);
-    if (!pp) narrow = fa::fwd_uses_narrow(launch, every);
+    if (!pp) narrow = fa::fwd_uses_narrow(launch, every) || near_narrow(launch, every);
     int limit = FLASH_MAX_SPLITS;
     if (n_blocks < limit) limit = n_blocks;
     int best_s = 1, prev_per = -1;
@@ -318,7 +336,7 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
         // as high, two unpaired work-groups to a CU: B2 H16 Nq111 Nk20468 d64 16 -> 8 splits 46.4 -> 42.4 us, B10 H4 Nq240 Nk9594 d72 6 -> 3
         // 56.6 -> 51.8, B6 H1 Nq459 Nk28734 d64 21 -> 10 40.0 -> 34.9.)
         launch.num_splits = s;
-        const bool paired = !pp && !every && k == 1 && fa::fwd_uses_pair(launch, 32 * bucket, tiled_variant(p) & 6);
+        const bool paired = !pp && !every && k == 1 && Nq > 32 && fa::fwd_uses_pair(launch, 32 * bucket, tiled_variant(p) & 6);
         float t = (float)k * a / rho + (paired ? 1.0f + 0.92f * b * chain : b * chain);
         if (s == 1 && narrow) {
             // 32-row work-groups with a visible key, and the time per tile of a wave on its own, measured: x 1.15 with
@@ -332,7 +350,8 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
             const float rhon = kn >= 2 && p->d <= 32 ? rho2 : 1.0f;
             const float bn = (p->d <= 64 ? ((p->d & 1) ? 1.955f : 1.15f) : bucket == 3 ? (p->d == 96 ? 1.3f : 1.6f) : p->d == 128 ? 1.6f : 2.3f) * b;
             const float later = p->is_causal && 2 * p->Nq >= p->Nk ? 0.5f : 1.0f;
-            t = (3.0f + (float)kn * (a - 1.0f) + bn * ((float)((tmax + 3) / 4) + later * (float)(kn - 1) * (float)tiles / (float)groups / 4.0f)) / rhon;
+            // (the launch takes the faster of the two)
+            t = fminf(t, (3.0f + (float)kn * (a - 1.0f) + bn * ((float)((tmax + 3) / 4) + later * (float)(kn - 1) * (float)tiles / (float)groups / 4.0f)) / rhon);
         }
         if (s > 1) t += c0 + (float)s * (c1 + partials);
         if (s == 1 || t < best_t) {

@@ -39,3 +39,25 @@ def test_features_in_every_bucket(fa, oracle, d, alibi, p):
         kw, okw = dict(kw, dropout_p=p, seed=7, offset=8), dict(okw, keep_mask=torch.from_numpy(keep), p_drop=p)
     O, L = oracle_forward_batched(oracle, q, k, v, **okw)
     check_o_lse(*fa.flash_forward(q, k, v, **kw), O, L, f"d {d} {sorted(kw)}")
+
+
+@pytest.mark.parametrize("B,H,Hk,Nq,Nk,d,p,kw", [
+    (2, 65, 65, 140, 2050, 32, 0.0, dict()), (1, 54, 54, 600, 2049, 24, 0.0, dict(causal=True)),  # 128-row work-groups past the CUs
+    (2, 130, 65, 50, 4100, 32, 0.0, dict()),                                     # folded, a second round at two per CU
+    (1, 9, 9, 930, 1540, 64, 0.0, dict()), (1, 9, 9, 930, 1540, 40, 0.2, dict()),  # K and V in L2
+    (1, 11, 11, 900, 2000, 50, 0.0, dict(window=(-1, 30))),                      # later work-groups with fewer keys
+    (1, 8, 8, 300, 2000, 128, 0.0, dict(window=(900, 20))), (1, 8, 4, 300, 2000, 100, 0.2, dict(window=(900, -1))),  # one stage per wave:
+    (1, 4, 4, 700, 400, 128, 0.0, dict(causal=True)), (1, 4, 4, 700, 450, 96, 0.2, dict(causal=True)),  # tiles and rows without a key
+    (1, 5, 5, 290, 130, 72, 0.0, dict(window=(40, -1))), (1, 14, 14, 1213, 2304, 112, 0.0, dict(causal=True)),
+])
+def test_more_rounds_and_one_stage_loops(fa, oracle, B, H, Hk, Nq, Nk, d, p, kw):
+    import torch
+
+    q, k, v = randn_f16_gpu((B, H, Nq, d), 1), randn_f16_gpu((B, Hk, Nk, d), 2), randn_f16_gpu((B, Hk, Nk, d), 3)
+    okw = dict(kw)
+    if p:
+        kw = dict(kw, dropout_p=p, seed=7, offset=8)
+        okw.update(keep_mask=torch.from_numpy(oracle.dropout_keep_mask(7, 8, p, B, H, Nq, Nk)), p_drop=p)
+    kr, vr = (t.repeat_interleave(H // Hk, dim=1).contiguous() for t in (k, v))
+    O, L = oracle_forward_batched(oracle, q, kr, vr, **okw)
+    check_o_lse(*fa.flash_forward(q, k, v, **kw), O, L, f"{B} {H} {Hk} {Nq} {Nk} {d} {kw}")
