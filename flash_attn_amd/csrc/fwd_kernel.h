@@ -1269,13 +1269,13 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
 //    5.9 / 5.7 / 6.8 / 7.2 -> 5.2 / 5.2 / 6.3 / 7.4; window of 100 keys N600, 4 tiles, 8.0 / 8.1 / 10.1 / 10.3 -> 5.3 / 5.3 / 6.7 / 7.8).
 //    Launches of up to 64 of them, which would gain as much, stay where they were below 4 tiles, 5 under a window: the tests
 //    of the 128-row instances' stage stamps ask for them there.
-//  * More rounds where the later work-groups are the light ones of a causal mask over about as many keys as rows (up to 512 of them else:
-//    with 1.9 keys per row B1 H14 N1213 d112, 532 of them, 33 against 44 us), the more tiles the more of them: D >= 96 from 8 + (groups -
-//    256) / 16 tiles on (narrow / 128 rows: 0.6 ... 1.0 there; B1 H3 N3748 d100, 354 of them: 48 -> 31 us; B8 H3 N1344 d64, 1008 of them: 19 ->
-//    25), D = 64 from 8 + (groups - 256) / 12 on, both up to 640; d = 32: a tile for every 40 of them (B1 H11 N2402: 20.0 -> 15.8), shorter
-//    rows, whose requests a wave alone hides less well, up to 640 from 16 on, 800 from 32 on; with dropout, whose tiles cost more
-//    beside the same fixed part, D >= 96 up to 512 from 8 + (groups - 256) / 32 on and up to 640 from 26 on, D = 64 the same beyond 18 tiles
-//    (B1 H11 N1267 21.9 -> 16.2), D = 32 up to 640 from 10 on (B1 H12 N1261 d128 30.1 -> 23.0, B1 H7 N2635 d96 45.2 -> 39.6).
+//  * More rounds where the later work-groups are the light ones of a causal mask over about as many keys as rows, the more tiles the more
+//    of them that see a key: D >= 96 from (groups - 256) / 16 tiles on, up to 640, 720 from 60 tiles, 800 from 100 on (narrow / 128 rows: B1
+//    H5 N4105 d96, 645 of them, 36.7 / 44.7 us; H14 N1001 d96, 448, 13.0 / 15.6; H16 Nq586 d128, 304, 10.9 / 13.4; but H10 N2833 d80, 890, 37.2 / 33.7);
+//    D = 64 from 8 + (groups - 256) / 12 tiles on up to 560, 640 from 36 on; d = 32: a tile for every 40 of them (B1 H11 N2402: 20.0 -> 15.8), shorter
+//    rows, whose requests a wave alone hides less well, up to 640 from 16 on, 800 from 32 on; D = 64 with dropout like D >= 96 beyond 18 tiles
+//    (B1 H11 N1267 21.9 -> 16.2), D = 32 with dropout from 10 tiles on.  With more keys than 5/4 of the rows (4/3 with dropout) the lightest ones
+//    are heavy too: up to 512, from 8 + (groups - 256) / 16 tiles on, / 32 with dropout (1.9 keys per row, B1 H14 N1213 d112, 532 of them, 44 / 33 us).
 //  * Short rows over many tiles in more rounds, any mask, where the 128-row work-groups are more than the CUs and so cannot be paired
 //    (B5 H8 H_kv4 Nq785 Nk20772 d32, 260 of them: 270 -> 172 us), or the last rounds are light, or there are few rounds; while K and V, which
 //    the narrow ones read once per 32 rows, stay in the 32 MiB of L2 (117 slices of 20695 keys d32, 310 MB, ten work-groups each:
@@ -1299,12 +1299,13 @@ inline bool fwd_uses_narrow(const FwdArgs& a, bool every)
     const bool dropout = a.drop_thr != 0;
     const long long rows = a.fold_rows ? a.fold_rows : a.Nq;
     if (a.causal && 2 * rows >= a.Nk) {
-        const bool to_nothing = (dropout ? 4 : 8) * rows >= (dropout ? 3 : 7) * (long long)a.Nk;  // the lightest work-groups see few keys
         if (bucket == 1) return (whole && 40 * tiles >= groups) || (groups <= (tiles >= 32 ? 800 : 640) && tiles >= (dropout ? 10 : 16));
-        if (groups > (to_nothing ? 640 : 2 * kNumCus)) return false;
-        if (bucket == 2 && !(dropout && tiles > 18)) return 12 * (tiles - 8) >= groups - kNumCus && (groups <= 560 || tiles >= 36);
-        if (dropout) return 32 * (tiles - 8) >= groups - kNumCus && (groups <= 512 || tiles >= 26);
-        return 16 * (tiles - 8) >= groups - kNumCus && (groups <= 576 || tiles >= 36);
+        const long long seeing = rows > a.Nk ? groups * a.Nk / rows : groups;  // the others leave at once
+        const bool to_nothing = (dropout ? 4 : 5) * rows >= (dropout ? 3 : 4) * (long long)a.Nk;  // the lightest work-groups see few keys
+        if (seeing > (to_nothing ? 800 : 2 * kNumCus)) return false;
+        if (bucket == 2 && !(dropout && tiles > 18)) return 12 * (tiles - 8) >= seeing - kNumCus && (seeing <= 560 || (seeing <= 640 && tiles >= 36));
+        if (to_nothing) return 16 * tiles >= seeing - kNumCus && seeing <= (tiles >= 100 ? 800 : tiles >= 60 ? 720 : 640);
+        return (dropout ? 32 : 16) * (tiles - 8) >= seeing - kNumCus;
     }
     if (bucket > 2 || (a.d % 2 != 0 && !dropout)) return false;
     const long long groups128 = (long long)a.Tr * a.B * a.H;

@@ -48,6 +48,7 @@ def test_features_in_every_bucket(fa, oracle, d, alibi, p):
     (1, 11, 11, 900, 2000, 50, 0.0, dict(window=(-1, 30))),                      # later work-groups with fewer keys
     (1, 8, 8, 300, 2000, 128, 0.0, dict(window=(900, 20))), (1, 8, 4, 300, 2000, 100, 0.2, dict(window=(900, -1))),  # one stage per wave:
     (1, 4, 4, 700, 400, 128, 0.0, dict(causal=True)), (1, 4, 4, 700, 450, 96, 0.2, dict(causal=True)),  # tiles and rows without a key
+    (1, 14, 14, 1001, 1001, 96, 0.0, dict(causal=True)), (1, 6, 6, 1288, 772, 128, 0.2, dict(causal=True)),  # 448 and 246 that see a key
     (1, 5, 5, 290, 130, 72, 0.0, dict(window=(40, -1))), (1, 14, 14, 1213, 2304, 112, 0.0, dict(causal=True)),
 ])
 def test_more_rounds_and_one_stage_loops(fa, oracle, B, H, Hk, Nq, Nk, d, p, kw):
