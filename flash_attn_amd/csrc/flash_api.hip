@@ -342,13 +342,18 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
             // 32-row work-groups with a visible key, and the time per tile of a wave on its own, measured: x 1.15 with
             // two LDS stages per wave (d <= 64); with one, where the next tile's requests are only partly hidden, x 1.3 at
             // d = 96 and x 1.6 at d = 128, x 1.6 and x 2.3 for rows shorter than those buckets (2.05 us per tile at d = 100,
-            // 1.3 at d = 80), x 1.7 on top up to d = 64 for odd d (every second row off a 4-byte boundary: slower requests,
+            // 1.3 at d = 80) -- a sixth less under a causal mask since the loop above d = 64 has a body per kind
+            // of tile, half of that with dropout, and not where K and V come from HBM (90 shapes whose count this changed: 1.32 in the mean, B3 H2
+            // N1610 d80 5 -> 1 split 21.2 -> 11.9 us; without a mask 0.9 ... 1.4, left as it was) --, x 1.7 on top up to d = 64 for odd d (every second row off a 4-byte boundary: slower requests,
             // which a wave on its own cannot hide); under a causal mask with about as many rows as keys the work-groups that
             // follow another on their CU are the light ones of rows that found their tiles in L2 already, and take half of that
             const long long gn = (groups * ((Nq + 31) / 32) + Tr - 1) / Tr;
             const long long kn = (gn + kNumCU - 1) / kNumCU;
             const float rhon = kn >= 2 && p->d <= 32 ? rho2 : 1.0f;
-            const float bn = (p->d <= 64 ? ((p->d & 1) ? 1.955f : 1.15f) : bucket == 3 ? (p->d == 96 ? 1.3f : 1.6f) : p->d == 128 ? 1.6f : 2.3f) * b;
+            const bool in_l2 = 4LL * p->d * p->Nk * p->B * (p->H_kv > 0 ? p->H_kv : p->H) <= (32 << 20);
+            const float apart = !in_l2 || !p->is_causal ? 1.0f : p->dropout_p > 0.0f ? 0.92f : 0.84f;
+            const float bn = (p->d <= 64 ? ((p->d & 1) ? 1.955f : 1.15f)
+                              : (bucket == 3 ? (p->d == 96 ? 1.3f : 1.6f) : p->d == 128 ? 1.6f : 2.3f) * apart) * b;
             const float later = p->is_causal && 2 * p->Nq >= p->Nk ? 0.5f : 1.0f;
             // (the launch takes the faster of the two)
             t = fminf(t, (3.0f + (float)kn * (a - 1.0f) + bn * ((float)((tmax + 3) / 4) + later * (float)(kn - 1) * (float)tiles / (float)groups / 4.0f)) / rhon);
