@@ -418,45 +418,62 @@ constexpr int kMaskRight = 1, kMaskLeft = 2, kMaskAbove = 4, kMaskBelow = 8, kMa
     ".if fa_in == 2\n\t.ifnc \\fa_c,:\n\t.set fa_last, fa_last * 10 + \\fa_c\n\t.endif\n\t.endif\n\t" \
     ".ifc \\fa_c,[\n\t.set fa_in, 1\n\t.endif\n\t.endr\n\t" \
     ".if fa_last - " SYM " - 15\n\t.error \"an accumulator of sixteen registers\"\n\t.endif\n\t"
-// register, its key in the lower half of the lanes, in the upper half, and the lower one counted from the tile's start
-#define FA_MASK_16A(X) X("fa_a+0", 0, 4, 0) X("fa_a+1", 1, 5, 1) X("fa_a+2", 2, 6, 2) X("fa_a+3", 3, 7, 3) X("fa_a+4", 8, 12, 8) \
-    X("fa_a+5", 9, 13, 9) X("fa_a+6", 10, 14, 10) X("fa_a+7", 11, 15, 11) X("fa_a+8", 16, 20, 16) X("fa_a+9", 17, 21, 17) \
-    X("fa_a+10", 18, 22, 18) X("fa_a+11", 19, 23, 19) X("fa_a+12", 24, 28, 24) X("fa_a+13", 25, 29, 25) X("fa_a+14", 26, 30, 26) \
-    X("fa_a+15", 27, 31, 27)
-#define FA_MASK_16B(X) X("fa_b+0", 0, 4, 32) X("fa_b+1", 1, 5, 33) X("fa_b+2", 2, 6, 34) X("fa_b+3", 3, 7, 35) X("fa_b+4", 8, 12, 40) \
-    X("fa_b+5", 9, 13, 41) X("fa_b+6", 10, 14, 42) X("fa_b+7", 11, 15, 43) X("fa_b+8", 16, 20, 48) X("fa_b+9", 17, 21, 49) \
-    X("fa_b+10", 18, 22, 50) X("fa_b+11", 19, 23, 51) X("fa_b+12", 24, 28, 56) X("fa_b+13", 25, 29, 57) X("fa_b+14", 26, 30, 58) \
-    X("fa_b+15", 27, 31, 59)
-#define FA_MASK_RIGHT(R, K, K4, T) \
+// register, its key in the lower half of the lanes and in the upper half
+#define FA_MASK_16A(X) X("fa_a+0", 0, 4) X("fa_a+1", 1, 5) X("fa_a+2", 2, 6) X("fa_a+3", 3, 7) X("fa_a+4", 8, 12) \
+    X("fa_a+5", 9, 13) X("fa_a+6", 10, 14) X("fa_a+7", 11, 15) X("fa_a+8", 16, 20) X("fa_a+9", 17, 21) \
+    X("fa_a+10", 18, 22) X("fa_a+11", 19, 23) X("fa_a+12", 24, 28) X("fa_a+13", 25, 29) X("fa_a+14", 26, 30) \
+    X("fa_a+15", 27, 31)
+#define FA_MASK_16B(X) X("fa_b+0", 0, 4) X("fa_b+1", 1, 5) X("fa_b+2", 2, 6) X("fa_b+3", 3, 7) X("fa_b+4", 8, 12) \
+    X("fa_b+5", 9, 13) X("fa_b+6", 10, 14) X("fa_b+7", 11, 15) X("fa_b+8", 16, 20) X("fa_b+9", 17, 21) \
+    X("fa_b+10", 18, 22) X("fa_b+11", 19, 23) X("fa_b+12", 24, 28) X("fa_b+13", 25, 29) X("fa_b+14", 26, 30) \
+    X("fa_b+15", 27, 31)
+#define FA_MASK_RIGHT(R, K, K4) \
     "s_bfm_b32 vcc_lo, " #K ", 0\n\ts_bfm_b32 vcc_hi, " #K4 ", 0\n\tv_cndmask_b32_e32 v[" R "], v[" R "], %[ninf], vcc\n\t"
-#define FA_MASK_LEFT(R, K, K4, T) \
+#define FA_MASK_LEFT(R, K, K4) \
     "s_bfm_b64 vcc, " #K4 "+1, 32\n\ts_bfm_b32 vcc_lo, " #K "+1, 0\n\tv_cndmask_b32_e32 v[" R "], %[ninf], v[" R "], vcc\n\t"
-#define FA_MASK_ABOVE(R, K, K4, T) "v_cmp_gt_i32_e32 vcc, " #T ", %[hi]\n\tv_cndmask_b32_e32 v[" R "], v[" R "], %[ninf], vcc\n\t"
-#define FA_MASK_BELOW(R, K, K4, T) "v_cmp_lt_i32_e32 vcc, " #T ", %[lo]\n\tv_cndmask_b32_e32 v[" R "], v[" R "], %[ninf], vcc\n\t"
-#define FA_MASK_WHOLE(R, K, K4, T) "v_mov_b32 v[" R "], %[ninf]\n\t"
+// (A v_cndmask wants two wait states behind the vector instruction that wrote its scalar operand, and inside a statement nobody but
+// the statement provides them.  Comparisons into vcc and into a scalar pair take turns, two of a block's scores ahead of their
+// selections: the instructions between are the neighbours' and cost nothing, where an s_nop 1 per score takes half as long again.)
+#define FA_MASK_CMP0(CMP, BOUND, T) CMP "_e32 vcc, " #T ", " BOUND "\n\t"
+#define FA_MASK_CMP1(CMP, BOUND, T) CMP "_e64 %[pair], " #T ", " BOUND "\n\t"
+#define FA_MASK_SEL0(A, R) "v_cndmask_b32_e32 v[" A "+" #R "], v[" A "+" #R "], %[ninf], vcc\n\t"
+#define FA_MASK_SEL1(A, R) "v_cndmask_b32_e64 v[" A "+" #R "], v[" A "+" #R "], %[ninf], %[pair]\n\t"
+#define FA_MASK_NEXT(CMP, BOUND, A, R0, R1, T0, T1) \
+    FA_MASK_SEL0(A, R0) FA_MASK_CMP0(CMP, BOUND, T0) FA_MASK_SEL1(A, R1) FA_MASK_CMP1(CMP, BOUND, T1)
+#define FA_MASK_BOUND(CMP, BOUND, A, T0, T1, T2, T3, T4, T5, T6, T7, T8, T9, T10, T11, T12, T13, T14, T15) \
+    FA_MASK_CMP0(CMP, BOUND, T0) FA_MASK_CMP1(CMP, BOUND, T1) "s_nop 0\n\t" \
+    FA_MASK_NEXT(CMP, BOUND, A, 0, 1, T2, T3) FA_MASK_NEXT(CMP, BOUND, A, 2, 3, T4, T5) FA_MASK_NEXT(CMP, BOUND, A, 4, 5, T6, T7) \
+    FA_MASK_NEXT(CMP, BOUND, A, 6, 7, T8, T9) FA_MASK_NEXT(CMP, BOUND, A, 8, 9, T10, T11) FA_MASK_NEXT(CMP, BOUND, A, 10, 11, T12, T13) \
+    FA_MASK_NEXT(CMP, BOUND, A, 12, 13, T14, T15) FA_MASK_SEL0(A, 14) "s_nop 0\n\t" FA_MASK_SEL1(A, 15)
+#define FA_MASK_BOUND_A(CMP, BOUND) FA_MASK_BOUND(CMP, BOUND, "fa_a", 0, 1, 2, 3, 8, 9, 10, 11, 16, 17, 18, 19, 24, 25, 26, 27)
+#define FA_MASK_BOUND_B(CMP, BOUND) FA_MASK_BOUND(CMP, BOUND, "fa_b", 32, 33, 34, 35, 40, 41, 42, 43, 48, 49, 50, 51, 56, 57, 58, 59)
+#define FA_MASK_ABOVE(BOUNDS) BOUNDS("v_cmp_gt_i32", "%[hi]")
+#define FA_MASK_BELOW(BOUNDS) BOUNDS("v_cmp_lt_i32", "%[lo]")
+#define FA_MASK_WHOLE(R, K, K4) "v_mov_b32 v[" R "], %[ninf]\n\t"
 // (a taken branch costs some twenty cycles: whole groups of modes are passed by together)
 #define FA_MASK_IF(BIT, NAME, BODY) "s_bitcmp1_b32 %[modes], " #BIT "\n\ts_cbranch_scc0 .Lfa_" NAME "%=\n\t" BODY ".Lfa_" NAME "%=:\n\t"
-#define FA_MASK_BLOCK(B, ANY, DIAG, WHOLE, B0, B1, B2, B3, REGS) \
+#define FA_MASK_BLOCK(B, ANY, DIAG, WHOLE, B0, B1, B2, B3, REGS, BOUNDS) \
     "s_and_b32 vcc_lo, %[modes], " ANY "\n\ts_cbranch_scc0 .Lfa_" B "z%=\n\t" \
     "s_and_b32 vcc_lo, %[modes], " DIAG "\n\ts_cbranch_scc0 .Lfa_" B "o%=\n\t" \
     FA_MASK_IF(B0, B "r", REGS(FA_MASK_RIGHT)) FA_MASK_IF(B1, B "l", REGS(FA_MASK_LEFT)) "s_branch .Lfa_" B "z%=\n\t" \
-    ".Lfa_" B "o%=:\n\t" FA_MASK_IF(B2, B "a", REGS(FA_MASK_ABOVE)) FA_MASK_IF(B3, B "b", REGS(FA_MASK_BELOW)) \
+    ".Lfa_" B "o%=:\n\t" FA_MASK_IF(B2, B "a", FA_MASK_ABOVE(BOUNDS)) FA_MASK_IF(B3, B "b", FA_MASK_BELOW(BOUNDS)) \
     "s_and_b32 vcc_lo, %[modes], " WHOLE "\n\ts_cbranch_scc0 .Lfa_" B "z%=\n\t" REGS(FA_MASK_WHOLE) ".Lfa_" B "z%=:\n\t"
 template <bool kDiagonals>
 __device__ __forceinline__ void mask_tile(v16f& s0, v16f& s1, int modes, int lo, int hi, float ninf)
 {
+    uint64_t pair;
     if constexpr (kDiagonals)
         asm(FA_FIRST_REGISTER("fa_a", "%[s0]") FA_FIRST_REGISTER("fa_b", "%[s1]") "s_nop 15\n\t"
-            FA_MASK_BLOCK("a", "31", "3", "16", 0, 1, 2, 3, FA_MASK_16A)
-            FA_MASK_BLOCK("b", "31*256", "3*256", "16*256", 8, 9, 10, 11, FA_MASK_16B)
-            : [s0] "+v"(s0), [s1] "+v"(s1)
+            FA_MASK_BLOCK("a", "31", "3", "16", 0, 1, 2, 3, FA_MASK_16A, FA_MASK_BOUND_A)
+            FA_MASK_BLOCK("b", "31*256", "3*256", "16*256", 8, 9, 10, 11, FA_MASK_16B, FA_MASK_BOUND_B)
+            : [s0] "+v"(s0), [s1] "+v"(s1), [pair] "=&s"(pair)
             : [modes] "s"(modes), [lo] "v"(lo), [hi] "v"(hi), [ninf] "v"(ninf)
             : "vcc", "scc");
     else
         asm(FA_FIRST_REGISTER("fa_a", "%[s0]") FA_FIRST_REGISTER("fa_b", "%[s1]") "s_nop 15\n\t"
-            FA_MASK_IF(2, "a", FA_MASK_16A(FA_MASK_ABOVE) FA_MASK_16B(FA_MASK_ABOVE))
-            FA_MASK_IF(3, "b", FA_MASK_16A(FA_MASK_BELOW) FA_MASK_16B(FA_MASK_BELOW))
-            : [s0] "+v"(s0), [s1] "+v"(s1)
+            FA_MASK_IF(2, "a", FA_MASK_ABOVE(FA_MASK_BOUND_A) FA_MASK_ABOVE(FA_MASK_BOUND_B))
+            FA_MASK_IF(3, "b", FA_MASK_BELOW(FA_MASK_BOUND_A) FA_MASK_BELOW(FA_MASK_BOUND_B))
+            : [s0] "+v"(s0), [s1] "+v"(s1), [pair] "=&s"(pair)
             : [modes] "s"(modes), [lo] "v"(lo), [hi] "v"(hi), [ninf] "v"(ninf)
             : "vcc", "scc");
 }

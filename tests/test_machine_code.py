@@ -1,0 +1,63 @@
+"""The distances between instructions that the hardware of gfx950 asks of the program, in the code as it was built.  The compiler
+keeps them for what it writes itself, and cannot for what stands inside an inline-assembly statement.  No GPU needed."""
+import os
+
+import machine_code as mc
+
+LIBRARY = os.path.join(mc.ROOT, "flash_attn_amd", "lib", "libflash_attn_mi355.so")
+
+# vector instructions whose second operand is a result too
+TWO_RESULTS = ("v_mad_u64_u32", "v_mad_i64_i32", "v_add_co_u32", "v_sub_co_u32", "v_subrev_co_u32", "v_addc_co_u32", "v_subb_co_u32",
+               "v_subbrev_co_u32", "v_div_scale_f32", "v_permlane32_swap", "v_permlane16_swap", "v_swap_b32")
+READS_VCC = ("v_cndmask_b32_e32", "v_addc_co_u32_e32", "v_subb_co_u32_e32", "v_div_fmas_f32")
+
+
+def too_close(body):
+    """(what, index of the reader) wherever a reader follows the writer of its operand with fewer wait states than these, the ones
+    that the compiler provides between instructions of its own (an s_nop n counts n + 1, every other instruction 1):
+      2   a vector instruction wrote a scalar register (vcc too), a vector instruction reads it
+      5   a vector instruction wrote a scalar register, a memory instruction reads it
+    Straight through the code, branches counted as one instruction: what is asked for holds on the path that falls through."""
+    now, scalar = 0, {}
+    for i, (m, text) in enumerate(body):
+        operands = [mc.registers(x) for x in text.split(",")]
+        if m.startswith("v_"):
+            results = 2 if m.startswith(TWO_RESULTS) else 1
+            written, read = set().union(*operands[:results]), set().union(*operands[results:])
+            if m in READS_VCC:
+                read |= mc.registers("vcc")
+            if any(now - scalar[r] <= 2 for r in read if r in scalar):
+                yield "scalar register written and read by vector instructions", i
+            for r in written:
+                if r[0] == "s":
+                    scalar[r] = now
+        elif m.startswith(("global_", "buffer_", "scratch_", "flat_", "ds_")):
+            if any(now - scalar[r] <= 5 for r in set().union(*operands) if r in scalar):
+                yield "scalar register written by a vector instruction, read by a memory instruction", i
+        elif m.startswith("s_") and not m.startswith(("s_cmp", "s_bitcmp", "s_cbranch", "s_nop", "s_wait", "s_barrier")):
+            for r in operands[0]:
+                scalar.pop(r, None)
+        now += 1 + (int(text, 0) if m == "s_nop" else 0)
+        if m in ("s_branch", "s_endpgm", "s_setpc_b64"):
+            scalar.clear()
+
+
+def test_the_check_sees_what_it_is_for():
+    compare, select = ("v_cmp_gt_i32_e32", "vcc, 5, v1"), ("v_cndmask_b32_e32", "v2, v2, v3, vcc")
+    other = ("v_mov_b32_e32", "v9, v8")
+    assert [i for _, i in too_close([compare, select])] == [1]
+    assert [i for _, i in too_close([compare, other, select])] == [2]
+    assert not list(too_close([compare, other, other, select])) and not list(too_close([compare, ("s_nop", "1"), select]))
+    assert list(too_close([("v_cmp_gt_i32_e64", "s[4:5], 5, v1"), ("v_cndmask_b32_e64", "v2, v2, v3, s[4:5]")]))
+    first = ("v_readfirstlane_b32", "s4, v1")
+    assert list(too_close([first, ("s_nop", "3"), ("global_load_lds_dwordx4", "v0, s[4:5]")]))
+    assert not list(too_close([first, ("s_nop", "4"), ("global_load_lds_dwordx4", "v0, s[4:5]")]))
+    assert not list(too_close([first, ("s_mov_b32", "s4, 0"), ("global_load_lds_dwordx4", "v0, s[4:5]")]))
+
+
+def test_wait_states():
+    found, seen = [], 0
+    for name, body in mc.kernels(LIBRARY):
+        seen += 1
+        found += [(name, i, what, body[max(0, i - 3):i + 1]) for what, i in too_close(body)]
+    assert seen > 300 and not found, (len(found), found[:3])
