@@ -612,6 +612,11 @@ __device__ __forceinline__ uint32_t keep_pair(uint32_t p2, uint32_t w, uint32_t 
     return x;
 }
 
+// An MFMA reads a register two wait states after the vector instruction that wrote it at the earliest; the compiler, which keeps
+// that distance in its own code, does not see which instruction a statement like keep_pair's ends with.  To stand between
+// operands that come out of such a statement and the MFMA.
+__device__ __forceinline__ void settle_for_mfma(v8h& p) { asm("s_nop 1" : "+v"(p)); }
+
 // 16-bit field f (0..7) of a Philox output
 __device__ __forceinline__ uint32_t philox_field16(const v4u& w, int f) { return (w[f >> 1] >> (16 * (f & 1))) & 0xffffu; }
 

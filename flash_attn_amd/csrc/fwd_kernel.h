@@ -789,6 +789,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                     p[2 * k] = pk.h[0];
                     p[2 * k + 1] = pk.h[1];
                 }
+                settle_for_mfma(p);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb) oacc[mb][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mb], p, oacc[mb][0], 0, 0, 0);

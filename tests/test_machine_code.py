@@ -16,9 +16,10 @@ def too_close(body):
     """(what, index of the reader) wherever a reader follows the writer of its operand with fewer wait states than these, the ones
     that the compiler provides between instructions of its own (an s_nop n counts n + 1, every other instruction 1):
       2   a vector instruction wrote a scalar register (vcc too), a vector instruction reads it
+      2   a vector instruction wrote a vector register, an MFMA reads it
       5   a vector instruction wrote a scalar register, a memory instruction reads it
     Straight through the code, branches counted as one instruction: what is asked for holds on the path that falls through."""
-    now, scalar = 0, {}
+    now, scalar, vector = 0, {}, {}
     for i, (m, text) in enumerate(body):
         operands = [mc.registers(x) for x in text.split(",")]
         if m.startswith("v_"):
@@ -28,9 +29,14 @@ def too_close(body):
                 read |= mc.registers("vcc")
             if any(now - scalar[r] <= 2 for r in read if r in scalar):
                 yield "scalar register written and read by vector instructions", i
-            for r in written:
-                if r[0] == "s":
-                    scalar[r] = now
+            if m.startswith("v_mfma"):
+                if any(now - vector[r] <= 2 for r in read if r in vector):
+                    yield "register written by a vector instruction, read by an MFMA", i
+                for r in written:
+                    vector.pop(r, None)
+            else:
+                vector.update({r: now for r in written if r[0] == "v"})
+            scalar.update({r: now for r in written if r[0] == "s"})
         elif m.startswith(("global_", "buffer_", "scratch_", "flat_", "ds_")):
             if any(now - scalar[r] <= 5 for r in set().union(*operands) if r in scalar):
                 yield "scalar register written by a vector instruction, read by a memory instruction", i
@@ -40,6 +46,7 @@ def too_close(body):
         now += 1 + (int(text, 0) if m == "s_nop" else 0)
         if m in ("s_branch", "s_endpgm", "s_setpc_b64"):
             scalar.clear()
+            vector.clear()
 
 
 def test_the_check_sees_what_it_is_for():
@@ -53,6 +60,9 @@ def test_the_check_sees_what_it_is_for():
     assert list(too_close([first, ("s_nop", "3"), ("global_load_lds_dwordx4", "v0, s[4:5]")]))
     assert not list(too_close([first, ("s_nop", "4"), ("global_load_lds_dwordx4", "v0, s[4:5]")]))
     assert not list(too_close([first, ("s_mov_b32", "s4, 0"), ("global_load_lds_dwordx4", "v0, s[4:5]")]))
+    packed, mfma = ("v_pk_mul_lo_u16", "v31, v33, v31"), ("v_mfma_f32_32x32x16_f16", "v[4:19], v[20:23], v[28:31], v[4:19]")
+    assert list(too_close([packed, ("s_waitcnt", "lgkmcnt(1)"), mfma])) and list(too_close([packed, mfma]))
+    assert not list(too_close([packed, ("s_nop", "1"), mfma])) and not list(too_close([mfma, mfma]))
 
 
 def test_wait_states():
