@@ -285,7 +285,8 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
     int limit = FLASH_MAX_SPLITS;
     if (n_blocks < limit) limit = n_blocks;
     int best_s = 1, prev_per = -1;
-    float best_t = 0.0f;
+    float best_t = 0.0f, t_whole = 0.0f;
+    bool whole = true;  // no count is faster than the unsplit launch by the price of unpaired work-groups
     for (int s = 1; s <= limit; ++s) {
         const int per = (n_blocks + s - 1) / s;
         if (per == prev_per) continue;  // the same ranges as s - 1 plus an empty split (src/main.cu:397-398)
@@ -337,7 +338,10 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
         // 56.6 -> 51.8, B6 H1 Nq459 Nk28734 d64 21 -> 10 40.0 -> 34.9.)
         launch.num_splits = s;
         const bool paired = !pp && !every && k == 1 && Nq > 32 && fa::fwd_uses_pair(launch, 32 * bucket, tiled_variant(p) & 6);
-        float t = (float)k * a / rho + (paired ? 1.0f + 0.92f * b * chain : b * chain);
+        // (How many splits, not whether to split: with that price launches that were whole in 32-row work-groups came out in a few
+        // splits, causal B1 H12 Nq425 Nk6429 d64 in 5, and callers who bring no workspace for them were refused.)
+        const float unpaired = (float)k * a / rho + b * chain;
+        float t = paired ? (float)k * a / rho + (1.0f + 0.92f * b * chain) : unpaired;
         if (s == 1 && narrow) {
             // 32-row work-groups with a visible key, and the time per tile of a wave on its own, measured: x 1.15 with
             // two LDS stages per wave (d <= 64); with one, where the next tile's requests are only partly hidden, x 1.3 at
@@ -358,13 +362,16 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
             // (the launch takes the faster of the two)
             t = fminf(t, (3.0f + (float)kn * (a - 1.0f) + bn * ((float)((tmax + 3) / 4) + later * (float)(kn - 1) * (float)tiles / (float)groups / 4.0f)) / rhon);
         }
-        if (s > 1) t += c0 + (float)s * (c1 + partials);
+        const float merge = s > 1 ? c0 + (float)s * (c1 + partials) : 0.0f;
+        t += merge;
+        if (s == 1) t_whole = fminf(t, unpaired);
+        else if (unpaired + merge < t_whole) whole = false;
         if (s == 1 || t < best_t) {
             best_t = t;
             best_s = s;
         }
     }
-    return best_s;
+    return whole ? 1 : best_s;
 }
 
 int resolve_splits(const flash_params* p)

@@ -141,3 +141,14 @@ def test_paired_launches_of_the_dropout_tests():
               for Nq, d in ((33, 128), (140, 100), (128, 64))]
     for c, r in zip(calls, record(calls)):
         assert r["launches"][0]["variant"] & (PAIR | NARROW | DROPOUT) == PAIR | DROPOUT, c
+
+
+def test_launches_that_are_whole_without_their_paired_form_need_no_workspace():
+    """Whether to split is not a matter of the paired work-groups' price: a caller of such a shape brings no workspace."""
+    shapes = [(1, 12, 12, 425, 6429, 64, 1, 0.0), (2, 16, 2, 436, 2828, 64, 1, 0.0), (4, 48, 12, 30, 3410, 64, 0, 0.0),
+              (2, 1, 1, 3543, 4219, 128, 0, 0.1), (6, 24, 12, 28, 2283, 72, 0, 0.0), (7, 2, 2, 525, 5976, 128, 1, 0.0)]
+    calls = [dict(entry="splitkv", B=B, H=H, H_kv=Hk, Nq=Nq, Nk=Nk, d=d, is_causal=c, dropout_p=p, num_splits=0)
+             for B, H, Hk, Nq, Nk, d, c, p in shapes]
+    calls.append(dict(entry="splitkv", B=3, H=3, Nq=996, Nk=996, d=40, window_left=1470, window_right=100, num_splits=0))
+    for c, r in zip(calls, record(calls)):
+        assert r["rc"] == 0 and r["splits"] == 1 and r["workspace"] == [0, 0] and len(r["launches"]) == 1, (c, r)
