@@ -36,7 +36,7 @@ constexpr float kLn2 = 0.6931471805599453f;
 // earlier (B1 H2 N128 d64 5.1 -> 4.8 us, decode B15 H2 Nk3200 d64 8.9 -> 8.5 us, B2 H8 N2560 d40 causal 34.1 -> 33.6).
 struct FastDiv {
     uint32_t mul, shift;
-    __device__ __forceinline__ int quotient(int n) const { return (int)(__umulhi(2u * (uint32_t)n, mul) >> shift); }
+    __host__ __device__ __forceinline__ int quotient(int n) const { return (int)((uint32_t)(((uint64_t)(2u * (uint32_t)n) * mul) >> 32) >> shift); }
 };
 inline FastDiv fast_div(long long divisor)
 {
@@ -215,7 +215,7 @@ __device__ __forceinline__ void store_empty_rows(const FwdArgs& a, int bh, int s
 // snake_end = min(work-groups, places), a multiple of 8) every second block of 256 therefore takes its items in reverse
 // CU order -- the CU with the heaviest item of one block gets the lightest of the next -- while i % 8, the XCD and with it
 // the L2 that a head slice's K and V sit in, stays as it is.
-__device__ __forceinline__ int work_position(int block, int snake_end)
+__host__ __device__ __forceinline__ int work_position(int block, int snake_end)
 {
     if (block < snake_end && (block & 256)) {
         const int base = block & ~255;
@@ -240,7 +240,7 @@ __device__ __forceinline__ int work_position(int block, int snake_end)
 // The launcher asks for it exactly where the plain order aliases: work-group x + 8 n of XCD x has split
 // (x / c + (8 / c) n) % S for c = 1, 2 or 4 slices per chunk, which reaches every split only if S is odd; other chunk
 // sizes mix by themselves, and rotating an order that already mixes measured 0 ... -14 %.
-__device__ __forceinline__ int split_of_rest(const FwdArgs& a, int rest, int* row_block_index)
+__host__ __device__ __forceinline__ int split_of_rest(const FwdArgs& a, int rest, int* row_block_index)
 {
     const int mi = a.by_splits.quotient(rest), s0 = rest - mi * a.num_splits;
     *row_block_index = mi;
@@ -253,7 +253,7 @@ inline int split_rotate_for(int num_splits, int slice_chunk)
     return num_splits > 1 && num_splits % 2 == 0 && (slice_chunk == 1 || slice_chunk == 2 || slice_chunk == 4) ? 1 : 0;
 }
 
-__device__ __forceinline__ int slice_of_position(const FwdArgs& a, int local)
+__host__ __device__ __forceinline__ int slice_of_position(const FwdArgs& a, int local)
 {
     if (a.group_xcd > 1) {
         const int x = local & 7, y = local >> 3, yg = a.by_xcd_group.quotient(y);
@@ -270,7 +270,7 @@ __device__ __forceinline__ int slice_of_position(const FwdArgs& a, int local)
 struct WorkItem {
     int bh, split, m_block;
 };
-__device__ __forceinline__ WorkItem work_item(const FwdArgs& a, int block)
+__host__ __device__ __forceinline__ WorkItem work_item(const FwdArgs& a, int block)
 {
     const int pos = work_position(block, a.snake_end);
     const int ch = a.by_chunk.quotient(pos), w = pos - ch * (a.slice_chunk * a.Tr * a.num_splits);

@@ -1234,6 +1234,23 @@ inline void set_slice_order(FwdArgs& b, int groups_per_slice, int resident)
     }
 }
 
+// order of the work-groups of launch_fwd_instance: slices, splits, places
+template <int D, int NB, int VAR>
+inline void set_work_order(FwdArgs& b)
+{
+    constexpr int kResident = ((VAR & kVarPair) != 0 ? 1 : NB == 1 ? fwd_groups_per_cu(D, NB, VAR) : 2) * kNumCus;
+    // (chunks as for three work-groups per CU at D = 64, where four measured +-1 % causal)
+    constexpr int kChunked = kResident < 3 * kNumCus ? kResident : 3 * kNumCus;
+    // (D = 96: chunks as for two work-groups per CU.  For three, causal B8 H32 N1000 d96 takes all its 256 slices as one chunk
+    // instead of 128 and finds fewer tiles in the caches: 74.9 -> 79.0 us, unmasked N = 1024 119.9 -> 133.7)
+    set_slice_order(b, b.Tr * b.num_splits, D == 96 ? 2 * kNumCus : kChunked);
+    b.split_rotate = split_rotate_for(b.num_splits, b.slice_chunk);
+    // (All places, the fourth at D = 64 too: with two row blocks per slice, whose second one is nearly empty, three of a CU's four
+    // work-groups were full ones on every other CU.  B32 H16 N130 d64 10.9 -> 9.9 us, B40 13.0 -> 12.3, B48 15.2 -> 14.8.)
+    b.snake_end = snake_end_for((long long)b.Tr * b.B * b.H * b.num_splits, kResident);
+    set_divisors(b, b.slice_chunk);
+}
+
 template <int D, int NB, int VAR>
 inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
 {
@@ -1245,17 +1262,7 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
     if (hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), smem, attr_done); e != hipSuccess) return e;
     const long long groups = (long long)a.Tr * a.B * a.H * a.num_splits;
     FwdArgs b = a;
-    constexpr int kResident = (kPair ? 1 : NB == 1 ? fwd_groups_per_cu(D, NB, VAR) : 2) * kNumCus;
-    // (chunks as for three work-groups per CU at D = 64, where four measured +-1 % causal)
-    constexpr int kChunked = kResident < 3 * kNumCus ? kResident : 3 * kNumCus;
-    // (D = 96: chunks as for two work-groups per CU.  For three, causal B8 H32 N1000 d96 takes all its 256 slices as one chunk
-    // instead of 128 and finds fewer tiles in the caches: 74.9 -> 79.0 us, unmasked N = 1024 119.9 -> 133.7)
-    set_slice_order(b, a.Tr * a.num_splits, D == 96 ? 2 * kNumCus : kChunked);
-    b.split_rotate = split_rotate_for(b.num_splits, b.slice_chunk);
-    // (All places, the fourth at D = 64 too: with two row blocks per slice, whose second one is nearly empty, three of a CU's four
-    // work-groups were full ones on every other CU.  B32 H16 N130 d64 10.9 -> 9.9 us, B40 13.0 -> 12.3, B48 15.2 -> 14.8.)
-    b.snake_end = snake_end_for(groups, kResident);
-    set_divisors(b, b.slice_chunk);
+    set_work_order<D, NB, VAR>(b);
     return launch_kernel(kern, dim3((unsigned)groups), dim3(kPair ? 512 : 256), smem, st, b);
 }
 
