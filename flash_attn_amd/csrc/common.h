@@ -75,7 +75,8 @@ struct FwdArgs {
     int alibi_left;      // ALiBi and no visible key lies right of its row (causal, or right window 0)
     int slice_chunk;     // head slices per chunk of the work-group order (set by the kernel's launcher)
     int snake_end;       // work-groups below this index sit on the GPU together; odd 256-blocks of them run reversed (launcher)
-    int group_xcd;       // > 1: query heads per K/V head, and the slice order keeps the heads of a K/V head on one XCD (launcher)
+    int group_xcd;       // query heads per K/V head where the slice order keeps the heads of a K/V head on one XCD (launcher):
+    int group_span;      // for the first so many slices of a chunk, 0: for none (slice_of_position)
     int split_rotate;    // 1: the split index of a work-group is rotated by its row block (launcher; split_of_rest)
     // divisions of the work-group index and of the head slice (launcher: set_divisors)
     FastDiv by_chunk, by_slices, by_splits, by_xcd_group, by_kv_group, by_heads;
@@ -230,8 +231,8 @@ __host__ __device__ __forceinline__ int work_position(int block, int snake_end)
 // the work-groups).  With grouped K/V heads the G = group_xcd query heads of a K/V head are G consecutive slices and would
 // land on G different XCDs, each pulling the same K and V into its own L2 (measured on B4 H32 H_kv4 N4096 d128 causal:
 // 3.7 times the K/V/Q bytes fetched).  Instead position (x, y) = (p % 8, p / 8) takes query head y % G of K/V slice
-// 8 (y / G) + x: the heads of a K/V head share an XCD and follow each other there.  A bijection on chunks whose size is
-// a multiple of 8 G (the launcher sets group_xcd only then).
+// 8 (y / G) + x: the heads of a K/V head share an XCD and follow each other there.  A bijection on the first multiple of 8 G
+// positions; what is left of a chunk that is no such multiple keeps the plain order.
 // Split index and row-block index of the position `rest` inside a slice (splits fastest).  Where the slices of a chunk
 // are not a multiple of 8, the XCD of a work-group depends on its split: with 4 slices and 2 splits, XCDs 0-3 get
 // every first split and XCDs 4-7 every second one, and under a causal mask, whose first splits are the long ones, half the
@@ -255,7 +256,7 @@ inline int split_rotate_for(int num_splits, int slice_chunk)
 
 __host__ __device__ __forceinline__ int slice_of_position(const FwdArgs& a, int local)
 {
-    if (a.group_xcd > 1) {
+    if (local < a.group_span) {
         const int x = local & 7, y = local >> 3, yg = a.by_xcd_group.quotient(y);
         return (yg * 8 + x) * a.group_xcd + y - yg * a.group_xcd;
     }

@@ -1219,19 +1219,20 @@ inline int slice_chunk_for(int slices, int groups_per_slice, int resident, bool 
     return slices;
 }
 
-// slice_chunk and group_xcd of a launch: with grouped K/V heads the chunks are multiples of 8 G slices where the slice
-// count allows, so that the heads of a K/V head can share an XCD (slice_of_position)
+// slice_chunk, group_xcd and group_span of a launch: with grouped K/V heads the chunks are multiples of 8 G slices where the
+// slice count allows, so that the heads of every K/V head share an XCD (slice_of_position); otherwise the heads of as many
+// K/V heads do as fill whole rounds of eight, and the chunks are the large ones, of which whole rounds are the most.
+// Ragged slice counts, plain order -> like this: with dropout (heads not folded) B1 H596 H_kv149 Nq20 Nk14594 d64 349 -> 255 us,
+// d128 893 -> 639, H600 H_kv150 in one chunk instead of 24 slices 323 -> 255; window of 500 B3 H56 H_kv7 N3000 d64 100 -> 92.5;
+// causal B5 H28 H_kv7 N2048 d128 (8-wave kernel) 180 -> 172, B3 H40 H_kv10 N1777 d64 63.3 -> 62.5; unmasked B7 H24 H_kv6 N1000 d80 78.8
+// -> 78.1, B17 H48 H_kv6 Nq100 Nk5000 d128 326 -> 295; 24 shapes, none slower.
 inline void set_slice_order(FwdArgs& b, int groups_per_slice, int resident)
 {
-    const int slices = b.B * b.H;
-    const bool alike = !b.causal && b.wl < 0 && b.wr < 0 && b.num_splits == 1;
-    b.group_xcd = 0;
-    if (b.kv_group > 1 && slices % (8 * b.kv_group) == 0) {
-        b.slice_chunk = slice_chunk_for(slices, groups_per_slice, resident, alike, 8 * b.kv_group);
-        if (b.slice_chunk % (8 * b.kv_group) == 0) b.group_xcd = b.kv_group;
-    } else {
-        b.slice_chunk = slice_chunk_for(slices, groups_per_slice, resident, alike);
-    }
+    const int slices = b.B * b.H, round = 8 * b.kv_group;
+    const bool alike = !b.causal && b.wl < 0 && b.wr < 0 && b.num_splits == 1 && (b.kv_group == 1 || slices % round == 0);
+    b.slice_chunk = slice_chunk_for(slices, groups_per_slice, resident, alike, slices % round == 0 ? round : 8);
+    b.group_xcd = b.kv_group;
+    b.group_span = b.kv_group > 1 && b.slice_chunk % b.kv_group == 0 ? b.slice_chunk / round * round : 0;
 }
 
 // order of the work-groups of launch_fwd_instance: slices, splits, places

@@ -16,7 +16,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["bijection", "places"])
+@pytest.mark.parametrize("check", ["bijection", "places", "shared_heads"])
 def test_work_order(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -63,10 +63,36 @@ static int places()
     return 0;
 }
 
+// The query heads of a K/V head on one XCD (work-group i runs on i % 8), except for those of the last, incomplete round of eight
+// K/V heads.
+static int shared_heads()
+{
+    for (int G : {2, 3, 4, 7, 8})
+        for (int Hk : {8, 11, 16, 75, 149})
+            for (int Tr : {1, 3})
+                for (int splits : {1, 3}) {
+                    fa::FwdArgs a = args(1, Hk * G, G, 128 * Tr, splits, splits == 3);
+                    fa::set_work_order<64, 1, kPlain>(a);
+                    if (a.slice_chunk != a.H) continue;  // (chunks that are no multiple of G cannot)
+                    std::vector<int> xcd(Hk * Tr * splits, -1), apart(Hk * Tr * splits);
+                    for (int i = 0; i < a.H * Tr * splits; ++i) {
+                        const fa::WorkItem it = fa::work_item(a, i);
+                        const int k = (it.bh / G * splits + it.split) * Tr + it.m_block;
+                        if (xcd[k] >= 0 && xcd[k] != i % 8) apart[k] = 1;
+                        xcd[k] = i % 8;
+                    }
+                    int heads = 0;
+                    for (int x : apart) heads += !x;
+                    CHECK(heads >= Hk / 8 * 8 * Tr * splits);
+                }
+    return 0;
+}
+
 int main(int, char** argv)
 {
     const char* what = argv[1];
     if (!std::strcmp(what, "bijection")) return bijection();
     if (!std::strcmp(what, "places")) return places();
+    if (!std::strcmp(what, "shared_heads")) return shared_heads();
     return 2;
 }
