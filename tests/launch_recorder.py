@@ -37,6 +37,23 @@ def record(calls):
     return json.loads(out.stdout)
 
 
+def form(launch):
+    """What a tiled launch's work-groups are: "narrow" (32 rows), "paired" (two halves of four waves), "tall" (256 rows, four waves),
+    "8-wave" (256 rows) or "plain" (128 rows)."""
+    if "fwd_pp_kernel" in launch["kernel"]:
+        return "8-wave"
+    if launch["variant"] & (NARROW | PAIR):
+        return "narrow" if launch["variant"] & NARROW else "paired"
+    return "tall" if launch["kernel"].split("ELi")[1] == "2" else "plain"
+
+
+def call(B, H, Hk, Nq, Nk, d, p=0.0, causal=False, window=(-1, -1), alibi=False, num_splits=1, kernel_hint=0):
+    """A call in the words of the GPU tests, for record()."""
+    c = dict(entry="splitkv" if num_splits != 1 else "forward", B=B, H=H, H_kv=Hk, Nq=Nq, Nk=Nk, d=d, is_causal=int(causal),
+             window_left=window[0], window_right=window[1], dropout_p=p, num_splits=num_splits, kernel_hint=kernel_hint)
+    return dict(c, alibi_slopes=0xA00000) if alibi else c
+
+
 def _child(so):
     sys.path.insert(0, ROOT)
     sys.modules["torch"] = None  # (the binding loads torch's HIP runtime first where there is one)

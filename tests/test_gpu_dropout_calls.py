@@ -10,18 +10,22 @@ from helpers import check_o_lse, oracle_forward_batched, randn_f16_gpu
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("B,H,Nq,Nk,d,kw", [
-    (1, 2, 130, 1090, 64, {}),                                      # narrow, two stages per wave
-    (1, 2, 700, 1090, 100, dict(causal=True)),                      # narrow, one stage per wave
-    (2, 4, 1090, 1090, 96, dict(causal=True)),                      # paired
-    (3, 30, 600, 600, 63, dict(causal=True)),                       # a work-group's tiles one after the other, odd rows
-    (3, 30, 520, 1030, 96, dict(window=(300, 0))),                  # starts inside a table
-    (3, 30, 600, 600, 64, dict(causal=True, alibi=True)),           # from the last tile to the first
-    (1, 3, 1100, 1100, 128, dict(causal=True, kernel_hint=2)),      # 8-wave kernel
-    (1, 3, 300, 1100, 128, dict(window=(700, 0), kernel_hint=2)),   # 8-wave kernel, waves that start later than others
-    (1, 2, 40, 1600, 72, dict(num_splits=3)),                       # splits that begin and end inside a table
-])
-def test_keep_decisions_across_call_tables(fa, oracle, B, H, Nq, Nk, d, kw):
+WALKS = [  # (the last field: what the launch is, which tests/test_launch_geometry.py holds the rules to)
+    (1, 2, 130, 1090, 64, {}, "narrow"),                                    # two stages per wave
+    (1, 2, 700, 1090, 100, dict(causal=True), "narrow"),                    # one stage per wave
+    (2, 4, 1090, 1090, 96, dict(causal=True), "narrow"),                    # two rounds of work-groups
+    (1, 11, 1090, 1090, 64, dict(causal=True), "paired"), (1, 20, 800, 800, 100, dict(causal=True), "paired"),
+    (3, 30, 600, 600, 63, dict(causal=True), "plain"),                      # a work-group's tiles one after the other, odd rows
+    (3, 30, 520, 1030, 96, dict(window=(300, 0)), "plain"),                 # starts inside a table
+    (3, 30, 600, 600, 64, dict(causal=True, alibi=True), "plain"),          # from the last tile to the first
+    (1, 3, 1100, 1100, 128, dict(causal=True, kernel_hint=2), "8-wave"),
+    (1, 3, 300, 1100, 128, dict(window=(700, 0), kernel_hint=2), "8-wave"), # waves that start later than others
+    (1, 2, 40, 1600, 72, dict(num_splits=3), "paired"),                     # splits that begin and end inside a table
+]
+
+
+@pytest.mark.parametrize("B,H,Nq,Nk,d,kw,form", WALKS)
+def test_keep_decisions_across_call_tables(fa, oracle, B, H, Nq, Nk, d, kw, form):
     import torch
     kw = dict(kw)
     okw = {k: v for k, v in kw.items() if k in ("causal", "window")}

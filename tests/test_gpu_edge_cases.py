@@ -106,7 +106,7 @@ def test_8wave_kernel_on_shorter_rows(fa, oracle, d):
 # multiple of 32, a last tile of one key), causal rows whose upper waves get no tile at all, Nq != Nk in both directions
 # (leading row blocks without a visible key), wide windows, grouped K/V heads, head dims in both buckets: whole chunks,
 # the bucket width, every alignment.  kernel_hint = KERNEL_4WAVE runs the 128-row instances on the same request.
-@pytest.mark.parametrize("B,H,Hk,Nq,Nk,d,kw", [
+NARROW_SHAPES = [
     (1, 8, 8, 1021, 1021, 31, dict()),                      # the reference's checked-in run (src/main.cu:39-49)
     (1, 8, 8, 1021, 1021, 31, dict(causal=True)),
     (1, 4, 4, 1000, 1025, 64, dict(causal=True)),
@@ -117,8 +117,7 @@ def test_8wave_kernel_on_shorter_rows(fa, oracle, d):
     (2, 2, 2, 515, 515, 56, dict(causal=True, window=(600, -1))),
     (1, 5, 5, 640, 640, 32, dict(window=(-1, 64))),
     (1, 4, 4, 1, 3000, 20, dict(dropout_p=0.0)),            # one row: the decode kernel, not these instances
-    # above d = 64 a wave has one LDS stage and requests K and V of its next tile separately (rows of the bucket's
-    # width only: the shorter rows in this list run the 128-row instances)
+    # above d = 64 a wave has one LDS stage and requests K and V of its next tile separately
     (1, 8, 8, 1024, 1024, 128, dict(causal=True)),
     (1, 4, 2, 777, 1100, 96, dict(window=(1000, 20))),
     (1, 2, 2, 600, 700, 128, dict(causal=True, dropout_p=0.3, seed=9, offset=2)),
@@ -132,7 +131,10 @@ def test_8wave_kernel_on_shorter_rows(fa, oracle, d):
     (1, 3, 3, 500, 1100, 31, dict(alibi=True)),
     (1, 2, 2, 600, 600, 48, dict(causal=True, dropout_p=0.2, seed=5, offset=77)),
     (2, 2, 1, 333, 900, 27, dict(window=(800, 30), alibi=True, dropout_p=0.5, seed=2 ** 35, offset=1)),
-])
+]
+
+
+@pytest.mark.parametrize("B,H,Hk,Nq,Nk,d,kw", NARROW_SHAPES)
 def test_narrow_instances(fa, oracle, B, H, Hk, Nq, Nk, d, kw):
     import torch
     q = randn_f16_gpu((B, H, Nq, d), 41)
@@ -682,20 +684,25 @@ def test_stage_stamps(fa, oracle, hint, N, d, kw):
     assert (np.diff(st2.cpu().numpy()[:, :7], axis=1) >= 0).all()
 
 
-@pytest.mark.parametrize("B,H,Hk,Nq,Nk,d,S,kw", [
-    (1, 3, 3, 700, 700, 64, 1, dict(causal=True)),      # 32-row work-groups, two stages per wave
-    (1, 3, 3, 700, 700, 128, 1, dict()),                # 32-row work-groups, one stage
-    (2, 2, 2, 200, 1740, 31, 3, dict(causal=True)),     # eight waves in two halves
-    (1, 8, 8, 1664, 1664, 100, 1, dict(causal=True)),
-    (2, 16, 4, 20, 700, 128, 3, dict(causal=True)),     # folded heads
-    (1, 8, 2, 30, 1740, 72, 2, dict()),                 # folded heads in two halves
-    (2, 32, 4, 64, 64, 96, 1, dict(window=(20, 5))),    # folded heads, several row blocks
-    (4, 16, 16, 1, 700, 128, 2, dict(dropout_p=0.1)),
-    (1, 8, 8, 100, 2000, 64, 12, dict(causal=True, window=(60, -1))),  # splits without a key
-    (1, 2, 2, 300, 40, 64, 1, dict(causal=True)),       # row blocks without a key
-    (32, 32, 32, 256, 70, 64, 1, dict()),               # 256-row work-groups
-])
-def test_stage_stamps_of_every_launch_form(fa, B, H, Hk, Nq, Nk, d, S, kw):
+STAMPED_FORMS = [  # (the last field: what the launch is, which tests/test_launch_geometry.py holds the rules to)
+    (1, 3, 3, 700, 700, 64, 1, dict(causal=True), "narrow"),        # two stages per wave
+    (1, 3, 3, 700, 700, 128, 1, dict(), "narrow"),                  # one stage
+    (1, 8, 8, 1664, 1664, 100, 1, dict(causal=True), "narrow"),     # two rounds of work-groups
+    (2, 2, 2, 200, 1740, 31, 3, dict(causal=True), "paired"),       # eight waves in two halves
+    (1, 28, 28, 1283, 1283, 100, 1, dict(causal=True), "paired"),   # two of them one after the other
+    (2, 16, 4, 20, 700, 128, 3, dict(causal=True), "plain"),        # folded heads
+    (1, 8, 2, 30, 1740, 72, 2, dict(), "paired"),                   # folded heads in two halves
+    (2, 32, 4, 64, 64, 96, 1, dict(window=(20, 5)), "plain"),       # folded heads, several row blocks
+    (4, 16, 16, 1, 700, 128, 2, dict(dropout_p=0.1), "plain"),
+    (1, 8, 8, 100, 2000, 64, 12, dict(causal=True, window=(60, -1)), "plain"),  # splits without a key
+    (1, 2, 2, 300, 40, 64, 1, dict(causal=True), "plain"),          # row blocks without a key
+    (32, 32, 32, 256, 70, 64, 1, dict(), "plain"),                  # two tiles, four work-groups per CU
+    (32, 32, 32, 256, 1030, 64, 1, dict(), "tall"),
+]
+
+
+@pytest.mark.parametrize("B,H,Hk,Nq,Nk,d,S,kw,form", STAMPED_FORMS)
+def test_stage_stamps_of_every_launch_form(fa, B, H, Hk, Nq, Nk, d, S, kw, form):
     """The instrumented twin of whatever instance serves the call: the same results bit by bit, and a row of ordered
     stamps from each work-group."""
     import torch

@@ -20,7 +20,11 @@ def test_paired_halves(fa, oracle, Nq, G, d, kw):
         check_o_lse(*fa.flash_forward_splitkv(q, k, v, num_splits=S, **kw), O, L, f"split {S}")
 
 
-@pytest.mark.parametrize("B,H,N,d", [(1, 8, 1664, 100), (2, 4, 1311, 112), (1, 16, 1244, 31), (1, 11, 1090, 64)])
+# (tests/test_launch_geometry.py holds these three lists against the rule)
+UNSPLIT = [(1, 17, 1290, 100), (1, 20, 900, 112), (1, 20, 1100, 31), (1, 11, 1090, 64)]
+
+
+@pytest.mark.parametrize("B,H,N,d", UNSPLIT)
 def test_paired_halves_unsplit(fa, oracle, B, H, N, d):
     """Unsplit causal launches of 64 to 256 work-groups, too many rows for the narrow instances."""
     q, k, v = (randn_f16_gpu((B, H, N, d), s) for s in (4, 5, 6))
@@ -39,9 +43,12 @@ def test_paired_halves_dropout(fa, oracle, Nq, d):
     check_o_lse(*fa.flash_forward_splitkv(q, k, v, num_splits=3, causal=True, dropout_p=p, seed=9), O, L, "dropout")
 
 
-@pytest.mark.parametrize("B,H,N,d,kw", [(1, 20, 700, 128, dict(causal=True)), (1, 11, 1090, 64, dict(causal=True)),
-                                        (1, 20, 900, 100, dict(causal=True, window=(390, -1))), (1, 16, 1100, 96, dict(window=(600, 0))),
-                                        (1, 34, 800, 31, dict(causal=True))])
+UNSPLIT_DROPOUT = [(1, 20, 700, 128, dict(causal=True)), (1, 11, 1090, 64, dict(causal=True)),
+                   (1, 20, 900, 100, dict(causal=True, window=(390, -1))), (1, 16, 1100, 96, dict(window=(600, 0))),
+                   (1, 34, 800, 31, dict(causal=True))]
+
+
+@pytest.mark.parametrize("B,H,N,d,kw", UNSPLIT_DROPOUT)
 def test_paired_halves_unsplit_dropout(fa, oracle, B, H, N, d, kw):
     """Whole launches with dropout, under a mask and under a window, and the decisions that the two halves store."""
     import torch
@@ -70,8 +77,10 @@ def test_paired_halves_windowed_dropout(fa, oracle, Nq, d):
     check_o_lse(*fa.flash_forward_splitkv(q, k, v, num_splits=3, dropout_p=p, seed=9, **kw), O, L, "windowed dropout")
 
 
-@pytest.mark.parametrize("B,H,Hk,Nq,Nk,d,p", [(1, 28, 28, 1283, 1283, 100, 0.0), (2, 12, 4, 1700, 1921, 40, 0.0), (1, 26, 26, 1281, 1300, 64, 0.2),
-                                              (1, 24, 24, 1925, 1870, 72, 0.0)])
+FOLLOWING = [(1, 28, 28, 1283, 1283, 100, 0.0), (2, 12, 4, 1700, 1921, 40, 0.0), (1, 26, 26, 1281, 1300, 64, 0.2), (1, 24, 24, 1925, 1870, 72, 0.0)]
+
+
+@pytest.mark.parametrize("B,H,Hk,Nq,Nk,d,p", FOLLOWING)
 def test_paired_halves_one_after_the_other(fa, oracle, B, H, Hk, Nq, Nk, d, p):
     """Causal launches of 257 to 512 work-groups, two of them one after the other on a CU; rows that see no key among them."""
     import torch

@@ -7,8 +7,12 @@ from helpers import check_o_lse, randn_f16_gpu, to_f32_np
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("B,H,Hk,Nq,Nk", [(32, 32, 32, 256, 256), (32, 32, 8, 225, 225), (16, 32, 32, 512, 64),
-                                          (16, 32, 32, 385, 130), (3, 28, 28, 3329, 65)])
+# (the rule takes them from 1024 keys on; tests/test_launch_geometry.py holds these shapes against it)
+SHAPES = [(32, 32, 32, 256, 1024), (32, 32, 8, 225, 1055), (16, 32, 32, 512, 1088), (16, 32, 32, 449, 1030), (3, 28, 28, 3329, 2049)]
+CHUNKS = [(16, 32, 32, 512, 1024), (16, 32, 8, 481, 1090), (3, 28, 28, 3329, 1025), (13, 40, 40, 512, 1087)]
+
+
+@pytest.mark.parametrize("B,H,Hk,Nq,Nk", SHAPES)
 def test_tall_blocks(fa, oracle, B, H, Hk, Nq, Nk):
     import torch
 
@@ -20,7 +24,7 @@ def test_tall_blocks(fa, oracle, B, H, Hk, Nq, Nk):
     check_o_lse(o[-1:, -1:], lse[-1:, -1:], O, L, "last head")
 
 
-@pytest.mark.parametrize("B,H,Hk,Nq,Nk", [(16, 32, 32, 512, 1024), (16, 32, 8, 481, 1090), (3, 28, 28, 3329, 1025), (13, 40, 40, 512, 1087)])
+@pytest.mark.parametrize("B,H,Hk,Nq,Nk", CHUNKS)
 def test_tall_blocks_and_slice_chunks_of_long_key_ranges(fa, oracle, B, H, Hk, Nq, Nk):
-    """The rule takes them from 1024 keys on; slice counts that do and do not divide into chunks of sixteen."""
+    """Slice counts that do and do not divide into chunks of sixteen."""
     test_tall_blocks(fa, oracle, B, H, Hk, Nq, Nk)

@@ -1,7 +1,7 @@
 """What the library launches against the buffers it told the caller to bring, without a GPU (tests/launch_recorder.py)."""
 import numpy as np
 
-from launch_recorder import ALIBI, DROPOUT, EVERY, FOLD, FULL_D, KV_ONCE, NARROW, PAIR, STAMP, record
+from launch_recorder import ALIBI, DROPOUT, EVERY, FOLD, FULL_D, KV_ONCE, NARROW, PAIR, STAMP, call, form, record
 
 STAMPS = 0x900000  # a stage-stamp buffer
 
@@ -132,15 +132,33 @@ def test_non_temporal_requests_only_where_no_other_work_group_asks_for_the_tiles
     assert {(True, True, False, True), (True, False, False, True), (True, False, True, True), (True, True, True, True)} <= seen
 
 
-def test_paired_launches_of_the_dropout_tests():
-    """The shapes of tests/test_gpu_paired_halves.py that are about paired launches with dropout are such launches."""
-    calls = [dict(entry="forward", B=1, H=H, Nq=N, Nk=N, d=d, is_causal=c, window_left=left, window_right=right, dropout_p=0.2)
-             for H, N, d, c, left, right in ((20, 700, 128, 1, -1, -1), (11, 1090, 64, 1, -1, -1), (20, 900, 100, 1, 390, -1),
-                                             (16, 1100, 96, 0, 600, 0), (34, 800, 31, 1, -1, -1))]
-    calls += [dict(entry="splitkv", B=1, H=2, Nq=Nq, Nk=1740, d=d, num_splits=3, is_causal=1, window_left=390, dropout_p=0.2)
-              for Nq, d in ((33, 128), (140, 100), (128, 64))]
-    for c, r in zip(calls, record(calls)):
-        assert r["launches"][0]["variant"] & (PAIR | NARROW | DROPOUT) == PAIR | DROPOUT, c
+def test_launch_forms_of_the_gpu_tests():
+    """The shapes of the GPU tests that are about a launch form are launched in that form."""
+    import test_gpu_dropout_calls as calls_
+    import test_gpu_edge_cases as edge
+    import test_gpu_narrow_rule as narrow
+    import test_gpu_paired_halves as paired
+    import test_gpu_tall_blocks as tall
+
+    rows = [("tall", call(*s, 64)) for s in tall.SHAPES + tall.CHUNKS]
+    rows += [(f, call(B, H, H, N, N, d, **kw)) for B, H, N, d, kw, f in narrow.LINES]
+    rows += [("narrow", call(*shape, p, **kw)) for *shape, p, kw in narrow.ROUNDS]
+    rows += [(f, call(B, H, H, Nq, Nk, d, 0.3, **kw)) for B, H, Nq, Nk, d, kw, f in calls_.WALKS]
+    rows += [("paired", call(B, H, H, N, N, d, causal=True)) for B, H, N, d in paired.UNSPLIT]
+    rows += [("paired", call(B, H, H, N, N, d, 0.2, **kw)) for B, H, N, d, kw in paired.UNSPLIT_DROPOUT]
+    rows += [("paired", call(1, 2, 2, Nq, 1740, d, 0.2, num_splits=3, causal=True, window=(390, -1))) for Nq, d in ((33, 128), (140, 100), (128, 64))]
+    rows += [("paired", call(*s, causal=True)) for s in paired.FOLLOWING]
+    for *shape, S, kw, f in edge.STAMPED_FORMS:
+        kw = dict(kw)
+        rows.append((f, call(*shape, kw.pop("dropout_p", 0.0), num_splits=S, **kw)))
+    for *shape, kw in edge.NARROW_SHAPES:
+        if shape[3] > 1:  # (one row: the decode kernel)
+            kw = {k: v for k, v in kw.items() if k not in ("seed", "offset")}
+            rows.append(("narrow", call(*shape, kw.pop("dropout_p", 0.0), **kw)))
+    for (f, c), r in zip(rows, record([c for _, c in rows])):
+        launch = r["launches"][0]
+        assert form(launch) == f, (f, c, launch)
+        assert bool(launch["variant"] & DROPOUT) == (c["dropout_p"] > 0.0), (c, launch)
 
 
 def test_launches_that_are_whole_without_their_paired_form_need_no_workspace():
