@@ -1,6 +1,7 @@
 """The native front end of the binding (csrc/py_binding.cpp) against binding.py's own path, which the debug outputs take:
 same kernels, so bit-identical results whatever way the arguments come."""
 import os
+import shutil
 import subprocess
 import sys
 import types
@@ -86,6 +87,7 @@ def test_leaves_what_it_cannot_serve_to_the_binding(fa):
 
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "flash_attn_amd", "csrc")
+DRIVER = os.path.join(os.path.dirname(os.path.abspath(__file__)), "driver")
 
 
 def _dry_run(*args):
@@ -96,6 +98,20 @@ def _dry_run(*args):
 
 def test_the_library_builds_without_python():
     assert "flash_api.hip" in (out := _dry_run("-B", "PYTHON=false")) and "py_binding.cpp" not in out
+
+
+@pytest.mark.parametrize("folder,target", [(CSRC, "build/fwd_d64.o"), (DRIVER, "mfma_rate")])
+def test_a_failed_compilation_fails_the_build(tmp_path, folder, target):
+    """Also where the result of an earlier build is there: it does not stand in for the one that was not made."""
+    tree = tmp_path / "flash_attn_amd" / "csrc"
+    shutil.copytree(folder, tree, ignore=shutil.ignore_patterns("*.o"))
+    (tmp_path / "include").mkdir()
+    (tmp_path / "include" / "flash_attn_mi355.h").touch()
+    (tree / "build").mkdir(exist_ok=True)
+    (tree / target).touch(0o777)
+    os.utime(tree / target, (1, 1))
+    r = subprocess.run(["make", "-C", str(tree), target, "HIPCC=false"], capture_output=True, text=True, timeout=120)
+    assert r.returncode != 0, r.stdout
 
 
 def test_the_front_end_is_rebuilt_for_another_torch():
