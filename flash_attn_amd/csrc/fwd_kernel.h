@@ -142,7 +142,8 @@ constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarSt
 // work-groups per CU (narrow: one or two by their LDS; held to 256 VGPRs all the same, without which the compiler keeps more
 // than there are and moves them to and from accumulation registers): three up to D = 96 (168 VGPRs), except for the instance that
 // serves every request, which stages its tiles through registers, and at D = 96 those with sixteen registers of bias constants
-// and dropout, which would spill.  Four at D = 64 without either (128 VGPRs: B32 H32 N512 d64 in 128-row blocks 100.3 -> 91.1 us
+// and dropout, which would spill (bias and dropout without those constants, two per CU -> three: B8 H32 N1000 d96 168 -> 158 us, B16 H16
+// N512 d80 47.8 -> 46.8, but B4 H12 N777 d88 32.4 -> 33.5).  Four at D = 64 without either (128 VGPRs: B32 H32 N512 d64 in 128-row blocks 100.3 -> 91.1 us
 // together with the shorter chunks below); with the bias constants four spill in the loop (window of 256 keys with ALiBi B2
 // H16 N4096 d64 22.9 -> 24.4).
 constexpr int fwd_groups_per_cu(int D, int NB, int VAR)
@@ -289,6 +290,9 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
             }
         }
         diagonals = diagonal_sides(straight, lo_min, lo_max, hi_min, hi_max);
+        // (At D = 96 with bias and dropout this one register of the vector unit was one too many and lived in scratch memory.  On the scalar
+        // unit everywhere: B2 H8 N2000 causal with bias d31 28.1 -> 29.0 us, d31 with dropout as well 41.9 -> 40.7.)
+        if constexpr (D == 96 && kAlibi && kDropout) diagonals = wave_uniform(diagonals);
         // (a wave whose rows all lie past Nq sees nothing: it only helps to stage the tiles)
         live0 = (lo_min >> 6) - tile_begin;
         nlive = q0 + wave_row0 < Nq ? max(0, (hi_max >> 6) - tile_begin - live0 + 1) : 0;

@@ -1,7 +1,9 @@
 """The distances between instructions that the hardware of gfx950 asks of the program, in the code as it was built.  The compiler
 keeps them for what it writes itself, and cannot for what stands inside an inline-assembly statement.  No GPU needed."""
 import os
+import re
 
+import launch_recorder as lr
 import machine_code as mc
 
 LIBRARY = os.path.join(mc.ROOT, "flash_attn_amd", "lib", "libflash_attn_mi355.so")
@@ -71,3 +73,12 @@ def test_wait_states():
         seen += 1
         found += [(name, i, what, body[max(0, i - 3):i + 1]) for what, i in too_close(body)]
     assert seen > 300 and not found, (len(found), found[:3])
+
+
+def test_registers_suffice():
+    """No kernel moves registers to and from scratch memory, other than the instance that serves every request and the
+    instrumented twins."""
+    kernels = mc.metadata(LIBRARY)
+    spills = [name for name, m in kernels.items() if m["private_segment_fixed_size"] or m["vgpr_spill_count"]]
+    variant = {name: int(re.match(r".*fwd_(?:pp_)?kernelILi\d+E(?:Li\d+E)?Li(\d+)EEE", name)[1]) for name in spills}
+    assert len(kernels) > 300 and not [name for name in spills if not variant[name] & (lr.EVERY | lr.STAMP)], spills
