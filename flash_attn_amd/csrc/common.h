@@ -387,7 +387,9 @@ __device__ __forceinline__ void mul_wide_u32(uint32_t m, uint32_t x, uint32_t& h
     lo = (uint32_t)r;
 }
 
-// both products of a Philox round (one statement: between two of the above the compiler puts a wait state that nothing needs)
+// Both products of a Philox round in one statement: between two of the above the compiler puts a wait state, in case the first ends with
+// an instruction that writes part of a register, whose result the next instruction must not read.  v_mad_u64_u32 writes whole
+// registers, and neither of the two reads what the other writes (vcc is carry out alone).
 __device__ __forceinline__ void mul_wide_pair(uint32_t m0, uint32_t x0, uint32_t m1, uint32_t x1, uint32_t& hi0, uint32_t& lo0,
                                               uint32_t& hi1, uint32_t& lo1)
 {

@@ -191,8 +191,9 @@ long long tiled_groups(const flash_params* p, const fa::FwdArgs& a)
 // side by side costing the sum of its tiles over the gain of n, b = microseconds per 64-key tile of a work-group alone
 // on its CU.  Over 21 swept shapes the count it picks is within 5 % of the best measured one on 19 (the others: 6 % and
 // 9 %); the reference's rule with 256 CUs: 9 of 21, the worst 3.1 times slower than the best count.  It knows
-// which launches will be narrow or paired.  Its constants and the lines
-// of fwd_uses_narrow are fits to the kernels as they are; a change of either wants both measured again.
+// of narrow launches, and of paired ones with one work-group per CU; paired launches of 257 to 512 work-groups have the price of
+// unpaired ones, and the fourth work-group per CU at d = 64 and the third at d = 96 that of rounds of three and two.  Its constants
+// and the lines of fwd_uses_narrow are fits to the kernels as they are; a change of either wants both measured again.
 int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode);
 bool folds_heads(const flash_params* p);
 void fold_heads(fa::FwdArgs* a);
@@ -225,9 +226,11 @@ int auto_splits_tiled(const flash_params* p, int n_blocks, bool decode = false)
     return splits;
 }
 
-// Unsplit launches of several rounds of 32-row work-groups at the edge of what the narrow instances take: the 128-row instances
-// are as fast there or a little faster, but the estimate, which prices those too high when K and V stay in L2, would split them.
-// They stay whole: a call of such a shape needs no workspace, and none that exceeds the built-in scratch.
+// Unsplit launches of several rounds of 32-row work-groups at the edge of what the narrow instances take.  They run 128-row
+// work-groups, as fast there or a little faster, and have the price of narrow ones, since the price of 128 rows is too high for most of
+// them: the estimate would split launches that are faster whole.  The lines are those up to which launches were narrow when the
+// prices were fitted, and the price is no promise to stay whole: where it is higher than that of a split (few rows over many
+// keys: B9 H10 H_kv5 Nq90 Nk10270 d40 in 8) the launch is split.
 bool near_narrow(const fa::FwdArgs& a, bool every)
 {
     const long long groups = (long long)a.B * a.H * ((a.Nq + 31) / 32);

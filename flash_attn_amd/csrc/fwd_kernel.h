@@ -461,12 +461,8 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         else issue(std::true_type{});
     };
     auto dma_tile = [&](int tile, int stage) { dma_tile_parts(tile, stage, std::true_type{}, std::true_type{}); };
-    // wait until at most the requests of one tile (the youngest) are still in flight / until none is
-    auto dma_wait = [&](bool one_tile_in_flight) {
-        if (!one_tile_in_flight) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        else if (k_extra) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NKX + NVX) : "memory");
-        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NKX + NVX - 1) : "memory");
-    };
+    // wait until every request has landed
+    auto dma_wait = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
 
     // ---- accumulators
     v16f oacc[MB][NB];
@@ -938,7 +934,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         set_bounds();
         read_slope();
         stamps.take(1);
-        dma_wait(false);
+        dma_wait();
         pin_q();
         stamps.take(2);
         second_tile(late);
@@ -948,7 +944,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         for (int t = 0; t < rounds; ++t) {
             if (!kPair || nth(t) < ntiles) tile_math(nth(t), buf);
             if (kStamp && t == 0) stamps.take(4);
-            dma_wait(false);
+            dma_wait();
             __syncthreads();
             // (the request stands at the end so that the first tile, whose successor is on its way already, is no case of its own:
             // a copy of the tile's code costs a launch of few tiles its way through a cold instruction cache)
@@ -1282,8 +1278,10 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
 //  * One round -- no more 32-row work-groups than places for them, one per CU by their LDS, two at D = 32 (from 4 tiles on): from 2
 //    tiles on, 3 at 96 < d < 128 (N150, 3 tiles, d31 / 64 / 128 / 100 6.2 / 6.2 / 7.8 / 8.3 -> 5.1 / 5.2 / 6.6 / 7.6 us; N120, 2 tiles,
 //    5.9 / 5.7 / 6.8 / 7.2 -> 5.2 / 5.2 / 6.3 / 7.4; window of 100 keys N600, 4 tiles, 8.0 / 8.1 / 10.1 / 10.3 -> 5.3 / 5.3 / 6.7 / 7.8).
-//    Launches of up to 64 of them, which would gain as much, stay where they were below 4 tiles, 5 under a window: the tests
-//    of the 128-row instances' stage stamps ask for them there.
+//    Launches of up to 64 of them keep the 128-row form below 4 tiles, 5 under a window, at a cost (128 rows / narrow, d32 / 64 / 96 / 128: H8
+//    N128 3.7 / 4.5 / 5.0 / 5.9 against 3.3 / 4.0 / 4.3 / 5.3 us, N190 4.6 / 5.6 / 6.3 / 7.4 against 3.6 / 4.4 / 4.7 / 5.8, H4 N300 under a window of
+//    100 keys 6.1 / 7.3 / 8.1 / 9.4 against 3.7 / 4.5 / 4.8 / 5.9; back to back the first are at the host's rate of 4.9 us per call either way): a
+//    stamped call runs as the call without, and readers of the stamps count on a row per 128 query rows there (test_stage_stamps).
 //  * More rounds where the later work-groups are the light ones of a causal mask over about as many keys as rows, the more tiles the more
 //    of them that see a key: D >= 96 from (groups - 256) / 16 tiles on, up to 640, 720 from 60 tiles, 800 from 100 on (narrow / 128 rows: B1
 //    H5 N4105 d96, 645 of them, 36.7 / 44.7 us; H14 N1001 d96, 448, 13.0 / 15.6; H16 Nq586 d128, 304, 10.9 / 13.4; but H10 N2833 d80, 890, 37.2 / 33.7);
