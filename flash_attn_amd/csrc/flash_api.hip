@@ -227,10 +227,10 @@ int auto_splits_tiled(const flash_params* p, int n_blocks, bool decode = false)
 }
 
 // Unsplit launches of several rounds of 32-row work-groups at the edge of what the narrow instances take.  They run 128-row
-// work-groups, as fast there or a little faster, and have the price of narrow ones, since the price of 128 rows is too high for most of
-// them: the estimate would split launches that are faster whole.  The lines are those up to which launches were narrow when the
-// prices were fitted, and the price is no promise to stay whole: where it is higher than that of a split (few rows over many
-// keys: B9 H10 H_kv5 Nq90 Nk10270 d40 in 8) the launch is split.
+// work-groups, as fast there or a little faster, at the price of narrow ones: the estimate's price of 128 rows splits more of them than
+// gain by it (24 random shapes whose count this decides: whole faster on 15, split / whole 1.02 in the mean, 0.78 ... 1.21, and a
+// whole launch needs no workspace).  The lines are those up to which launches were narrow when the prices were fitted; it is no promise to
+// stay whole (B9 H10 H_kv5 Nq90 Nk10270 d40: 8 splits).
 bool near_narrow(const fa::FwdArgs& a, bool every)
 {
     const long long groups = (long long)a.B * a.H * ((a.Nq + 31) / 32);
