@@ -3,8 +3,6 @@
 #pragma once
 #include "common.h"
 
-#define FLASH_MAX_SPLITS_K 128  // must equal FLASH_MAX_SPLITS of the public header
-
 namespace fa {
 
 template <int CTRL>

@@ -7,6 +7,8 @@
 
 #include <atomic>
 
+#define FLASH_MAX_SPLITS_K 128  // must equal FLASH_MAX_SPLITS of the public header
+
 namespace fa {
 
 typedef _Float16 half_t;
@@ -46,6 +48,8 @@ inline FastDiv fast_div(long long divisor)
     while ((1ull << l) < d) ++l;
     return {(uint32_t)(((1ull << (31 + l)) + d - 1) / d), l};
 }
+
+__host__ __device__ __forceinline__ constexpr FastDiv fast_div_by_one() { return {0x80000000u, 0u}; }
 
 // Arguments of the tiled forward kernel and of the decode/combine kernels, filled by the host from flash_params
 // (which is itself the superset of the reference's mykernelParamType, include/utils.h:21-44).
@@ -92,11 +96,6 @@ struct FwdArgs {
     __device__ __forceinline__ int head(int bh) const { return bh - by_heads.quotient(bh) * H; }
 };
 
-// What every work-group needs of the order lies in sixteen words that one scalar load fetches.  With by_heads half outside, a second
-// load stood behind the first tile's requests: B2 H8 N2000 causal with bias d31 28.2 -> 27.6 us, d100 44.4 -> 43.6, with dropout
-// as well d31 42.0 -> 40.5; B9 H2 N3456 d31 52.9 -> 51.8.
-static_assert(offsetof(FwdArgs, by_heads) + sizeof(FastDiv) - offsetof(FwdArgs, snake_end) <= 64, "one load");
-
 // Divisors of a launch, once its slice order is set (the decode kernel, whose order has no chunks, deals out
 // `slices` groups of query heads per split)
 inline void set_divisors(FwdArgs& b, long long slices)
@@ -108,6 +107,96 @@ inline void set_divisors(FwdArgs& b, long long slices)
     b.by_kv_group = fast_div(b.kv_group);
     b.by_heads = fast_div(b.H);
     b.by_fold = fast_div(b.fold_rows);
+}
+
+// ---- FwdArgs as the tiled kernels get it.  A launch takes the longer the more its arguments are: what an otherwise host-bound
+// stream of launches needs per launch is 2.62 ... 2.72 us with 32 ... 112 bytes, 3.24 with 128, 3.35 with the 272 bytes of FwdArgs (an empty
+// kernel, sizes in random order).  FwdArgs -> packed, B5 H4 Nq1 Nk256 d128 6.01 -> 5.68 us, B8 H8 H_kv1 Nq1 Nk812 d96 (two launches)
+// 9.25 -> 8.65, B1 H2 N128 d64 4.94 -> 4.79; long launches +-0.  So the kernels get 108 bytes, narrow fields packed, and unpack them at their start; what only
+// ALiBi, dropout and debug outputs need follows in PackedMore.  Split launches find their partial results where the others have O and LSE.
+// (The words that tell a work-group its place in the order come first: one scalar load.)
+struct Packed {
+    int snake_end, slice_chunk, Tr;
+    uint32_t shifts;  // of by_chunk, by_slices, by_splits, by_xcd_group, by_kv_group (folded: by_fold): five bits each; bit 25: split_rotate, bit 26: causal
+    uint32_t sizes;   // d, num_splits: eight bits each; group_xcd: sixteen
+    uint32_t mul_chunk, mul_slices, mul_splits;
+    int group_span_or_fold_rows;      // folded launches have one query head per K/V head
+    uint32_t mul_xcd_or_fold_group;
+    uint32_t mul_kv_or_fold;
+    int Nq, Nk, wl, wr, keys_per_split;
+    const half_t *Q, *K, *V;
+    void *O, *LSE;
+    float scale_log2;
+};
+struct PackedMore : Packed {
+    int H;
+    FastDiv by_heads;
+    uint32_t drop_thr, drop_sub2;
+    float drop_rscale;
+    uint32_t seed_lo, seed_hi, off_lo;
+    const float* alibi;
+    uint8_t* keep_out;
+    float* scores_out;
+    uint64_t* stamps;
+};
+constexpr size_t kCheapArgs = 112;  // bytes up to which a launch costs its least
+static_assert(offsetof(Packed, scale_log2) + sizeof(float) <= kCheapArgs && sizeof(Packed) <= kCheapArgs, "cheap launches");
+static_assert(FLASH_MAX_SPLITS_K < 256, "eight bits");
+
+inline PackedMore packed(const FwdArgs& a)
+{
+    PackedMore p{};
+    const bool fold = a.fold_rows > 0, xcd = a.group_xcd < 65536;  // (more heads per K/V head than that keep the plain order)
+    p.snake_end = a.snake_end, p.slice_chunk = a.slice_chunk, p.Tr = a.Tr;
+    p.shifts = a.by_chunk.shift | a.by_slices.shift << 5 | a.by_splits.shift << 10 | (fold || !xcd ? 0u : a.by_xcd_group.shift) << 15 |
+               (fold ? a.by_fold : a.by_kv_group).shift << 20 | (a.split_rotate ? 1u << 25 : 0u) | (a.causal ? 1u << 26 : 0u);
+    p.sizes = (uint32_t)a.d | (uint32_t)a.num_splits << 8 | (xcd ? (uint32_t)a.group_xcd : 1u) << 16;
+    p.mul_chunk = a.by_chunk.mul, p.mul_slices = a.by_slices.mul, p.mul_splits = a.by_splits.mul;
+    p.group_span_or_fold_rows = fold ? a.fold_rows : xcd ? a.group_span : 0;
+    p.mul_xcd_or_fold_group = fold ? (uint32_t)a.fold_group : a.by_xcd_group.mul;
+    p.mul_kv_or_fold = (fold ? a.by_fold : a.by_kv_group).mul;
+    p.Nq = a.Nq, p.Nk = a.Nk, p.wl = a.wl, p.wr = a.wr, p.keys_per_split = a.keys_per_split;
+    p.Q = a.Q, p.K = a.K, p.V = a.V;
+    p.O = a.num_splits > 1 ? static_cast<void*>(a.O_partial) : a.O;
+    p.LSE = a.num_splits > 1 ? a.LSE_partial : a.LSE;
+    p.scale_log2 = a.scale_log2;
+    p.H = a.H, p.by_heads = a.by_heads;
+    p.drop_thr = a.drop_thr, p.drop_sub2 = a.drop_sub2, p.drop_rscale = a.drop_rscale;
+    p.seed_lo = a.seed_lo, p.seed_hi = a.seed_hi, p.off_lo = a.off_lo;
+    p.alibi = a.alibi, p.keep_out = a.keep_out, p.scores_out = a.scores_out, p.stamps = a.stamps;
+    return p;
+}
+
+// what packed() was given, as far as the kernels ask for it
+template <bool kFold, typename P>
+__host__ __device__ __forceinline__ FwdArgs unpacked(const P& p)
+{
+    FwdArgs a{};
+    auto div = [&](uint32_t mul, int k) __attribute__((always_inline)) { return FastDiv{mul, p.shifts >> (5 * k) & 31u}; };
+    a.snake_end = p.snake_end, a.slice_chunk = p.slice_chunk, a.Tr = p.Tr;
+    a.by_chunk = div(p.mul_chunk, 0), a.by_slices = div(p.mul_slices, 1), a.by_splits = div(p.mul_splits, 2);
+    a.split_rotate = p.shifts >> 25 & 1u, a.causal = p.shifts >> 26 & 1u;
+    a.d = p.sizes & 255u, a.num_splits = p.sizes >> 8 & 255u;
+    a.by_kv_group = fast_div_by_one();
+    if constexpr (kFold) {
+        a.fold_rows = p.group_span_or_fold_rows, a.fold_group = (int)p.mul_xcd_or_fold_group;
+        a.by_fold = div(p.mul_kv_or_fold, 4);
+    } else {
+        a.group_span = p.group_span_or_fold_rows, a.group_xcd = p.sizes >> 16;
+        a.by_xcd_group = div(p.mul_xcd_or_fold_group, 3), a.by_kv_group = div(p.mul_kv_or_fold, 4);
+    }
+    a.Nq = p.Nq, a.Nk = p.Nk, a.wl = p.wl, a.wr = p.wr, a.keys_per_split = p.keys_per_split;
+    a.Q = p.Q, a.K = p.K, a.V = p.V;
+    a.O = static_cast<half_t*>(p.O), a.O_partial = static_cast<float*>(p.O);
+    a.LSE = a.LSE_partial = static_cast<float*>(p.LSE);
+    a.scale_log2 = p.scale_log2;
+    if constexpr (sizeof(P) > sizeof(Packed)) {
+        a.H = p.H, a.by_heads = p.by_heads;
+        a.drop_thr = p.drop_thr, a.drop_sub2 = p.drop_sub2, a.drop_rscale = p.drop_rscale;
+        a.seed_lo = p.seed_lo, a.seed_hi = p.seed_hi, a.off_lo = p.off_lo;
+        a.alibi = p.alibi, a.keep_out = p.keep_out, a.scores_out = p.scores_out, a.stamps = p.stamps;
+    }
+    return a;
 }
 
 // Folded launches: the G query heads of a K/V head, n rows each, are one problem of G n rows over that K/V head -- in

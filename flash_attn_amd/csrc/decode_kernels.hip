@@ -17,11 +17,44 @@
 
 namespace fa {
 
+// Arguments of the decode kernel: see Packed in common.h
+struct DecodeArgs {
+    uint32_t mul_slices, mul_kv, mul_heads;
+    uint32_t shifts;  // of by_slices, by_kv_group, by_heads: five bits each; d, num_splits: eight bits each; bit 31: combine_waves is 4
+    int slices, H, Nk, wl, keys_per_split;  // slices: groups of G query heads
+    float scale_log2;
+    const half_t *Q, *K, *V;
+    half_t* O;
+    float *LSE, *O_partial, *LSE_partial;
+    uint32_t* counters;
+    const float* alibi;
+};
+static_assert(sizeof(DecodeArgs) <= kCheapArgs, "cheap launches");
+static DecodeArgs decode_args(const FwdArgs& a, int slices)
+{
+    return {a.by_slices.mul, a.by_kv_group.mul, a.by_heads.mul,
+            a.by_slices.shift | a.by_kv_group.shift << 5 | a.by_heads.shift << 10 | (uint32_t)a.d << 15 | (uint32_t)a.num_splits << 23 |
+                (a.combine_waves == 4 ? 1u << 31 : 0u),
+            slices, a.H, a.Nk, a.wl, a.keys_per_split, a.scale_log2, a.Q, a.K, a.V, a.O, a.LSE, a.O_partial, a.LSE_partial, a.counters, a.alibi};
+}
+__device__ __forceinline__ FwdArgs unpacked(const DecodeArgs& p)
+{
+    FwdArgs a{};
+    auto div = [&](uint32_t mul, int k) __attribute__((always_inline)) { return FastDiv{mul, p.shifts >> (5 * k) & 31u}; };
+    a.by_slices = div(p.mul_slices, 0), a.by_kv_group = div(p.mul_kv, 1), a.by_heads = div(p.mul_heads, 2);
+    a.d = p.shifts >> 15 & 255u, a.num_splits = p.shifts >> 23 & 255u, a.combine_waves = p.shifts >> 31 ? 4 : 1;
+    a.H = p.H, a.Nk = p.Nk, a.wl = p.wl, a.keys_per_split = p.keys_per_split, a.scale_log2 = p.scale_log2;
+    a.Q = p.Q, a.K = p.K, a.V = p.V, a.O = p.O, a.LSE = p.LSE, a.O_partial = p.O_partial, a.LSE_partial = p.LSE_partial;
+    a.counters = p.counters, a.alibi = p.alibi;
+    return a;
+}
+
 // G = query heads served by one work-group: the G consecutive heads share one K/V head (grouped-query attention), so
 // the K/V stream is read once for all of them.  G == 1 is the plain one-K/V-head-per-query-head case.
 template <int LPK, bool kAlibi, int G>
-__global__ void __launch_bounds__(256) decode_split_kernel(const FwdArgs a)
+__global__ void __launch_bounds__(256) decode_split_kernel(const DecodeArgs packed_args)
 {
+    const FwdArgs a = unpacked(packed_args);
     constexpr int KPI = 64 / LPK;      // keys per wave instruction
     constexpr int U = G > 2 ? 4 : 8;   // load instructions in flight per tensor
     constexpr int KB = U * KPI;        // keys per wave block
@@ -37,7 +70,7 @@ __global__ void __launch_bounds__(256) decode_split_kernel(const FwdArgs a)
     const int c = lane % LPK;
     const int kg = lane / LPK;
     const int split = a.by_slices.quotient(blockIdx.x);
-    const int bh0 = (blockIdx.x - split * (a.B * a.H / G)) * G;  // first of the G query slices of this work-group
+    const int bh0 = (blockIdx.x - split * packed_args.slices) * G;  // first of the G query slices of this work-group
     const int d = a.d, Nk = a.Nk;
     // Rows of any length from eight elements on, at any 2-byte alignment: a lane behind the row's whole chunks works
     // on the row's last 16 bytes, columns d - 8 ... d - 1 (no load leaves the row), with q zeroed where the lane before
@@ -252,8 +285,8 @@ static hipError_t launch_decode_instance(const FwdArgs& a, hipStream_t st)
     const unsigned groups = (unsigned)(slices * a.num_splits);
     FwdArgs b = a;
     set_divisors(b, slices);
-    if (a.alibi != nullptr) return launch_kernel(decode_split_kernel<LPK, true, G>, dim3(groups), dim3(256), 0, st, b);
-    return launch_kernel(decode_split_kernel<LPK, false, G>, dim3(groups), dim3(256), 0, st, b);
+    if (a.alibi != nullptr) return launch_kernel(decode_split_kernel<LPK, true, G>, dim3(groups), dim3(256), 0, st, decode_args(b, (int)slices));
+    return launch_kernel(decode_split_kernel<LPK, false, G>, dim3(groups), dim3(256), 0, st, decode_args(b, (int)slices));
 }
 
 template <int LPK>

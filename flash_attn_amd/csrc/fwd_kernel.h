@@ -139,6 +139,10 @@ constexpr float kNothingSeen = -3.402823466e38f;
 constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarStamp = 16, kVarAlibiLeft = 32, kVarKvOnce = 64,
               kVarEvery = 128, kVarNarrow = 256, kVarFold = 512, kVarPair = 1024;
 
+// arguments of an instance
+template <int VAR>
+using KernelArgs = std::conditional_t<(VAR & (kVarAlibi | kVarDropout | kVarStamp | kVarEvery)) != 0, PackedMore, Packed>;
+
 // work-groups per CU (narrow: one or two by their LDS; held to 256 VGPRs all the same, without which the compiler keeps more
 // than there are and moves them to and from accumulation registers): three up to D = 96 (168 VGPRs), except for the instance that
 // serves every request, which stages its tiles through registers, and at D = 96 those with sixteen registers of bias constants
@@ -155,8 +159,9 @@ constexpr int fwd_groups_per_cu(int D, int NB, int VAR)
 }
 
 template <int D, int NB, int VAR>
-__global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel(const FwdArgs a)
+__global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel(const KernelArgs<VAR> packed_args)
 {
+    const FwdArgs a = unpacked<(VAR & kVarFold) != 0>(packed_args);
     constexpr bool kVec = (VAR & kVarVec) != 0, kAlibi = (VAR & kVarAlibi) != 0, kDropout = (VAR & kVarDropout) != 0,
                    kFullD = (VAR & kVarFullD) != 0, kStamp = (VAR & kVarStamp) != 0, kKvOnce = (VAR & kVarKvOnce) != 0;
     using C = FwdCfg<D, NB, (VAR & kVarNarrow) != 0>;
@@ -1264,7 +1269,7 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
     const long long groups = (long long)a.Tr * a.B * a.H * a.num_splits;
     FwdArgs b = a;
     set_work_order<D, NB, VAR>(b);
-    return launch_kernel(kern, dim3((unsigned)groups), dim3(kPair ? 512 : 256), smem, st, b);
+    return launch_kernel(kern, dim3((unsigned)groups), dim3(kPair ? 512 : 256), smem, st, packed(b));
 }
 
 // The instances of a bucket: {d == bucket, d % 8 == 0} x {plain, ALiBi, ALiBi with every visible key at or left of its
@@ -1347,7 +1352,7 @@ inline hipError_t launch_fwd_narrow_instance(const FwdArgs& a, hipStream_t st)
     b.split_rotate = 0;
     b.snake_end = snake_end_for(groups, kNumCus);
     set_divisors(b, b.slice_chunk);
-    return launch_kernel(kern, dim3((unsigned)groups), dim3(256), smem, st, b);
+    return launch_kernel(kern, dim3((unsigned)groups), dim3(256), smem, st, packed(b));
 }
 
 // Paired work-groups (kPair in fwd_kernel): launches of at most one 128-row work-group per CU, whose SIMDs would have one

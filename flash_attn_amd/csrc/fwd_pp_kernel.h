@@ -68,8 +68,9 @@ __device__ __forceinline__ void lds_barrier_keep(void)
 }
 
 template <int D, int VAR>
-__global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const FwdArgs a)
+__global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const KernelArgs<VAR> packed_args)
 {
+    const FwdArgs a = unpacked<false>(packed_args);
     constexpr bool kAlibi = (VAR & kVarAlibi) != 0, kDropout = (VAR & kVarDropout) != 0, kStamp = (VAR & kVarStamp) != 0,
                    kFullD = (VAR & kVarFullD) != 0;
     using C = PPCfg<D>;
@@ -657,7 +658,7 @@ inline hipError_t launch_fwd_pp_instance(const FwdArgs& a, hipStream_t st)
     b.split_rotate = split_rotate_for(b.num_splits, b.slice_chunk);
     b.snake_end = snake_end_for(groups, kNumCus);
     set_divisors(b, b.slice_chunk);
-    return launch_kernel(kern, dim3((unsigned)groups), dim3(512), C::SMEM, st, b);
+    return launch_kernel(kern, dim3((unsigned)groups), dim3(512), C::SMEM, st, packed(b));
 }
 
 // {d == D, shorter rows} x {plain, ALiBi, dropout, both}; ST = kVarStamp: their instrumented twins

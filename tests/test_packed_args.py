@@ -1,0 +1,30 @@
+"""The arguments that the tiled kernels get, packed and unpacked on the host (tests/packed_args_test.cpp), and their size in the code
+as it was built.  No GPU needed."""
+import os
+import re
+import subprocess
+
+import launch_recorder as lr
+import machine_code as mc
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+LIBRARY = os.path.join(mc.ROOT, "flash_attn_amd", "lib", "libflash_attn_mi355.so")
+
+
+def test_round_trip(tmp_path):
+    exe = str(tmp_path / "packed_args_test")
+    subprocess.check_call(["/opt/rocm/bin/hipcc", "-x", "hip", "--offload-host-only", "--offload-arch=gfx950", "-std=c++17", "-O1", "-I",
+                           os.path.join(os.path.dirname(HERE), "flash_attn_amd", "csrc"), os.path.join(HERE, "packed_args_test.cpp"), "-o", exe])
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_arguments_are_few():
+    """112 bytes at most, hidden arguments included, for every kernel without ALiBi, dropout and debug outputs, and for decode."""
+    seen = 0
+    for name, fields in mc.metadata(LIBRARY).items():
+        m = re.match(r".*fwd_(?:pp_)?kernelILi\d+E(?:Li\d+E)?Li(\d+)EEE", name)
+        if (m and not int(m[1]) & (lr.ALIBI | lr.DROPOUT | lr.STAMP | lr.EVERY)) or "decode_split_kernel" in name or "combine_kernel" in name:
+            seen += 1
+            assert fields["kernarg_segment_size"] <= 112, (name, fields["kernarg_segment_size"])
+    assert seen > 100
