@@ -33,14 +33,21 @@
 namespace fa {
 
 
-template <int D, int NB, bool kNarrow = false>
+template <int D, int NB, bool kNarrow = false, bool kShort = false>
 struct FwdCfg {
     static constexpr int kWaves = 4;
     static constexpr int RW = 32 * NB;        // query rows per wave
     static constexpr int BR = kWaves * RW;    // query rows per work-group
     static constexpr int BC = 64;             // keys per tile
     static constexpr int CH = D / 8;          // 16-byte chunks per row
-    static constexpr int KS = D / 16;         // k-steps of the QK^T contraction
+    // Rows of at most D - 16 elements (kShort: d = 40 in 64 columns, 72 and 80 in 96, 100 and 112 in 128) leave out the last k-step,
+    // its share of K in LDS and of the requests for it: a tile is bound by what it issues and moves, and one in twelve of its MFMAs at D = 96
+    // met zeroes of Q.  With the k-step -> without: causal B3 H12 N1777 d80 34.7 -> 32.9 us, B4 H16 N2048 d80 106.8 -> 101.0, d72 causal
+    // 60.1 -> 57.6, B10 H16 H_kv8 N1216 d40 74.7 -> 70.3, B15 H16 N1536 d100 causal 187 -> 178 (8-wave), B1 H4 N2048 d100 16.8 -> 15.6
+    // (narrow), causal with dropout B8 H32 N1000 d80 91.0 -> 86.3; split over 8409 keys B3 H16 Nq192 d72, bound by HBM, +-0.  (At run time, one branch around the
+    // MFMAs, it gave 1-3 % there and cost the other rows 0.3-1 %.)
+    static constexpr int KS = D / 16 - (kShort ? 1 : 0);  // k-steps of the QK^T contraction
+    static constexpr int CHK = 2 * KS;        // 16-byte chunks per K row
     static constexpr int MB = D / 32;         // 32-wide head-dim blocks of O^T
     // LDS rows.  K rows are read 16 bytes per lane by 32 consecutive rows, which have to be spread over all banks.
     // Either the rows are padded by one 16-byte chunk (kPadK: stride / 16 odd), or the chunks of row r are permuted by
@@ -54,12 +61,14 @@ struct FwdCfg {
     // V rows are read by ds_read_b64_tr_b16, four consecutive rows of 64 bytes per half wave: a stride of 64 (mod 128)
     // puts the four rows on disjoint bank groups.
     static constexpr bool kPadK = D == 128 && !kNarrow;
-    static constexpr int CK = CH + (kPadK ? 1 : 0);  // chunks of a K row in LDS
+    static constexpr int CK = CHK + (kPadK ? 1 : 0);  // chunks of a K row in LDS
     static constexpr int SK = CK * 16;
     static constexpr int SV = D * 2;
     static constexpr __host__ __device__ int kswz(int r)
     {
-        return kPadK ? 0 : D == 128 ? r & 15 : D == 64 ? (r >> 1) & 7 : (r >> 2) & 3;  // rows of 256 / 128 / 192 or 64 bytes
+        if (kPadK) return 0;
+        if (kShort) return (r >> 3) & 1;  // rows of 224 / 160 / 96 bytes, an odd multiple of 32: eight rows spread by themselves
+        return D == 128 ? r & 15 : D == 64 ? (r >> 1) & 7 : (r >> 2) & 3;  // rows of 256 / 128 / 192 or 64 bytes
     }
     // Where the row length is a multiple of 128 bytes, the two 64-byte halves of each 128 bytes are exchanged in rows
     // 2, 3 (mod 4), which has the same effect without padding.
@@ -73,7 +82,7 @@ struct FwdCfg {
     static constexpr int NKX = (CK + 3) / 4;      // 1 KiB blocks of a K tile (CK of them) per wave, rounded up
     static constexpr int NVX = CH / 4;            // 1 KiB blocks of a V tile (CH of them) per wave
     static constexpr int NLD = BC * CH / 256;  // 16-byte chunks per thread per tile (K and V each)
-    static_assert(D % 32 == 0 && D <= 128, "head-dim bucket");
+    static_assert(D % 32 == 0 && D <= 128 && (!kShort || D >= 64), "head-dim bucket");
     static_assert((BC * CH) % 256 == 0, "tile chunks must divide over the group");
 };
 
@@ -136,8 +145,9 @@ constexpr float kNothingSeen = -3.402823466e38f;
 // each, see kNarrow below.
 // kVarPair (without ALiBi): eight waves in two halves that take every other tile each, see kPair below.
 // kVarFold (no other feature): the rows are the query heads of a K/V head, see row_position in common.h.
+// kVarShort (D >= 64, not kVarFullD, kVarEvery or kVarFold): rows of at most D - 16 elements, see FwdCfg::kShort.
 constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarStamp = 16, kVarAlibiLeft = 32, kVarKvOnce = 64,
-              kVarEvery = 128, kVarNarrow = 256, kVarFold = 512, kVarPair = 1024;
+              kVarEvery = 128, kVarNarrow = 256, kVarFold = 512, kVarPair = 1024, kVarShort = 2048;
 
 // arguments of an instance
 template <int VAR>
@@ -164,7 +174,8 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     const FwdArgs a = unpacked<(VAR & kVarFold) != 0>(packed_args);
     constexpr bool kVec = (VAR & kVarVec) != 0, kAlibi = (VAR & kVarAlibi) != 0, kDropout = (VAR & kVarDropout) != 0,
                    kFullD = (VAR & kVarFullD) != 0, kStamp = (VAR & kVarStamp) != 0, kKvOnce = (VAR & kVarKvOnce) != 0;
-    using C = FwdCfg<D, NB, (VAR & kVarNarrow) != 0>;
+    using C = FwdCfg<D, NB, (VAR & kVarNarrow) != 0, (VAR & kVarShort) != 0>;
+    static_assert((VAR & kVarShort) == 0 || (VAR & (kVarFullD | kVarEvery | kVarFold)) == 0, "shorter rows");
     Stamps<kStamp> stamps;
     stamps.take(0);
     constexpr int BC = C::BC, KS = C::KS, MB = C::MB, CH = C::CH, SK = C::SK, SV = C::SV, NLD = C::NLD;
@@ -401,9 +412,11 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     auto chunk_offset = [&](int c) { return kFullD ? c * 16 : (c * 8 + 8 <= d ? c * 16 : (d - 8) * 2); };
     // (narrow: every block of a tile is the wave's own, and so is the buffer; both permutations repeat every 16 rows, which are
     // CH / 4 blocks, so that only the first CH / 4 requests need offsets of their own and all others are the same some
-    // multiple of 16 rows further on, which goes into the scalar base address: 66 registers less at D = 128)
-    constexpr int NKX = kNarrow ? CH : C::NKX, NVX = kNarrow ? CH : C::NVX;
-    constexpr int NKO = kNarrow ? CH / 4 : NKX, NVO = kNarrow ? CH / 4 : NVX;  // offsets held
+    // multiple of 16 rows further on, which goes into the scalar base address: 66 registers less at D = 128; where 16 rows
+    // of K are no whole number of blocks, 32 are)
+    constexpr int NKX = kNarrow ? C::CHK : C::NKX, NVX = kNarrow ? CH : C::NVX;
+    constexpr int kKeyRows = C::CHK % 4 == 0 ? 16 : 32;  // rows of K after which the offsets repeat
+    constexpr int NKO = kNarrow ? C::CHK * kKeyRows / 64 : NKX, NVO = kNarrow ? CH / 4 : NVX;  // offsets held
     auto block_of = [&](int i) { return kNarrow ? i : wave + 4 * i; };
     uint32_t koff[NKO], voff[NVO];
     int krow[NKO], vrow[NVO];
@@ -413,7 +426,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
             const int q = 64 * block_of(i) + lane;
             krow[i] = q / C::CK;
             const int c = q % C::CK;
-            koff[i] = (uint32_t)(krow[i] * row_bytes + chunk_offset((c < CH ? c : CH - 1) ^ C::kswz(krow[i])));
+            koff[i] = (uint32_t)(krow[i] * row_bytes + chunk_offset((c < C::CHK ? c : C::CHK - 1) ^ C::kswz(krow[i])));
         }
 #pragma unroll
         for (int i = 0; i < NVO; ++i) {
@@ -454,7 +467,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
 #pragma unroll
             for (int i = 0; i < NKX; ++i) {
                 if (!decltype(k_part)::value || (i == NKX - 1 && !k_extra)) break;
-                request(Kb, koff[i % NKO], krow[i % NKO], i / NKO * 16, kst + block_of(i) * 1024);
+                request(Kb, koff[i % NKO], krow[i % NKO], i / NKO * kKeyRows, kst + block_of(i) * 1024);
             }
 #pragma unroll
             for (int i = 0; i < NVX; ++i) {
@@ -1260,7 +1273,7 @@ inline void set_work_order(FwdArgs& b)
 template <int D, int NB, int VAR>
 inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
 {
-    using C = FwdCfg<D, NB>;
+    using C = FwdCfg<D, NB, false, (VAR & kVarShort) != 0>;
     auto kern = fwd_kernel<D, NB, VAR>;
     static DeviceFlags attr_done;  // per instantiation and device
     constexpr bool kPair = (VAR & kVarPair) != 0;
@@ -1274,7 +1287,7 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
 
 // The instances of a bucket: {d == bucket, d % 8 == 0} x {plain, ALiBi, ALiBi with every visible key at or left of its
 // row, dropout, both}, for rows at any alignment (d % 8 != 0) {plain, ALiBi, dropout, both}, and the one that serves
-// every other request; the narrow, paired and folded ones below.  ST = kVarStamp selects their instrumented twins (debug
+// every other request; those for shorter rows (all but the last) once more for d <= D - 16; the narrow, paired and folded ones below.  ST = kVarStamp selects their instrumented twins (debug
 // time stamps).  Nothing else looks at the stamp pointer: a stamped call is launched as the same call without.
 // The narrow instances (kNarrow in fwd_kernel) serve unsplit launches whose time is the chain of key tiles that a work-group
 // walks through, which they cut to a quarter for a fixed cost of about 1 us (a wave's own requests, the merge of four).
@@ -1340,7 +1353,7 @@ inline bool fwd_uses_narrow(const FwdArgs& a, bool every)
 template <int D, int VAR>
 inline hipError_t launch_fwd_narrow_instance(const FwdArgs& a, hipStream_t st)
 {
-    using C = FwdCfg<D, 1, true>;
+    using C = FwdCfg<D, 1, true, (VAR & kVarShort) != 0>;
     auto kern = fwd_kernel<D, 1, VAR | kVarNarrow>;
     static DeviceFlags attr_done;  // per instantiation and device
     constexpr int smem = 4 * (D <= 64 ? 2 : 1) * (C::KBUF + C::VBUF);  // two stages per wave up to D = 64, one above
@@ -1418,6 +1431,13 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
     hipError_t e;
     const int feat = variant & (kVarAlibi | kVarDropout);
     constexpr int AL = kVarAlibi | kVarAlibiLeft;  // ALiBi with no visible key right of its row
+    // launch(kVarShort) where rows are at most D - 16 elements long, launch(0) otherwise
+    auto by_length = [&](auto launch) {
+        if constexpr (D >= 64) {
+            if (a.d <= D - 16) return launch(std::integral_constant<int, kVarShort>{});
+        }
+        return launch(std::integral_constant<int, 0>{});
+    };
     if (fwd_uses_narrow(a, fwd_needs_every_instance(a, variant))) {
         // plain: by row length like the others; with ALiBi or dropout: the instances for rows at any alignment, which serve
         // every row length from eight elements on, and above 64 the ones for rows of the bucket's width
@@ -1437,13 +1457,20 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
             return (int)launch_fwd_narrow_instance<D, ST | kVarFold>(a, st);
         }
         if (a.d == D) return (int)launch_fwd_narrow_instance<D, ST | kVarVec | kVarFullD>(a, st);
-        if (variant & kVarVec) return (int)launch_fwd_narrow_instance<D, ST | kVarVec>(a, st);
-        return (int)launch_fwd_narrow_instance<D, ST>(a, st);
+        if (variant & kVarVec) return (int)by_length([&](auto sh) { return launch_fwd_narrow_instance<D, ST | kVarVec | decltype(sh)::value>(a, st); });
+        return (int)by_length([&](auto sh) { return launch_fwd_narrow_instance<D, ST | decltype(sh)::value>(a, st); });
     }
     const bool pair = fwd_uses_pair(a, D, feat);
     auto halves = [&](auto var) {
         constexpr int V = decltype(var)::value;
         return pair ? launch_fwd_instance<D, NB, V | kVarPair>(a, st) : launch_fwd_instance<D, NB, V>(a, st);
+    };
+    // rows shorter than the bucket: V with paired work-groups where they fit, or alone
+    auto shorter_rows = [&](auto var) {
+        return by_length([&](auto sh) { return halves(std::integral_constant<int, decltype(var)::value | decltype(sh)::value>{}); });
+    };
+    auto shorter_rows_alone = [&](auto var) {
+        return by_length([&](auto sh) { return launch_fwd_instance<D, NB, decltype(var)::value | decltype(sh)::value>(a, st); });
     };
     // (several row blocks per K/V head ask for the same tiles and have to find them in L2: folded launches of 129 rows or more,
     // non-temporal -> ordinary, 24 random shapes -1 ... +15 %, +4.4 % in the mean: B2 H32 H_kv8 Nq42 Nk3937 d128 23.5 -> 20.5 us, B16
@@ -1462,10 +1489,10 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
         // scores are scaled ahead of the row maximum), the score dump, rows of fewer than eight elements, a dropout
         // threshold of 0
         if (fwd_needs_every_instance(a, variant)) e = launch_fwd_instance<D, NB, ST | kVarAlibi | kVarDropout | kVarEvery>(a, st);
-        else if (feat == 0) e = halves(std::integral_constant<int, ST>{});
-        else if (feat == kVarAlibi) e = launch_fwd_instance<D, NB, ST | kVarAlibi>(a, st);
-        else if (feat == kVarDropout) e = halves(std::integral_constant<int, ST | kVarDropout>{});
-        else e = launch_fwd_instance<D, NB, ST | kVarAlibi | kVarDropout>(a, st);
+        else if (feat == 0) e = shorter_rows(std::integral_constant<int, ST>{});
+        else if (feat == kVarAlibi) e = shorter_rows_alone(std::integral_constant<int, ST | kVarAlibi>{});
+        else if (feat == kVarDropout) e = shorter_rows(std::integral_constant<int, ST | kVarDropout>{});
+        else e = shorter_rows_alone(std::integral_constant<int, ST | kVarAlibi | kVarDropout>{});
     } else if (a.d == D) {
         constexpr int V = ST | kVarVec | kVarFullD;
         if constexpr (D == 64) {
@@ -1481,10 +1508,10 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
         else e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL | kVarDropout>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi | kVarDropout>(a, st);
     } else {
         constexpr int V = ST | kVarVec;
-        if (feat == 0) e = halves(std::integral_constant<int, V>{});
-        else if (feat == kVarAlibi) e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi>(a, st);
-        else if (feat == kVarDropout) e = halves(std::integral_constant<int, V | kVarDropout>{});
-        else e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL | kVarDropout>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi | kVarDropout>(a, st);
+        if (feat == 0) e = shorter_rows(std::integral_constant<int, V>{});
+        else if (feat == kVarDropout) e = shorter_rows(std::integral_constant<int, V | kVarDropout>{});
+        else if (feat == kVarAlibi) e = a.alibi_left ? shorter_rows_alone(std::integral_constant<int, V | AL>{}) : shorter_rows_alone(std::integral_constant<int, V | kVarAlibi>{});
+        else e = a.alibi_left ? shorter_rows_alone(std::integral_constant<int, V | AL | kVarDropout>{}) : shorter_rows_alone(std::integral_constant<int, V | kVarAlibi | kVarDropout>{});
     }
     return (int)e;
 }

@@ -76,7 +76,10 @@ __global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const KernelArgs<VAR> pa
     using C = PPCfg<D>;
     Stamps<kStamp> stamps;
     stamps.take(0);
-    constexpr int BC = C::BC, KS = C::KS, MB = C::MB, NKL = C::NKL, NVL = C::NVL, NST = C::NST;
+    // (rows of at most D - 16 elements leave out the last k-step: fwd_kernel.h)
+    constexpr int KS = C::KS - ((VAR & kVarShort) != 0 ? 1 : 0);
+    static_assert((VAR & kVarShort) == 0 || (VAR & kVarFullD) == 0, "shorter rows");
+    constexpr int BC = C::BC, MB = C::MB, NKL = C::NKL, NVL = C::NVL, NST = C::NST;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     FA_LDS char* const Ks = (FA_LDS char*)smem;
     FA_LDS char* const Vs = Ks + NST * C::KBUF;
@@ -674,10 +677,14 @@ inline int launch_fwd_pp_bucket_st(const FwdArgs& a, int variant, hipStream_t st
         else if (feat == kVarDropout) e = launch_fwd_pp_instance<D, V | kVarDropout>(a, st);
         else e = launch_fwd_pp_instance<D, V | kVarAlibi | kVarDropout>(a, st);
     } else {
-        if (feat == 0) e = launch_fwd_pp_instance<D, ST>(a, st);
-        else if (feat == kVarAlibi) e = launch_fwd_pp_instance<D, ST | kVarAlibi>(a, st);
-        else if (feat == kVarDropout) e = launch_fwd_pp_instance<D, ST | kVarDropout>(a, st);
-        else e = launch_fwd_pp_instance<D, ST | kVarAlibi | kVarDropout>(a, st);
+        auto by_length = [&](auto var) {
+            constexpr int V = ST | decltype(var)::value;
+            return a.d <= D - 16 ? launch_fwd_pp_instance<D, V | kVarShort>(a, st) : launch_fwd_pp_instance<D, V>(a, st);
+        };
+        if (feat == 0) e = by_length(std::integral_constant<int, 0>{});
+        else if (feat == kVarAlibi) e = by_length(std::integral_constant<int, kVarAlibi>{});
+        else if (feat == kVarDropout) e = by_length(std::integral_constant<int, kVarDropout>{});
+        else e = by_length(std::integral_constant<int, kVarAlibi | kVarDropout>{});
     }
     return (int)e;
 }
