@@ -482,6 +482,14 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // wait until every request has landed
     auto dma_wait = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
 
+    // Narrow at D = 64: the scores of a wave's next tile are worked out beside the exponentials of the present one
+    // (tile_with_scores_ahead), since a wave alone on its SIMD otherwise leaves the vector unit idle for every MFMA and the matrix
+    // unit for every exponential.  One tile after the other -> ahead: B1 H8 N1024 d64 7.8 -> 7.55 us, N2048 causal 15.1 -> 14.4, B2 H3 N1792
+    // 19.2 -> 18.2, B1 H8 N1024 d40 7.45 -> 6.7, d63 causal with bias 13.7 -> 12.8; one tile per wave +-0.  At D = 32, where K Q^T is four
+    // MFMAs and two work-groups share a CU, it is +1 ... -3 %; above D = 64 there is no second stage for K.  With dropout
+    // the Philox rounds stand beside the MFMAs already.
+    constexpr bool kAheadQk = kNarrow && D == 64 && !kDropout;
+
     // ---- accumulators
     v16f oacc[MB][NB];
     float m_ref[NB], m_thr[NB], l_run[NB];
@@ -637,7 +645,8 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
 
     // online softmax of one tile (per query row = per lane); leaves P^T packed to fp16 in pf
     // masked: some row of the wave does not see all of the tile (wave-uniform)
-    auto softmax = [&](bool masked, int kb0, v16f (&s)[2][NB], v8h (&pf)[2][2][NB]) {
+    // ahead: stops in front of the exponentials (tile_with_scores_ahead below has them)
+    auto softmax = [&](bool masked, int kb0, v16f (&s)[2][NB], v8h (&pf)[2][2][NB], auto ahead) __attribute__((always_inline)) {
         constexpr bool folded = kFoldAlibi;
         if constexpr (kDropout) calls.cover(kb0, lane, (uint32_t)bh, a.off_lo, a.seed_lo, a.seed_hi);
         if constexpr (kDropout && !kEvery) first_part = calls.at(kb0, 0, g);  // (in time for pv)
@@ -724,6 +733,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
 #pragma unroll
                     for (int r = 0; r < 16; ++r) oacc[mb][nb][r] *= alpha;
             }
+            if constexpr (decltype(ahead)::value) continue;
             float rs = 0.0f;
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
@@ -767,17 +777,23 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         }
     };
 
-    // O^T += V^T P^T with the tile in V buffer `buf`
-    auto pv = [&](int buf, int kb0, v16f (&s)[2][NB], v8h (&pf)[2][2][NB]) {
-        // (a lane's rows all share bit 1 of the row index: the swizzle is one per-lane choice between two bases)
-        const char* const vb[2] = {Vs + buf * C::VBUF + v_rd + v_sw, Vs + buf * C::VBUF + v_rd + (v_sw ^ (C::VSWZ ? 64 : 0))};
-        auto v_frag = [&](int kb, int tt, int mb) __attribute__((always_inline)) {
-            const char* p0 = C::VSWZ ? vb[mb & 1] + (32 * kb + 16 * tt) * SV + (mb >> 1) * 128 : vb[0] + (32 * kb + 16 * tt) * SV + mb * 64;
+    // V^T fragment of the tile in V buffer `buf`: keys 32 kb + 16 tt ... + 15, columns of block mb
+    // (a lane's rows all share bit 1 of the row index: the swizzle is one per-lane choice between two bases)
+    auto v_frags = [&](int buf) __attribute__((always_inline)) {
+        const char* const b0 = Vs + buf * C::VBUF + v_rd + v_sw;
+        const char* const b1 = Vs + buf * C::VBUF + v_rd + (v_sw ^ (C::VSWZ ? 64 : 0));
+        return [=](int kb, int tt, int mb) __attribute__((always_inline)) {
+            const char* p0 = C::VSWZ ? ((mb & 1) ? b1 : b0) + (32 * kb + 16 * tt) * SV + (mb >> 1) * 128 : b0 + (32 * kb + 16 * tt) * SV + mb * 64;
             union { v4hp p[2]; v8h v; } af;
             af.p[0] = __builtin_amdgcn_ds_read_tr16_b64_v4f16((FA_LDS v4hp*)(p0));
             af.p[1] = __builtin_amdgcn_ds_read_tr16_b64_v4f16((FA_LDS v4hp*)(p0 + 8 * SV));
             return af.v;
         };
+    };
+
+    // O^T += V^T P^T with the tile in V buffer `buf`
+    auto pv = [&](int buf, int kb0, v16f (&s)[2][NB], v8h (&pf)[2][2][NB]) {
+        auto v_frag = v_frags(buf);
         if constexpr (kDropout && !kEvery) {
             // Dropout, 16 keys at a time (a step): drop iff field < threshold, row sum left undropped
             // (src/flash_forward.h:221-237); the survivors' factor 1/(1-p) is common to the whole row and multiplies O once in
@@ -829,6 +845,71 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         }
     };
 
+    // A wave alone on its SIMD: what softmax leaves to do of the tile whose scores (rows raised) are in s, and P V with it, while the
+    // matrix unit is at the scores of the tile to come, K in buffer kbuf.  The exponents leave the score registers first, so that
+    // the next scores take their place; then the MFMAs of K Q^T stand between the exponentials of the first 32 keys, and those of
+    // their P V between the exponentials of the others, step by step behind fences.  (The last tile has no successor: what is
+    // in the buffer then is multiplied all the same, and not looked at.)
+    auto tile_with_scores_ahead = [&](int vbuf, int kbuf, v16f (&s)[2][NB]) __attribute__((always_inline)) {
+        constexpr int n = 2 * KS, kAhead = 3;  // step i: k-step i / 2, key block i % 2
+        const char* const kbase = Ks + kbuf * C::KBUF + k_rd;
+        auto v_frag = v_frags(vbuf);
+        // (the fences order nothing that only computes; what passes through here is worked out by then)
+        auto pin = [](auto& v) __attribute__((always_inline)) { asm volatile("" : "+v"(v)); };
+        auto k_frag = [&](int i) { return *reinterpret_cast<const v8h*>(kbase + (i & 1) * 32 * SK + k_step(i >> 1)); };
+        v8h kf[n], vf[2 * 2 * MB];
+        union { uint32_t u[4]; v8h h; } p[2][2];
+        float x[2][16], rs = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) kf[i] = k_frag(i);
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                x[kb][r] = __builtin_fmaf(s[kb][0][r], cs, -m_ref[0]);
+                pin(x[kb][r]);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        // exponentials of scores r0 ... r0 + count - 1 of a key block, each pair packed
+        auto exps = [&](int kb, int r0, int count) __attribute__((always_inline)) {
+#pragma unroll
+            for (int r = r0; r < r0 + count; r += 2) {
+                const float p0 = fast_exp2(x[kb][r]), p1 = fast_exp2(x[kb][r + 1]);
+                rs = kb == 0 && r == 0 ? p0 + p1 : rs + p0 + p1;
+                union { v2h h; uint32_t u; } two;
+                two.h = pack_f16(p0, p1);
+                pin(two.u);
+                pin(rs);
+                p[kb][r >> 3].u[(r & 7) >> 1] = two.u;
+            }
+        };
+        constexpr int kPer = 16 / n & ~1;  // scores per step of K Q^T
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+            const v16f z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+            s[i & 1][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[i], qf[0][i >> 1], i < 2 ? z : s[i & 1][0], 0, 0, 0);
+            if (i + kAhead < n) kf[i + kAhead] = k_frag(i + kAhead);
+            // the first fragments of V behind the last ones of K
+            else if (i + kAhead - n < 2 * MB) vf[i + kAhead - n] = v_frag(0, (i + kAhead - n) / MB, (i + kAhead - n) % MB);
+            exps(0, kPer * i, i == n - 1 ? 16 - kPer * i : kPer);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = kAhead; i < 2 * MB; ++i) vf[i] = v_frag(0, i / MB, i % MB);
+        constexpr int kPerV = 16 / (2 * MB);
+#pragma unroll
+        for (int i = 0; i < 2 * MB; ++i) {
+            oacc[i % MB][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i], p[0][i / MB].h, oacc[i % MB][0], 0, 0, 0);
+            vf[2 * MB + i] = v_frag(1, i / MB, i % MB);
+            exps(1, kPerV * i, kPerV);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        l_run[0] += rs;
+#pragma unroll
+        for (int i = 0; i < 2 * MB; ++i)
+            oacc[i % MB][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[2 * MB + i], p[1][i / MB].h, oacc[i % MB][0], 0, 0, 0);
+    };
+
     // The Q fragments must have landed before the loop starts: a load still counted as outstanding at the loop
     // header makes the compiler guard every use of qf inside the loop with a vmcnt wait, and since vmcnt counts in
     // order, that wait would also drain the K/V prefetch of the same iteration.
@@ -851,7 +932,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
             v8h pf[2][2][NB];
             const int kb0 = (tile_begin + t) * BC;
             qk(buf, s);
-            softmax(tile_masked(t), kb0, s, pf);
+            softmax(tile_masked(t), kb0, s, pf, std::false_type{});
             pv(buf, kb0, s, pf);
             dump_keep(kb0);
         }
@@ -873,7 +954,37 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         pin_q();
         stamps.take(2);
         stamps.take(3);  // (no barrier in front of the loop)
-        if constexpr (NSTG == 2) {
+        if constexpr (kAheadQk) {
+            // K runs one tile ahead of V.  At the end of tile n the stage buffers K(n + 1) and V(n) have been read, K(n + 2) and V(n + 1)
+            // are on their way, K(n + 3) and V(n + 2) are requested.
+            v16f s[2][NB];
+            v8h none[2][2][NB];
+            auto request = [&](int n, int stage, auto k_part) {
+                if (n < nt) dma_tile_parts(tile_begin + wave + 4 * n, stage, k_part, std::integral_constant<bool, !decltype(k_part)::value>{});
+            };
+            if (nt == 1) {  // (no successor whose scores could be worked out)
+                tile_math(wave, 0);
+                stamps.take(4);
+            } else if (nt > 1) {
+                qk(0, s);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                request(2, 0, std::true_type{});
+                int buf = 0, n = 0;
+                do {
+                    const int t = wave + 4 * n;
+                    softmax(tile_masked(t), (tile_begin + t) * BC, s, none, std::true_type{});
+                    tile_with_scores_ahead(buf, buf ^ 1, s);
+                    if (kStamp && n == 0) stamps.take(4);
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                    request(n + 2, buf, std::false_type{});
+                    request(n + 3, buf ^ 1, std::true_type{});
+                    if (n + 3 < nt) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NKX + NVX) : "memory");
+                    else if (n + 2 < nt) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NVX) : "memory");
+                    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    buf ^= 1;
+                } while (++n < nt);
+            }
+        } else if constexpr (NSTG == 2) {
             int buf = 0;
             for (int n = 0; n < nt; ++n) {
                 tile_math(wave + 4 * n, buf);
@@ -905,7 +1016,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                     dma_tile_parts(tile_begin + wave + 4 * (n + 1), 0, std::true_type{}, std::false_type{});
                 }
-                if constexpr (kLive) softmax(tile_masked(t), (tile_begin + t) * BC, s, pf);
+                if constexpr (kLive) softmax(tile_masked(t), (tile_begin + t) * BC, s, pf, std::false_type{});
                 // V(n): older than the K request just issued
                 if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NKX) : "memory");
                 else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
