@@ -735,6 +735,11 @@ __device__ __forceinline__ void dma_kib(const char* base, uint32_t off, FA_LDS c
                  : "s"(m0v), "v"(off), "s"(base)
                  : "memory", "m0");
 }
+// A float at an address that is the same in all lanes, which nobody writes during the launch: a load of the scalar unit.
+__device__ __forceinline__ float read_uniform(const float* p)
+{
+    return *reinterpret_cast<const __attribute__((address_space(4))) float*>(reinterpret_cast<uintptr_t>(p));
+}
 // The same request marked non-temporal, for data that no other work-group will ask for (the K/V stream of a decode
 // launch): measured 5.4 -> 6.3 TB/s on grouped-query decode with eight query heads per K/V head.
 __device__ __forceinline__ void dma_kib_nt(const char* base, uint32_t off, FA_LDS char* lds_dst)

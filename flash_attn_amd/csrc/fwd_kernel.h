@@ -75,6 +75,7 @@ struct FwdCfg {
     static constexpr bool VSWZ = (D * 2) % 128 == 0;
     static constexpr int KBUF = BC * SK;
     static constexpr int VBUF = BC * SV;
+    static constexpr bool kQApart = kNarrow && D <= 64;  // Q has a place of its own behind the four waves' stages
     static constexpr int kTiles = 2 * KBUF + 2 * VBUF, kOut = 4 * NB * 32 * (2 * D + 16);
     static constexpr int SMEM = kTiles > kOut ? kTiles : kOut;
     static constexpr int NSTG = 2;
@@ -209,6 +210,14 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // (narrow: two stages per wave up to D = 64, one above: four waves' tiles of 26 / 33 KiB)
     constexpr int NSTG = kNarrow ? (D <= 64 ? 2 : 1) : kDma ? C::NSTG : 2;
     constexpr int BRW = kNarrow ? 32 : C::BR;  // query rows per work-group
+    // Narrow: Q is fetched like the first 32 rows of a K tile, so that the wave's first wait is for Q and tile 0 alone.  Loaded into
+    // registers -> so: B1 H8 N1021 d31 8.0 -> 7.3 us, d63 11.5 -> 10.2, N1024 d64 7.2 -> 7.0, N2048 causal d64 14.4 -> 13.9, N1024
+    // d128 10.8 -> 10.1, N300 d128 7.3 -> 6.75, B1 H2 N3000 d111 33.1 -> 31.9, d72, d80 and one or two tiles per wave +-1 %; d96
+    // -1 ... -2 % (8.5 -> 8.6, as much as the same code around the old loads), left as it is.
+    // Where to, and bytes from one wave's to the next one's
+    constexpr bool kQApart = C::kQApart;
+    constexpr int kQWave = kQApart ? 32 * C::SK : NSTG * (C::KBUF + C::VBUF);
+    constexpr int kQLds = kQApart ? 4 * NSTG * (C::KBUF + C::VBUF) : NSTG * C::KBUF + (NSTG - 1) * C::VBUF;
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
     const int tid = threadIdx.x;
@@ -324,7 +333,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // ---- Q fragments (B operand of S^T = K Q^T): lane holds row l32, columns 16*ks + 8*g .. +7
     v8h qf[NB][KS];
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
+    for (int nb = 0; nb < NB && !kNarrow; ++nb) {
         const int ic = row_i[nb] < Nq ? row_i[nb] : Nq - 1;
         const half_t* qrow = Qbh + (size_t)ic * d;
         if constexpr (kVec) {
@@ -420,14 +429,15 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     auto block_of = [&](int i) { return kNarrow ? i : wave + 4 * i; };
     uint32_t koff[NKO], voff[NVO];
     int krow[NKO], vrow[NVO];
+    auto k_offset = [&](int i) __attribute__((always_inline)) {
+        const int q = 64 * block_of(i) + lane;
+        krow[i] = q / C::CK;
+        const int c = q % C::CK;
+        koff[i] = (uint32_t)(krow[i] * row_bytes + chunk_offset((c < C::CHK ? c : C::CHK - 1) ^ C::kswz(krow[i])));
+    };
     if constexpr (kDma) {
 #pragma unroll
-        for (int i = 0; i < NKO; ++i) {
-            const int q = 64 * block_of(i) + lane;
-            krow[i] = q / C::CK;
-            const int c = q % C::CK;
-            koff[i] = (uint32_t)(krow[i] * row_bytes + chunk_offset((c < C::CHK ? c : C::CHK - 1) ^ C::kswz(krow[i])));
-        }
+        for (int i = 0; i < NKO && !kNarrow; ++i) k_offset(i);  // (narrow: request by request, below)
 #pragma unroll
         for (int i = 0; i < NVO; ++i) {
             const int q = 64 * block_of(i) + lane;
@@ -512,8 +522,10 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     const bool scale_late = !kEvery || c2 > 0.0f;
     const float cs = scale_late ? c2 : 1.0f;
     const float inv_cs = __builtin_amdgcn_rcpf(cs);  // (of the raise threshold alone: whether a row is rescaled is no matter of its last bit)
-    // The ALiBi slope of the head is read once the first tile requests are on their way (read_slope below): it is a
-    // vector load, the wait for it counts every older request as well, and nothing before the first softmax needs it.
+    // The ALiBi slope of the head is read once the first tile requests are on their way (read_slope below): nothing before the
+    // first softmax needs it.  Narrow: by the scalar unit, whose loads have a count of their own; the wait for a vector load takes in
+    // every tile request, V(1) among them (causal B1 H8 N1021 d63 12.8 -> 10.9 us, d31 8.7 -> 7.7, B1 H4 N600 d80 9.3 -> 8.3 together with
+    // what Q gains below).  The others wait for two tiles first anyway, and lose 1-3 % by a slope in a scalar register.
     float slope2 = 0.0f, nsig = 0.0f;
 
     // ALiBi where every visible key lies at or left of its row (causal mask, or a right window of 0: j <= i, keys right
@@ -525,7 +537,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     auto read_slope = [&]() {
         if constexpr (kAlibi) {
             // (only the kEvery instance is launched without a slope table)
-            slope2 = (!kEvery || a.alibi) ? a.alibi[a.head(bh)] * kLog2e : 0.0f;
+            slope2 = (!kEvery || a.alibi) ? (kNarrow ? read_uniform(a.alibi + a.head(bh)) : a.alibi[a.head(bh)]) * kLog2e : 0.0f;
             nsig = scale_late ? -slope2 / c2 : 0.0f;
             if constexpr (kFoldAlibi) {
 #pragma unroll
@@ -943,15 +955,59 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         // than those of tile n + 2) have been waited for.  No other wave reads or writes these buffers.
         const int nt = wave < ntiles ? (ntiles - wave + 3) / 4 : 0;
         static_assert(NKX + NVX <= 63, "vmcnt immediate");
+        // In front of tile 0 the wave waits for no more than Q, K(0) and, with two stages, V(0).  Q comes straight into LDS too: loaded
+        // into registers, it is waited for by a count that takes in every younger request, and comes in 16-byte pieces of 32 rows
+        // where these are whole ones.  With one stage it lies where V will be, whose request follows once Q is in registers (an
+        // area of its own and V requested at once: d96 -2 %, all waves' K then arrive behind some V).  With two stages V(1) goes
+        // out with the rest where rows are aligned; requests at 2-byte alignment take 15 ns per KiB and CU to issue where others take
+        // 5, so there it waits for its turn.
+        auto request = [&](int n, int stage, auto k_part) {
+            if (n < nt) dma_tile_parts(tile_begin + wave + 4 * n, stage, k_part, std::integral_constant<bool, !decltype(k_part)::value>{});
+        };
+        constexpr std::true_type k_part{};
+        constexpr std::false_type v_part{};
+        if (nt > 0) {
+            const char* const Qb = reinterpret_cast<const char*>(Qbh) + (size_t)q0 * (size_t)row_bytes;
+            const int rows_left = Nq - q0;
+            // (each offset is worked out right in front of its request; rows past Nq re-read the last one)
 #pragma unroll
-        for (int u = 0; u < NSTG; ++u)
-            if (u < nt) dma_tile(tile_begin + wave + 4 * u, u);
+            for (int i = 0; i < (NKO > C::CHK / 2 ? NKO : C::CHK / 2); ++i) {
+                if (i < NKO) k_offset(i);
+                asm volatile("" : "+v"(koff[i % NKO]));
+                if (i >= C::CHK / 2) continue;
+                const int further = i / NKO * kKeyRows;
+                const int over = max(krow[i % NKO] + further - (rows_left - 1), 0);
+                dma_kib(Qb, koff[i % NKO] + (uint32_t)__mul24(further - over, row_bytes), (FA_LDS char*)smem + kQLds + wave * kQWave + i * 1024);
+            }
+            request(0, 0, k_part);
+            if constexpr (NSTG == 2) {
+                request(0, 0, v_part);
+                request(1, 1, k_part);
+                if constexpr (kVec) request(1, 1, v_part);
+            }
+        }
         stamps.take(1);
         if constexpr (kStamp) __builtin_amdgcn_sched_barrier(0);  // (ahead of the work on Q, whose wait drains the requests too)
         set_bounds();
         read_slope();
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (NSTG == 2 && nt > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NKX + (kVec ? NVX : 0)) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        {
+            const char* const qbase = smem + kQLds + wave * kQWave + k_rd;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const v4u raw = *reinterpret_cast<const v4u*>(qbase + k_step(ks));
+                const int col = 16 * ks + 8 * g;
+                const v4u z = {0u, 0u, 0u, 0u};
+                union { v4u u; v8h h; } t;
+                t.u = kFullD || 16 * ks + 16 <= D - 32 || col < d ? raw : z;
+                // (d > D - 32: the columns before are all there)
+                qf[0][ks] = kVec || 16 * ks + 16 <= D - 32 ? t.h : mask_q_chunk_anyalign(raw, col, d);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
         pin_q();
+        if constexpr (NSTG == 1 || !kVec) request(NSTG - 1, NSTG - 1, v_part);
         stamps.take(2);
         stamps.take(3);  // (no barrier in front of the loop)
         if constexpr (kAheadQk) {
@@ -959,16 +1015,15 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
             // are on their way, K(n + 3) and V(n + 2) are requested.
             v16f s[2][NB];
             v8h none[2][2][NB];
-            auto request = [&](int n, int stage, auto k_part) {
-                if (n < nt) dma_tile_parts(tile_begin + wave + 4 * n, stage, k_part, std::integral_constant<bool, !decltype(k_part)::value>{});
-            };
             if (nt == 1) {  // (no successor whose scores could be worked out)
                 tile_math(wave, 0);
                 stamps.take(4);
             } else if (nt > 1) {
                 qk(0, s);
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                request(2, 0, std::true_type{});
+                request(2, 0, k_part);
+                if (nt > 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NVX + NKX) : "memory");  // K(1)
+                else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NVX) : "memory");
                 int buf = 0, n = 0;
                 do {
                     const int t = wave + 4 * n;
@@ -976,8 +1031,8 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                     tile_with_scores_ahead(buf, buf ^ 1, s);
                     if (kStamp && n == 0) stamps.take(4);
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                    request(n + 2, buf, std::false_type{});
-                    request(n + 3, buf ^ 1, std::true_type{});
+                    request(n + 2, buf, v_part);
+                    request(n + 3, buf ^ 1, k_part);
                     if (n + 3 < nt) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NKX + NVX) : "memory");
                     else if (n + 2 < nt) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NVX) : "memory");
                     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1467,7 +1522,7 @@ inline hipError_t launch_fwd_narrow_instance(const FwdArgs& a, hipStream_t st)
     using C = FwdCfg<D, 1, true, (VAR & kVarShort) != 0>;
     auto kern = fwd_kernel<D, 1, VAR | kVarNarrow>;
     static DeviceFlags attr_done;  // per instantiation and device
-    constexpr int smem = 4 * (D <= 64 ? 2 : 1) * (C::KBUF + C::VBUF);  // two stages per wave up to D = 64, one above
+    constexpr int smem = 4 * (D <= 64 ? 2 : 1) * (C::KBUF + C::VBUF) + (C::kQApart ? 4 * 32 * C::SK : 0);  // two stages per wave up to D = 64, one above
     if (hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), smem, attr_done); e != hipSuccess) return e;
     FwdArgs b = a;
     b.Tr = (a.Nq + 31) / 32;
