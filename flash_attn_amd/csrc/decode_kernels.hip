@@ -17,11 +17,24 @@
 
 namespace fa {
 
-// Arguments of the decode kernel: see Packed in common.h
+// Arguments of the decode kernel: at most 112 bytes, see Packed in common.h.  What every address depends on has words of its own where
+// there is room, without ALiBi: cut out of `shifts`, d and num_splits cost each launch 0.04 us of GPU time that nothing hides (B1 H32
+// Nk2048 d128 9.90 -> 9.85 us, Nk4096 d64 10.11 -> 10.07, B5 H4 Nk256 d128 5.64 -> 5.56; FwdArgs itself, 272 bytes, is a further 0.05 faster
+// where the GPU is the bound and 0.1 slower where the host is: B1 H4 Nk300 d64 5.4 -> 5.55).
+struct DecodeOwn {
+    int d, num_splits;
+};
+struct DecodeHeads {
+    int H;
+    uint32_t mul_heads;
+};
+template <bool kAlibi>
 struct DecodeArgs {
-    uint32_t mul_slices, mul_kv, mul_heads;
+    uint32_t mul_slices, mul_kv;
     uint32_t shifts;  // of by_slices, by_kv_group, by_heads: five bits each; d, num_splits: eight bits each; bit 31: combine_waves is 4
-    int slices, H, Nk, wl, keys_per_split;  // slices: groups of G query heads
+    int slices;       // groups of G query heads
+    std::conditional_t<kAlibi, DecodeHeads, DecodeOwn> own;
+    int Nk, wl, keys_per_split;
     float scale_log2;
     const half_t *Q, *K, *V;
     half_t* O;
@@ -29,30 +42,44 @@ struct DecodeArgs {
     uint32_t* counters;
     const float* alibi;
 };
-static_assert(sizeof(DecodeArgs) <= kCheapArgs, "cheap launches");
-static DecodeArgs decode_args(const FwdArgs& a, int slices)
+static_assert(sizeof(DecodeArgs<true>) <= kCheapArgs && sizeof(DecodeArgs<false>) <= kCheapArgs, "cheap launches");
+template <bool kAlibi>
+static DecodeArgs<kAlibi> decode_args(const FwdArgs& a, int slices)
 {
-    return {a.by_slices.mul, a.by_kv_group.mul, a.by_heads.mul,
-            a.by_slices.shift | a.by_kv_group.shift << 5 | a.by_heads.shift << 10 | (uint32_t)a.d << 15 | (uint32_t)a.num_splits << 23 |
-                (a.combine_waves == 4 ? 1u << 31 : 0u),
-            slices, a.H, a.Nk, a.wl, a.keys_per_split, a.scale_log2, a.Q, a.K, a.V, a.O, a.LSE, a.O_partial, a.LSE_partial, a.counters, a.alibi};
+    DecodeArgs<kAlibi> p{};
+    p.mul_slices = a.by_slices.mul, p.mul_kv = a.by_kv_group.mul, p.slices = slices;
+    p.shifts = a.by_slices.shift | a.by_kv_group.shift << 5 | a.by_heads.shift << 10 | (uint32_t)a.d << 15 | (uint32_t)a.num_splits << 23 |
+               (a.combine_waves == 4 ? 1u << 31 : 0u);
+    if constexpr (kAlibi) p.own = {a.H, a.by_heads.mul};
+    else p.own = {a.d, a.num_splits};
+    p.Nk = a.Nk, p.wl = a.wl, p.keys_per_split = a.keys_per_split, p.scale_log2 = a.scale_log2;
+    p.Q = a.Q, p.K = a.K, p.V = a.V, p.O = a.O, p.LSE = a.LSE, p.O_partial = a.O_partial, p.LSE_partial = a.LSE_partial;
+    p.counters = a.counters, p.alibi = a.alibi;
+    return p;
 }
-__device__ __forceinline__ FwdArgs unpacked(const DecodeArgs& p)
+template <bool kAlibi>
+__device__ __forceinline__ FwdArgs unpacked(const DecodeArgs<kAlibi>& p)
 {
     FwdArgs a{};
     auto div = [&](uint32_t mul, int k) __attribute__((always_inline)) { return FastDiv{mul, p.shifts >> (5 * k) & 31u}; };
-    a.by_slices = div(p.mul_slices, 0), a.by_kv_group = div(p.mul_kv, 1), a.by_heads = div(p.mul_heads, 2);
-    a.d = p.shifts >> 15 & 255u, a.num_splits = p.shifts >> 23 & 255u, a.combine_waves = p.shifts >> 31 ? 4 : 1;
-    a.H = p.H, a.Nk = p.Nk, a.wl = p.wl, a.keys_per_split = p.keys_per_split, a.scale_log2 = p.scale_log2;
+    a.by_slices = div(p.mul_slices, 0), a.by_kv_group = div(p.mul_kv, 1);
+    a.combine_waves = p.shifts >> 31 ? 4 : 1;
+    if constexpr (kAlibi) {
+        a.d = p.shifts >> 15 & 255u, a.num_splits = p.shifts >> 23 & 255u;
+        a.H = p.own.H, a.by_heads = div(p.own.mul_heads, 2), a.alibi = p.alibi;
+    } else {
+        a.d = p.own.d, a.num_splits = p.own.num_splits;
+    }
+    a.Nk = p.Nk, a.wl = p.wl, a.keys_per_split = p.keys_per_split, a.scale_log2 = p.scale_log2;
     a.Q = p.Q, a.K = p.K, a.V = p.V, a.O = p.O, a.LSE = p.LSE, a.O_partial = p.O_partial, a.LSE_partial = p.LSE_partial;
-    a.counters = p.counters, a.alibi = p.alibi;
+    a.counters = p.counters;
     return a;
 }
 
 // G = query heads served by one work-group: the G consecutive heads share one K/V head (grouped-query attention), so
 // the K/V stream is read once for all of them.  G == 1 is the plain one-K/V-head-per-query-head case.
 template <int LPK, bool kAlibi, int G>
-__global__ void __launch_bounds__(256) decode_split_kernel(const DecodeArgs packed_args)
+__global__ void __launch_bounds__(256) decode_split_kernel(const DecodeArgs<kAlibi> packed_args)
 {
     const FwdArgs a = unpacked(packed_args);
     constexpr int KPI = 64 / LPK;      // keys per wave instruction
@@ -285,8 +312,8 @@ static hipError_t launch_decode_instance(const FwdArgs& a, hipStream_t st)
     const unsigned groups = (unsigned)(slices * a.num_splits);
     FwdArgs b = a;
     set_divisors(b, slices);
-    if (a.alibi != nullptr) return launch_kernel(decode_split_kernel<LPK, true, G>, dim3(groups), dim3(256), 0, st, decode_args(b, (int)slices));
-    return launch_kernel(decode_split_kernel<LPK, false, G>, dim3(groups), dim3(256), 0, st, decode_args(b, (int)slices));
+    if (a.alibi != nullptr) return launch_kernel(decode_split_kernel<LPK, true, G>, dim3(groups), dim3(256), 0, st, decode_args<true>(b, (int)slices));
+    return launch_kernel(decode_split_kernel<LPK, false, G>, dim3(groups), dim3(256), 0, st, decode_args<false>(b, (int)slices));
 }
 
 template <int LPK>

@@ -28,3 +28,15 @@ def test_arguments_are_few():
             seen += 1
             assert fields["kernarg_segment_size"] <= 112, (name, fields["kernarg_segment_size"])
     assert seen > 100
+
+
+def test_decode_addresses_wait_for_no_bit_field():
+    """What the first addresses of the decode kernel need has words of its own where there is room for them: without ALiBi nothing but
+    shift counts, which shifts take as they are, is cut out of a word before the first request."""
+    seen = 0
+    for name, body in mc.kernels(LIBRARY):
+        if re.match(r".*decode_split_kernelILi\d+ELb0E", name):
+            seen += 1
+            first = next(i for i, (m, _) in enumerate(body) if m.startswith("global_load"))
+            assert not [x for x in body[:first] if x[0].startswith("s_bfe")], name
+    assert seen == 12
