@@ -1,7 +1,7 @@
 // Split-KV decode (one query row per head), split combine, and the stand-alone dropout keep-mask kernel.
 //
-// decode_split_kernel replaces forward_kernel_splitkv (src/flash_forward_splitkv.h:14-344) for Nq == 1, where the
-// reference's 128-row MMA tile would waste 127 of 128 rows: the work is a pure stream over K and V, bound by HBM.
+// decode_split_kernel and decode_stream_kernel (the same with longer arguments) replace forward_kernel_splitkv (src/flash_forward_splitkv.h:14-344)
+// for Nq == 1, where the reference's 128-row MMA tile would waste 127 of 128 rows: the work is a pure stream over K and V, bound by HBM.
 //   * one work-group per (head slice, split) -- per (G query heads of one K/V head, split) under grouped-query
 //     attention, so that K and V are streamed once per K/V head; its 4 waves take blocks of the split's keys in turn
 //   * a key row is spread over LPK lanes (16 bytes each), so one wave instruction reads 1 KiB of consecutive bytes
@@ -17,10 +17,12 @@
 
 namespace fa {
 
-// Arguments of the decode kernel: at most 112 bytes, see Packed in common.h.  What every address depends on has words of its own where
-// there is room, without ALiBi: cut out of `shifts`, d and num_splits cost each launch 0.04 us of GPU time that nothing hides (B1 H32
-// Nk2048 d128 9.90 -> 9.85 us, Nk4096 d64 10.11 -> 10.07, B5 H4 Nk256 d128 5.64 -> 5.56; FwdArgs itself, 272 bytes, is a further 0.05 faster
-// where the GPU is the bound and 0.1 slower where the host is: B1 H4 Nk300 d64 5.4 -> 5.55).
+// Arguments of the decode kernel.  What every address depends on has words of its own where there is room, without ALiBi: cut out of
+// `shifts`, d and num_splits cost each launch 0.04 us of GPU time that nothing hides.  112 bytes are what the host passes on fastest
+// (see Packed in common.h), but launches of a busy GPU follow each other 0.15-0.2 us faster where the arguments take more than 128
+// (120 and 128 like 112; 192, 256 and 272 alike): so launches that the GPU bounds, from 4 MiB of K and V on, get 192.  112 / 192 bytes: 2 MiB B1
+// H8 Nk512 d128 5.48 / 5.56 us, 0.3 MiB B1 H4 Nk300 d64 5.41 / 5.53, 4 MiB B1 H16 Nk512 d128 5.90 / 5.90, 6 MiB Nk768 6.55 / 6.42, 10 MiB B4 H8 Nk640
+// 6.70 / 6.48, 7.8 MiB B2 H8 Nk2000 d64 7.75 / 7.74, 9.4 MiB B1 H32 Nk1200 d64 6.55 / 6.36, Nk2048 d128 9.94 / 9.75, Nk4096 d128 14.59 / 14.41.
 struct DecodeOwn {
     int d, num_splits;
 };
@@ -42,6 +44,11 @@ struct DecodeArgs {
     uint32_t* counters;
     const float* alibi;
 };
+template <bool kAlibi>
+struct DecodeStreamArgs : DecodeArgs<kAlibi> {
+    uint32_t unused[20];
+};
+static_assert(sizeof(DecodeStreamArgs<true>) == 192 && sizeof(DecodeStreamArgs<false>) == 192, "more than 128 bytes");
 static_assert(sizeof(DecodeArgs<true>) <= kCheapArgs && sizeof(DecodeArgs<false>) <= kCheapArgs, "cheap launches");
 template <bool kAlibi>
 static DecodeArgs<kAlibi> decode_args(const FwdArgs& a, int slices)
@@ -78,8 +85,8 @@ __device__ __forceinline__ FwdArgs unpacked(const DecodeArgs<kAlibi>& p)
 
 // G = query heads served by one work-group: the G consecutive heads share one K/V head (grouped-query attention), so
 // the K/V stream is read once for all of them.  G == 1 is the plain one-K/V-head-per-query-head case.
-template <int LPK, bool kAlibi, int G>
-__global__ void __launch_bounds__(256) decode_split_kernel(const DecodeArgs<kAlibi> packed_args)
+template <int LPK, int G, bool kAlibi>
+__device__ __forceinline__ void decode_split(const DecodeArgs<kAlibi>& packed_args)
 {
     const FwdArgs a = unpacked(packed_args);
     constexpr int KPI = 64 / LPK;      // keys per wave instruction
@@ -268,6 +275,17 @@ __global__ void __launch_bounds__(256) decode_split_kernel(const DecodeArgs<kAli
     }
 }
 
+template <int LPK, bool kAlibi, int G>
+__global__ void __launch_bounds__(256) decode_split_kernel(const DecodeArgs<kAlibi> args)
+{
+    decode_split<LPK, G>(args);
+}
+template <int LPK, bool kAlibi, int G>
+__global__ void __launch_bounds__(256) decode_stream_kernel(const DecodeStreamArgs<kAlibi> args)
+{
+    decode_split<LPK, G, kAlibi>(args);
+}
+
 // one wave per query row, or one work-group (W = 4)
 template <int W>
 __global__ void __launch_bounds__(256) combine_kernel(const float* __restrict__ O_partial,
@@ -312,8 +330,15 @@ static hipError_t launch_decode_instance(const FwdArgs& a, hipStream_t st)
     const unsigned groups = (unsigned)(slices * a.num_splits);
     FwdArgs b = a;
     set_divisors(b, slices);
-    if (a.alibi != nullptr) return launch_kernel(decode_split_kernel<LPK, true, G>, dim3(groups), dim3(256), 0, st, decode_args<true>(b, (int)slices));
-    return launch_kernel(decode_split_kernel<LPK, false, G>, dim3(groups), dim3(256), 0, st, decode_args<false>(b, (int)slices));
+    const long long keys = a.wl >= 0 && a.wl < a.Nk ? a.wl + 1 : a.Nk;
+    const bool stream = 4 * keys * a.d * a.B * a.Hk >= 4 << 20;  // bytes of K and V
+    auto launch = [&](auto alibi) {
+        constexpr bool kAlibi = decltype(alibi)::value;
+        const DecodeArgs<kAlibi> args = decode_args<kAlibi>(b, (int)slices);
+        if (stream) return launch_kernel(decode_stream_kernel<LPK, kAlibi, G>, dim3(groups), dim3(256), 0, st, DecodeStreamArgs<kAlibi>{args, {}});
+        return launch_kernel(decode_split_kernel<LPK, kAlibi, G>, dim3(groups), dim3(256), 0, st, args);
+    };
+    return a.alibi != nullptr ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
 template <int LPK>
