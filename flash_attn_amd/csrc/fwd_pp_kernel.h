@@ -71,6 +71,7 @@ template <int D, int VAR>
 __global__ void __launch_bounds__(512, 2) fwd_pp_kernel(const KernelArgs<VAR> packed_args)
 {
     const FwdArgs a = unpacked<false>(packed_args);
+    ask_for_all_arguments<VAR>(a);
     constexpr bool kAlibi = (VAR & kVarAlibi) != 0, kDropout = (VAR & kVarDropout) != 0, kStamp = (VAR & kVarStamp) != 0,
                    kFullD = (VAR & kVarFullD) != 0;
     using C = PPCfg<D>;

@@ -40,3 +40,35 @@ def test_decode_addresses_wait_for_no_bit_field():
             first = next(i for i, (m, _) in enumerate(body) if m.startswith("global_load"))
             assert not [x for x in body[:first] if x[0].startswith("s_bfe")], name
     assert seen == 12
+
+
+def argument_lines(body):
+    """64-byte lines of the arguments that scalar loads ask for before the first wait for scalar loads, and behind it."""
+    first, later, waited = set(), set(), False
+    for m, text in body:
+        if m.startswith("s_load_dword"):
+            target, base, offset = (x.strip() for x in text.split(",")[:3])
+            if base != "s[0:1]":
+                continue
+            words = int(m.removeprefix("s_load_dword").removeprefix("x") or 1)
+            lines = range(int(offset, 0) // 64, (int(offset, 0) + 4 * words - 1) // 64 + 1)
+            (later if waited else first).update(lines)
+            if mc.registers(target) & {("s", 0), ("s", 1)}:
+                break
+        elif m == "s_waitcnt" and "lgkmcnt" in text:
+            waited = True
+    return first, later
+
+
+def test_no_line_of_the_arguments_comes_late():
+    """No tiled kernel asks for a line of its arguments for the first time once it has waited for others (ALiBi and dropout together, the
+    instances that serve every request and the instrumented twins apart)."""
+    seen = 0
+    for name, body in mc.kernels(LIBRARY):
+        m = re.match(r".*fwd_(?:pp_)?kernelILi\d+E(?:Li\d+E)?Li(\d+)EEE", name)
+        if not m or int(m[1]) & (lr.STAMP | lr.EVERY) or int(m[1]) & (lr.ALIBI | lr.DROPOUT) == lr.ALIBI | lr.DROPOUT:
+            continue
+        seen += 1
+        first, later = argument_lines(body)
+        assert later <= first, (name, first, later)
+    assert seen > 100
