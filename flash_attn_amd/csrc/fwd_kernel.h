@@ -603,12 +603,18 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // S^T = K Q^T of the tile in K buffer `buf`
     auto qk = [&](int buf, v16f (&s)[2][NB]) {
         constexpr bool folded = kFoldAlibi;
+        constexpr bool kInOrder = NB == 1 && (folded || (D == 32 && !kAlibi && !kDropout && !kNarrow && !kPair && !kFullD));
         const char* kbase = Ks + buf * C::KBUF + k_rd;
-        if constexpr (folded && NB == 1) {
-            // The first k-step's MFMAs are inline asm here (below), which the issue-order groups at the end of this
-            // function cannot name: with them in the stream the compiler fell back to waiting for every fragment right
-            // behind its request.  So this instance is written out in issue order, fenced step by step: three fragments
-            // ahead, then MFMA and read in turn.
+        // Written out in issue order, fenced step by step -- three fragments ahead, then MFMA and read in turn -- where the issue-order
+        // groups at the end of this function do not do:
+        //  * with the bias in the accumulator the first k-step's MFMAs are inline asm (below), which the groups cannot name: with
+        //    them in the stream the compiler fell back to waiting for every fragment right behind its request;
+        //  * at D = 32, where there are four MFMAs, the groups are lost in the plain instances as soon as what is around them changes,
+        //    and the compiler requests two fragments, waits for both, and does the same again.  So -> written out: causal B5 H2 Nq60 Nk5905 d31
+        //    (split) 11.0 -> 10.85 us, B1 H8 Nq200 Nk8000 d31 (split) 13.85 -> 13.5, B8 H16 N2000 d31 window of 128 keys 20.4 -> 20.2, causal B4
+        //    H16 N700 d24 9.40 -> 9.27.  Rows of the bucket's width hide the waits behind other waves, and lose 1-2 % by the
+        //    fences (B15 H64 H_kv8 N107 d32 7.25 -> 7.39, B4 H8 N2000 32.1 -> 32.5); the paired and narrow ones have their order.
+        if constexpr (kInOrder) {
             constexpr int n = 2 * KS, kAhead = 3;  // step i: k-step i / 2, key block i % 2
             v8h af[n];
 #pragma unroll
@@ -617,8 +623,12 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
 #pragma unroll
             for (int i = 0; i < n; ++i) {
                 const int ks = i >> 1, kb = i & 1;
-                if (ks == 0) asm("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(s[kb][0]) : "v"(af[i]), "v"(qf[0][ks]), "v"(calib));
-                else s[kb][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], qf[0][ks], s[kb][0], 0, 0, 0);
+                const v16f z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+                if constexpr (folded) {
+                    if (ks == 0) asm("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(s[kb][0]) : "v"(af[i]), "v"(qf[0][ks]), "v"(calib));
+                }
+                if (ks == 0 && !folded) s[kb][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], qf[0][ks], z, 0, 0, 0);
+                if (ks > 0) s[kb][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], qf[0][ks], s[kb][0], 0, 0, 0);
                 if (i + kAhead < n)
                     af[i + kAhead] = *reinterpret_cast<const v8h*>(kbase + ((i + kAhead) & 1) * 32 * SK + k_step((i + kAhead) >> 1));
                 __builtin_amdgcn_sched_barrier(0);

@@ -82,3 +82,29 @@ def test_registers_suffice():
     spills = [name for name, m in kernels.items() if m["private_segment_fixed_size"] or m["vgpr_spill_count"]]
     variant = {name: int(re.match(r".*fwd_(?:pp_)?kernelILi\d+E(?:Li\d+E)?Li(\d+)EEE", name)[1]) for name in spills}
     assert len(kernels) > 300 and not [name for name in spills if not variant[name] & (lr.EVERY | lr.STAMP)], spills
+
+
+def waits_at_products(body):
+    """How often a fragment's read is followed by a wait for every read and the MFMA that takes it, nothing in between: the latency of LDS
+    with nothing beside it."""
+    kinds = []
+    for m, text in body:
+        if m.startswith("v_mfma"):
+            kinds.append("M")
+        elif m == "ds_read_b128":
+            kinds.append("r")
+        elif m == "s_waitcnt" and "lgkmcnt" in text:
+            kinds.append("0" if "lgkmcnt(0)" in text else "w")
+    return len(re.findall("rw?0M", "".join(kinds)))
+
+
+def test_fragments_are_asked_for_ahead():
+    """The plain instances of the 32-column bucket for rows shorter than it, whose tile is four products of K and Q, ask for three
+    fragments before the first product and wait for none alone."""
+    assert waits_at_products([("ds_read_b128", "v[0:3], v9"), ("s_waitcnt", "lgkmcnt(0)"), ("v_mfma_f32_32x32x16_f16", "")]) == 1
+    found = {}
+    for name, body in mc.kernels(LIBRARY):
+        m = re.match(r".*fwd_kernelILi32ELi1ELi(\d+)EEE", name)
+        if m and int(m[1]) in (0, lr.VEC, lr.FOLD, lr.FOLD | lr.VEC):
+            found[int(m[1])] = waits_at_products(body)
+    assert found == {0: 0, lr.VEC: 0, lr.FOLD: 0, lr.FOLD | lr.VEC: 0}
