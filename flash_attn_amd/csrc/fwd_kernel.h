@@ -225,8 +225,12 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     constexpr int BRW = kNarrow ? 32 : C::BR;  // query rows per work-group
     // Narrow: Q is fetched like the first 32 rows of a K tile, so that the wave's first wait is for Q and tile 0 alone.  Loaded into
     // registers -> so: B1 H8 N1021 d31 8.0 -> 7.3 us, d63 11.5 -> 10.2, N1024 d64 7.2 -> 7.0, N2048 causal d64 14.4 -> 13.9, N1024
-    // d128 10.8 -> 10.1, N300 d128 7.3 -> 6.75, B1 H2 N3000 d111 33.1 -> 31.9, d72, d80 and one or two tiles per wave +-1 %; d96
-    // -1 ... -2 % (8.5 -> 8.6, as much as the same code around the old loads), left as it is.
+    // d128 10.8 -> 10.1, N300 d128 7.3 -> 6.75, B1 H2 N3000 d111 33.1 -> 31.9, d72, d80 and one or two tiles per wave +-1 %.  Whole rows of 96
+    // without bias keep the loads (kQLoads), with V of tile 0 requested at once: the other way it leaves only once Q is there, which costs launches
+    // of few tiles more than the rest gain (Q like a tile / loads: causal B14 H4 N120 4.89 / 4.73 us, B3 H3 N194 4.80 / 4.71, B1 H8 N400 6.00 / 5.94,
+    // with dropout N640 8.48 / 8.42; unmasked N120 4.84 / 4.68, N256 4.75 / 4.81, N1024 7.87 / 7.83, B1 H4 N2000 12.16 / 12.29).  With a bias the
+    // scalar load of the slope gains by the shorter first wait: causal B1 H4 N600 7.60 against 7.84.
+    constexpr bool kQLoads = kNarrow && D == 96 && kFullD && !kAlibi;
     // Where to, and bytes from one wave's to the next one's
     constexpr bool kQApart = C::kQApart;
     constexpr int kQWave = kQApart ? 32 * C::SK : NSTG * (C::KBUF + C::VBUF);
@@ -346,7 +350,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // ---- Q fragments (B operand of S^T = K Q^T): lane holds row l32, columns 16*ks + 8*g .. +7
     v8h qf[NB][KS];
 #pragma unroll
-    for (int nb = 0; nb < NB && !kNarrow; ++nb) {
+    for (int nb = 0; nb < NB && (!kNarrow || kQLoads); ++nb) {
         const int ic = row_i[nb] < Nq ? row_i[nb] : Nq - 1;
         const half_t* qrow = Qbh + (size_t)ic * d;
         if constexpr (kVec) {
@@ -450,7 +454,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     };
     if constexpr (kDma) {
 #pragma unroll
-        for (int i = 0; i < NKO && !kNarrow; ++i) k_offset(i);  // (narrow: request by request, below)
+        for (int i = 0; i < NKO && (!kNarrow || kQLoads); ++i) k_offset(i);  // (narrow: request by request, below)
 #pragma unroll
         for (int i = 0; i < NVO; ++i) {
             const int q = 64 * block_of(i) + lane;
@@ -546,6 +550,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // -nsig * (8 (r / 4) + r % 4), and a part per lane and 32-key block.  The first goes into the MFMA as the initial
     // accumulator value, the second into the addend of the exponent fma: no instruction per score is left.
     constexpr bool kFoldAlibi = kAlibi && kVec && (VAR & kVarAlibiLeft) != 0;
+    static_assert(!kAheadQk || !kFoldAlibi, "scores worked out ahead start from zero");
     v16f calib;
     auto read_slope = [&]() {
         if constexpr (kAlibi) {
@@ -989,15 +994,21 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         };
         constexpr std::true_type k_part{};
         constexpr std::false_type v_part{};
-        if (nt > 0) {
+        if constexpr (kQLoads) {
+            // (written as for any number of stages: as one statement the compiler puts the address arithmetic between the
+            // requests, and N1024 takes 8.12 us instead of 7.83)
+#pragma unroll
+            for (int u = 0; u < NSTG; ++u)
+                if (u < nt) dma_tile(tile_begin + wave + 4 * u, u);
+        } else if (nt > 0) {
             const char* const Qb = reinterpret_cast<const char*>(Qbh) + (size_t)q0 * (size_t)row_bytes;
             const int rows_left = Nq - q0;
+            static_assert(NKO <= C::CHK / 2, "offsets");
             // (each offset is worked out right in front of its request; rows past Nq re-read the last one)
 #pragma unroll
-            for (int i = 0; i < (NKO > C::CHK / 2 ? NKO : C::CHK / 2); ++i) {
+            for (int i = 0; i < C::CHK / 2; ++i) {
                 if (i < NKO) k_offset(i);
                 asm volatile("" : "+v"(koff[i % NKO]));
-                if (i >= C::CHK / 2) continue;
                 const int further = i / NKO * kKeyRows;
                 const int over = max(krow[i % NKO] + further - (rows_left - 1), 0);
                 dma_kib(Qb, koff[i % NKO] + (uint32_t)__mul24(further - over, row_bytes), (FA_LDS char*)smem + kQLds + wave * kQWave + i * 1024);
@@ -1015,7 +1026,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         read_slope();
         if (NSTG == 2 && nt > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NKX + (kVec ? NVX : 0)) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        {
+        if constexpr (!kQLoads) {
             const char* const qbase = smem + kQLds + wave * kQWave + k_rd;
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
@@ -1030,7 +1041,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         }
         pin_q();
-        if constexpr (NSTG == 1 || !kVec) request(NSTG - 1, NSTG - 1, v_part);
+        if constexpr (!kQLoads && (NSTG == 1 || !kVec)) request(NSTG - 1, NSTG - 1, v_part);
         stamps.take(2);
         stamps.take(3);  // (no barrier in front of the loop)
         if constexpr (kAheadQk) {
