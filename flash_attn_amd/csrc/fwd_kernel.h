@@ -181,11 +181,26 @@ constexpr int fwd_groups_per_cu(int D, int NB, int VAR)
     return NB == 1 && D <= 96 && (VAR & kVarEvery) == 0 ? 3 : 2;
 }
 
+// Arguments of fwd_kernel.  Two groups of instances got slower by what the compiler makes of the packed fields:
+//  * D = 96 without features: told that d and num_splits are eight bits wide it orders the work around the loop otherwise, at the same
+//    number of instructions in the loop.  Known -> not: causal B1 H64 H_kv8 N448 d96 9.64 -> 9.44 us, B8 H8 N200 7.26 -> 7.10, N192 6.23 -> 6.16,
+//    B14 H4 N120 d80 5.14 -> 5.07.  Narrow instances, other buckets, ALiBi and dropout stay or lose up to 3 %.
+//  * D = 32 at any alignment with ALiBi and dropout: 209 of the 321 8-byte instructions of its loop lay off 8-byte boundaries, with
+//    one more word in front of them 112: causal B2 H8 N2000 d31 41.6 -> 40.45 us.
+template <int D, int VAR>
+__device__ __forceinline__ FwdArgs fwd_arguments(const KernelArgs<VAR>& packed_args)
+{
+    FwdArgs a = unpacked<(VAR & kVarFold) != 0>(packed_args);
+    ask_for_all_arguments<VAR>(a);
+    if constexpr (D == 96 && (VAR & (kVarAlibi | kVarDropout | kVarNarrow)) == 0) asm("" : "+s"(a.d), "+s"(a.num_splits));
+    if constexpr (D == 32 && (VAR & ~kVarStamp) == (kVarAlibi | kVarDropout)) asm volatile("s_nop 0");
+    return a;
+}
+
 template <int D, int NB, int VAR>
 __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_per_cu(D, NB, VAR)) fwd_kernel(const KernelArgs<VAR> packed_args)
 {
-    const FwdArgs a = unpacked<(VAR & kVarFold) != 0>(packed_args);
-    ask_for_all_arguments<VAR>(a);
+    const FwdArgs a = fwd_arguments<D, VAR>(packed_args);
     constexpr bool kVec = (VAR & kVarVec) != 0, kAlibi = (VAR & kVarAlibi) != 0, kDropout = (VAR & kVarDropout) != 0,
                    kFullD = (VAR & kVarFullD) != 0, kStamp = (VAR & kVarStamp) != 0, kKvOnce = (VAR & kVarKvOnce) != 0;
     using C = FwdCfg<D, NB, (VAR & kVarNarrow) != 0, (VAR & kVarShort) != 0>;

@@ -50,6 +50,27 @@ def kernels(library):
                 yield name, body
 
 
+def addresses(library, pattern):
+    """[(address, mnemonic, operands)] of the one function of the library's device code whose name the pattern matches."""
+    found = []
+    with tempfile.TemporaryDirectory() as folder:
+        for n, image in enumerate(code_objects(library)):
+            path = os.path.join(folder, f"{n}.elf")
+            with open(path, "wb") as f:
+                f.write(image)
+            names = {line.split()[-1] for line in _tool("llvm-readelf", "-sW", path).splitlines() if " FUNC " in line}
+            for name in (x for x in names if re.match(pattern, x)):
+                body = []
+                for line in _tool("llvm-objdump", "-d", "--no-show-raw-insn", "--disassemble-symbols=" + name, path).splitlines():
+                    text, _, place = line.partition("//")
+                    if line.startswith("\t") and place.strip():
+                        mnemonic, _, rest = text.strip().partition(" ")
+                        body.append((int(place.split(":")[0], 16), mnemonic, rest.strip()))
+                found.append(body)
+    assert len(found) == 1, pattern
+    return found[0]
+
+
 def metadata(library):
     """Per kernel of the library: the integer fields of its metadata (vgpr_count, private_segment_fixed_size, ...)."""
     out = {}

@@ -108,3 +108,19 @@ def test_fragments_are_asked_for_ahead():
         if m and int(m[1]) in (0, lr.VEC, lr.FOLD, lr.FOLD | lr.VEC):
             found[int(m[1])] = waits_at_products(body)
     assert found == {0: 0, lr.VEC: 0, lr.FOLD: 0, lr.FOLD | lr.VEC: 0}
+
+
+def test_loop_lies_on_eight_byte_boundaries():
+    """32 columns, rows at any alignment, ALiBi and dropout: most of the 8-byte instructions of the key-tile loop lie on 8-byte boundaries."""
+    body = mc.addresses(LIBRARY, rf".*fwd_kernelILi32ELi1ELi{lr.ALIBI | lr.DROPOUT}EEE")
+    products = [at for at, m, _ in body if m.startswith("v_mfma")]
+    loops = []
+    for at, m, text in body:
+        if m.startswith(("s_branch", "s_cbranch")):
+            words = int(text.split()[0])
+            start = at + 4 + 4 * (words - 65536 if words > 32767 else words)
+            if start < at and sum(start <= x <= at for x in products) >= 8:
+                loops.append((at - start, start, at))
+    _, start, end = min(loops)
+    eight = [at for (at, _, _), (after, _, _) in zip(body, body[1:]) if start <= at <= end and after - at == 8]
+    assert len(eight) > 200 and sum(at % 8 != 0 for at in eight) <= len(eight) // 2, (len(eight), sum(at % 8 != 0 for at in eight))
