@@ -623,7 +623,8 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // S^T = K Q^T of the tile in K buffer `buf`
     auto qk = [&](int buf, v16f (&s)[2][NB]) {
         constexpr bool folded = kFoldAlibi;
-        constexpr bool kInOrder = NB == 1 && (folded || (D == 32 && !kAlibi && !kDropout && !kNarrow && !kPair && !kFullD));
+        constexpr bool kInOrder = NB == 1 && (folded || (D == 32 && !kAlibi && !kDropout && !kNarrow && !kPair && !kFullD) ||
+                                              (D == 96 && kNarrow && kAlibi && kDropout));
         const char* kbase = Ks + buf * C::KBUF + k_rd;
         // Written out in issue order, fenced step by step -- three fragments ahead, then MFMA and read in turn -- where the issue-order
         // groups at the end of this function do not do:
@@ -633,7 +634,9 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         //    and the compiler requests two fragments, waits for both, and does the same again.  So -> written out: causal B5 H2 Nq60 Nk5905 d31
         //    (split) 11.0 -> 10.85 us, B1 H8 Nq200 Nk8000 d31 (split) 13.85 -> 13.5, B8 H16 N2000 d31 window of 128 keys 20.4 -> 20.2, causal B4
         //    H16 N700 d24 9.40 -> 9.27.  Rows of the bucket's width hide the waits behind other waves, and lose 1-2 % by the
-        //    fences (B15 H64 H_kv8 N107 d32 7.25 -> 7.39, B4 H8 N2000 32.1 -> 32.5); the paired and narrow ones have their order.
+        //    fences (B15 H64 H_kv8 N107 d32 7.25 -> 7.39, B4 H8 N2000 32.1 -> 32.5); the paired and narrow ones have their order;
+        //  * nor, for the same reason, in the narrow instance of D = 96 with ALiBi and dropout: causal B1 H8 N640 9.72 -> 9.39 us, B1 H4 N1000
+        //    11.74 -> 11.31, B1 H8 N1021 without a mask 11.98 -> 11.56.
         if constexpr (kInOrder) {
             constexpr int n = 2 * KS, kAhead = 3;  // step i: k-step i / 2, key block i % 2
             v8h af[n];

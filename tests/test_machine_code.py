@@ -99,15 +99,16 @@ def waits_at_products(body):
 
 
 def test_fragments_are_asked_for_ahead():
-    """The plain instances of the 32-column bucket for rows shorter than it, whose tile is four products of K and Q, ask for three
-    fragments before the first product and wait for none alone."""
+    """Instances whose products of K and Q stand written out in issue order: plain, 32 columns, rows shorter than those; narrow, 96 columns,
+    ALiBi and dropout.  They ask for three fragments before the first product and wait for none alone."""
     assert waits_at_products([("ds_read_b128", "v[0:3], v9"), ("s_waitcnt", "lgkmcnt(0)"), ("v_mfma_f32_32x32x16_f16", "")]) == 1
+    wanted = {(32, 0), (32, lr.VEC), (32, lr.FOLD), (32, lr.FOLD | lr.VEC), (96, lr.NARROW | lr.VEC | lr.FULL_D | lr.ALIBI | lr.DROPOUT)}
     found = {}
     for name, body in mc.kernels(LIBRARY):
-        m = re.match(r".*fwd_kernelILi32ELi1ELi(\d+)EEE", name)
-        if m and int(m[1]) in (0, lr.VEC, lr.FOLD, lr.FOLD | lr.VEC):
-            found[int(m[1])] = waits_at_products(body)
-    assert found == {0: 0, lr.VEC: 0, lr.FOLD: 0, lr.FOLD | lr.VEC: 0}
+        m = re.match(r".*fwd_kernelILi(\d+)ELi1ELi(\d+)EEE", name)
+        if m and (int(m[1]), int(m[2])) in wanted:
+            found[int(m[1]), int(m[2])] = waits_at_products(body)
+    assert found == dict.fromkeys(wanted, 0)
 
 
 def test_loop_lies_on_eight_byte_boundaries():
