@@ -331,7 +331,7 @@ static hipError_t launch_decode_instance(const FwdArgs& a, hipStream_t st)
     FwdArgs b = a;
     set_divisors(b, slices);
     const long long keys = a.wl >= 0 && a.wl < a.Nk ? a.wl + 1 : a.Nk;
-    const bool stream = 4 * keys * a.d * a.B * a.Hk >= 4 << 20;  // bytes of K and V
+    const bool stream = keys * a.B * a.Hk >= ((1 << 20) + a.d - 1) / a.d;  // 4 MiB of K and V, 4 d bytes a key
     auto launch = [&](auto alibi) {
         constexpr bool kAlibi = decltype(alibi)::value;
         const DecodeArgs<kAlibi> args = decode_args<kAlibi>(b, (int)slices);
