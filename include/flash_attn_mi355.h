@@ -112,7 +112,10 @@ typedef struct flash_params {
      * without the buffer, with the instrumented twin of the same kernel instance: same split count, same work-groups, same
      * results bit by bit.  Where the waves of a work-group share out its key tiles (see kernel_hint) the readings are those of
      * its first wave, which has every fourth or every other tile; with 32 rows per work-group there is no barrier in front of
-     * the loop, and reading 3 follows reading 2.  With a split count above 1 the combine step is not stamped.  The only instrumentation of the reference is the event
+     * the loop and the requests go out in steps: reading 1 is taken once Q and K of the wave's first tile are requested (up to 64
+     * columns its V and K of the second tile as well), reading 2 once Q is in registers and that K has landed, reading 3 right
+     * after it, reading 4 behind the first whole tile, which at 33 to 64 columns without dropout takes in the scores of the
+     * second.  With a split count above 1 the combine step is not stamped.  The only instrumentation of the reference is the event
      * pair around its launches (src/main.cu:195-213). */
     uint64_t *stage_stamps_out;
     /* Optional: device memory of split_counters_len 32-bit words, all zero, which lets flash_forward_splitkv merge the
