@@ -109,11 +109,13 @@ inline void set_divisors(FwdArgs& b, long long slices)
     b.by_fold = fast_div(b.fold_rows);
 }
 
-// ---- FwdArgs as the tiled kernels get it.  A launch takes the longer the more its arguments are: what an otherwise host-bound
-// stream of launches needs per launch is 2.62 ... 2.72 us with 32 ... 112 bytes, 3.24 with 128, 3.35 with the 272 bytes of FwdArgs (an empty
-// kernel, sizes in random order).  FwdArgs -> packed, B5 H4 Nq1 Nk256 d128 6.01 -> 5.68 us, B8 H8 H_kv1 Nq1 Nk812 d96 (two launches)
-// 9.25 -> 8.65, B1 H2 N128 d64 4.94 -> 4.79; long launches +-0.  So the kernels get 108 bytes, narrow fields packed, and unpack them at their start; what only
-// ALiBi, dropout and debug outputs need follows in PackedMore.  Split launches find their partial results where the others have O and LSE.
+// ---- FwdArgs as the tiled kernels get it.  A launch takes the host the longer the more its arguments are: back to back an empty
+// kernel takes 2.6 us with 32 ... 112 bytes, 3.5-3.7 with 120 ... 272 (sizes in random order).  So the kernels get 112 bytes,
+// narrow fields packed, and unpack them at their start; what only ALiBi, dropout and debug outputs need follows in
+// PackedMore, 184 bytes.  FwdArgs (272 bytes) -> packed: B1 H2 N64 d64 3.65 -> 3.44 us, N128 d32 3.75 -> 3.55, B1 H8 N200 d64 4.5 -> 4.3 (medians; the runs spread by 10-20 %);
+// where the GPU is the bound a launch of up to 128 bytes starts 0.15-0.2 us later behind the one before than a longer
+// one (the decode kernel goes by that, decode_kernels.hip), 1 % of a launch of 20 us.  Split launches find their partial
+// results where the others have O and LSE.
 // (The words that tell a work-group its place in the order come first: one scalar load.)
 struct Packed {
     int snake_end, slice_chunk, Tr;
