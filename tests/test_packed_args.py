@@ -20,7 +20,8 @@ def test_round_trip(tmp_path):
 
 
 def test_arguments_are_few():
-    """112 bytes at most, hidden arguments included, for every kernel without ALiBi, dropout and debug outputs, and for decode."""
+    """112 bytes at most, hidden arguments included, for every kernel without ALiBi, dropout and debug outputs, and for decode below the
+    line from which on its launches get more on purpose."""
     seen = 0
     for name, fields in mc.metadata(LIBRARY).items():
         m = re.match(r".*fwd_(?:pp_)?kernelILi\d+E(?:Li\d+E)?Li(\d+)EEE", name)
