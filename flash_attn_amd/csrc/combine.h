@@ -55,6 +55,19 @@ __device__ __forceinline__ void store_partial(float* p, float v, bool shared)
     if (shared) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else *p = v;
 }
+// four columns on a 16-byte boundary
+__device__ __forceinline__ void store_partial4(float* p, v4f v, bool shared)
+{
+    if (shared) {
+        union { v4f f; uint64_t u[2]; } r;
+        r.f = v;
+        uint64_t* const q = reinterpret_cast<uint64_t*>(p);
+        __hip_atomic_store(q, r.u[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(q + 1, r.u[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+        *reinterpret_cast<v4f*>(p) = v;
+    }
+}
 // Called by every thread of the work-group, behind its last store_partial; `flag` is an LDS word nobody else uses.
 __device__ __forceinline__ bool last_to_arrive(uint32_t* counter, int num_splits, int* flag)
 {

@@ -86,7 +86,7 @@ struct FwdArgs {
     FastDiv by_chunk, by_slices, by_splits, by_xcd_group, by_kv_group, by_heads;
     int fold_rows;       // > 0: the query heads of a K/V head are the rows of one problem, this many rows each (see RowSpan)
     int fold_group;      // query heads folded into one
-    FastDiv by_fold;
+    FastDiv by_fold, by_row_blocks;
     uint32_t* counters;  // nullptr, or where the work-groups of a split launch count themselves in (combine.h)
     int combine_waves;   // waves that merge a row's partial results: 1 or 4 (combine_waves_for)
     int alibi_left;      // ALiBi and no visible key lies right of its row (causal, or right window 0)
@@ -107,6 +107,7 @@ inline void set_divisors(FwdArgs& b, long long slices)
     b.by_kv_group = fast_div(b.kv_group);
     b.by_heads = fast_div(b.H);
     b.by_fold = fast_div(b.fold_rows);
+    b.by_row_blocks = fast_div(b.Tr);
 }
 
 // ---- FwdArgs as the tiled kernels get it.  A launch takes the host the longer the more its arguments are: back to back an empty
@@ -144,6 +145,58 @@ struct PackedMore : Packed {
 constexpr size_t kCheapArgs = 112;  // bytes up to which a launch costs its least
 static_assert(offsetof(Packed, scale_log2) + sizeof(float) <= kCheapArgs && sizeof(Packed) <= kCheapArgs, "cheap launches");
 static_assert(FLASH_MAX_SPLITS_K < 256, "eight bits");
+
+// Arguments of launches of few rows per slice (kVarRows of fwd_kernel.h), whose last work-groups may merge the partial results: 112 bytes
+// hold results and partial results both.  One query head per K/V head; order of the work-groups: rows_item.
+constexpr int kRowsLimit = 32;  // rows of a work-group
+struct PackedRows {
+    uint32_t mul_slices, mul_row_blocks;
+    int slices;
+    uint32_t shifts;  // of by_slices, by_row_blocks, by_kv_group (folded: by_fold): five bits each; bit 15: causal, bit 16: combine_waves is 4; fold_rows (64 at most, kFoldRows): eight bits from 24 on
+    uint32_t sizes;   // d, num_splits: eight bits each; fold_group: sixteen
+    int Nq, Nk, keys_per_split, wl, wr;
+    const half_t *Q, *K, *V;
+    half_t* O;
+    float *LSE, *O_partial, *LSE_partial;
+    uint32_t* counters;
+    uint32_t mul_kv_or_fold;
+    float scale_log2;
+};
+struct PackedRowsMore : PackedRows {
+    uint64_t* stamps;
+};
+static_assert(sizeof(PackedRows) <= kCheapArgs, "cheap launches");
+
+inline PackedRowsMore packed_rows(const FwdArgs& a)
+{
+    PackedRowsMore p{};
+    p.mul_slices = a.by_slices.mul, p.mul_row_blocks = a.by_row_blocks.mul, p.slices = a.B * a.H;
+    p.shifts = a.by_slices.shift | a.by_row_blocks.shift << 5 | (a.fold_rows ? a.by_fold : a.by_kv_group).shift << 10 | (a.causal ? 1u << 15 : 0u) | (a.combine_waves == 4 ? 1u << 16 : 0u) |
+               (uint32_t)a.fold_rows << 24;
+    p.sizes = (uint32_t)a.d | (uint32_t)a.num_splits << 8 | (uint32_t)a.fold_group << 16;
+    p.Nq = a.Nq;
+    p.Nk = a.Nk, p.keys_per_split = a.keys_per_split, p.wl = a.wl, p.wr = a.wr;
+    p.Q = a.Q, p.K = a.K, p.V = a.V, p.O = a.O, p.LSE = a.LSE, p.O_partial = a.O_partial, p.LSE_partial = a.LSE_partial;
+    p.counters = a.counters, p.mul_kv_or_fold = (a.fold_rows ? a.by_fold : a.by_kv_group).mul, p.scale_log2 = a.scale_log2;
+    p.stamps = a.stamps;
+    return p;
+}
+template <bool kFold, typename P>
+__host__ __device__ __forceinline__ FwdArgs unpacked_rows(const P& p)
+{
+    FwdArgs a{};
+    a.by_slices = FastDiv{p.mul_slices, p.shifts & 31u}, a.by_row_blocks = FastDiv{p.mul_row_blocks, p.shifts >> 5 & 31u};
+    (kFold ? a.by_fold : a.by_kv_group) = FastDiv{p.mul_kv_or_fold, p.shifts >> 10 & 31u};
+    if (kFold) a.by_kv_group = fast_div_by_one();
+    a.causal = p.shifts >> 15 & 1u, a.combine_waves = p.shifts >> 16 & 1u ? 4 : 1, a.fold_rows = p.shifts >> 24;
+    a.d = p.sizes & 255u, a.num_splits = p.sizes >> 8 & 255u, a.fold_group = p.sizes >> 16;
+    a.Nq = p.Nq, a.Tr = (p.Nq + 31) / 32, a.slice_chunk = p.slices;
+    a.Nk = p.Nk, a.keys_per_split = p.keys_per_split, a.wl = p.wl, a.wr = p.wr;
+    a.Q = p.Q, a.K = p.K, a.V = p.V, a.O = p.O, a.LSE = p.LSE, a.O_partial = p.O_partial, a.LSE_partial = p.LSE_partial;
+    a.counters = p.counters, a.scale_log2 = p.scale_log2;
+    if constexpr (sizeof(P) > sizeof(PackedRows)) a.stamps = p.stamps;
+    return a;
+}
 
 inline PackedMore packed(const FwdArgs& a)
 {
@@ -379,6 +432,26 @@ __host__ __device__ __forceinline__ WorkItem work_item(const FwdArgs& a, int blo
     it.split = split_of_rest(a, rest, &mi);
     it.m_block = a.Tr - 1 - mi;
     return it;
+}
+
+// The same of PackedRows: slices vary fastest, then splits, and the row blocks of a split, which read the same keys, run on one XCD (its
+// L2 sees them once): position p of eight neighbours takes indices 8 Tr (p / 8) + p % 8 + 8 m, the last few, that are no eight, plain order.  With
+// the row blocks slowest they were on as many XCDs as the split count made it: causal B3 H2 Nq128 Nk8000 d128 in 9 splits 20.9 -> 16.4 us.
+template <bool kOneBlock>
+__host__ __device__ __forceinline__ WorkItem rows_item(const FwdArgs& a, int block)
+{
+    int p = block, m = 0;
+    if constexpr (!kOneBlock) {
+        const int pairs = a.slice_chunk * a.num_splits, whole = pairs & ~7, q = a.by_row_blocks.quotient(block >> 3);
+        p = 8 * q + (block & 7), m = (block >> 3) - q * a.Tr;
+        if (block >= whole * a.Tr) {
+            p = block - whole * a.Tr;
+            for (m = 0; p >= pairs - whole; ++m) p -= pairs - whole;
+            p += whole;
+        }
+    }
+    const int split = a.by_slices.quotient(p);
+    return {p - split * a.slice_chunk, split, a.Tr - 1 - m};
 }
 
 // snake_end for a launch of `groups` work-groups with `resident` places on the GPU

@@ -375,7 +375,11 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
             best_s = s;
         }
     }
-    return whole ? 1 : best_s;
+    if (whole) return 1;
+    // Launches of few rows (fa::fwd_uses_rows; decode calls come here with the heads as rows) have a count of their own.  Never a higher
+    // one, and never one where the launch was whole: who brings a workspace for the estimate's count has enough for this one.
+    const int few = !every && fa::rows_form_serves(launch, tiled_variant(p)) ? fa::rows_form_splits(slices, Nq, p->d, p->Nk) : 0;
+    return few > 0 && few < best_s ? few : best_s;
 }
 
 int resolve_splits(const flash_params* p)
@@ -522,7 +526,9 @@ int run_splitkv(const flash_params* p, int splits, hipStream_t st)
     // (a slice of the decode kernel has one row per query head, which its last work-group merges in a microsecond)
     if (route == kRouteStream && splits > 1 && p->split_counters && (long long)p->B * p->H <= p->split_counters_len)
         a.counters = p->split_counters;
-    a.combine_waves = fa::combine_waves_for(splits, route == kRouteStream ? fa::decode_heads_per_group(a.kv_group) : 1);
+    const bool rows = route == kRouteTiled && !needs_every_instance(p) && fa::fwd_uses_rows(a, tiled_variant(p));
+    if (rows && splits > 1 && p->split_counters && a.Nq <= 4 && splits * p->d <= 1024 && (long long)a.B * a.H <= p->split_counters_len) a.counters = p->split_counters;
+    a.combine_waves = fa::combine_waves_for(splits, route == kRouteStream ? fa::decode_heads_per_group(a.kv_group) : rows && a.Nq <= 32 ? a.Nq : 1);
     // (a launch is limited to 2^32 - 1 threads: a work-group per row reaches 2^24 rows, a wave per row 2^26)
     if ((long long)p->B * p->H * p->Nq >= 1LL << 24) a.combine_waves = 1;
     const int e = route == kRouteStream ? record_hip(fa::launch_decode_split(a, st)) : launch_tiled(p, a, st);

@@ -28,10 +28,10 @@
 #pragma once
 #include <type_traits>
 
+#include "combine.h"
 #include "common.h"
 
 namespace fa {
-
 
 template <int D, int NB, bool kNarrow = false, bool kShort = false>
 struct FwdCfg {
@@ -147,12 +147,15 @@ constexpr float kNothingSeen = -3.402823466e38f;
 // kVarPair (without ALiBi): eight waves in two halves that take every other tile each, see kPair below.
 // kVarFold (no other feature): the rows are the query heads of a K/V head, see row_position in common.h.
 // kVarShort (D >= 64, not kVarFullD, kVarEvery or kVarFold): rows of at most D - 16 elements, see FwdCfg::kShort.
+// kVarRows (with kVarNarrow; no other feature but kVarFold): launches of few rows per slice, whole or in splits, see kRows below.
+// kVarManyRows (with kVarRows): more than 32 rows, whose row blocks ask for the same tiles.
 constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarStamp = 16, kVarAlibiLeft = 32, kVarKvOnce = 64,
-              kVarEvery = 128, kVarNarrow = 256, kVarFold = 512, kVarPair = 1024, kVarShort = 2048;
+              kVarEvery = 128, kVarNarrow = 256, kVarFold = 512, kVarPair = 1024, kVarShort = 2048, kVarRows = 4096, kVarManyRows = 8192;
 
 // arguments of an instance
 template <int VAR>
-using KernelArgs = std::conditional_t<(VAR & (kVarAlibi | kVarDropout | kVarStamp | kVarEvery)) != 0, PackedMore, Packed>;
+using KernelArgs = std::conditional_t<(VAR & kVarRows) != 0, std::conditional_t<(VAR & kVarStamp) != 0, PackedRowsMore, PackedRows>,
+                                      std::conditional_t<(VAR & (kVarAlibi | kVarDropout | kVarStamp | kVarEvery)) != 0, PackedMore, Packed>>;
 
 // The arguments take up two lines of 64 bytes, PackedMore three.  Left to the compiler nothing of the last one is asked for before the
 // work-group knows its place -- with ALiBi or dropout, before Q is on its way --, and the first tile requests wait until it has come from memory; so
@@ -190,11 +193,17 @@ constexpr int fwd_groups_per_cu(int D, int NB, int VAR)
 template <int D, int VAR>
 __device__ __forceinline__ FwdArgs fwd_arguments(const KernelArgs<VAR>& packed_args)
 {
-    FwdArgs a = unpacked<(VAR & kVarFold) != 0>(packed_args);
-    ask_for_all_arguments<VAR>(a);
-    if constexpr (D == 96 && (VAR & (kVarAlibi | kVarDropout | kVarNarrow)) == 0) asm("" : "+s"(a.d), "+s"(a.num_splits));
-    if constexpr (D == 32 && (VAR & ~kVarStamp) == (kVarAlibi | kVarDropout)) asm volatile("s_nop 0");
-    return a;
+    if constexpr ((VAR & kVarRows) != 0) {
+        const FwdArgs a = unpacked_rows<(VAR & kVarFold) != 0>(packed_args);
+        asm volatile("" : : "s"(a.scale_log2));  // (the second line of the arguments with the first)
+        return a;
+    } else {
+        FwdArgs a = unpacked<(VAR & kVarFold) != 0>(packed_args);
+        ask_for_all_arguments<VAR>(a);
+        if constexpr (D == 96 && (VAR & (kVarAlibi | kVarDropout | kVarNarrow)) == 0) asm("" : "+s"(a.d), "+s"(a.num_splits));
+        if constexpr (D == 32 && (VAR & ~kVarStamp) == (kVarAlibi | kVarDropout)) asm volatile("s_nop 0");
+        return a;
+    }
 }
 
 template <int D, int NB, int VAR>
@@ -228,6 +237,11 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // of a split -- in the same launch, where a split count of four would need the combine launch behind it.
     constexpr bool kNarrow = (VAR & kVarNarrow) != 0;
     static_assert(!kNarrow || (kDma && NB == 1 && !kKvOnce), "narrow instances");
+    // The narrow form for launches of few rows per slice (fwd_uses_rows says which), in splits too: their partial results leave the merge
+    // as whole rows of floats, and where a caller has brought counters (combine.h) and the rows are four or fewer, the last work-group
+    // of a slice merges the splits.  With up to 32 rows nobody else asks for the tiles, and the requests are non-temporal.
+    constexpr bool kRows = (VAR & kVarRows) != 0, kRowsOnce = kRows && (VAR & kVarManyRows) == 0;
+    static_assert(!kRows || (kNarrow && !kAlibi && !kDropout), "few rows");
     constexpr bool kFold = (VAR & kVarFold) != 0;
     static_assert(!kFold || (!kAlibi && !kDropout), "folded instances");
     // A launch of one work-group per CU leaves a SIMD one wave, whose score, softmax and output phases follow one another:
@@ -244,8 +258,9 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // without bias keep the loads (kQLoads), with V of tile 0 requested at once: the other way it leaves only once Q is there, which costs launches
     // of few tiles more than the rest gain (Q like a tile / loads: causal B14 H4 N120 4.89 / 4.73 us, B3 H3 N194 4.80 / 4.71, B1 H8 N400 6.00 / 5.94,
     // with dropout N640 8.48 / 8.42; unmasked N120 4.84 / 4.68, N256 4.75 / 4.81, N1024 7.87 / 7.83, B1 H4 N2000 12.16 / 12.29).  With a bias the
-    // scalar load of the slope gains by the shorter first wait: causal B1 H4 N600 7.60 against 7.84.
-    constexpr bool kQLoads = kNarrow && D == 96 && kFullD && !kAlibi;
+    // scalar load of the slope gains by the shorter first wait: causal B1 H4 N600 7.60 against 7.84.  With few rows (kRows) at D = 128, too, V goes
+    // out at once, its tiles coming from HBM: B4 H32 H_kv8 Nk8192 25.8 -> 25.4, B1 Nk32768 26.1 -> 25.8 (shorter rows, loaded piece by piece: 12.7 -> 14.8).
+    constexpr bool kQLoads = kNarrow && kFullD && ((D == 96 && !kAlibi) || (D == 128 && kRows));
     // Where to, and bytes from one wave's to the next one's
     constexpr bool kQApart = C::kQApart;
     constexpr int kQWave = kQApart ? 32 * C::SK : NSTG * (C::KBUF + C::VBUF);
@@ -264,7 +279,9 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     const int l32 = lane & 31;
     const int g = lane >> 5;
 
-    const WorkItem item = work_item(a, blockIdx.x);
+    WorkItem item;
+    if constexpr (kRows) item = rows_item<kRowsOnce>(a, blockIdx.x);
+    else item = work_item(a, blockIdx.x);
     const int bh = item.bh, split = item.split, m_block = item.m_block;
     const int Nq = a.Nq, Nk = a.Nk, d = kFullD ? D : a.d;
     const int shift = Nk - (kFold ? a.fold_rows : Nq);
@@ -287,7 +304,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     }
     const int tile_begin = kmin / BC;
     const int ntiles = kmax > kmin ? (kmax + BC - 1) / BC - tile_begin : 0;
-    if (!kStamp && ntiles == 0) {  // (the instrumented twins take the long way and report their stages)
+    if (!kStamp && !kRows && ntiles == 0) {  // (the instrumented twins take the long way and report their stages, kRows to count itself in)
         store_empty_rows<kFold>(a, bh, split, q0, q0 + BRW < Nq ? q0 + BRW : Nq, tid, kPair ? 512 : 256);
         return;
     }
@@ -503,7 +520,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                 } else {
                     base += (size_t)further * (size_t)row_bytes;
                 }
-                if constexpr (kKvOnce) dma_kib_nt(base, off, dst);
+                if constexpr (kKvOnce || kRowsOnce) dma_kib_nt(base, off, dst);
                 else dma_kib(base, off, dst);
             };
 #pragma unroll
@@ -1268,6 +1285,52 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         }
         const float inv = L > 0.0f ? (kDropout ? a.drop_rscale : 1.0f) / L : 0.0f;
         const int gi = q0 + row;
+        if constexpr (kRows) {
+            if (a.num_splits > 1) {
+                const bool here = a.counters != nullptr;
+                if (gi < Nq) {
+                    const size_t prow = partial_row<kFold>(a, bh, split, gi);
+                    float* const op = a.O_partial + prow * d;
+                    const int cfull = d & ~7, rem = d & 7;
+#pragma unroll
+                    for (int k = 0; k < D / 32; ++k) {
+                        const int cc = 4 * ((tid & 7) + 8 * k);
+                        v4f o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                        for (int w = 0; w < 4; ++w) {
+                            const v4f p = *reinterpret_cast<const v4f*>(so + (w * 32 + row) * SM + cc);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(wgt[w], p[e], o[e]);
+                        }
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) o[e] *= inv;
+                        if constexpr (kFullD) {
+                            store_partial4(op + cc, o, here);
+                        } else if (cc < cfull || (rem != 0 && cc < cfull + 8)) {
+                            float* const oc = op + (cc < cfull ? cc : cc - (8 - rem));
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) store_partial(oc + e, o[e], here);
+                        }
+                    }
+                    if ((tid & 7) == 0) store_partial(a.LSE_partial + prow, L > 0.0f ? __builtin_fmaf(M, kLn2, fast_log2(L) * kLn2) : -INFINITY, here);
+                }
+                if (here && last_to_arrive(a.counters + bh, a.num_splits, reinterpret_cast<int*>(smem))) {
+                    float* const lds = reinterpret_cast<float*>(smem) + 64;
+                    auto merge_row = [&](int r, auto waves_c) __attribute__((always_inline)) {
+                        const int hq = kFold ? a.by_fold.quotient(r) : 0;
+                        combine_row<true, decltype(waves_c)::value>(a.O_partial, a.LSE_partial, a.O, a.LSE, kFold ? bh * a.fold_group + hq : bh,
+                                                                    kFold ? r - hq * a.fold_rows : r, kFold ? a.fold_rows : Nq, d, a.num_splits, lds);
+                    };
+                    if (a.combine_waves == 1) {
+                        for (int r = wave; r < Nq; r += 4) merge_row(r, std::integral_constant<int, 1>{});
+                    } else {
+                        for (int r = 0; r < Nq; ++r) merge_row(r, std::integral_constant<int, 4>{});
+                    }
+                }
+                store_stamps();
+                return;
+            }
+        }
         if (gi < Nq) {
             half_t* const op = a.O + ((size_t)bh * Nq + gi) * d;
             const int cfull = d & ~7, rem = d & 7;
@@ -1568,13 +1631,20 @@ inline bool fwd_uses_narrow(const FwdArgs& a, bool every)
     return tiles >= (no_pair ? 32 : 64) && rounds_pay && fed;
 }
 
+// LDS of a narrow work-group: two stages per wave up to D = 64, one above
+template <int D, int VAR>
+constexpr int narrow_lds()
+{
+    using C = FwdCfg<D, 1, true, (VAR & kVarShort) != 0>;
+    return 4 * (D <= 64 ? 2 : 1) * (C::KBUF + C::VBUF) + (C::kQApart ? 4 * 32 * C::SK : 0);
+}
+
 template <int D, int VAR>
 inline hipError_t launch_fwd_narrow_instance(const FwdArgs& a, hipStream_t st)
 {
-    using C = FwdCfg<D, 1, true, (VAR & kVarShort) != 0>;
     auto kern = fwd_kernel<D, 1, VAR | kVarNarrow>;
     static DeviceFlags attr_done;  // per instantiation and device
-    constexpr int smem = 4 * (D <= 64 ? 2 : 1) * (C::KBUF + C::VBUF) + (C::kQApart ? 4 * 32 * C::SK : 0);  // two stages per wave up to D = 64, one above
+    constexpr int smem = narrow_lds<D, VAR>();
     if (hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), smem, attr_done); e != hipSuccess) return e;
     FwdArgs b = a;
     b.Tr = (a.Nq + 31) / 32;
@@ -1584,6 +1654,72 @@ inline hipError_t launch_fwd_narrow_instance(const FwdArgs& a, hipStream_t st)
     b.snake_end = snake_end_for(groups, kNumCus);
     set_divisors(b, b.slice_chunk);
     return launch_kernel(kern, dim3((unsigned)groups), dim3(256), smem, st, packed(b));
+}
+
+// Launches of few rows (kRows in fwd_kernel), no features, no window.  Old form (128-row work-groups, one wave of which has rows) / this one, each
+// with its best split count, inputs that no cache holds, us:
+//  * Up to 32 rows per slice (decode with heads as rows, folded heads, speculative tokens), whole, 128 ... 256 slices, one work-group
+//    per CU: what the non-temporal requests give the narrow form.  B32 H32 H_kv8 Nk4096 d128 91.1 / 79.7, Nk1024 25.2 / 22.7, Nk512 14.4 / 13.0, B20
+//    54.0 / 49.8, B32 d64 47.2 / 41.6, B64 H16 H_kv4 Nk3000 d96 51.0 / 44.7, B24 H64 H_kv8 d80 33.8 / 30.4, B30 H8 Nq8 Nk3000 d128 62.8 / 53.8; a second
+//    round costs (320 slices 54.8 / 60.3, 512 77.9 / 81.7).
+//  * Up to 32 rows in splits, four tiles or more each, at most 32 of them, up to eight tiles per wave: B1 H32 H_kv8 Nk1920 d64 8.8 / 7.3, B1 H16 H_kv4
+//    Nk3584 d64 8.9 / 7.5, B4 H32 H_kv8 Nk8192 d128 26.2 / 25.2, B1 Nk32768 28.2 / 26.0, B12 H32 H_kv4 Nq3 Nk8396 d80 29.0 / 26.0, B4 H8 Nq16 Nk8192
+//    d128 28.6 / 25.7.  Above d = 64, where Q of a short launch comes a memory latency ahead of V, only launches that fill the GPU gain (B1 H32 H_kv8
+//    Nk2048 d128, 128 work-groups, 8.5 / 8.8; B5 H4 H_kv1 Nk7937 d96 9.9 / 10.1); with more tiles per wave both run at the rate of HBM (B16 H32
+//    H_kv4 Nk16384 83.2 / 83).
+//  * Up to 512 rows, in splits: a quarter of the splits, and of the partial results, fills the GPU, at the price of a tile fetched once per 32
+//    rows, so that the tiles per wave are bounded.  B2 H8 Nq64 Nk4096 d128 17.1 / 14.2, B4 H4 Nq128 Nk4096 20.9 / 17.9, B1 H8 Nq128 Nk16384 29.3 / 26.4,
+//    B1 H4 Nq512 Nk4096 20.7 / 15.3, B1 H8 H_kv4 Nq120 Nk6000 18.6 / 14.2, B1 H16 H_kv2 Nq40 Nk9000 (folded) 17.0 / 13.5, B1 H8 Nq128 Nk8192 d80 17.4 / 14.8, B1
+//    H2 Nq128 Nk4096 d64 10.3 / 8.5; with more tiles than that: B4 H4 Nq130 Nk7000 d128 (10) 25.8 / 27.8, B2 H8 Nq100 Nk8000 d64 (8) 16.0 / 16.4, B1 H12
+//    H_kv2 Nq100 Nk7000 d100 (6) 18.1 / 19.9, B1 H32 Nq128 Nk16384 d128 (32) 63 / 80.  Launches of fewer than 96 work-groups, which only a
+//    caller's own split count makes, are launched as they always were.
+inline bool rows_form_fits(long long slices, int rows, int d, int Nk, int splits, int keys_per_split)
+{
+    const int places = d <= 32 ? 2 * kNumCus : kNumCus;
+    const long long groups = slices * ((rows + 31) / 32) * splits;
+    if (rows > 512 || groups > places) return false;
+    if (splits == 1) return rows <= 32 && groups >= 128 && groups <= kNumCus && Nk >= 512;
+    const int per_wave = (keys_per_split + 255) / 256;
+    if (splits > 32 || keys_per_split < 256) return false;
+    if (rows > 32) return groups >= 96 && per_wave <= (d == 128 ? 8 : d % 32 == 0 ? 7 : 4);
+    return groups >= (d <= 64 ? 48 : 192) && per_wave <= 8 && slices >= 4;
+}
+inline bool rows_form_serves(const FwdArgs& a, int variant)
+{
+    return (a.kv_group == 1 || a.Nq > kRowsLimit) && (variant & (kVarAlibi | kVarDropout)) == 0 && a.wl < 0 && a.wr < 0 && a.kernel_hint == 0;
+}
+inline bool fwd_uses_rows(const FwdArgs& a, int variant)
+{
+    return rows_form_serves(a, variant) && rows_form_fits((long long)a.B * a.H, a.Nq, a.d, a.Nk, a.num_splits, a.keys_per_split);
+}
+// split count with which such a launch fills the GPU, 0 if there is none that rows_form_fits
+inline int rows_form_splits(long long slices, int rows, int d, int Nk)
+{
+    const int n_blocks = (Nk + 127) / 128;
+    const long long groups = slices * ((rows + 31) / 32);
+    if (rows > 512 || groups < 1) return 0;
+    if (rows <= 32 && groups >= 144 && groups <= kNumCus && Nk >= 512) return 1;
+    if (rows <= 32 && slices >= 16 && Nk <= 1280) return 0;
+    long long s = (d <= 32 ? 2 * kNumCus : kNumCus) / groups;
+    if (s > (n_blocks + 1) / 2) s = (n_blocks + 1) / 2;
+    if (s > 32) s = 32;
+    if (s < 2) return 0;
+    const int per = (int)((n_blocks + s - 1) / s), even = (n_blocks + per - 1) / per;  // all of them with keys
+    return even >= 2 && rows_form_fits(slices, rows, d, Nk, even, 128 * per) ? even : 0;
+}
+
+template <int D, int VAR>
+inline hipError_t launch_fwd_rows_instance(const FwdArgs& a, hipStream_t st)
+{
+    auto kern = fwd_kernel<D, 1, VAR | kVarNarrow | kVarRows>;
+    static DeviceFlags attr_done;  // per instantiation and device
+    constexpr int smem = narrow_lds<D, 0>();
+    if (hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), smem, attr_done); e != hipSuccess) return e;
+    FwdArgs b = a;
+    b.Tr = (a.Nq + 31) / 32;
+    const long long slices = (long long)a.B * a.H;
+    set_divisors(b, slices);
+    return launch_kernel(kern, dim3((unsigned)(slices * a.num_splits * b.Tr)), dim3(256), smem, st, packed_rows(b));
 }
 
 // Paired work-groups (kPair in fwd_kernel): launches of at most one 128-row work-group per CU, whose SIMDs would have one
@@ -1639,7 +1775,7 @@ inline int fwd_rows_per_group(const FwdArgs& a, int variant)
     const bool every = fwd_needs_every_instance(a, variant);
     if (!a.fold_rows && fwd_uses_pingpong(a.d, !every, a.Nq, a.Nk, a.causal, a.wl, a.wr, (long long)a.B * a.H * a.num_splits, a.kernel_hint))
         return 256;
-    if (fwd_uses_narrow(a, every)) return 32;
+    if (fwd_uses_narrow(a, every) || (!every && fwd_uses_rows(a, variant))) return 32;
     return fwd_uses_tall(a, variant) ? 256 : 128;
 }
 
@@ -1656,6 +1792,16 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
         }
         return launch(std::integral_constant<int, 0>{});
     };
+    if (!fwd_needs_every_instance(a, variant) && fwd_uses_rows(a, variant)) {
+        // rows of the bucket's width, or any length from eight elements on
+        auto rows = [&](auto full_c) {
+            constexpr int R = ST | (decltype(full_c)::value ? kVarVec | kVarFullD : 0);
+            if (a.Nq <= kRowsLimit) return (int)(a.fold_rows ? launch_fwd_rows_instance<D, R | kVarFold>(a, st) : launch_fwd_rows_instance<D, R>(a, st));
+            constexpr int M = R | kVarManyRows;
+            return (int)(a.fold_rows ? launch_fwd_rows_instance<D, M | kVarFold>(a, st) : launch_fwd_rows_instance<D, M>(a, st));
+        };
+        return a.d == D ? rows(std::true_type{}) : rows(std::false_type{});
+    }
     if (fwd_uses_narrow(a, fwd_needs_every_instance(a, variant))) {
         // plain: by row length like the others; with ALiBi or dropout: the instances for rows at any alignment, which serve
         // every row length from eight elements on, and above 64 the ones for rows of the bucket's width
