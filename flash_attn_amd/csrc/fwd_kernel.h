@@ -1734,18 +1734,28 @@ inline hipError_t launch_fwd_rows_instance(const FwdArgs& a, hipStream_t st)
 //  * up to 32 rows only one wave of four has any, and a second one beside it gained 7-11 % at d = 32, but lost 4 % at
 //    d = 112 (B2 H16 H_kv4 Nq2 Nk16960 18.2 -> 19.0).
 //  * causal, unsplit and up to twice as many: two work-groups of a CU side by side last as long as the longer one, whose SIMDs
-//    have one wave each once its light neighbour is done; as paired ones they follow each other, eight waves at a time.  From
-//    1280 keys on up to 384 work-groups (1.0 ... 1.2 times as fast over d = 40 ... 128), with dropout up to 512, from 1856 on up to
-//    512 without (0.98 ... 1.1): B1 H32 N1500 d128 32.5 -> 29.2 us, B3 H8 N1777 d100 34.4 -> 29.3, B1 H16 N4096 d128 83.1 -> 75.2, B4 H8
-//    N2000 d96 35.3 -> 33.3, with dropout B3 H12 N1777 d80 45.1 -> 41.8.  Below (B2 H24 N1000 d128 23.3 -> 24.1) and above (B5 H8 N1777
-//    d100 42.5 -> 47.8, 560 of them) it loses.
+//    have one wave each once its light neighbour is done; as paired ones they follow each other, eight waves at a time.  The lines lie where 150
+//    random launches cross over.  Up to 384 work-groups (unpaired / paired): N1238 d64 17.9 / 15.7 us, N1117 d80 19.2 / 16.0, N1184 d100 23.1 / 19.5, N1000
+//    d40 14.7 / 13.7; with dropout N1267 d64 27.3 / 22.7, N640 d64 15.5 / 13.2, N1021 d128 28.7 / 24.0, N680 d128 20.8 / 18.3; below the lines N675 d64
+//    11.35 / 11.46, N926 d96 16.4 / 17.3, N660 d128 17.8 / 20.6, with dropout N668 d32 13.4 / 13.4, N556 d128 20.3 / 23.2.  More of them: B1 H16 N4096
+//    d128 83.1 / 75.2, B4 H8 N2000 d96 36.1 / 34.2, N1645 d96 (390 of them) 28.5 / 25.9, N1672 d80 (448) 26.4 / 24.9, B3 H12 N1777 d80 31.1 / 30.4, B4 H8 N2000 d80 with dropout 44.6 / 40.9, N1246 d64 (400 of them) 17.4 / 16.4;
+//    below N1424 d80 24.7 / 26.8, N1785 d96 (504) 32.6 / 33.0, N1227 d64 with dropout 25.8 / 25.9.  Above 512 it loses (B5 H8 N1777 d100 42.5 / 47.8, 560 of them).
+inline long long following_keys(int d, long long groups, bool dropout)
+{
+    const int bucket = (d + 31) / 32;
+    constexpr int kPlain[4] = {704, 704, 960, 1104}, kDropout[4] = {960, 608, 608, 640};
+    if (groups <= 384) return dropout ? kDropout[bucket - 1] : kPlain[bucket - 1];
+    if (dropout) return 1280;
+    if (bucket == 3) return groups <= 448 ? 1600 : d <= 80 ? 1760 : 1856;
+    return bucket <= 2 && groups <= 416 ? 1184 : 1856;
+}
 inline bool fwd_uses_pair(const FwdArgs& a, int bucket_d, int feat)
 {
     if ((feat & kVarAlibi) != 0 || a.kernel_hint != 0 || (a.Nq <= 32 && bucket_d > 32)) return false;
     const long long groups = (long long)a.Tr * a.B * a.H * a.num_splits;
     const long long left = a.wl >= 0 ? a.wl : a.Nk, right = a.causal ? 0 : a.wr >= 0 ? a.wr : a.Nk;
     if (a.causal && a.wl < 0 && a.num_splits == 1 && !a.fold_rows && 2 * (long long)a.Nq >= a.Nk && groups > kNumCus)
-        return groups <= 2 * kNumCus && a.Nk >= (groups <= 384 || feat != 0 ? 1280 : 1856);
+        return groups <= 2 * kNumCus && a.Nk >= following_keys(a.d, groups, feat != 0);
     return groups <= kNumCus && a.Nk >= 8 * 64 * a.num_splits && left + right + 128 >= 8 * 64;
 }
 
