@@ -144,7 +144,7 @@ constexpr float kNothingSeen = -3.402823466e38f;
 // kVarEvery (with kVarAlibi and kVarDropout, without kVarVec): the instance that serves every request, see kEvery below.
 // kVarNarrow (unsplit launches): the four waves of a work-group share 32 query rows and take every fourth key tile
 // each, see kNarrow below.
-// kVarPair (without ALiBi): eight waves in two halves that take every other tile each, see kPair below.
+// kVarPair (with ALiBi: keys at or left of the row alone, no dropout): eight waves in two halves that take every other tile each, see kPair below.
 // kVarFold (no other feature): the rows are the query heads of a K/V head, see row_position in common.h.
 // kVarShort (D >= 64, not kVarFullD, kVarEvery or kVarFold): rows of at most D - 16 elements, see FwdCfg::kShort.
 // kVarRows (with kVarNarrow; no other feature but kVarFold): launches of few rows per slice, whole or in splits, see kRows below.
@@ -1170,8 +1170,12 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         // grows towards the row, so in rising order the row maximum outgrew kLazyTau, and O was rescaled, in tile after
         // tile.  Causal window of 1650 keys B9 H3 N5649 d72: 112.3 -> 104.4 us, B4 H4 N3392 d128 with 704 keys 32.8 -> 31.0,
         // B2 H16 N4096 d64 with 256 keys (a third of whose heads rescaled per tile) 23.8 -> 23.3.
-        auto nth = [&](int t) { return kFoldAlibi ? ntiles - 1 - t : kPair ? 2 * t + half : t; };
+        auto nth = [&](int t) {
+            const int i = kPair ? 2 * t + half : t;
+            return kFoldAlibi ? ntiles - 1 - i : i;
+        };
         // (paired: both halves go round as often, for the barrier; the second one's last tile may not exist)
+        auto there = [&](int t) { return !kPair || 2 * t + half < ntiles; };
         const int rounds = kPair ? (ntiles + 1) / 2 : ntiles;
         static_assert(NSTG == 2, "a stage that is read and one that is filled");
         // (Launches whose every tile has one reader take them from HBM, all work-groups at once: they request the second tile only
@@ -1180,9 +1184,9 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         // work-groups, whose halves have a tile each on its way, -2 %.)
         constexpr bool late = (kFold || kKvOnce) && !kPair;
         auto second_tile = [&](bool now) {
-            if (now && 1 < rounds && (!kPair || nth(1) < ntiles)) dma_tile(tile_begin + nth(1), 1);
+            if (now && 1 < rounds && there(1)) dma_tile(tile_begin + nth(1), 1);
         };
-        if (0 < rounds && (!kPair || nth(0) < ntiles)) dma_tile(tile_begin + nth(0), 0);
+        if (0 < rounds && there(0)) dma_tile(tile_begin + nth(0), 0);
         second_tile(!late);
         set_bounds();
         read_slope();
@@ -1195,13 +1199,13 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         stamps.take(3);
         int buf = 0;  // stage of tile t
         for (int t = 0; t < rounds; ++t) {
-            if (!kPair || nth(t) < ntiles) tile_math(nth(t), buf);
+            if (there(t)) tile_math(nth(t), buf);
             if (kStamp && t == 0) stamps.take(4);
             dma_wait();
             __syncthreads();
             // (the request stands at the end so that the first tile, whose successor is on its way already, is no case of its own:
             // a copy of the tile's code costs a launch of few tiles its way through a cold instruction cache)
-            if (kPair ? nth(t + 2) < ntiles : t + 2 < ntiles) dma_tile(tile_begin + nth(t + 2), buf);
+            if (kPair ? there(t + 2) : t + 2 < ntiles) dma_tile(tile_begin + nth(t + 2), buf);
             buf ^= 1;
         }
     } else {
@@ -1731,6 +1735,11 @@ inline hipError_t launch_fwd_rows_instance(const FwdArgs& a, hipStream_t st)
 //    N683 d128 22.7 -> 20.1.
 //  * eight tiles or more per work-group, a window's included: with fewer the merge costs what the shorter chain saves.
 //    (Window of 500 keys B1 H16 N1500 d64 12.7 -> 10.7 us, of 1000 B2 H4 N2500 d96 21.5 -> 18.0.)
+//  * with ALiBi and no visible key right of its row, whole: from 5 tiles on, 8 above d = 96, the chain of a tile being the longer one (110 random launches of
+//    up to 512 work-groups, unpaired / paired): windows B1 H8 N3835 d40 of 1390 keys 21.3 / 17.4 us, B4 H2 N3551 d64 of 1858 26.8 / 21.8, B2 H8 N1533
+//    d64 of 196 9.2 / 8.6, B1 H8 N1792 d96 of 1052 21.0 / 17.5, B1 H12 N1281 d100 of 1108 30.3 / 25.0, B2 H4 N1230 d128 of 941 22.1 / 19.5; causal N3502 d72
+//    46.1 / 37.2, N848 d32 11.1 / 9.4; up to 512 of them under the lines without dropout (next but one) N2253 d100 48.6 / 38.5, N7577 d64 88.0 / 72.2, N875 d40 13.6 / 11.6;
+//    left out: d128 windows of 159 ... 396 keys 11.0 / 11.1, of 257 to 512 work-groups 15.9 / 20.2.  Two-sided ALiBi, and with dropout, stay as they are.
 //  * up to 32 rows only one wave of four has any, and a second one beside it gained 7-11 % at d = 32, but lost 4 % at
 //    d = 112 (B2 H16 H_kv4 Nq2 Nk16960 18.2 -> 19.0).
 //  * causal, unsplit and up to twice as many: two work-groups of a CU side by side last as long as the longer one, whose SIMDs
@@ -1751,12 +1760,15 @@ inline long long following_keys(int d, long long groups, bool dropout)
 }
 inline bool fwd_uses_pair(const FwdArgs& a, int bucket_d, int feat)
 {
-    if ((feat & kVarAlibi) != 0 || a.kernel_hint != 0 || (a.Nq <= 32 && bucket_d > 32)) return false;
+    const bool alibi = (feat & kVarAlibi) != 0, dropout = (feat & kVarDropout) != 0;
+    if (alibi && (dropout || !a.alibi_left || a.num_splits != 1)) return false;
+    if (a.kernel_hint != 0 || (a.Nq <= 32 && bucket_d > 32)) return false;
     const long long groups = (long long)a.Tr * a.B * a.H * a.num_splits;
     const long long left = a.wl >= 0 ? a.wl : a.Nk, right = a.causal ? 0 : a.wr >= 0 ? a.wr : a.Nk;
     if (a.causal && a.wl < 0 && a.num_splits == 1 && !a.fold_rows && 2 * (long long)a.Nq >= a.Nk && groups > kNumCus)
-        return groups <= 2 * kNumCus && a.Nk >= following_keys(a.d, groups, feat != 0);
-    return groups <= kNumCus && a.Nk >= 8 * 64 * a.num_splits && left + right + 128 >= 8 * 64;
+        return groups <= 2 * kNumCus && a.Nk >= following_keys(a.d, groups, dropout);
+    const long long keys = alibi && bucket_d <= 96 ? 4 * 64 + 1 : 8 * 64;
+    return groups <= kNumCus && a.Nk >= keys * a.num_splits && left + right + 128 >= keys;
 }
 
 // 64 query rows per wave at d = 64 (NB = 2, 199 VGPRs, two work-groups of 256 rows per CU): a K or V fragment read from LDS
@@ -1864,7 +1876,7 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
         // threshold of 0
         if (fwd_needs_every_instance(a, variant)) e = launch_fwd_instance<D, NB, ST | kVarAlibi | kVarDropout | kVarEvery>(a, st);
         else if (feat == 0) e = shorter_rows(std::integral_constant<int, ST>{});
-        else if (feat == kVarAlibi) e = shorter_rows_alone(std::integral_constant<int, ST | kVarAlibi>{});
+        else if (feat == kVarAlibi) e = shorter_rows(std::integral_constant<int, ST | kVarAlibi>{});
         else if (feat == kVarDropout) e = shorter_rows(std::integral_constant<int, ST | kVarDropout>{});
         else e = shorter_rows_alone(std::integral_constant<int, ST | kVarAlibi | kVarDropout>{});
     } else if (a.d == D) {
@@ -1877,14 +1889,14 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
             }
         }
         if (feat == 0) e = kv_once ? halves(std::integral_constant<int, V | kVarKvOnce>{}) : halves(std::integral_constant<int, V>{});
-        else if (feat == kVarAlibi) e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi>(a, st);
+        else if (feat == kVarAlibi) e = a.alibi_left ? halves(std::integral_constant<int, V | AL>{}) : launch_fwd_instance<D, NB, V | kVarAlibi>(a, st);
         else if (feat == kVarDropout) e = halves(std::integral_constant<int, V | kVarDropout>{});
         else e = a.alibi_left ? launch_fwd_instance<D, NB, V | AL | kVarDropout>(a, st) : launch_fwd_instance<D, NB, V | kVarAlibi | kVarDropout>(a, st);
     } else {
         constexpr int V = ST | kVarVec;
         if (feat == 0) e = shorter_rows(std::integral_constant<int, V>{});
         else if (feat == kVarDropout) e = shorter_rows(std::integral_constant<int, V | kVarDropout>{});
-        else if (feat == kVarAlibi) e = a.alibi_left ? shorter_rows_alone(std::integral_constant<int, V | AL>{}) : shorter_rows_alone(std::integral_constant<int, V | kVarAlibi>{});
+        else if (feat == kVarAlibi) e = a.alibi_left ? shorter_rows(std::integral_constant<int, V | AL>{}) : shorter_rows_alone(std::integral_constant<int, V | kVarAlibi>{});
         else e = a.alibi_left ? shorter_rows_alone(std::integral_constant<int, V | AL | kVarDropout>{}) : shorter_rows_alone(std::integral_constant<int, V | kVarAlibi | kVarDropout>{});
     }
     return (int)e;
