@@ -1735,11 +1735,16 @@ inline hipError_t launch_fwd_rows_instance(const FwdArgs& a, hipStream_t st)
 //    N683 d128 22.7 -> 20.1.
 //  * eight tiles or more per work-group, a window's included: with fewer the merge costs what the shorter chain saves.
 //    (Window of 500 keys B1 H16 N1500 d64 12.7 -> 10.7 us, of 1000 B2 H4 N2500 d96 21.5 -> 18.0.)
-//  * with ALiBi and no visible key right of its row, whole: from 5 tiles on, 8 above d = 96, the chain of a tile being the longer one (110 random launches of
+//  * with ALiBi and no visible key right of its row, whole: from 5 tiles on, 8 at d = 128, the chain of a tile being the longer one (110 random launches of
 //    up to 512 work-groups, unpaired / paired): windows B1 H8 N3835 d40 of 1390 keys 21.3 / 17.4 us, B4 H2 N3551 d64 of 1858 26.8 / 21.8, B2 H8 N1533
 //    d64 of 196 9.2 / 8.6, B1 H8 N1792 d96 of 1052 21.0 / 17.5, B1 H12 N1281 d100 of 1108 30.3 / 25.0, B2 H4 N1230 d128 of 941 22.1 / 19.5; causal N3502 d72
 //    46.1 / 37.2, N848 d32 11.1 / 9.4; up to 512 of them under the lines without dropout (next but one) N2253 d100 48.6 / 38.5, N7577 d64 88.0 / 72.2, N875 d40 13.6 / 11.6;
 //    left out: d128 windows of 159 ... 396 keys 11.0 / 11.1, of 257 to 512 work-groups 15.9 / 20.2.  Two-sided ALiBi, and with dropout, stay as they are.
+//  * under a window that ends at the row, whole, without dropout: from 5 tiles on below d = 128, too (130 random launches, unpaired / paired, us): N4064 d32 of 219 keys 8.03 /
+//    6.78, N904 d40 of 184 8.15 / 7.53, N3367 d64 of 212 9.48 / 8.80, N1554 d64 of 146 8.32 / 8.07, N1911 d72 of 208 10.51 / 9.58, N907 d100 of 231 12.50 / 11.69, N1126 d112 of
+//    159 10.34 / 9.99; but d128 of 202 12.74 / 13.77, of 293 14.44 / 14.85, and without a window N300 d96 7.94 / 8.42.  At 32 < d <= 64 up to 400 work-groups,
+//    from 7 tiles on, without ALiBi: B1 H8 N4178 d64 of 480 12.02 / 10.58, B2 H32 N623 d64 of 346 11.27 / 10.21, B1 H12 N4037 d40 of 878 21.5 / 20.2, B4 H2 N6294 d64 of 1121 27.9 /
+//    25.9; with 5 tiles N791 d40 8.93 / 9.06, d32 of 417 10.84 / 11.19, and above d = 64 0.7 ... 0.9 times as fast (d72 of 163 12.3 / 16.5).
 //  * up to 32 rows only one wave of four has any, and a second one beside it gained 7-11 % at d = 32, but lost 4 % at
 //    d = 112 (B2 H16 H_kv4 Nq2 Nk16960 18.2 -> 19.0).
 //  * causal, unsplit and up to twice as many: two work-groups of a CU side by side last as long as the longer one, whose SIMDs
@@ -1767,8 +1772,10 @@ inline bool fwd_uses_pair(const FwdArgs& a, int bucket_d, int feat)
     const long long left = a.wl >= 0 ? a.wl : a.Nk, right = a.causal ? 0 : a.wr >= 0 ? a.wr : a.Nk;
     if (a.causal && a.wl < 0 && a.num_splits == 1 && !a.fold_rows && 2 * (long long)a.Nq >= a.Nk && groups > kNumCus)
         return groups <= 2 * kNumCus && a.Nk >= following_keys(a.d, groups, dropout);
-    const long long keys = alibi && bucket_d <= 96 ? 4 * 64 + 1 : 8 * 64;
-    return groups <= kNumCus && a.Nk >= keys * a.num_splits && left + right + 128 >= keys;
+    const bool window = left + right + 128 < a.Nk && right == 0 && a.num_splits == 1 && !dropout;
+    if (groups > kNumCus) return window && !alibi && bucket_d == 64 && groups <= 400 && left + 128 > 6 * 64;
+    const long long keys = a.d < 128 && (alibi || window) ? 4 * 64 + 1 : 8 * 64;
+    return a.Nk >= keys * a.num_splits && left + right + 128 >= keys;
 }
 
 // 64 query rows per wave at d = 64 (NB = 2, 199 VGPRs, two work-groups of 256 rows per CU): a K or V fragment read from LDS
