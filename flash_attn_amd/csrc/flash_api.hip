@@ -193,7 +193,7 @@ long long tiled_groups(const flash_params* p, const fa::FwdArgs& a)
 // 9 %); the reference's rule with 256 CUs: 9 of 21, the worst 3.1 times slower than the best count.  It knows
 // of narrow launches, and of paired ones with one work-group per CU; paired launches of 257 to 512 work-groups have the price of
 // unpaired ones, and the fourth work-group per CU at d = 64 and the third at d = 96 that of rounds of three and two.  Its constants
-// and the lines of fwd_uses_narrow and fwd_uses_pair are fits to the kernels as they were before narrow launches got 2-17 % faster
+// and the lines of fwd_uses_narrow are fits to the kernels as they were before narrow launches got 2-17 % faster
 // (odd d most) and rows of at most 16 columns less than their bucket 3-8 %: they err on the side of the wider work-groups, and want measuring again.
 int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode);
 bool folds_heads(const flash_params* p);

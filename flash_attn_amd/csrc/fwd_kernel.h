@@ -1733,7 +1733,7 @@ inline hipError_t launch_fwd_rows_instance(const FwdArgs& a, hipStream_t st)
 //    Nq128 Nk16384 d128 63.3 -> 60.6 (bound by HBM for half of it).
 //  * causal with dropout: B2 H2 N2112 d100 59.9 -> 46.2 us, B2 H4 N1986 d96 50.1 -> 38.9, B1 H8 N3061 d64 65.2 -> 52.6, B4 H8
 //    N683 d128 22.7 -> 20.1.
-//  * eight tiles or more per work-group, a window's included: with fewer the merge costs what the shorter chain saves.
+//  * eight tiles or more per work-group, a window's included (five where the last points say so): with fewer the merge costs what the shorter chain saves.
 //    (Window of 500 keys B1 H16 N1500 d64 12.7 -> 10.7 us, of 1000 B2 H4 N2500 d96 21.5 -> 18.0.)
 //  * with ALiBi and no visible key right of its row, whole: from 5 tiles on, 8 at d = 128, the chain of a tile being the longer one (110 random launches of
 //    up to 512 work-groups, unpaired / paired): windows B1 H8 N3835 d40 of 1390 keys 21.3 / 17.4 us, B4 H2 N3551 d64 of 1858 26.8 / 21.8, B2 H8 N1533
