@@ -1320,15 +1320,11 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                 }
                 if (here && last_to_arrive(a.counters + bh, a.num_splits, reinterpret_cast<int*>(smem))) {
                     float* const lds = reinterpret_cast<float*>(smem) + 64;
-                    auto merge_row = [&](int r, auto waves_c) __attribute__((always_inline)) {
+                    // (a wave per row: two to four rows of at most 32 splits take no fewer batches in a row with all four waves on each, see combine_waves_for)
+                    for (int r = wave; r < Nq; r += 4) {
                         const int hq = kFold ? a.by_fold.quotient(r) : 0;
-                        combine_row<true, decltype(waves_c)::value>(a.O_partial, a.LSE_partial, a.O, a.LSE, kFold ? bh * a.fold_group + hq : bh,
-                                                                    kFold ? r - hq * a.fold_rows : r, kFold ? a.fold_rows : Nq, d, a.num_splits, lds);
-                    };
-                    if (a.combine_waves == 1) {
-                        for (int r = wave; r < Nq; r += 4) merge_row(r, std::integral_constant<int, 1>{});
-                    } else {
-                        for (int r = 0; r < Nq; ++r) merge_row(r, std::integral_constant<int, 4>{});
+                        combine_row<true, 1>(a.O_partial, a.LSE_partial, a.O, a.LSE, kFold ? bh * a.fold_group + hq : bh, kFold ? r - hq * a.fold_rows : r,
+                                             kFold ? a.fold_rows : Nq, d, a.num_splits, lds);
                     }
                 }
                 store_stamps();
