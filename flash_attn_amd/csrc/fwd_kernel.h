@@ -148,7 +148,7 @@ constexpr float kNothingSeen = -3.402823466e38f;
 // kVarFold (no other feature): the rows are the query heads of a K/V head, see row_position in common.h.
 // kVarShort (D >= 64, not kVarFullD, kVarEvery or kVarFold): rows of at most D - 16 elements, see FwdCfg::kShort.
 // kVarRows (with kVarNarrow; no other feature but kVarFold): launches of few rows per slice, whole or in splits, see kRows below.
-// kVarManyRows (with kVarRows): more than 32 rows, whose row blocks ask for the same tiles.
+// kVarManyRows (with kVarRows): more than 32 rows, whose row blocks ask for the same tiles, or tiles that the caches serve (rows_read_once).
 constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarStamp = 16, kVarAlibiLeft = 32, kVarKvOnce = 64,
               kVarEvery = 128, kVarNarrow = 256, kVarFold = 512, kVarPair = 1024, kVarShort = 2048, kVarRows = 4096, kVarManyRows = 8192;
 
@@ -239,7 +239,8 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     static_assert(!kNarrow || (kDma && NB == 1 && !kKvOnce), "narrow instances");
     // The narrow form for launches of few rows per slice (fwd_uses_rows says which), in splits too: their partial results leave the merge
     // as whole rows of floats, and where a caller has brought counters (combine.h) and the rows are four or fewer, the last work-group
-    // of a slice merges the splits.  With up to 32 rows nobody else asks for the tiles, and the requests are non-temporal.
+    // of a slice merges the splits.  With up to 32 rows nobody else asks for the tiles, and the requests are non-temporal where that pays
+    // (rows_read_once).
     constexpr bool kRows = (VAR & kVarRows) != 0, kRowsOnce = kRows && (VAR & kVarManyRows) == 0;
     static_assert(!kRows || (kNarrow && !kAlibi && !kDropout), "few rows");
     constexpr bool kFold = (VAR & kVarFold) != 0;
@@ -1308,8 +1309,8 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                         }
 #pragma unroll
                         for (int e = 0; e < 4; ++e) o[e] *= inv;
-                        if constexpr (kFullD) {
-                            store_partial4(op + cc, o, here);
+                        if constexpr (kVec) {
+                            if (kFullD || cc < d) store_partial4(op + cc, o, here);
                         } else if (cc < cfull || (rem != 0 && cc < cfull + 8)) {
                             float* const oc = op + (cc < cfull ? cc : cc - (8 - rem));
 #pragma unroll
@@ -1708,12 +1709,26 @@ inline int rows_form_splits(long long slices, int rows, int d, int Nk)
     return even >= 2 && rows_form_fits(slices, rows, d, Nk, even, 128 * per) ? even : 0;
 }
 
+// Whether such a launch asks for its tiles with non-temporal requests (kRowsOnce in fwd_kernel).  Up to 32 rows nobody else asks for them; but
+// rows that are no multiple of 64 bytes share lines with their neighbours, which other requests ask for, and where K and V fit the 32 MiB of L2
+// those are still there.  Ordinary / non-temporal over 575 random launches of d = 31 ... 112, by bytes of K and V: 12-16 MiB 0.91 ... 0.96, 18-20 0.91 ... 0.98,
+// 20-22 0.95 ... 1.02, 22-24 1.00 ... 1.03, 30-48 1.02 ... 1.07, above 1.04 ... 1.10: in splits B18 H4 H_kv1 Nk7763 d31 (16 MiB)
+// 9.59 / 10.50 us, B2 H32 H_kv8 Nk3997 d72 (18) 8.96 / 9.40, B5 H64 H_kv8 Nk5952 d40 (36) 12.84 / 12.04; whole B25 H32 H_kv8 Nk896 d31 (21) 8.07 / 8.45, B24 Nk1282
+// d40 (38) 10.95 / 10.40.  With fewer than 160 work-groups 0.95 ... 1.02 at any size, ordinary ones mostly the faster.
+constexpr long long kOnceBytes = 22 << 20;
+inline bool rows_read_once(const FwdArgs& a, int bucket_d)
+{
+    if (a.Nq > kRowsLimit) return false;
+    const long long slices = (long long)a.B * a.H;
+    return a.d == bucket_d || (slices * a.num_splits >= 160 && 4 * slices * a.Nk * a.d >= kOnceBytes);
+}
+
 template <int D, int VAR>
 inline hipError_t launch_fwd_rows_instance(const FwdArgs& a, hipStream_t st)
 {
     auto kern = fwd_kernel<D, 1, VAR | kVarNarrow | kVarRows>;
     static DeviceFlags attr_done;  // per instantiation and device
-    constexpr int smem = narrow_lds<D, 0>();
+    constexpr int smem = narrow_lds<D, VAR>();
     if (hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), smem, attr_done); e != hipSuccess) return e;
     FwdArgs b = a;
     b.Tr = (a.Nq + 31) / 32;
@@ -1818,14 +1833,24 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
         return launch(std::integral_constant<int, 0>{});
     };
     if (!fwd_needs_every_instance(a, variant) && fwd_uses_rows(a, variant)) {
-        // rows of the bucket's width, or any length from eight elements on
-        auto rows = [&](auto full_c) {
-            constexpr int R = ST | (decltype(full_c)::value ? kVarVec | kVarFullD : 0);
-            if (a.Nq <= kRowsLimit) return (int)(a.fold_rows ? launch_fwd_rows_instance<D, R | kVarFold>(a, st) : launch_fwd_rows_instance<D, R>(a, st));
-            constexpr int M = R | kVarManyRows;
-            return (int)(a.fold_rows ? launch_fwd_rows_instance<D, M | kVarFold>(a, st) : launch_fwd_rows_instance<D, M>(a, st));
+        // By row length and alignment like the narrow ones; in the bucket of 32 columns rows at any alignment serve every shorter length.  When they served
+        // all shorter lengths -> now, us: B4 H16 H_kv4 Nk6004 d40 in 16 splits 11.90 -> 11.06, B2 H32 H_kv8 Nk3264 d72 in 13 11.17 -> 10.47, B2 H4 Nq20 Nk6190 d80
+        // in 25 11.01 -> 9.49, B2 H16 H_kv2 Nq8 Nk9000 d112 in 24 13.00 -> 12.27, B2 H8 Nq11 Nk11200 d100 in 15 19.82 -> 19.60; whole B20 H64 H_kv8 Nk5263 d80 46.66
+        // -> 46.52.  Rows of whole chunks give 4 % of it, short ones 1-2, ordinary requests below rows_read_once's line 3-8.
+        auto rows = [&](auto var) {
+            auto folded = [&](auto cached) {
+                constexpr int V = ST | decltype(var)::value | decltype(cached)::value;
+                if (a.fold_rows) return (int)launch_fwd_rows_instance<D, V | kVarFold>(a, st);
+                if constexpr ((V & kVarFullD) != 0) return (int)launch_fwd_rows_instance<D, V>(a, st);
+                else return (int)by_length([&](auto sh) { return launch_fwd_rows_instance<D, V | decltype(sh)::value>(a, st); });
+            };
+            return rows_read_once(a, D) ? folded(std::integral_constant<int, 0>{}) : folded(std::integral_constant<int, kVarManyRows>{});
         };
-        return a.d == D ? rows(std::true_type{}) : rows(std::false_type{});
+        if (a.d == D) return rows(std::integral_constant<int, kVarVec | kVarFullD>{});
+        if constexpr (D > 32) {
+            if (variant & kVarVec) return rows(std::integral_constant<int, kVarVec>{});
+        }
+        return rows(std::integral_constant<int, 0>{});
     }
     if (fwd_uses_narrow(a, fwd_needs_every_instance(a, variant))) {
         // plain: by row length like the others; with ALiBi or dropout: the instances for rows at any alignment, which serve
