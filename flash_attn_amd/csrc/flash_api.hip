@@ -528,7 +528,7 @@ int run_splitkv(const flash_params* p, int splits, hipStream_t st)
         a.counters = p->split_counters;
     // Rows that a work-group merges: those of a slice where the split launch may do it, with counters given or not, so that a result is the
     // same bit by bit either way; one behind a launch of its own.
-    const bool in_launch = route == kRouteTiled && !needs_every_instance(p) && fa::fwd_uses_rows(a, tiled_variant(p)) && a.Nq <= 4 && splits * p->d <= 1024;
+    const bool in_launch = route == kRouteTiled && !needs_every_instance(p) && fa::fwd_uses_rows(a, tiled_variant(p)) && fa::rows_form_merges(a);
     if (in_launch && splits > 1 && p->split_counters && (long long)a.B * a.H <= p->split_counters_len) a.counters = p->split_counters;
     a.combine_waves = fa::combine_waves_for(splits, route == kRouteStream ? fa::decode_heads_per_group(a.kv_group) : in_launch ? a.Nq : 1);
     // (a launch is limited to 2^32 - 1 threads: a work-group per row reaches 2^24 rows, a wave per row 2^26)

@@ -1292,7 +1292,7 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
         const int gi = q0 + row;
         if constexpr (kRows) {
             if (a.num_splits > 1) {
-                const bool here = a.counters != nullptr;
+                const bool here = kFullD && a.counters != nullptr;
                 if (gi < Nq) {
                     const size_t prow = partial_row<kFold>(a, bh, split, gi);
                     float* const op = a.O_partial + prow * d;
@@ -1314,18 +1314,19 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
                         } else if (cc < cfull || (rem != 0 && cc < cfull + 8)) {
                             float* const oc = op + (cc < cfull ? cc : cc - (8 - rem));
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) store_partial(oc + e, o[e], here);
+                            for (int e = 0; e < 4; ++e) oc[e] = o[e];
                         }
                     }
                     if ((tid & 7) == 0) store_partial(a.LSE_partial + prow, L > 0.0f ? __builtin_fmaf(M, kLn2, fast_log2(L) * kLn2) : -INFINITY, here);
                 }
-                if (here && last_to_arrive(a.counters + bh, a.num_splits, reinterpret_cast<int*>(smem))) {
-                    float* const lds = reinterpret_cast<float*>(smem) + 64;
-                    // (a wave per row: two to four rows of at most 32 splits take no fewer batches in a row with all four waves on each, see combine_waves_for)
-                    for (int r = wave; r < Nq; r += 4) {
-                        const int hq = kFold ? a.by_fold.quotient(r) : 0;
-                        combine_row<true, 1>(a.O_partial, a.LSE_partial, a.O, a.LSE, kFold ? bh * a.fold_group + hq : bh, kFold ? r - hq * a.fold_rows : r,
-                                             kFold ? a.fold_rows : Nq, d, a.num_splits, lds);
+                if constexpr (kFullD) {  // (no other instance gets counters: rows_form_merges)
+                    if (here && last_to_arrive(a.counters + bh, a.num_splits, reinterpret_cast<int*>(smem))) {
+                        float* const lds = reinterpret_cast<float*>(smem) + 64;
+                        for (int r = wave; r < Nq; r += 4) {  // (a wave per row, whose splits are one batch)
+                            const int hq = kFold ? a.by_fold.quotient(r) : 0;
+                            combine_row<true, 1>(a.O_partial, a.LSE_partial, a.O, a.LSE, kFold ? bh * a.fold_group + hq : bh, kFold ? r - hq * a.fold_rows : r,
+                                                 kFold ? a.fold_rows : Nq, d, a.num_splits, lds);
+                        }
                     }
                 }
                 store_stamps();
@@ -1692,6 +1693,17 @@ inline bool rows_form_serves(const FwdArgs& a, int variant)
 inline bool fwd_uses_rows(const FwdArgs& a, int variant)
 {
     return rows_form_serves(a, variant) && rows_form_fits((long long)a.B * a.H, a.Nq, a.d, a.Nk, a.num_splits, a.keys_per_split);
+}
+// Whether the last work-group of such a launch to arrive at a slice's counter merges its partial results.  A merge by a launch of its own takes 1.5-2 us,
+// which the arrival (a store, an atomic and a load from memory in a row) and partial results written through and read past the L2 use up
+// soon.  Its own launch / here, time over time, over 451 random launches of whole buckets: up to four rows and 12 splits, by splits * d up to 512 / 768 /
+// 1024 / 1536, 1.04 / 1.04 / 1.02 / 1.00 (d = 32, up to 8 splits 1.02, 9 to 12 0.99); 13 to 16 splits 0.93 ... 0.96, more, two batches of a wave, 0.88 ... 0.94; five to eight rows
+// 0.92 ... 0.96, more 0.5 ... 0.8; rows between the buckets, up to four, 0.85 ... 1.00.  B11 H16 H_kv4 Nk1142 d128 in 5 splits 11.10 / 10.50 us, B6 H4 H_kv1 Nk2240 d64 in
+// 9 7.89 / 7.24, B1 H16 H_kv4 Nk2957 d64 in 12 7.82 / 7.23; B4 H16 H_kv4 Nk4800 d64 in 13 9.76 / 10.58, B8 H8 H_kv2 Nk8000 d128 in 16 15.67 / 16.90, B6 H4 H_kv1 Nk8132
+// d32 in 32 7.45 / 9.11, B6 H32 H_kv4 (eight rows) Nk1792 d64 in 7 8.61 / 9.48.
+inline bool rows_form_merges(const FwdArgs& a)
+{
+    return a.Nq <= 4 && a.d % 32 == 0 && a.num_splits <= (a.d == 32 ? 8 : 12) && a.num_splits * a.d <= 1024;
 }
 // split count with which such a launch fills the GPU, 0 if there is none that rows_form_fits
 inline int rows_form_splits(long long slices, int rows, int d, int Nk)
