@@ -148,7 +148,7 @@ constexpr float kNothingSeen = -3.402823466e38f;
 // kVarFold (no other feature): the rows are the query heads of a K/V head, see row_position in common.h.
 // kVarShort (D >= 64, not kVarFullD, kVarEvery or kVarFold): rows of at most D - 16 elements, see FwdCfg::kShort.
 // kVarRows (with kVarNarrow; no other feature but kVarFold): launches of few rows per slice, whole or in splits, see kRows below.
-// kVarManyRows (with kVarRows): more than 32 rows, whose row blocks ask for the same tiles, or tiles that the caches serve (rows_read_once).
+// kVarManyRows (with kVarRows): more than 32 rows, whose row blocks ask for the same tiles.
 constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarStamp = 16, kVarAlibiLeft = 32, kVarKvOnce = 64,
               kVarEvery = 128, kVarNarrow = 256, kVarFold = 512, kVarPair = 1024, kVarShort = 2048, kVarRows = 4096, kVarManyRows = 8192;
 
@@ -239,8 +239,9 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     static_assert(!kNarrow || (kDma && NB == 1 && !kKvOnce), "narrow instances");
     // The narrow form for launches of few rows per slice (fwd_uses_rows says which), in splits too: their partial results leave the merge
     // as whole rows of floats, and where a caller has brought counters (combine.h) and the rows are four or fewer, the last work-group
-    // of a slice merges the splits.  With up to 32 rows nobody else asks for the tiles, and the requests are non-temporal where that pays
-    // (rows_read_once).
+    // of a slice merges the splits.  With up to 32 rows nobody else asks for the tiles, and the requests are non-temporal.
+    // Ordinary / non-temporal, time over time, over 1000 random launches: K and V that no cache holds, up to 8 MiB 1.02 ... 1.04, 40 MiB 1.03 ... 1.05, 128 MiB 1.05 ... 1.09, more
+    // 1.11; called again and again with the same K and V, up to 20 MiB 0.99 ... 1.00, 20-40 MiB (the L2 holds 32) 0.94 ... 0.99, more 0.98 ... 1.06.
     constexpr bool kRows = (VAR & kVarRows) != 0, kRowsOnce = kRows && (VAR & kVarManyRows) == 0;
     static_assert(!kRows || (kNarrow && !kAlibi && !kDropout), "few rows");
     constexpr bool kFold = (VAR & kVarFold) != 0;
@@ -1696,14 +1697,12 @@ inline bool fwd_uses_rows(const FwdArgs& a, int variant)
 }
 // Whether the last work-group of such a launch to arrive at a slice's counter merges its partial results.  A merge by a launch of its own takes 1.5-2 us,
 // which the arrival (a store, an atomic and a load from memory in a row) and partial results written through and read past the L2 use up
-// soon.  Its own launch / here, time over time, over 451 random launches of whole buckets: up to four rows and 12 splits, by splits * d up to 512 / 768 /
-// 1024 / 1536, 1.04 / 1.04 / 1.02 / 1.00 (d = 32, up to 8 splits 1.02, 9 to 12 0.99); 13 to 16 splits 0.93 ... 0.96, more, two batches of a wave, 0.88 ... 0.94; five to eight rows
-// 0.92 ... 0.96, more 0.5 ... 0.8; rows between the buckets, up to four, 0.85 ... 1.00.  B11 H16 H_kv4 Nk1142 d128 in 5 splits 11.10 / 10.50 us, B6 H4 H_kv1 Nk2240 d64 in
-// 9 7.89 / 7.24, B1 H16 H_kv4 Nk2957 d64 in 12 7.82 / 7.23; B4 H16 H_kv4 Nk4800 d64 in 13 9.76 / 10.58, B8 H8 H_kv2 Nk8000 d128 in 16 15.67 / 16.90, B6 H4 H_kv1 Nk8132
-// d32 in 32 7.45 / 9.11, B6 H32 H_kv4 (eight rows) Nk1792 d64 in 7 8.61 / 9.48.
+// soon.  Its own launch / here, time over time, over 230 random launches of whole buckets, K and V from memory (called again with the same ones 1 % more):
+// two to four rows, up to 4 / 5 to 8 splits d32 1.07 / 1.05, d64 1.05 / 1.05, d96 1.03 / 1.04, d128 1.03 / 1.03, none below 1.00; 9 to 12 0.98 ... 1.04, 13 to 16 0.89 ... 1.00, more,
+// two batches of a wave, 0.79 ... 0.95; five to eight rows 0.98 ... 0.99 / 0.96 ... 0.98, more 0.5 ... 0.8; rows between the buckets, up to four, 0.85 ... 1.00.
 inline bool rows_form_merges(const FwdArgs& a)
 {
-    return a.Nq <= 4 && a.d % 32 == 0 && a.num_splits <= (a.d == 32 ? 8 : 12) && a.num_splits * a.d <= 1024;
+    return a.Nq <= 4 && a.d % 32 == 0 && a.num_splits <= 8;
 }
 // split count with which such a launch fills the GPU, 0 if there is none that rows_form_fits
 inline int rows_form_splits(long long slices, int rows, int d, int Nk)
@@ -1719,20 +1718,6 @@ inline int rows_form_splits(long long slices, int rows, int d, int Nk)
     if (s < 2) return 0;
     const int per = (int)((n_blocks + s - 1) / s), even = (n_blocks + per - 1) / per;  // all of them with keys
     return even >= 2 && rows_form_fits(slices, rows, d, Nk, even, 128 * per) ? even : 0;
-}
-
-// Whether such a launch asks for its tiles with non-temporal requests (kRowsOnce in fwd_kernel).  Up to 32 rows nobody else asks for them; but
-// rows that are no multiple of 64 bytes share lines with their neighbours, which other requests ask for, and where K and V fit the 32 MiB of L2
-// those are still there.  Ordinary / non-temporal over 575 random launches of d = 31 ... 112, by bytes of K and V: 12-16 MiB 0.91 ... 0.96, 18-20 0.91 ... 0.98,
-// 20-22 0.95 ... 1.02, 22-24 1.00 ... 1.03, 30-48 1.02 ... 1.07, above 1.04 ... 1.10: in splits B18 H4 H_kv1 Nk7763 d31 (16 MiB)
-// 9.59 / 10.50 us, B2 H32 H_kv8 Nk3997 d72 (18) 8.96 / 9.40, B5 H64 H_kv8 Nk5952 d40 (36) 12.84 / 12.04; whole B25 H32 H_kv8 Nk896 d31 (21) 8.07 / 8.45, B24 Nk1282
-// d40 (38) 10.95 / 10.40.  With fewer than 160 work-groups 0.95 ... 1.02 at any size, ordinary ones mostly the faster.
-constexpr long long kOnceBytes = 22 << 20;
-inline bool rows_read_once(const FwdArgs& a, int bucket_d)
-{
-    if (a.Nq > kRowsLimit) return false;
-    const long long slices = (long long)a.B * a.H;
-    return a.d == bucket_d || (slices * a.num_splits >= 160 && 4 * slices * a.Nk * a.d >= kOnceBytes);
 }
 
 template <int D, int VAR>
@@ -1846,17 +1831,16 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
     };
     if (!fwd_needs_every_instance(a, variant) && fwd_uses_rows(a, variant)) {
         // By row length and alignment like the narrow ones; in the bucket of 32 columns rows at any alignment serve every shorter length.  When they served
-        // all shorter lengths -> now, us: B4 H16 H_kv4 Nk6004 d40 in 16 splits 11.90 -> 11.06, B2 H32 H_kv8 Nk3264 d72 in 13 11.17 -> 10.47, B2 H4 Nq20 Nk6190 d80
-        // in 25 11.01 -> 9.49, B2 H16 H_kv2 Nq8 Nk9000 d112 in 24 13.00 -> 12.27, B2 H8 Nq11 Nk11200 d100 in 15 19.82 -> 19.60; whole B20 H64 H_kv8 Nk5263 d80 46.66
-        // -> 46.52.  Rows of whole chunks give 4 % of it, short ones 1-2, ordinary requests below rows_read_once's line 3-8.
+        // all shorter lengths -> now, us, K and V from memory: B2 H4 Nq20 Nk6190 d80 in 25 splits 11.10 -> 9.85, B2 H16 H_kv2 Nq8 Nk9000 d112 in 24 14.01 -> 12.72, B2 H8
+        // Nq11 Nk11200 d100 in 15 19.88 -> 19.25, whole B20 H64 H_kv8 Nk5263 d80 46.62 -> 46.62; rows of whole chunks give 4 % of it, short ones 1-2.
         auto rows = [&](auto var) {
-            auto folded = [&](auto cached) {
-                constexpr int V = ST | decltype(var)::value | decltype(cached)::value;
+            auto folded = [&](auto many) {
+                constexpr int V = ST | decltype(var)::value | decltype(many)::value;
                 if (a.fold_rows) return (int)launch_fwd_rows_instance<D, V | kVarFold>(a, st);
                 if constexpr ((V & kVarFullD) != 0) return (int)launch_fwd_rows_instance<D, V>(a, st);
                 else return (int)by_length([&](auto sh) { return launch_fwd_rows_instance<D, V | decltype(sh)::value>(a, st); });
             };
-            return rows_read_once(a, D) ? folded(std::integral_constant<int, 0>{}) : folded(std::integral_constant<int, kVarManyRows>{});
+            return a.Nq <= kRowsLimit ? folded(std::integral_constant<int, 0>{}) : folded(std::integral_constant<int, kVarManyRows>{});
         };
         if (a.d == D) return rows(std::integral_constant<int, kVarVec | kVarFullD>{});
         if constexpr (D > 32) {

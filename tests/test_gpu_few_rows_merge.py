@@ -11,12 +11,10 @@ ROWS = 1 << 12
 
 # B, H, Hk, Nq, Nk, d, splits, launches
 LINES = [
-    (8, 32, 8, 1, 4000, 128, 4, 1), (4, 32, 8, 1, 4000, 128, 8, 1), (7, 16, 4, 1, 4000, 128, 9, 2),      # 1024 floats per row
-    (25, 4, 1, 1, 4000, 96, 10, 1), (23, 4, 1, 1, 4000, 96, 11, 2),
-    (1, 32, 8, 1, 4000, 64, 12, 1), (1, 32, 8, 1, 4000, 64, 13, 2),                                      # 12 splits
-    (2, 32, 8, 1, 4000, 32, 8, 1), (2, 32, 8, 1, 4000, 32, 9, 2),                                        # d = 32: 8
-    (6, 8, 8, 4, 4000, 64, 4, 1), (6, 8, 8, 5, 4000, 64, 4, 2), (12, 8, 4, 2, 4000, 128, 4, 1), (12, 8, 4, 3, 4000, 128, 4, 2),  # four rows
-    (8, 32, 8, 1, 4000, 100, 4, 2), (8, 32, 8, 1, 4000, 120, 4, 2), (4, 32, 8, 1, 4000, 40, 8, 2), (4, 32, 8, 1, 4000, 31, 8, 2),
+    (4, 32, 8, 1, 4000, 128, 8, 1), (7, 16, 4, 1, 4000, 128, 9, 2), (25, 4, 1, 1, 4000, 96, 8, 1), (25, 4, 1, 1, 4000, 96, 9, 2),  # eight splits
+    (1, 32, 8, 1, 4000, 64, 8, 1), (1, 32, 8, 1, 4000, 64, 9, 2), (2, 32, 8, 1, 4000, 32, 8, 1), (2, 32, 8, 1, 4000, 32, 9, 2),
+    (6, 8, 8, 4, 4000, 64, 4, 1), (6, 8, 8, 5, 4000, 64, 4, 2), (12, 8, 4, 2, 4000, 128, 4, 1), (12, 8, 4, 3, 4000, 128, 4, 2),    # four rows
+    (8, 32, 8, 1, 4000, 100, 4, 2), (8, 32, 8, 1, 4000, 120, 4, 2), (4, 32, 8, 1, 4000, 40, 8, 2), (4, 32, 8, 1, 4000, 31, 8, 2),  # whole buckets
 ]
 
 
@@ -31,7 +29,7 @@ def test_lines():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,H,Hk,Nq,d,S", [(8, 32, 8, 1, 128, 4), (6, 16, 4, 1, 128, 8), (8, 32, 8, 1, 96, 4), (20, 8, 2, 1, 96, 5), (8, 16, 8, 2, 96, 3), (16, 6, 6, 3, 128, 2),
-                                           (1, 32, 8, 1, 64, 12), (2, 8, 8, 4, 64, 5), (1, 32, 8, 1, 32, 8), (3, 8, 4, 2, 32, 6)])
+                                           (1, 32, 8, 1, 64, 8), (2, 8, 8, 4, 64, 5), (1, 32, 8, 1, 32, 8), (3, 8, 4, 2, 32, 6)])
 def test_one_launch(fa, oracle, B, H, Hk, Nq, d, S):
     """Against the oracle, and the same bits as the merge by a launch of its own, call after call; the counters end at zero.  A last tile of three
     keys, and splits of unequal length."""
