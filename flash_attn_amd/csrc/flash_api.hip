@@ -523,14 +523,12 @@ int run_splitkv(const flash_params* p, int splits, hipStream_t st)
     fa::FwdArgs a;
     fill_args(p, splits, &a);
     const int route = splitkv_route(p, &a);
-    // (a slice of the decode kernel has one row per query head, which its last work-group merges in a microsecond)
-    if (route == kRouteStream && splits > 1 && p->split_counters && (long long)p->B * p->H <= p->split_counters_len)
-        a.counters = p->split_counters;
-    // Rows that a work-group merges: those of a slice where the split launch may do it, with counters given or not, so that a result is the
-    // same bit by bit either way; one behind a launch of its own.
-    const bool in_launch = route == kRouteTiled && !needs_every_instance(p) && fa::fwd_uses_rows(a, tiled_variant(p)) && fa::rows_form_merges(a);
-    if (in_launch && splits > 1 && p->split_counters && (long long)a.B * a.H <= p->split_counters_len) a.counters = p->split_counters;
-    a.combine_waves = fa::combine_waves_for(splits, route == kRouteStream ? fa::decode_heads_per_group(a.kv_group) : in_launch ? a.Nq : 1);
+    // Few rows per slice are merged by the split launch itself: the decode kernel's, one per query head, and up to four of the tiled kernel's
+    // (fa::rows_form_merges).  Either way the rows of a work-group decide the waves per row, so that a result is the same bit by bit with and without counters.
+    const bool merges = route == kRouteStream ||
+                        (!needs_every_instance(p) && fa::fwd_uses_rows(a, tiled_variant(p)) && fa::rows_form_merges(a));
+    if (merges && splits > 1 && p->split_counters && (long long)p->B * p->H <= p->split_counters_len) a.counters = p->split_counters;
+    a.combine_waves = fa::combine_waves_for(splits, !merges ? 1 : route == kRouteStream ? fa::decode_heads_per_group(a.kv_group) : a.Nq);
     // (a launch is limited to 2^32 - 1 threads: a work-group per row reaches 2^24 rows, a wave per row 2^26)
     if ((long long)p->B * p->H * p->Nq >= 1LL << 24) a.combine_waves = 1;
     const int e = route == kRouteStream ? record_hip(fa::launch_decode_split(a, st)) : launch_tiled(p, a, st);

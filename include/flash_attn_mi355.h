@@ -119,10 +119,12 @@ typedef struct flash_params {
      * pair around its launches (src/main.cu:195-213). */
     uint64_t *stage_stamps_out;
     /* Optional: device memory of split_counters_len 32-bit words, all zero, which lets flash_forward_splitkv merge the
-     * partial results of few query rows (16 or fewer per K/V head or query head) inside the split kernel instead of in a
-     * second launch; the results are the same bit by bit.  The call leaves the words zero.  Calls that may overlap on the GPU must
-     * not share them: one such array per stream will do (and none for calls captured into a graph that may be replayed
-     * beside others).  Used where there are at least B * H words; NULL, or fewer words: the second launch. */
+     * partial results inside the split kernel instead of in a second launch where that is the faster way: one query row per head,
+     * less than four query heads per K/V head (any number with ALiBi or a left window), and up to four rows per K/V head of
+     * heads of 32, 64, 96 or 128 elements in up to eight splits.  The results are the same bit by bit.  The call leaves the words zero.
+     * Calls that may overlap on the GPU must not share them: one such array per stream will do (and none for calls captured
+     * into a graph that may be replayed beside others).  Used where there are at least B * H words; NULL, or fewer
+     * words: the second launch. */
     uint32_t *split_counters;
     int split_counters_len;
 } flash_params;

@@ -18,13 +18,21 @@ LINES = [
 ]
 
 
-def recorded(cases):
-    return record([dict(call(*c[:6], num_splits=c[6]), entry="splitkv", split_counters=0xB00000, split_counters_len=c[0] * c[1]) for c in cases])
+def recorded(cases, missing=0):
+    return record([dict(call(*c[:6], num_splits=c[6]), entry="splitkv", split_counters=0xB00000, split_counters_len=c[0] * c[1] - missing)
+                   for c in cases])
 
 
 def test_lines():
     for c, r in zip(LINES, recorded(LINES)):
         assert r["rc"] == 0 and r["splits"] == c[6] and r["launches"][0]["variant"] & ROWS and len(r["launches"]) == c[7], (c, r)
+
+
+def test_words():
+    """A word per query head, however many of them share a slice; with one less, a launch of its own."""
+    cases = [c for c in LINES if c[7] == 1] + [(2, 16, 16, 1, 4000, 64, 8, 1), (2, 16, 8, 1, 4000, 64, 8, 1)]
+    assert [len(r["launches"]) for r in recorded(cases)] == [1] * len(cases)
+    assert [len(r["launches"]) for r in recorded(cases, missing=1)] == [2] * len(cases)
 
 
 @pytest.mark.gpu
