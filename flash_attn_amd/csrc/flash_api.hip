@@ -379,7 +379,7 @@ int auto_splits_tiled_uncached(const flash_params* p, int n_blocks, bool decode)
     // Launches of few rows (fa::fwd_uses_rows; decode calls come here with the heads as rows) have a count of their own.  Never a higher
     // one, and never one where the launch was whole: who brings a workspace for the estimate's count has enough for this one.
     const int few = !every && fa::rows_form_serves(launch, tiled_variant(p)) ? fa::rows_form_splits(slices, Nq, p->d, p->Nk) : 0;
-    return few > 0 && few < best_s ? few : best_s;
+    return few > 0 && few < best_s && fa::rows_form_lowers(slices, Nq, p->d, p->Nk, few, best_s) ? few : best_s;
 }
 
 int resolve_splits(const flash_params* p)

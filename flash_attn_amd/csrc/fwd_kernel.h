@@ -1704,7 +1704,10 @@ inline bool rows_form_merges(const FwdArgs& a)
 {
     return a.Nq <= 4 && a.d % 32 == 0 && a.num_splits <= 8;
 }
-// split count with which such a launch fills the GPU, 0 if there is none that rows_form_fits
+// Split count with which such a launch fills the GPU, 0 if there is none that rows_form_fits.  Where the estimate splits: whole from 144 slices on (128 ... 143 0.96 ... 1.09
+// times as fast as its count, 144 ... 168 1.00 ... 1.15); not up to 1280 keys of 16 slices or more, which come out in two to five splits of 256 keys and gain nothing (720 ... 1268
+// keys d31 0.95 ... 1.01, d64 0.98 ... 1.02, d40 1.00 ... 1.05; 1407 ... 1520 d40, d32 1.05).  More than 32 rows with d < 32 take 256 work-groups, one per CU: 1.03 ... 1.16 there, 0.84 ... 1.00
+// with two per CU (more than 1024 keys per split 0.54 ... 1.0 either way).
 inline int rows_form_splits(long long slices, int rows, int d, int Nk)
 {
     const int n_blocks = (Nk + 127) / 128;
@@ -1712,12 +1715,28 @@ inline int rows_form_splits(long long slices, int rows, int d, int Nk)
     if (rows > 512 || groups < 1) return 0;
     if (rows <= 32 && groups >= 144 && groups <= kNumCus && Nk >= 512) return 1;
     if (rows <= 32 && slices >= 16 && Nk <= 1280) return 0;
-    long long s = (d <= 32 ? 2 * kNumCus : kNumCus) / groups;
+    long long s = (d == 32 || (d < 32 && rows <= kRowsLimit) ? 2 * kNumCus : kNumCus) / groups;
     if (s > (n_blocks + 1) / 2) s = (n_blocks + 1) / 2;
     if (s > 32) s = 32;
     if (s < 2) return 0;
     const int per = (int)((n_blocks + s - 1) / s), even = (n_blocks + per - 1) / per;  // all of them with keys
     return even >= 2 && rows_form_fits(slices, rows, d, Nk, even, 128 * per) ? even : 0;
+}
+
+// Whether it is the better one where the estimate for 128-row work-groups, whose count is never lower than this one, says `estimate`.  Time at the
+// estimate's count / here over 760 random launches with such a count, K and V from memory:
+//  * up to 32 rows, d = 64: 256 keys per split 0.93 ... 0.98 (1.00 ... 1.09 where the launch merges itself), more keys, one work-group per CU by the estimate, whose splits are
+//    then more than 32, 0.98 ... 1.26, two per CU 0.93 ... 1.03, 0.985 in the mean; d = 96, two per CU, 0.97 ... 1.01; but d = 128 0.98 ... 1.07, d = 32 0.98 ... 1.22, rows between
+//    the buckets 1.02 ... 1.25.  B8 H16 H_kv2 Nk1739 d64 7.2 us in 14 splits, 7.6 in 7, B8 H64 H_kv8 Nk5941 d64 19.8 in 8, 20.4 in 4, B13 H32 H_kv4 Nk5210 d96 21.1 in 9,
+//    21.8 in 4; B6 H8 H_kv1 Nk31104 d64 16.0 in 41, 13.6 in 31.
+//  * more rows, two row blocks, 256 keys per split, above d = 32, 96 ... 159 work-groups 0.90 ... 1.02 (33 to 50 rows; 56 to 59 rows up to 1.10), 160 on 1.02 ... 1.05 (B8 H4 H_kv1 Nq9 Nk1306
+//    d128 9.4 in 11, 10.4 in 6; B17 H4 H_kv4 Nq57 Nk1700 d128 1.05 times as fast).
+inline bool rows_form_lowers(long long slices, int rows, int d, int Nk, int splits, int estimate)
+{
+    const int n_blocks = (Nk + 127) / 128, keys_per_split = 128 * ((n_blocks + splits - 1) / splits);
+    if (rows > kRowsLimit) return d <= 32 || rows > 64 || keys_per_split > 256 || 2 * slices * splits >= 160;
+    if (splits == 1 || (d != 64 && d != 96)) return true;
+    return (rows <= 4 && splits <= 8) || (slices * estimate <= kNumCus && keys_per_split >= 512);
 }
 
 template <int D, int VAR>
