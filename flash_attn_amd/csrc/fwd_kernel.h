@@ -1674,8 +1674,13 @@ inline hipError_t launch_fwd_narrow_instance(const FwdArgs& a, hipStream_t st)
 //    rows, so that the tiles per wave are bounded.  B2 H8 Nq64 Nk4096 d128 17.1 / 14.2, B4 H4 Nq128 Nk4096 20.9 / 17.9, B1 H8 Nq128 Nk16384 29.3 / 26.4,
 //    B1 H4 Nq512 Nk4096 20.7 / 15.3, B1 H8 H_kv4 Nq120 Nk6000 18.6 / 14.2, B1 H16 H_kv2 Nq40 Nk9000 (folded) 17.0 / 13.5, B1 H8 Nq128 Nk8192 d80 17.4 / 14.8, B1
 //    H2 Nq128 Nk4096 d64 10.3 / 8.5; with more tiles than that: B4 H4 Nq130 Nk7000 d128 (10) 25.8 / 27.8, B2 H8 Nq100 Nk8000 d64 (8) 16.0 / 16.4, B1 H12
-//    H_kv2 Nq100 Nk7000 d100 (6) 18.1 / 19.9, B1 H32 Nq128 Nk16384 d128 (32) 63 / 80.  Launches of fewer than 96 work-groups, which only a
-//    caller's own split count makes, are launched as they always were.
+//    H_kv2 Nq100 Nk7000 d100 (6) 18.1 / 19.9, B1 H32 Nq128 Nk16384 d128 (32) 63 / 80.  Fewer than 96 work-groups
+//    (0.92 ... 1.13) stay as they are.
+//  * The other lines, 1260 random launches, old form at the estimate's count / this one.  At that count the form gains whatever the number of slices and work-groups: 96 to 191
+//    of them above d = 64 1.05 ... 1.22 times as fast, one to three slices 1.05 ... 1.22, 33 to 64 splits 1.02 ... 1.17 in the mean; but such launches are rare, and most calls of few
+//    slices come here with a count cut to 32: one to three slices, 32 to 96 work-groups, 0.80 ... 1.01 at whole buckets, 4 slices on 0.90 ... 0.94 above d = 64 up to 143 work-groups,
+//    from 144 on 1.00 ... 1.03, up to d = 64 0.97 up to 95, 1.01 ... 1.07 beyond.  Whole, whole buckets: 64 to 95 slices 0.97 ... 1.02, 96 to 127 1.00 ... 1.04 (single ones 0.93), 128 to
+//    159 1.05 ... 1.07, 160 to 256 1.09 ... 1.13.
 inline bool rows_form_fits(long long slices, int rows, int d, int Nk, int splits, int keys_per_split)
 {
     const int places = d <= 32 ? 2 * kNumCus : kNumCus;
@@ -1779,8 +1784,12 @@ inline hipError_t launch_fwd_rows_instance(const FwdArgs& a, hipStream_t st)
 //    random launches cross over.  Up to 384 work-groups (unpaired / paired): N1238 d64 17.9 / 15.7 us, N1117 d80 19.2 / 16.0, N1184 d100 23.1 / 19.5, N1000
 //    d40 14.7 / 13.7; with dropout N1267 d64 27.3 / 22.7, N640 d64 15.5 / 13.2, N1021 d128 28.7 / 24.0, N680 d128 20.8 / 18.3; below the lines N675 d64
 //    11.35 / 11.46, N926 d96 16.4 / 17.3, N660 d128 17.8 / 20.6, with dropout N668 d32 13.4 / 13.4, N556 d128 20.3 / 23.2.  More of them: B1 H16 N4096
-//    d128 83.1 / 75.2, B4 H8 N2000 d96 36.1 / 34.2, N1645 d96 (390 of them) 28.5 / 25.9, N1672 d80 (448) 26.4 / 24.9, B3 H12 N1777 d80 31.1 / 30.4, B4 H8 N2000 d80 with dropout 44.6 / 40.9, N1246 d64 (400 of them) 17.4 / 16.4;
+//    d128 83.1 / 75.2, B4 H8 N2000 d96 36.1 / 34.2, N1645 d96 (390 of them) 28.5 / 25.9, N1672 d80 (448) 26.4 / 24.9, B4 H8 N2000 d80 with dropout 44.6 / 40.9, N1246 d64 (400 of them) 17.4 / 16.4;
 //    below N1424 d80 24.7 / 26.8, N1785 d96 (504) 32.6 / 33.0, N1227 d64 with dropout 25.8 / 25.9.  Above 512 it loses (B5 H8 N1777 d100 42.5 / 47.8, 560 of them).
+//    At 64 < d <= 96, 449 to 512 of them, d <= 80 has the instances for shorter rows and crosses over earlier: 220 launches of d = 72, 80 / 88, 96, unpaired / paired, time over
+//    time, with K and V from memory and again with the same ones, N1650-1700 0.975, 0.998 / 0.956, 0.979, N1760-1855 0.991, 1.011 / 0.971, 0.994, N1880-1910 1.022, 1.048 / 1.006,
+//    1.028; their number decides as much (450 to 480 of them up to 0.04 above, 490 to 510 below): N1700 d80 (490) 31.9 / 33.9, N1760 d72 (476) 31.7 / 31.2, N1825 d80 (480) 31.7 / 30.4;
+//    N1760 d96 (490) 36.5 / 39.2, N1825 d88 (465) 35.3 / 36.2.
 inline long long following_keys(int d, long long groups, bool dropout)
 {
     const int bucket = (d + 31) / 32;
