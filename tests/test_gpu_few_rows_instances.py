@@ -36,3 +36,14 @@ def test_few_rows_of_shorter_heads(fa, oracle, d, B, H, Hk, Nq):
     kr, vr = (t.repeat_interleave(H // Hk, dim=1).contiguous() for t in (k, v))
     O, L = oracle_forward_batched(oracle, q, kr, vr, causal=True)
     check_o_lse(*fa.flash_forward_splitkv(q, k, v, num_splits=SPLITS, causal=True), O, L)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [31, 40, 64, 96, 100, 128])
+def test_last_split_of_one_key(fa, oracle, d):
+    B, H, Nq, Nk, S = 3, 16, 32, 3 * 384 + 1, 4
+    r, = record([dict(call(B, H, H, Nq, Nk, d, causal=True, num_splits=S), entry="splitkv")])
+    assert r["launches"][0]["variant"] & ROWS and r["splits"] == S
+    q, k, v = randn_f16_gpu((B, H, Nq, d), 1), randn_f16_gpu((B, H, Nk, d), 2), randn_f16_gpu((B, H, Nk, d), 3)
+    O, L = oracle_forward_batched(oracle, q, k, v, causal=True)
+    check_o_lse(*fa.flash_forward_splitkv(q, k, v, num_splits=S, causal=True), O, L)
