@@ -1771,10 +1771,11 @@ inline hipError_t launch_fwd_rows_instance(const FwdArgs& a, hipStream_t st)
 //    up to 512 work-groups, unpaired / paired): windows B1 H8 N3835 d40 of 1390 keys 21.3 / 17.4 us, B4 H2 N3551 d64 of 1858 26.8 / 21.8, B2 H8 N1533
 //    d64 of 196 9.2 / 8.6, B1 H8 N1792 d96 of 1052 21.0 / 17.5, B1 H12 N1281 d100 of 1108 30.3 / 25.0, B2 H4 N1230 d128 of 941 22.1 / 19.5; causal N3502 d72
 //    46.1 / 37.2, N848 d32 11.1 / 9.4; up to 512 of them under the lines without dropout (next but one) N2253 d100 48.6 / 38.5, N7577 d64 88.0 / 72.2, N875 d40 13.6 / 11.6;
+//    from six on where no window cuts (290 to 320 keys, causal, unpaired / paired, time over time d64 0.97 ... 1.01, d72-96 0.96 ... 0.99; 337 on 1.01 ... 1.07: N320 d64 7.70 / 7.91 us);
 //    left out: d128 windows of 159 ... 396 keys 11.0 / 11.1, of 257 to 512 work-groups 15.9 / 20.2.  Two-sided ALiBi, and with dropout, stay as they are.
 //  * under a window that ends at the row, whole, without dropout: from 5 tiles on below d = 128, too (130 random launches, unpaired / paired, us): N4064 d32 of 219 keys 8.03 /
 //    6.78, N904 d40 of 184 8.15 / 7.53, N3367 d64 of 212 9.48 / 8.80, N1554 d64 of 146 8.32 / 8.07, N1911 d72 of 208 10.51 / 9.58, N907 d100 of 231 12.50 / 11.69, N1126 d112 of
-//    159 10.34 / 9.99; but d128 of 202 12.74 / 13.77, of 293 14.44 / 14.85, and without a window N300 d96 7.94 / 8.42.  At 32 < d <= 64 up to 400 work-groups,
+//    159 10.34 / 9.99 (five tiles at 96 < d < 128 up to 128 work-groups; 192 to 240 of them 0.95 ... 0.99, six tiles 1.00 ... 1.05: N1984 d112 of 192 12.23 / 12.82); but d128 of 202 12.74 / 13.77, of 293 14.44 / 14.85, and without a window N300 d96 7.94 / 8.42.  At 32 < d <= 64 up to 400 work-groups,
 //    from 7 tiles on, without ALiBi: B1 H8 N4178 d64 of 480 12.02 / 10.58, B2 H32 N623 d64 of 346 11.27 / 10.21, B1 H12 N4037 d40 of 878 21.5 / 20.2, B4 H2 N6294 d64 of 1121 27.9 /
 //    25.9; with 5 tiles N791 d40 8.93 / 9.06, d32 of 417 10.84 / 11.19, and above d = 64 0.7 ... 0.9 times as fast (d72 of 163 12.3 / 16.5).
 //  * up to 32 rows only one wave of four has any, and a second one beside it gained 7-11 % at d = 32, but lost 4 % at
@@ -1782,7 +1783,8 @@ inline hipError_t launch_fwd_rows_instance(const FwdArgs& a, hipStream_t st)
 //  * causal, unsplit and up to twice as many: two work-groups of a CU side by side last as long as the longer one, whose SIMDs
 //    have one wave each once its light neighbour is done; as paired ones they follow each other, eight waves at a time.  The lines lie where 150
 //    random launches cross over.  Up to 384 work-groups (unpaired / paired): N1238 d64 17.9 / 15.7 us, N1117 d80 19.2 / 16.0, N1184 d100 23.1 / 19.5, N1000
-//    d40 14.7 / 13.7; with dropout N1267 d64 27.3 / 22.7, N640 d64 15.5 / 13.2, N1021 d128 28.7 / 24.0, N680 d128 20.8 / 18.3; below the lines N675 d64
+//    d40 14.7 / 13.7; with dropout N1267 d64 27.3 / 22.7, N640 d64 15.5 / 13.2, N1021 d128 28.7 / 24.0, N680 d128 20.8 / 18.3
+//    (above d = 64 and 324 of them from 896 on: N704 d128 22.2 / 24.2, N822 d80 22.3 / 24.5, N842 d128 28.4 / 30.9, N749 d128 25.5 / 26.4, N921 d80 23.6 / 23.8; 1.00 ... 1.10 times as fast beyond); below the lines N675 d64
 //    11.35 / 11.46, N926 d96 16.4 / 17.3, N660 d128 17.8 / 20.6, with dropout N668 d32 13.4 / 13.4, N556 d128 20.3 / 23.2.  More of them: B1 H16 N4096
 //    d128 83.1 / 75.2, B4 H8 N2000 d96 36.1 / 34.2, N1645 d96 (390 of them) 28.5 / 25.9, N1672 d80 (448) 26.4 / 24.9, B4 H8 N2000 d80 with dropout 44.6 / 40.9, N1246 d64 (400 of them) 17.4 / 16.4;
 //    below N1424 d80 24.7 / 26.8, N1785 d96 (504) 32.6 / 33.0, N1227 d64 with dropout 25.8 / 25.9.  Above 512 it loses (B5 H8 N1777 d100 42.5 / 47.8, 560 of them).
@@ -1794,7 +1796,7 @@ inline long long following_keys(int d, long long groups, bool dropout)
 {
     const int bucket = (d + 31) / 32;
     constexpr int kPlain[4] = {704, 704, 960, 1104}, kDropout[4] = {960, 608, 608, 640};
-    if (groups <= 384) return dropout ? kDropout[bucket - 1] : kPlain[bucket - 1];
+    if (groups <= 384) return !dropout ? kPlain[bucket - 1] : groups > 324 && bucket > 2 ? 896 : kDropout[bucket - 1];
     if (dropout) return 1280;
     if (bucket == 3) return groups <= 448 ? 1600 : d <= 80 ? 1760 : 1856;
     return bucket <= 2 && groups <= 416 ? 1184 : 1856;
@@ -1810,7 +1812,8 @@ inline bool fwd_uses_pair(const FwdArgs& a, int bucket_d, int feat)
         return groups <= 2 * kNumCus && a.Nk >= following_keys(a.d, groups, dropout);
     const bool window = left + right + 128 < a.Nk && right == 0 && a.num_splits == 1 && !dropout;
     if (groups > kNumCus) return window && !alibi && bucket_d == 64 && groups <= 400 && left + 128 > 6 * 64;
-    const long long keys = a.d < 128 && (alibi || window) ? 4 * 64 + 1 : 8 * 64;
+    const bool six = alibi ? !window : a.d > 96 && groups > 128;  // tiles, where five are not enough
+    const long long keys = a.d < 128 && (alibi || window) ? (six ? 5 * 64 + 1 : 4 * 64 + 1) : 8 * 64;
     return a.Nk >= keys * a.num_splits && left + right + 128 >= keys;
 }
 
