@@ -48,8 +48,8 @@ __device__ __forceinline__ float wave_max(float v)
 // The last one leaves the counter at zero for the next launch on the stream.
 // Two launches -> one, GPU time per call: decode B1 H4 Nk487 d128 in 4 splits 7.1 -> 5.5 us, B3 H12 Nk1152 d64 in 5 splits
 // 7.8 -> 6.6, B1 H32 Nk4096 d128 in 8 splits 15.4 -> 14.7 (the arrival costs a store, an atomic and a load from memory in a
-// row, about 2 us).  The tiled kernels, whose rows leave in 16-byte pieces, do not do this: written through piece by
-// piece their partial results took longer than the second launch (B3 H8 H_kv1 Nk7296 d64: 9.7 -> 14.2 us).
+// row, about 2 us).  Of the tiled kernels those for few rows do it, for up to four rows in up to eight splits (rows_form_merges in fwd_kernel.h); the others
+// have many rows, whose partial results, written through piece by piece, took longer than the second launch (B3 H8 H_kv1 Nk7296 d64: 9.7 -> 14.2 us).
 __device__ __forceinline__ void store_partial(float* p, float v, bool shared)
 {
     if (shared) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

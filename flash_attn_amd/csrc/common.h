@@ -147,12 +147,12 @@ static_assert(offsetof(Packed, scale_log2) + sizeof(float) <= kCheapArgs && size
 static_assert(FLASH_MAX_SPLITS_K < 256, "eight bits");
 
 // Arguments of launches of few rows per slice (kVarRows of fwd_kernel.h), whose last work-groups may merge the partial results: 112 bytes
-// hold results and partial results both.  One query head per K/V head; order of the work-groups: rows_item.
+// hold results and partial results both.  Up to 32 rows, or folded: one query head per K/V head; order of the work-groups: rows_item.
 constexpr int kRowsLimit = 32;  // rows of a work-group
 struct PackedRows {
     uint32_t mul_slices, mul_row_blocks;
     int slices;
-    uint32_t shifts;  // of by_slices, by_row_blocks, by_kv_group (folded: by_fold): five bits each; bit 15: causal, bit 16: combine_waves is 4; fold_rows (64 at most, kFoldRows): eight bits from 24 on
+    uint32_t shifts;  // of by_slices, by_row_blocks, by_kv_group (folded: by_fold): five bits each; bit 15: causal, bit 16: combine_waves is 4 (the kernel merges with one wave per row whatever it says: up to eight splits are one batch); fold_rows (64 at most, kFoldRows): eight bits from 24 on
     uint32_t sizes;   // d, num_splits: eight bits each; fold_group: sixteen
     int Nq, Nk, keys_per_split, wl, wr;
     const half_t *Q, *K, *V;

@@ -142,13 +142,13 @@ constexpr float kNothingSeen = -3.402823466e38f;
 // one row block per slice and one query head (folded: all the query heads) per K/V head, the shape of a decode launch -- and
 // its requests are non-temporal.
 // kVarEvery (with kVarAlibi and kVarDropout, without kVarVec): the instance that serves every request, see kEvery below.
-// kVarNarrow (unsplit launches): the four waves of a work-group share 32 query rows and take every fourth key tile
+// kVarNarrow (unsplit launches; in splits with kVarRows): the four waves of a work-group share 32 query rows and take every fourth key tile
 // each, see kNarrow below.
 // kVarPair (with ALiBi: keys at or left of the row alone, no dropout): eight waves in two halves that take every other tile each, see kPair below.
 // kVarFold (no other feature): the rows are the query heads of a K/V head, see row_position in common.h.
 // kVarShort (D >= 64, not kVarFullD, kVarEvery or kVarFold): rows of at most D - 16 elements, see FwdCfg::kShort.
 // kVarRows (with kVarNarrow; no other feature but kVarFold): launches of few rows per slice, whole or in splits, see kRows below.
-// kVarManyRows (with kVarRows): more than 32 rows, whose row blocks ask for the same tiles.
+// kVarManyRows (with kVarRows): more than 32 rows, whose row blocks ask for the same tiles, or rows of d < 32: ordinary requests.
 constexpr int kVarVec = 1, kVarAlibi = 2, kVarDropout = 4, kVarFullD = 8, kVarStamp = 16, kVarAlibiLeft = 32, kVarKvOnce = 64,
               kVarEvery = 128, kVarNarrow = 256, kVarFold = 512, kVarPair = 1024, kVarShort = 2048, kVarRows = 4096, kVarManyRows = 8192;
 
@@ -241,7 +241,8 @@ __global__ void __launch_bounds__((VAR & kVarPair) != 0 ? 512 : 256, fwd_groups_
     // as whole rows of floats, and where a caller has brought counters (combine.h) and the rows are four or fewer, the last work-group
     // of a slice merges the splits.  With up to 32 rows nobody else asks for the tiles, and the requests are non-temporal.
     // Ordinary / non-temporal, time over time, over 1000 random launches: K and V that no cache holds, up to 8 MiB 1.02 ... 1.04, 40 MiB 1.03 ... 1.05, 128 MiB 1.05 ... 1.09, more
-    // 1.11; called again and again with the same K and V, up to 20 MiB 0.99 ... 1.00, 20-40 MiB (the L2 holds 32) 0.94 ... 0.99, more 0.98 ... 1.06.
+    // 1.11; called again and again with the same K and V, up to 20 MiB 0.99 ... 1.00, 20-40 MiB (the L2 holds 32) 0.94 ... 0.99, more 0.98 ... 1.06 (whole launches 0.88 ... 1.12).
+    // Not with d < 32 (launch_fwd_bucket_st).
     constexpr bool kRows = (VAR & kVarRows) != 0, kRowsOnce = kRows && (VAR & kVarManyRows) == 0;
     static_assert(!kRows || (kNarrow && !kAlibi && !kDropout), "few rows");
     constexpr bool kFold = (VAR & kVarFold) != 0;
@@ -1573,7 +1574,7 @@ inline hipError_t launch_fwd_instance(const FwdArgs& a, hipStream_t st)
 // row, dropout, both}, for rows at any alignment (d % 8 != 0) {plain, ALiBi, dropout, both}, and the one that serves
 // every other request; those for shorter rows (all but the last) once more for d <= D - 16; the narrow, paired and folded ones below.  ST = kVarStamp selects their instrumented twins (debug
 // time stamps).  Nothing else looks at the stamp pointer: a stamped call is launched as the same call without.
-// The narrow instances (kNarrow in fwd_kernel) serve unsplit launches whose time is the chain of key tiles that a work-group
+// The narrow instances (kNarrow in fwd_kernel; those of few rows have rules of their own, below) serve unsplit launches whose time is the chain of key tiles that a work-group
 // walks through, which they cut to a quarter for a fixed cost of about 1 us (a wave's own requests, the merge of four).
 // Measured against the 128-row instances, paired ones among them, on 1240 random launches of up to 1600 work-groups of 32 rows;
 // the lines below lie where the ratio of the two crosses one:
@@ -1871,7 +1872,13 @@ inline int launch_fwd_bucket_st(const FwdArgs& a, int variant, hipStream_t st)
                 if constexpr ((V & kVarFullD) != 0) return (int)launch_fwd_rows_instance<D, V>(a, st);
                 else return (int)by_length([&](auto sh) { return launch_fwd_rows_instance<D, V | decltype(sh)::value>(a, st); });
             };
-            return a.Nq <= kRowsLimit ? folded(std::integral_constant<int, 0>{}) : folded(std::integral_constant<int, kVarManyRows>{});
+            // (rows of less than 64 bytes share lines, which neighbouring requests ask for: called again with K and V that the caches hold, ordinary requests take 0.66 ... 0.93 of
+            // the time from 20 to 300 MiB on, from memory 1.03 ... 1.07: B21 H8 Nq3 Nk5952 d31 24.7 / 35.5 us and 38.4 / 37.0)
+            constexpr bool kNarrowRows = D == 32 && (decltype(var)::value & kVarFullD) == 0;
+            if constexpr (!kNarrowRows) {
+                if (a.Nq <= kRowsLimit) return folded(std::integral_constant<int, 0>{});
+            }
+            return folded(std::integral_constant<int, kVarManyRows>{});
         };
         if (a.d == D) return rows(std::integral_constant<int, kVarVec | kVarFullD>{});
         if constexpr (D > 32) {

@@ -19,7 +19,7 @@ def bucket(d):
 def test_instances(B, H, Hk, Nq):
     wanted = []
     for d in DIMS:
-        bits = NARROW | ROWS | (FOLD if Hk < H else 0) | (MANY_ROWS if Nq * (H // Hk) > 32 else 0)
+        bits = NARROW | ROWS | (FOLD if Hk < H else 0) | (MANY_ROWS if Nq * (H // Hk) > 32 or d < 32 else 0)
         if d > 32:
             bits |= (VEC if d % 8 == 0 else 0) | (SHORT if Hk == H and d <= bucket(d) - 16 else 0)
         wanted.append(bits)
